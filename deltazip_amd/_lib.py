@@ -33,6 +33,7 @@ SIGNATURES = {
     "dz_pack_2of4": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp]),
     "dz_hessian_add": (_i, [_vp, _vp, _i, _i, _i, C.c_float, C.c_float, _vp]),
     "dz_obs_sweep": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
+    "dz_obs_sweep_ahead": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _i, _vp, _vp, _vp]),
     "dz_multi_delta_linear_batch": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _vp,
                                          _vp, C.c_size_t, _vp]),
     "dz_multi_delta_linear_batch_tiled": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,

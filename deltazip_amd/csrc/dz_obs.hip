@@ -4,198 +4,494 @@
 //   dz_hessian_add   H <- H * s0 + (s1 x)^T (s1 x)                         (sparsegpt.py:27-40)
 //   dz_obs_sweep     the sweep over blocks of 128 columns                   (sparsegpt.py:92-146)
 //
-// Rows of the weight are independent given the inverse Hessian, so one wavefront sweeps one row:
-// its 128 block columns sit in two registers per lane, the column being processed is broadcast
-// with v_readlane, the update of the columns to its right is one multiply and one subtract per
-// lane.  Between blocks the accumulated errors are carried to the remaining columns by a tiled
-// product.  Every sum runs in ascending index order with one rounding per operation (no fused
-// multiply-add), so that the result is the same bit for bit as a plain fp32 restatement with
-// that order; speed is secondary here (the sweep runs once per layer, offline).
+// Every sum runs in ascending index order with one rounding per operation (no fused multiply-add
+// in the sums), so that the result is the same bit for bit as a plain fp32 restatement with that
+// order: the work is v_mul_f32 / v_add_f32, not matrix instructions, whose order of summation is
+// not specified.  In their two-operand form these two run at twice the rate of a three-operand
+// instruction once a SIMD has two wavefronts (measured with register-only loops: 62 T lane
+// operations per second against 39 T, and 31 T with one wavefront), which is the rate the two
+// products below are built for.
+#include <type_traits>
+#include <utility>
+
 #include "../../include/dz_amd.h"
 #include "dz_device.h"
 
 namespace {
 
 constexpr int OBS_BLOCK = 128;
+constexpr int OBS_TRI = 136 * 64;   // floats of a block of hinv on and above its diagonal, in 8 x 8 pieces
 
-// ---- H <- H * s0 + sum_t (s1 x[t, a]) * (s1 x[t, b]), t ascending.  64 x 64 outputs per
-// workgroup, 4 x 4 per thread, 32 tokens staged at a time.
+typedef f4_t f4u_t __attribute__((aligned(4)));   // 16 bytes of an array that is aligned to its elements only
+
+// acc[i][j] += va[i] * vb[j], product and sum rounded separately.  The products of a row are made
+// while the row before is summed: an addition that follows its own product at once runs at three
+// quarters of the rate.
+template <int NI, int NJ>
+__device__ __forceinline__ void outer_add(float (&acc)[NI][NJ], const float (&va)[NI], const float (&vb)[NJ]) {
+#pragma clang fp contract(off)
+  float p[2][NJ];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) p[0][j] = va[0] * vb[j];
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    if (i + 1 < NI) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) p[(i + 1) & 1][j] = va[i + 1] * vb[j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = acc[i][j] + p[i & 1][j];
+    __builtin_amdgcn_sched_barrier(0);
+  }
+}
+
+// N steps of acc += a b^T over operands staged in LDS: a 4 values at pa + k * lda, b 4 values each at
+// pb + k * ldb and pb + k * ldb + second.  The operands of a step are read while the step before is summed.
+template <int N>
+__device__ __forceinline__ void outer_steps(float (&acc)[4][8], const float* pa, int lda, const float* pb, int ldb,
+                                            int second) {
+  f4_t a = *(const f4_t*)pa, b = *(const f4_t*)pb, c = *(const f4_t*)(pb + second);
+#pragma unroll 4
+  for (int k = 0; k < N; ++k) {
+    // (the read behind the last step repeats the first)
+    pa = k + 1 < N ? pa + lda : pa - (N - 1) * lda;
+    pb = k + 1 < N ? pb + ldb : pb - (N - 1) * ldb;
+    const f4_t an = *(const f4_t*)pa, bn = *(const f4_t*)pb, cn = *(const f4_t*)(pb + second);
+    __builtin_amdgcn_sched_barrier(0);
+    const float va[4] = {a[0], a[1], a[2], a[3]}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
+    outer_add(acc, va, vb);
+    a = an;
+    b = bn;
+    c = cn;
+  }
+}
+
+// ---- H <- H * s0 + sum_t (s1 x[t, a]) * (s1 x[t, b]), t ascending.
+// Bound by the multiply-add rate.  The product of columns a and b has the same bits as that of b
+// and a, so only the tiles on and above the diagonal are summed and each is written to both places
+// (H itself need not be symmetric: either place scales its own old value).  64 x 64 outputs per
+// workgroup of two wavefronts, 4 x 8 per thread (three 16-byte LDS reads per 64 instructions; with
+// 4 x 4 per thread the LDS is the bound), 32 tokens staged at a time and the next 32 on their way
+// in registers.  The tile is this small because the tiles of a launch are equal and all run at
+// once: 2080 of them at K = 4096 are 8.1 per CU, a loss of a tenth where 64 x 128 would lose a fifth.
+// K = 4096, 2048 tokens: 1.38 -> 0.79 ms.
 template <typename XT>
-__global__ __launch_bounds__(256) void dz_hessian_kernel(float* __restrict__ H, const XT* __restrict__ x, int T,
+__global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ H, const XT* __restrict__ x, int T,
                                                          int K, float s0, float s1) {
 #pragma clang fp contract(off)
-  __shared__ float xa[32][64], xb[32][64];
-  const int a0 = blockIdx.y * 64, b0 = blockIdx.x * 64;
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  float acc[4][4];
+  constexpr int TC = sizeof(XT) == 2 ? 32 : 16;   // tokens per stage
+  constexpr int PER = 16 / sizeof(XT);         // elements per 16-byte load
+  constexpr int ROWL = 64 / PER;               // loads per (token, 64 columns)
+  constexpr int NL = TC * ROWL / 128;          // loads per thread, stage and side
+  constexpr int TSTEP = 128 / ROWL;            // tokens between a thread's loads
+  __shared__ __attribute__((aligned(16))) float st[2][32][64];   // [a | b][token][column]; the mirrored tile at the end
+  // tile number -> (ta <= tb): number = tb (tb + 1) / 2 + ta
+  const int n = blockIdx.x;
+  int tb = (int)((sqrtf(8.f * (float)n + 1.f) - 1.f) * 0.5f);
+  while (tb * (tb + 1) / 2 > n) --tb;
+  while ((tb + 1) * (tb + 2) / 2 <= n) ++tb;
+  const int ta = n - tb * (tb + 1) / 2;
+  const int a0 = ta * 64, b0 = tb * 64;
+  const int tid = threadIdx.x, tr = tid >> 3, tc = tid & 7;   // rows 4 tr .. + 3, columns 4 tc .. + 3 and 32 + 4 tc .. + 3
+  float acc[4][8];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int t0 = 0; t0 < T; t0 += 32) {
-    __syncthreads();
-    for (int e = tid; e < 32 * 64; e += 256) {
-      const int tt = e >> 6, c = e & 63;
-      const bool in = t0 + tt < T;
-      xa[tt][c] = in ? s1 * (float)x[(size_t)(t0 + tt) * K + a0 + c] : 0.f;
-      xb[tt][c] = in ? s1 * (float)x[(size_t)(t0 + tt) * K + b0 + c] : 0.f;
+    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+
+  typedef XT xv_t __attribute__((ext_vector_type(PER), aligned(sizeof(XT))));
+  const int lt = tid / ROWL, lc = (tid % ROWL) * PER;
+  xv_t next[2][NL];
+  // tokens beyond T: the last one again, placed as zeros (adding 0 changes no sum: none is -0)
+  auto fetch = [&](int t0) {
+    const XT* base = x + (size_t)t0 * K;
+#pragma unroll
+    for (int l = 0; l < NL; ++l) {
+      const unsigned off = (unsigned)min(lt + l * TSTEP, T - 1 - t0) * (unsigned)K + (unsigned)lc;
+      next[0][l] = *(const xv_t*)(base + a0 + off);
+      next[1][l] = *(const xv_t*)(base + b0 + off);
     }
+  };
+  fetch(0);
+  for (int t0 = 0; t0 < T; t0 += TC) {
     __syncthreads();
-    const int nt = min(32, T - t0);
-    for (int tt = 0; tt < nt; ++tt) {
-      float va[4], vb[4];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        va[i] = xa[tt][tr * 4 + i];
-        vb[i] = xb[tt][tc * 4 + i];
-      }
+    for (int l = 0; l < NL; ++l) {
+      const float sv = t0 + lt + l * TSTEP < T ? s1 : 0.f;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+      for (int side = 0; side < 2; ++side)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float p = va[i] * vb[j];
-          acc[i][j] = acc[i][j] + p;
+        for (int v = 0; v < PER; v += 4) {
+          const xv_t& q = next[side][l];
+          f4_t f = {(float)q[v], (float)q[v + 1], (float)q[v + 2], (float)q[v + 3]};
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f[e] = sv == 0.f ? 0.f : sv * f[e];
+          *(f4_t*)&st[side][lt + l * TSTEP][lc + v] = f;
         }
     }
+    __syncthreads();
+    if (t0 + TC < T) fetch(t0 + TC);
+    outer_steps<TC>(acc, &st[0][0][4 * tr], 64, &st[1][0][4 * tc], 64, 32);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float* h = H + (size_t)(a0 + tr * 4 + i) * K + b0 + tc * 4 + j;
-      const float scaled = *h * s0;
-      *h = scaled + acc[i][j];
-    }
-}
-
-__device__ __forceinline__ float lane_value(float v, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
-}
-
-// ---- one block of 128 columns, one wavefront per row (sparsegpt.py:98-142)
-template <bool QUANT>
-__global__ __launch_bounds__(256) void dz_obs_block_kernel(float* __restrict__ W, const float* __restrict__ hinv,
-                                                           const float* __restrict__ scale, int N, int K, int i1,
-                                                           float maxq, float zero, int prunen, int prunem,
-                                                           float* __restrict__ err, float* __restrict__ loss) {
-#pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63;
-  const int row = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (row >= N) return;
-  float* wr = W + (size_t)row * K + i1;
-  float w0 = wr[lane], w1 = wr[64 + lane];
-  float q0 = 0.f, q1 = 0.f, e0 = 0.f, e1 = 0.f, lsum = 0.f;
-  const float sc = QUANT ? scale[row] : 1.f;
-  unsigned pruned_bits = 0;   // bit c: column (start of the current group) + c is pruned
-  for (int i = 0; i < OBS_BLOCK; ++i) {
-    const float* hr = hinv + (size_t)(i1 + i) * K + i1;
-    const float h0 = hr[lane], h1 = hr[64 + lane];
-    const int li = i & 63;
-    const bool hi = i >= 64;
-    if (prunen != 0 && i % prunem == 0) {
-      // w^2 / diag^2 of the group's columns (the same half of the block: prunem divides 64); the
-      // prunen smallest are pruned, ties keep the lower column (sparsegpt.py:123-125)
-      float t[8];
+    for (int j = 0; j < 8; j += 4) {
+      f4u_t* h = (f4u_t*)(H + (size_t)(a0 + 4 * tr + i) * K + b0 + 8 * j + 4 * tc);
+      const f4_t old = *h;
+      f4_t v;
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        t[c] = 0.f;
-        if (c < prunem) {
-          const float wv = lane_value(hi ? w1 : w0, li + c);
-          const float dv = hinv[(size_t)(i1 + i + c) * K + i1 + i + c];
-          t[c] = (wv * wv) / (dv * dv);
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float scaled = old[e] * s0;
+        v[e] = scaled + acc[i][j + e];
       }
-      pruned_bits = 0;
+      *h = v;
+    }
+  if (ta == tb) return;
+  // the mirrored tile, turned in LDS (16-byte chunks of a row rotated by the row: no shared banks)
+  float* turn = &st[0][0][0];
+  __syncthreads();
 #pragma unroll
-      for (int a = 0; a < 8; ++a) {
-        int rank = 0;
-#pragma unroll
-        for (int b = 0; b < 8; ++b)
-          if (a != b && b < prunem) rank += (b > a) ? (t[b] > t[a]) : (t[b] >= t[a]);
-        if (a < prunem && rank >= prunem - prunen) pruned_bits |= 1u << a;
-      }
-    }
-    const float w = lane_value(hi ? w1 : w0, li);
-    const float d = lane_value(hi ? h1 : h0, li);
-    const bool pruned = prunen != 0 && ((pruned_bits >> (i % prunem)) & 1u);
-    float q = pruned ? 0.f : w;
-    if (QUANT) {
-      const float code = fminf(fmaxf(rintf(q / sc) + zero, 0.f), maxq);
-      q = sc * (code - zero);
-    }
-    const float diff = w - q;
-    lsum = lsum + (diff * diff) / (d * d);
-    const float er = diff / d;
-    const float p0 = er * h0, p1 = er * h1;
-    if (!hi) {
-      if (lane >= li) w0 = w0 - p0;
-      w1 = w1 - p1;
-      if (lane == li) {
-        q0 = q;
-        e0 = er;
-      }
-    } else {
-      if (lane >= li) w1 = w1 - p1;
-      if (lane == li) {
-        q1 = q;
-        e1 = er;
-      }
-    }
-  }
-  wr[lane] = q0;
-  wr[64 + lane] = q1;
-  err[(size_t)row * OBS_BLOCK + lane] = e0;
-  err[(size_t)row * OBS_BLOCK + 64 + lane] = e1;
-  if (lane == 0) loss[row] = loss[row] + lsum / 2.f;
-}
-
-// ---- W[:, i2:] -= Err @ hinv[i1:i2, i2:], the sum over the block's 128 columns in ascending
-// order (sparsegpt.py:146).  64 rows x 64 columns per workgroup, 4 x 4 per thread.
-__global__ __launch_bounds__(256) void dz_obs_propagate_kernel(float* __restrict__ W, const float* __restrict__ err,
-                                                               const float* __restrict__ hinv, int N, int K, int i1,
-                                                               int i2) {
-#pragma clang fp contract(off)
-  __shared__ float es[64][OBS_BLOCK], hs[OBS_BLOCK][64];
-  const int r0 = blockIdx.y * 64, c0 = i2 + blockIdx.x * 64;
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;
-  for (int e = tid; e < 64 * OBS_BLOCK; e += 256) {
-    const int r = e / OBS_BLOCK, k = e % OBS_BLOCK;
-    es[r][k] = r0 + r < N ? err[(size_t)(r0 + r) * OBS_BLOCK + k] : 0.f;
-  }
-  for (int e = tid; e < OBS_BLOCK * 64; e += 256) {
-    const int k = e >> 6, c = e & 63;
-    hs[k][c] = hinv[(size_t)(i1 + k) * K + c0 + c];
+  for (int j = 0; j < 8; ++j) {
+    const int b = (j < 4 ? 0 : 28) + 4 * tc + j;
+    *(f4_t*)(turn + b * 64 + (((tr + b + (b >> 4)) & 15) << 2)) = (f4_t){acc[0][j], acc[1][j], acc[2][j], acc[3][j]};
   }
   __syncthreads();
-  float acc[4][4];
+#pragma unroll
+  for (int l = 0; l < 8; ++l) {
+    const int b = l * 8 + (tid >> 4), ch = tid & 15;
+    const f4_t s = *(const f4_t*)(turn + b * 64 + (((ch + b + (b >> 4)) & 15) << 2));
+    f4u_t* h = (f4u_t*)(H + (size_t)(b0 + b) * K + a0 + 4 * ch);
+    const f4_t old = *h;
+    f4_t v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float scaled = old[e] * s0;
+      v[e] = scaled + s[e];
+    }
+    *h = v;
+  }
+}
+
+// ---- one block of 128 columns (sparsegpt.py:98-142)
+// x / b for b in [2^-40, 2^40], |x| in [2^-80, 2^80], y = 1 / b correctly rounded: two residual steps.
+// After the first the quotient is within one unit in the last place, from where the second rounds
+// correctly (P. Markstein, "Computation of elementary functions on the IBM RISC System/6000
+// processor", IBM J. Res. Dev. 34, 1990); nothing under- or overflows in these ranges.
+__device__ __forceinline__ float div_by(float x, float b, float y) {
+  const float q0 = x * y;
+  const float q1 = __builtin_fmaf(__builtin_fmaf(-b, q0, x), y, q0);
+  return __builtin_fmaf(__builtin_fmaf(-b, q1, x), y, q1);
+}
+constexpr float W_MIN = 0x1p-40f, X_MIN = 0x1p-80f, X_MAX = 0x1p40f, B_MIN = 0x1p-20f, B_MAX = 0x1p20f;
+
+template <int L>
+__device__ __forceinline__ float row_lane(float v) {   // the value of lane L of each row of 16 lanes
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+template <typename F, int... L>
+__device__ __forceinline__ void for_each_lane(F&& f, std::integer_sequence<int, L...>) {
+  (f(std::integral_constant<int, L>{}), ...);
+}
+
+// Bound by the chain of one column's decision on the one before it.  A row is swept by 16 lanes,
+// 8 neighbouring columns each, so the 8 columns of a lane -- whole pruning groups -- are decided in
+// that lane's registers and only the column's error travels, by one cross-lane move; a wavefront
+// sweeps 4 rows, which gives the 4096 rows of a projection one wavefront per SIMD (with a
+// wavefront per row four of them shared a SIMD and each repeated every decision in 64 lanes).
+// Sixteen turns of 8 columns: after each the registers move down by one lane, so that the deciding
+// lane is always the first of its 16.  The rows of hinv come from LDS.  Divisions by the diagonal
+// and by the row's scale use their reciprocals (`div_by`); a turn that meets a value outside the
+// range where that is the correctly rounded quotient -- zeros among them -- is run again with
+// ordinary divisions.  err_prev: errors of the block before, not yet carried to these columns (they
+// are first), or nullptr.  4096 rows, per block: 145 -> 28 us.
+template <bool QUANT, int M>   // M: columns per pruning group, 0: no pruning
+__device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* __restrict__ hinv,
+                                           const float* __restrict__ scale, int N, int K, int i1, float maxq,
+                                           float zero, int prunen, const float* __restrict__ err_prev,
+                                           float* __restrict__ err, float* __restrict__ loss, int wg, float* sm) {
+#pragma clang fp contract(off)
+  float* hs = sm;                                   // 8 x 8 pieces (row group o, column group j >= o), see `piece`
+  float* cst = sm + OBS_TRI;                        // [4][128]: d, 1 / d, d^2, 1 / d^2
+  float* outs = cst + 4 * OBS_BLOCK;                // [16 rows][132]: errors of the block before, then w - q
+  constexpr int OLD = OBS_BLOCK + 4;
+  const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, rg = tid >> 4;   // rg: row within the workgroup
+  const int row = wg * 16 + rg, rowc = min(row, N - 1);
+  auto piece = [](int o, int j) { return (((o * (33 - o)) >> 1) + j - o) * 64; };
+  // all loads of hinv by a thread are on their way before the first is used
+  f4_t hl[16], hh[8];
+  auto fetch_tri = [&]() {     // the block's own rows, on and right of the diagonal pieces
+#pragma unroll
+    for (int l = 0; l < 16; ++l) {
+      const int r = l * 8 + (tid >> 5), c = (tid & 31) * 4;
+      if ((c >> 3) >= (r >> 3)) hl[l] = *(const f4u_t*)(hinv + (size_t)(i1 + r) * K + i1 + c);
+    }
+  };
+  auto fetch_half = [&](int r0) {   // 64 rows of the block before, all 128 columns
+#pragma unroll
+    for (int l = 0; l < 8; ++l)
+      hh[l] = *(const f4u_t*)(hinv + (size_t)(r0 + l * 8 + (tid >> 5)) * K + i1 + (tid & 31) * 4);
+  };
+  auto place_half = [&]() {
+#pragma unroll
+    for (int l = 0; l < 8; ++l) ((f4_t*)hs)[l * 256 + tid] = hh[l];
+  };
+  if (err_prev) fetch_half(i1 - OBS_BLOCK);
+  bool odd = false;   // a divisor outside the range of div_by: every turn takes ordinary divisions
+  if (tid < OBS_BLOCK) {
+    const float d = hinv[(size_t)(i1 + tid) * K + i1 + tid], dd = d * d;
+    cst[tid] = d;
+    cst[OBS_BLOCK + tid] = 1.f / d;
+    cst[2 * OBS_BLOCK + tid] = dd;
+    cst[3 * OBS_BLOCK + tid] = 1.f / dd;
+    odd = !(d >= B_MIN && d <= B_MAX);
+  }
+  float w[8];
+  {
+    const float* wr = W + (size_t)rowc * K + i1 + 8 * p;
+    const f4_t v0 = *(const f4u_t*)wr, v1 = *(const f4u_t*)(wr + 4);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      w[e] = v0[e];
+      w[4 + e] = v1[e];
+    }
+  }
+  const float sc = QUANT ? scale[rowc] : 1.f, ysc = 1.f / sc;
+  odd = odd || (QUANT && !(sc >= W_MIN && sc <= X_MAX));
+  if (err_prev) {
+    const float* ep = err_prev + (size_t)rowc * OBS_BLOCK + 8 * p;
+    *(f4_t*)(outs + rg * OLD + 8 * p) = *(const f4u_t*)ep;
+    *(f4_t*)(outs + rg * OLD + 8 * p + 4) = *(const f4u_t*)(ep + 4);
+    float acc[1][8] = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      place_half();
+      __syncthreads();
+      if (half == 0) fetch_half(i1 - OBS_BLOCK / 2);
+#pragma unroll 2
+      for (int k = 0; k < OBS_BLOCK / 2; k += 4) {
+        const f4_t e4 = *(const f4_t*)(outs + rg * OLD + half * (OBS_BLOCK / 2) + k);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const f4_t b = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 8 * p), c = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 8 * p + 4);
+          const float va[1] = {e4[u]}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
+          outer_add(acc, va, vb);
+        }
+      }
+      __syncthreads();
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) w[e] = w[e] - acc[0][e];
+  }
+  fetch_tri();
+#pragma unroll
+  for (int l = 0; l < 16; ++l) {
+    const int r = l * 8 + (tid >> 5), c = (tid & 31) * 4;
+    if ((c >> 3) >= (r >> 3)) *(f4_t*)(hs + piece(r >> 3, c >> 3) + (r & 7) * 8 + (c & 4)) = hl[l];
+  }
+  odd = __syncthreads_or(odd);
+
+  for (int o = 0; o < 16; ++o) {
+    const float* hp = hs + piece(o, o + min(p, 15 - o));   // (lanes that have wrapped around hold columns that are done)
+    // constants of the turn's 8 columns, the same for every lane
+    float d[8], y[8], dd[8], ydd[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      d[e] = cst[8 * o + e];
+      y[e] = cst[OBS_BLOCK + 8 * o + e];
+      dd[e] = cst[2 * OBS_BLOCK + 8 * o + e];
+      ydd[e] = cst[3 * OBS_BLOCK + 8 * o + e];
+    }
+    float q[8], er[8], df[8], ws[8];
+    bool bad = false;
+    auto turn = [&](auto fast_c) {
+      constexpr bool FAST = decltype(fast_c)::value;
+      float wmin = 1.f, xmin = 1.f, xmax = 1.f;
+      unsigned pruned = 0;   // bit r: column r of the group that is being decided
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        if constexpr (M > 0) {
+          if (r % M == 0) {
+            // w^2 / diag^2 of the group's columns; the prunen smallest are pruned, ties keep the
+            // lower column (sparsegpt.py:123-125)
+            float t[M];
+#pragma unroll
+            for (int c = 0; c < M; ++c) {
+              const float ww = w[r + c] * w[r + c];
+              t[c] = FAST ? div_by(ww, dd[r + c], ydd[r + c]) : ww / dd[r + c];
+              if (FAST) {
+                wmin = fminf(wmin, fabsf(w[r + c]));
+                xmax = fmaxf(xmax, fabsf(w[r + c]));
+              }
+            }
+            pruned = 0;
+#pragma unroll
+            for (int a = 0; a < M; ++a) {
+              int rank = 0;
+#pragma unroll
+              for (int b = 0; b < M; ++b)
+                if (a != b) rank += (b > a) ? (t[b] > t[a]) : (t[b] >= t[a]);
+              if (rank >= M - prunen) pruned |= 1u << a;
+            }
+          }
+        }
+        const bool pr = M > 0 && ((pruned >> (r % (M > 0 ? M : 1))) & 1u);
+        float qv = pr ? 0.f : w[r];
+        if (QUANT) {
+          // (a pruned column's code is the zero-point: rint(0 / sc) + zero)
+          const float quo = FAST ? div_by(w[r], sc, ysc) : w[r] / sc;
+          const float code = fminf(fmaxf(rintf(pr ? 0.f : quo) + zero, 0.f), maxq);
+          qv = sc * (code - zero);
+        }
+        const float diff = w[r] - qv;
+        float e;
+        if (FAST) {
+          // without rounding a column that stays has no error
+          e = QUANT || pr ? div_by(diff, d[r], y[r]) : 0.f;
+          xmin = fminf(fminf(xmin, fabsf(w[r])), QUANT ? fabsf(diff) : X_MAX);
+          xmax = fmaxf(xmax, fabsf(w[r]));
+        } else {
+          e = diff / d[r];
+        }
+        q[r] = qv;
+        df[r] = diff;
+        er[r] = e;
+        const float eb = row_lane<0>(e);
+        const f4_t h0 = *(const f4_t*)(hp + 8 * r), h1 = *(const f4_t*)(hp + 8 * r + 4);
+        const float h[8] = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
+        // columns that are done -- the first lane's up to r, and whole lanes that have wrapped around
+        // -- are changed too; nothing reads them any more
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const float pp = eb * h[c];
+          w[c] = w[c] - pp;
+        }
+      }
+      if (FAST) bad = !(wmin >= W_MIN && xmin >= X_MIN && xmax <= X_MAX);
+    };
+    if (!odd) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) ws[e] = w[e];
+      turn(std::true_type{});
+    }
+    if (odd || __builtin_amdgcn_ballot_w64(bad && p == 0) != 0) {
+      if (!odd) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) w[e] = ws[e];
+      }
+      turn(std::false_type{});
+    }
+    if (p == 0) {
+      float* wr = W + (size_t)rowc * K + i1 + 8 * o;      // (rows beyond N sweep the last row again: the same values)
+      float* ep = err + (size_t)rowc * OBS_BLOCK + 8 * o;
+#pragma unroll
+      for (int e = 0; e < 8; e += 4) {
+        *(f4u_t*)(wr + e) = (f4_t){q[e], q[e + 1], q[e + 2], q[e + 3]};
+        *(f4u_t*)(ep + e) = (f4_t){er[e], er[e + 1], er[e + 2], er[e + 3]};
+        *(f4_t*)(outs + rg * OLD + 8 * o + e) = (f4_t){df[e], df[e + 1], df[e + 2], df[e + 3]};
+      }
+    }
+    // the next lane's columns move into the deciding lane (row_ror:15 = one lane down)
+#pragma unroll
+    for (int e = 0; e < 8; ++e)
+      w[e] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(w[e]), 0x12F, 0xF, 0xF, true));
+  }
+  // the row's losses, summed in column order: each lane continues the sum of the lane before it
+  float term[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float diff = outs[rg * OLD + 8 * p + e], dd = cst[2 * OBS_BLOCK + 8 * p + e];
+    term[e] = (diff * diff) / dd;
+  }
+  float lsum = 0.f;
+  auto chain = [&](auto l_c) {
+    float s = lsum;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s = s + term[e];
+    lsum = row_lane<decltype(l_c)::value>(s);
+  };
+  for_each_lane(chain, std::make_integer_sequence<int, 16>{});
+  if (row < N && p == 0) loss[row] = loss[row] + lsum / 2.f;
+}
+
+constexpr size_t OBS_LDS = (size_t)(OBS_TRI + 4 * OBS_BLOCK + 16 * (OBS_BLOCK + 4)) * 4;   // 44 KiB: three workgroups per CU
+
+// ---- W[:, c0 .. c0 + 127] -= Err @ hinv[i1 .. i1 + 127, c0 ..] for 64 rows, the sum over the block's
+// 128 columns in ascending order (sparsegpt.py:146).  Bound by the multiply-add rate: 4 x 8 values
+// per thread as in dz_hessian_kernel; the errors are staged with the row index innermost (with the
+// column innermost the four rows of a thread fell on one bank) and in stages of 32 columns, so that
+// several workgroups fit a CU.
+__device__ __forceinline__ void propagate_tile(float* __restrict__ W, const float* __restrict__ err,
+                                               const float* __restrict__ hinv, int N, int K, int i1, int r0, int c0,
+                                               float* sm) {
+#pragma clang fp contract(off)
+  constexpr int KC = 32, ELD = 64 + 4;
+  float* es = sm;                   // [KC][ELD]
+  float* hs = sm + KC * ELD;        // [KC][128]
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;   // rows 4 tr .. + 3, columns 4 tc .. + 3 and 64 + 4 tc .. + 3
+  float acc[4][8];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
-  for (int k = 0; k < OBS_BLOCK; ++k) {
-    float va[4], vb[4];
+    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+  // stage loads: errors as 16 bytes of a row (row tid / 8 and + 32, columns 4 (tid % 8) .. + 3)
+  f4_t en[2], hn[4];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      va[i] = es[tr * 4 + i][k];
-      vb[i] = hs[k][tc * 4 + i];
-    }
+    for (int l = 0; l < 2; ++l)
+      en[l] = *(const f4u_t*)(err + (size_t)min(r0 + l * 32 + (tid >> 3), N - 1) * OBS_BLOCK + k0 + 4 * (tid & 7));
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int l = 0; l < 4; ++l)
+      hn[l] = *(const f4u_t*)(hinv + (size_t)(i1 + k0 + l * 8 + (tid >> 5)) * K + c0 + 4 * (tid & 31));
+  };
+  fetch(0);
+  for (int k0 = 0; k0 < OBS_BLOCK; k0 += KC) {
+    __syncthreads();
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float p = va[i] * vb[j];
-        acc[i][j] = acc[i][j] + p;
-      }
+    for (int l = 0; l < 2; ++l)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) es[(4 * (tid & 7) + e) * ELD + l * 32 + (tid >> 3)] = en[l][e];
+#pragma unroll
+    for (int l = 0; l < 4; ++l) *(f4_t*)(hs + (l * 8 + (tid >> 5)) * 128 + 4 * (tid & 31)) = hn[l];
+    __syncthreads();
+    if (k0 + KC < OBS_BLOCK) fetch(k0 + KC);
+    outer_steps<KC>(acc, es + 4 * tr, ELD, hs + 4 * tc, 128, 64);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    const int r = r0 + tr * 4 + i;
+    const int r = r0 + 4 * tr + i;
     if (r >= N) continue;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float* w = W + (size_t)r * K + c0 + tc * 4 + j;
-      *w = *w - acc[i][j];
+    for (int j = 0; j < 8; j += 4) {
+      f4u_t* wp = (f4u_t*)(W + (size_t)r * K + c0 + 16 * j + 4 * tc);
+      f4_t v = *wp;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = v[e] - acc[i][j + e];
+      *wp = v;
     }
+  }
+}
+
+// One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
+// carrying the errors of the block before, err_prev, to their own columns), the others carry
+// err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
+// the products fill them: at 4096 x 4096, 8.4 -> 2.05 ms for the whole sweep
+// (one kernel after the other: 2.6 ms).
+template <bool QUANT, int M>
+__global__ __launch_bounds__(256, 3) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
+                                                          const float* __restrict__ scale, int N, int K, int i1,
+                                                          float maxq, float zero, int prunen, int nsweep,
+                                                          const float* __restrict__ err_sweep, float* __restrict__ err,
+                                                          const float* __restrict__ err_prev, int i_prev, int c_lo,
+                                                          float* __restrict__ loss) {
+  extern __shared__ __attribute__((aligned(16))) float sm[];
+  const int wg = blockIdx.x;
+  if (wg < nsweep) {
+    sweep_rows<QUANT, M>(W, hinv, scale, N, K, i1, maxq, zero, prunen, err_sweep, err, loss, wg, sm);
+  } else {
+    const int nr = (N + 63) / 64, t = wg - nsweep;
+    propagate_tile(W, err_prev, hinv, N, K, i_prev, (t % nr) * 64, c_lo + (t / nr) * 128, sm);
   }
 }
 
@@ -208,37 +504,73 @@ int dz_hessian_add(float* H, const void* x, int x_is_fp16, int T, int K, float s
   if (!H || !x) return DZ_EINVAL;
   if (T < 1 || K < 64 || K % 64) return DZ_ESHAPE;
   hipStream_t st = (hipStream_t)stream;
-  const dim3 grid(K / 64, K / 64);
+  const int nt = K / 64;
+  const dim3 grid((unsigned)(nt * (nt + 1) / 2));
   if (x_is_fp16)
-    hipLaunchKernelGGL(dz_hessian_kernel<_Float16>, grid, dim3(256), 0, st, H, (const _Float16*)x, T, K, scale_h,
+    hipLaunchKernelGGL(dz_hessian_kernel<_Float16>, grid, dim3(128), 0, st, H, (const _Float16*)x, T, K, scale_h,
                        scale_x);
   else
-    hipLaunchKernelGGL(dz_hessian_kernel<float>, grid, dim3(256), 0, st, H, (const float*)x, T, K, scale_h,
+    hipLaunchKernelGGL(dz_hessian_kernel<float>, grid, dim3(128), 0, st, H, (const float*)x, T, K, scale_h,
                        scale_x);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
-int dz_obs_sweep(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
-                 int prunem, float* err_workspace, float* loss, void* stream) {
-  if (!W || !hinv_upper || !err_workspace || !loss) return DZ_EINVAL;
+// err: errors of two neighbouring blocks (`ahead`), or of one.
+static int obs_sweep(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
+                     int prunem, float* err, bool ahead, float* loss, void* stream) {
+  if (!W || !hinv_upper || !err || !loss) return DZ_EINVAL;
   if (N < 1 || K < OBS_BLOCK || K % OBS_BLOCK) return DZ_ESHAPE;
   if (scale && bits != 2 && bits != 3 && bits != 4 && bits != 8) return DZ_EBITS;
   if (prunen < 0 || prunem < 0 || (prunen != 0 && (prunem > 8 || prunen >= prunem || 64 % prunem))) return DZ_ESHAPE;
   hipStream_t st = (hipStream_t)stream;
   const float maxq = (float)((1 << bits) - 1), zero = (float)(1 << (bits - 1));
-  for (int i1 = 0; i1 < K; i1 += OBS_BLOCK) {
-    const int i2 = i1 + OBS_BLOCK;
-    if (scale)
-      hipLaunchKernelGGL(dz_obs_block_kernel<true>, dim3((N + 3) / 4), dim3(256), 0, st, W, hinv_upper, scale, N, K,
-                         i1, maxq, zero, prunen, prunem, err_workspace, loss);
-    else
-      hipLaunchKernelGGL(dz_obs_block_kernel<false>, dim3((N + 3) / 4), dim3(256), 0, st, W, hinv_upper, scale, N,
-                         K, i1, maxq, zero, prunen, prunem, err_workspace, loss);
-    if (i2 < K)
-      hipLaunchKernelGGL(dz_obs_propagate_kernel, dim3((K - i2) / 64, (N + 63) / 64), dim3(256), 0, st, W,
-                         err_workspace, hinv_upper, N, K, i1, i2);
+  static std::atomic<unsigned long long> attr_done[8];
+  const int which = (scale ? 4 : 0) + (prunen == 0 ? 0 : prunem == 2 ? 1 : prunem == 4 ? 2 : 3);
+  const int nsweep = (N + 15) / 16, nr = (N + 63) / 64;
+  auto sweep = [&](auto kern) -> int {
+    if (!dz_lds_limit_once(attr_done[which], (const void*)kern, (int)OBS_LDS)) return DZ_ELAUNCH;
+    auto step = [&](int ns, int i1, const float* err_sweep, float* err_cur, const float* err_prev, int i_prev, int c_lo) {
+      const int grid = ns + (err_prev ? nr * ((K - c_lo) / OBS_BLOCK) : 0);
+      hipLaunchKernelGGL(kern, dim3(grid), dim3(256), OBS_LDS, st, W, hinv_upper, scale, N, K, i1, maxq, zero, prunen,
+                         ns, err_sweep, err_cur, err_prev, i_prev, c_lo, loss);
+    };
+    for (int i1 = 0, b = 0; i1 < K; i1 += OBS_BLOCK, ++b) {
+      const int i2 = i1 + OBS_BLOCK;
+      if (ahead) {
+        // the next block's columns are brought up to date by its own sweep, one launch later; what
+        // lies beyond them by the other workgroups of that launch
+        float *cur = err + (size_t)(b & 1) * N * OBS_BLOCK, *prev = err + (size_t)((b & 1) ^ 1) * N * OBS_BLOCK;
+        step(nsweep, i1, b ? prev : nullptr, cur, b && i2 < K ? prev : nullptr, i1 - OBS_BLOCK, i2);
+      } else {
+        step(nsweep, i1, nullptr, err, nullptr, 0, K);
+        if (i2 < K) step(0, i1, nullptr, nullptr, err, i1, i2);
+      }
+    }
+    return DZ_OK;
+  };
+  int rc;
+  switch (which) {
+    case 0: rc = sweep(dz_obs_step_kernel<false, 0>); break;
+    case 1: rc = sweep(dz_obs_step_kernel<false, 2>); break;
+    case 2: rc = sweep(dz_obs_step_kernel<false, 4>); break;
+    case 3: rc = sweep(dz_obs_step_kernel<false, 8>); break;
+    case 4: rc = sweep(dz_obs_step_kernel<true, 0>); break;
+    case 5: rc = sweep(dz_obs_step_kernel<true, 2>); break;
+    case 6: rc = sweep(dz_obs_step_kernel<true, 4>); break;
+    default: rc = sweep(dz_obs_step_kernel<true, 8>); break;
   }
+  if (rc) return rc;
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
+}
+
+int dz_obs_sweep(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
+                 int prunem, float* err_workspace, float* loss, void* stream) {
+  return obs_sweep(W, hinv_upper, scale, N, K, bits, prunen, prunem, err_workspace, false, loss, stream);
+}
+
+int dz_obs_sweep_ahead(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
+                       int prunem, float* err_workspace, float* loss, void* stream) {
+  return obs_sweep(W, hinv_upper, scale, N, K, bits, prunen, prunem, err_workspace, true, loss, stream);
 }
 
 }  // extern "C"

@@ -338,11 +338,12 @@ def obs_sweep(W: torch.Tensor, hinv_upper: torch.Tensor, scale: Optional[torch.T
         raise ValueError("hinv_upper must be a contiguous float32 [K, K] tensor")
     if scale is not None and (scale.dtype != torch.float32 or scale.numel() != N or not scale.is_contiguous()):
         raise ValueError("scale must be a contiguous float32 tensor with one entry per row")
-    err = torch.empty((N, 128), dtype=torch.float32, device=W.device)
+    err = torch.empty((2, N, 128), dtype=torch.float32, device=W.device)
     loss = torch.zeros(N, dtype=torch.float32, device=W.device)
-    rc = _lib.lib().dz_obs_sweep(W.data_ptr(), hinv_upper.data_ptr(), scale.data_ptr() if scale is not None else None,
-                                 N, K, bits, prunen, prunem, err.data_ptr(), loss.data_ptr(), _stream())
-    _lib.check(rc, "dz_obs_sweep")
+    rc = _lib.lib().dz_obs_sweep_ahead(W.data_ptr(), hinv_upper.data_ptr(),
+                                       scale.data_ptr() if scale is not None else None, N, K, bits, prunen, prunem,
+                                       err.data_ptr(), loss.data_ptr(), _stream())
+    _lib.check(rc, "dz_obs_sweep_ahead")
     return loss
 
 

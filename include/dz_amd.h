@@ -177,6 +177,11 @@ int dz_hessian_add(float* H, const void* x, int x_is_fp16, int T, int K, float s
 int dz_obs_sweep(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
                  int prunem, float* err_workspace, float* loss, void* stream);
 
+/* The same sweep, the same result, with err_workspace of 2 * N * 128 floats: the products that carry
+ * one block's errors to the right then run beside the next block's sweep instead of before it. */
+int dz_obs_sweep_ahead(float* W, const float* hinv_upper, const float* scale, int N, int K, int bits, int prunen,
+                       int prunem, float* err_workspace, float* loss, void* stream);
+
 /* Bytes of device workspace dz_multi_delta_linear needs for these sizes.  The workspace must be
  * zero-filled once before first use; calls leave it zero-filled for the next call, whatever their
  * sizes (it carries the partial sums of a K dimension split over workgroups; an empty slot is all

@@ -56,6 +56,54 @@ def test_obs_sweep_bit_exact(dev, n, k, bits, quant, prune):
     assert np.array_equal(loss.cpu().numpy(), want_loss)
 
 
+@pytest.mark.parametrize("k,tokens,half", [(64, 1, True), (128, 31, True), (192, 33, False), (320, 64, True), (320, 95, False)])
+def test_hessian_tiles_bit_exact(dev, k, tokens, half):
+    """Edges of the 64-column tiles and 32-token stages; the old value need not be symmetric, since
+    either side of the diagonal scales its own."""
+    rng = np.random.default_rng(k + tokens)
+    x = rng.standard_normal((tokens, k)).astype(np.float16 if half else np.float32)
+    H0 = rng.standard_normal((k, k)).astype(np.float32)
+    buf = torch.zeros(tokens * k + 1, dtype=torch.float16 if half else torch.float32, device=dev)
+    buf[1:] = torch.from_numpy(x).to(dev).view(-1)
+    for xd in (torch.from_numpy(x).to(dev), buf[1:].view(tokens, k)):          # aligned, and to its elements only
+        H = torch.from_numpy(H0.copy()).to(dev)
+        assert ops.hessian_add(H, xd, 2, 1) == 3
+        want, _ = o.hessian_add_batch_ref(H0.copy(), 2, x.reshape(1, tokens, k))
+        assert np.array_equal(H.cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("n,k,quant,prune", [(1, 128, True, (2, 4)), (17, 256, True, (2, 4)), (17, 256, False, (2, 4)),
+                                             (50, 384, True, (1, 8)), (50, 384, False, (3, 8)), (16, 128, True, (1, 2)),
+                                             (65, 256, False, (0, 0))])
+def test_obs_sweep_values_outside_the_fast_range(dev, n, k, quant, prune):
+    """Zeros, values too small or too large for division by a reciprocal, a zero row, rows whose scale
+    is out of range and a diagonal entry out of range: the ordinary divisions take over, and the result
+    stays the oracle's bit for bit."""
+    bits = 4
+    W, X = _inputs(n, k, 1024, 90 + n + k)
+    H, _ = o.hessian_add_batch_ref(np.zeros((k, k), np.float32), 0, X)
+    hinv, W0 = o.hinv_upper_ref(H, W)
+    rng = np.random.default_rng(5)
+    W0[rng.random((n, k)) < 0.02] = 0
+    W0[:, 9] = 0                                                   # a dead column
+    W0[rng.random((n, k)) < 0.01] *= np.float32(1e-30)
+    if n > 16:
+        W0[3, 40] = np.float32(3e13)
+        W0[5] = 0
+        W0[7] *= np.float32(2.0 ** -60)                            # and with it the row's scale
+    if n == 50:
+        hinv[k - 3, k - 3] = np.float32(2.0 ** -25)
+    sc = o.find_params_sym(W0, bits)[0][:, 0].copy() if quant else None
+    pn, pm = prune
+    want, want_loss = o.obs_sweep_ref(W0.copy(), hinv, sc, bits, pn, pm)
+    Wd = torch.from_numpy(W0.copy()).to(dev)
+    loss = ops.obs_sweep(Wd, torch.from_numpy(hinv).to(dev), torch.from_numpy(sc).to(dev) if quant else None,
+                         bits, pn, pm)
+    torch.cuda.synchronize()
+    assert np.array_equal(Wd.cpu().numpy(), want, equal_nan=True)
+    assert np.array_equal(loss.cpu().numpy(), want_loss, equal_nan=True)
+
+
 @pytest.mark.parametrize("n,k,bits,gs", [(64, 512, 4, -1), (96, 1024, 2, -1), (32, 512, 4, 128), (64, 256, 2, 64)])
 def test_scales_with_the_search_over_the_clipping_range(dev, n, k, bits, gs):
     """dz_quant_scales_mse against the oracle's restatement of quant.py:85-101.  The candidates'
