@@ -25,6 +25,9 @@ SIGNATURES = {
     "dz_segment": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
     "dz_embedding_select": (_i, [_vp, _vp, _vp, _vp, C.c_longlong, _i, _vp, _i, _i, _i, _i, _vp]),
     "dz_build_tiles": (_i, [_vp, _i, _vp, _i, _vp]),
+    "dz_build_tiles_either": (_i, [_vp, _i, _vp, _i, _vp, _i, _vp]),
+    "dz_build_tiles_rows": (_i, [_vp, _i, _i, _vp, _i, _vp]),
+    "dz_multi_delta_gemm_rows": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_multi_delta_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_multi_delta_gemm_tiled": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_compress_2of4": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),

@@ -467,33 +467,77 @@ __global__ __launch_bounds__(512, 2) void dz_gemm24_kernel(const Gemm24Params P)
 }
 
 // Row blocks from segment offsets: segment k (k = 0: tokens without a delta, k >= 1: slot k - 1)
-// is cut into blocks of at most 256 rows; unused entries of the table are left empty.
-__global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S,
-                                                              dz_gemm_tile* __restrict__ tiles, int max_tiles) {
+// is cut into blocks of at most `rows` rows; unused entries of the table are left empty.  With a
+// second table (blocks of rows2 < rows) one of the two gets all rows and the other stays empty: the
+// second one where the first one's blocks would be less than three quarters full.  There the short
+// blocks' kernel is the faster one although it reads the weights more often (5120 x 27648, 2-bit,
+// 256 against 128 rows: 4096 tokens of 16 deltas, 65 % full: 2064 against 1837 us; 2000 tokens of 8,
+// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).
+__global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S, int rows,
+                                                              dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
+                                                              dz_gemm_tile* __restrict__ tiles2, int max_tiles2) {
   extern __shared__ int first[];    // first[k]: index of segment k's first block; first[S + 1]: total
   const int tid = threadIdx.x, nseg = S + 1;
-  for (int k = tid; k < nseg; k += 1024) first[k + 1] = (seg_off[k + 1] - seg_off[k] + BM - 1) / BM;
-  if (tid == 0) first[0] = 0;
-  __syncthreads();
-  if (tid == 0)
-    for (int k = 1; k <= nseg; ++k) first[k] += first[k - 1];
-  __syncthreads();
-  for (int k = tid; k < nseg; k += 1024) {
-    const int lo = seg_off[k], hi = seg_off[k + 1];
-    for (int t = first[k], r = lo; r < hi && t < max_tiles; ++t, r += BM)
-      tiles[t] = dz_gemm_tile{r, min(r + BM, hi), k - 1, 0};
+  auto count = [&](int r) {
+    for (int k = tid; k < nseg; k += 1024) first[k + 1] = (seg_off[k + 1] - seg_off[k] + r - 1) / r;
+    if (tid == 0) first[0] = 0;
+    __syncthreads();
+    if (tid == 0)
+      for (int k = 1; k <= nseg; ++k) first[k] += first[k - 1];
+    __syncthreads();
+  };
+  auto fill = [&](dz_gemm_tile* t, int max_t, int r) {
+    for (int k = tid; k < nseg; k += 1024) {
+      const int lo = seg_off[k], hi = seg_off[k + 1];
+      for (int b = first[k], p = lo; p < hi && b < max_t; ++b, p += r) t[b] = dz_gemm_tile{p, min(p + r, hi), k - 1, 0};
+    }
+    for (int b = first[nseg] + tid; b < max_t; b += 1024) t[b] = dz_gemm_tile{0, 0, -1, 0};
+  };
+  auto empty = [&](dz_gemm_tile* t, int max_t) {
+    for (int b = tid; b < max_t; b += 1024) t[b] = dz_gemm_tile{0, 0, -1, 0};
+  };
+  count(rows);
+  if (!tiles2) {
+    fill(tiles, max_tiles, rows);
+    return;
   }
-  for (int t = first[nseg] + tid; t < max_tiles; t += 1024) tiles[t] = dz_gemm_tile{0, 0, -1, 0};
+  const long long held = seg_off[nseg] - seg_off[0], room = (long long)first[nseg] * rows;
+  if (4 * held >= 3 * room) {
+    fill(tiles, max_tiles, rows);
+    empty(tiles2, max_tiles2);
+  } else {
+    __syncthreads();                // everyone has read the total of the first count
+    count(rows2);
+    fill(tiles2, max_tiles2, rows2);
+    empty(tiles, max_tiles);
+  }
 }
 
 }  // namespace
 
-extern "C" int dz_build_tiles(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles, void* stream) {
+static int build_tiles(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, int rows2,
+                       dz_gemm_tile* tiles2, int max_tiles2, void* stream) {
   if (!seg_off || !tiles) return DZ_EINVAL;
-  if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || max_tiles < 1) return DZ_ESHAPE;
+  if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || max_tiles < 1 || rows < 1) return DZ_ESHAPE;
   hipLaunchKernelGGL(dz_build_tiles_kernel, dim3(1), dim3(1024), (size_t)(S + 2) * 4, (hipStream_t)stream,
-                     seg_off, S, tiles, max_tiles);
+                     seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
+}
+
+extern "C" int dz_build_tiles(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles, void* stream) {
+  return build_tiles(seg_off, S, BM, tiles, max_tiles, 0, nullptr, 0, stream);
+}
+
+extern "C" int dz_build_tiles_rows(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles,
+                                   void* stream) {
+  return build_tiles(seg_off, S, rows, tiles, max_tiles, 0, nullptr, 0, stream);
+}
+
+extern "C" int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles,
+                                     dz_gemm_tile* short_tiles, int max_short, void* stream) {
+  if (!short_tiles) return DZ_EINVAL;
+  if (max_short < 1) return DZ_ESHAPE;
+  return build_tiles(seg_off, S, BM, tiles, max_tiles, DZ_SHORT_ROWS, short_tiles, max_short, stream);
 }
 
 static int multi_delta_gemm(const uint16_t* x, const uint16_t* w_base, bool w_tiled, const void* codes_stacked,

@@ -359,7 +359,7 @@ class DeltaModelManager:
         if 32 < T <= ops.MAX_TOKENS_FUSED:
             ops.token_order(self.base_indices[:T], self.delta_slots, out=self.token_order)
         self.row_blocks[0] = None
-        if T > ops.MAX_TOKENS_FUSED and not ops.takes_fused_chunks(T, self.delta_slots):
+        if T > ops.MAX_TOKENS_FUSED and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
             self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots)
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)

@@ -158,29 +158,63 @@ def segment(indices: torch.Tensor, num_slots: int):
     return perm, off
 
 
+SHORT_ROWS = 128               # row blocks of the kernel for few tokens per delta (DZ_SHORT_ROWS)
+MAX_SLOTS_SEGMENT = 768        # DZ_MAX_SLOTS_SEGMENT
+
+
 class RowBlocks:
     """A batch of more than 128 tokens ordered by delta id and cut into row blocks of one delta each
     (what dz_segment and dz_build_tiles write): depends on the indices only, so it can be made once
-    per batch and passed to every layer call of the step (`order=`)."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S")
+    per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
+    256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None."""
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short")
 
-    def __init__(self, perm, tiles, max_tiles, T, S):
+    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
+        self.short, self.max_short = short, max_short
 
 
-def row_blocks(indices: torch.Tensor, num_slots: int) -> RowBlocks:
+def _block_table(T: int, num_slots: int, rows: int, device):
+    n = (T + rows - 1) // rows + min(num_slots + 1, T)
+    return torch.empty((n, 4), dtype=torch.int32, device=device), n
+
+
+def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
-    (serving/vllm/delta/models.py:421-435).  Two small launches, nothing read back to the host."""
+    (serving/vllm/delta/models.py:421-435).  Two small launches, nothing read back to the host.
+
+    Which of the two kernels serves the batch.  Tiles of 256 features x 256 tokens want full
+    blocks and some 256 of them; tiles of 128 x 128 read the weights twice as often but fill the GPU
+    with a quarter of the tokens and multiply few rows that are not there.
+      up to 1024 tokens   short blocks: even with a single delta there are too few long ones to fill
+                          the GPU (5120 x 5120, 2-bit, 1024 tokens, 1 / 16 / 64 deltas: 103 / 147 / 266
+                          against 187 / 241 / 640 us; 5120 x 27648: 437 / 602 / 1382 against 757 / 959 /
+                          3251; the exception, one delta and many features at 512 tokens, 232 against
+                          204, stays within the launches it saves)
+      above, 256 tokens   long blocks: they are at least half full, and at 8192 tokens of 16 deltas
+      per slot and more   the larger tile is the faster one
+      between             the number of deltas in the batch is known on the device only: it picks
+                          (dz_build_tiles_either), and both products are launched, one of them empty
+    `long_only`: the table of 256-token blocks alone, whatever the batch."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
     T = indices.numel()
     perm, seg_off = segment(indices, num_slots)
-    max_tiles = (T + 255) // 256 + min(num_slots + 1, T)
-    tiles = torch.empty((max_tiles, 4), dtype=torch.int32, device=indices.device)
-    _lib.check(_lib.lib().dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), max_tiles, _stream()),
-               "dz_build_tiles")
-    return RowBlocks(perm, tiles, max_tiles, T, num_slots)
+    L, dev, st = _lib.lib(), indices.device, _stream()
+    if not long_only and T <= 1024:
+        short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
+        _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
+                   "dz_build_tiles_rows")
+        return RowBlocks(perm, None, 0, T, num_slots, short, ns)
+    tiles, n = _block_table(T, num_slots, 256, dev)
+    if not long_only and T < 256 * (num_slots + 1):
+        short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
+        _lib.check(L.dz_build_tiles_either(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, short.data_ptr(), ns, st),
+                   "dz_build_tiles_either")
+        return RowBlocks(perm, tiles, n, T, num_slots, short, ns)
+    _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
+    return RowBlocks(perm, tiles, n, T, num_slots)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,
@@ -227,7 +261,7 @@ def apply_delta_uncompressed(x: torch.Tensor, delta_weights: torch.Tensor, indic
         raise ValueError("shapes: x [T, K], delta_weights [S, N, K], base_embedding [N, K], indices [T]")
     if not (delta_weights.is_contiguous() and base_embedding.is_contiguous() and x.is_contiguous()):
         raise ValueError("x and the weights must be contiguous")
-    blocks = row_blocks(indices, S)
+    blocks = row_blocks(indices, S, long_only=True)
     out = torch.empty((T, N), dtype=torch.float16, device=x.device)
     _lib.check(_lib.lib().dz_gemm_f16_select(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K,
                                              blocks.tiles.data_ptr(), blocks.max_tiles, blocks.perm.data_ptr(),
@@ -569,14 +603,10 @@ def _check_tiled(base_tiled, base_weight, N: int, K: int, device) -> None:
 
 
 def takes_fused_chunks(T: int, S: int) -> bool:
-    """Whether a batch above the fused kernel's 128 tokens goes through it in chunks of 128 rather than
-    through the matrix-core kernel.  That kernel works on row blocks of up to 256 tokens of one delta
-    and needs some 256 x (N / 256) of them to fill the GPU: a few hundred tokens, the more so when
-    they are spread over many deltas, leave most of it idle (5120 x 5120, 2-bit, tiled base weight;
-    chunks against the matrix-core kernel with 1 / 16 / 64 deltas in the batch: 384 tokens 0.15 / 0.16
-    / 0.21 ms against 0.19 / 0.24 / 0.57 ms; 512 tokens 0.20 / 0.21 / 0.26 against 0.19 / 0.24 / 0.57;
-    768 tokens 0.29 / 0.30 / 0.34 against 0.20 / 0.24 / 0.58).  The number of distinct deltas is
-    known on the device only, so the number of slots stands in for it."""
+    """Whether a batch above the fused kernel's 128 tokens can go through it in chunks of 128 (sizes at
+    which that costs no more than row blocks of 256 tokens).  Row blocks of 128 tokens are faster at
+    every one of them (5120 x 5120, 2-bit, 192 / 333 / 512 tokens of 16 deltas: 84 / 58 / 95 us against
+    132 / 153 / 262), so chunks serve only what `segment` cannot order: more than 768 slots."""
     return T <= 3 * MAX_TOKENS_FUSED or (T <= 4 * MAX_TOKENS_FUSED and S >= 16)
 
 
@@ -632,7 +662,7 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             raise ValueError("out must be float16 [T, N] with unit column stride")
     ldy = out.stride(0)
     if T > MAX_TOKENS_FUSED:
-        if takes_fused_chunks(T, S):
+        if S > MAX_SLOTS_SEGMENT and takes_fused_chunks(T, S):
             for r in range(0, T, MAX_TOKENS_FUSED):
                 multi_delta_linear(x2[r:r + MAX_TOKENS_FUSED], base_weight, qweight_stacked, scales_stacked,
                                    meta_stacked, indices[r:r + MAX_TOKENS_FUSED], bits=bits,
@@ -640,6 +670,8 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             return out
         from .prefill import multi_delta_linear_prefill
         blocks = order if isinstance(order, RowBlocks) else None
+        if blocks is not None and (blocks.T != T or blocks.S != S) and takes_fused_chunks(T, S):
+            blocks = None                             # (at these sizes a stale order was never an error)
         if blocks is not None and (blocks.T != T or blocks.S != S):
             raise ValueError("row blocks were made for another batch size or number of slots")
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
@@ -724,7 +756,11 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     G = scales_stacked[0][0].numel() // base_weight[0].shape[0]
     S = qweight_stacked[0].shape[0]
     if T > MAX_TOKENS_FUSED:
+        if not isinstance(order, RowBlocks) and n > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
+                and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
+            order = row_blocks(indices, S)            # once for all projections
         return [apply_delta(xs[j], qweight_stacked[j], scales_stacked[j], meta_stacked[j], indices, base_weight[j],
+                            order=order if isinstance(order, RowBlocks) and order.S == S and order.T == T else None,
                             base_tiled=None if base_tiled is None else base_tiled[j])
                 for j in range(n)]
     _need_cuda(indices, *xs, *qweight_stacked, *scales_stacked, *meta_stacked, *base_weight)

@@ -38,7 +38,7 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
                                *, bits: int, out: torch.Tensor, accumulate: bool, blocks=None,
                                base_tiled=None) -> torch.Tensor:
     """T > 128: tokens are ordered by delta id on the device (dz_segment), the order is cut into
-    row blocks of one delta each (dz_build_tiles) and one launch of dz_multi_delta_gemm multiplies
+    row blocks of one delta each (ops.row_blocks) and dz_multi_delta_gemm or dz_multi_delta_gemm_rows multiplies
     every block by the base weight and by its delta in packed form.  Nothing is read back to the
     host, gathered, scattered or dequantised to memory.  `blocks`: ops.row_blocks(indices, S) when
     the caller made it once for the batch (else made here, per call).  `base_tiled`: the base weight
@@ -62,12 +62,20 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
     stream = torch.cuda.current_stream().cuda_stream
     if blocks is None:
         blocks = row_blocks(indices, S)
-    fn, wptr = lib.dz_multi_delta_gemm, base_weight.data_ptr() if base_weight is not None else None
-    if base_tiled is not None:
-        fn, wptr = lib.dz_multi_delta_gemm_tiled, base_tiled.data_ptr()
-    rc = fn(x2.data_ptr(), wptr,
-                                 qweight_stacked.data_ptr(), meta_stacked.data_ptr(), scales_stacked.data_ptr(),
-                                 S, bits, group_size, blocks.tiles.data_ptr(), blocks.max_tiles, blocks.perm.data_ptr(),
-                                 out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), stream)
-    _lib.check(rc, "dz_multi_delta_gemm")
+    row_major = base_weight.data_ptr() if base_weight is not None else None
+    if blocks.tiles is not None:
+        fn, wptr = lib.dz_multi_delta_gemm, row_major
+        if base_tiled is not None:
+            fn, wptr = lib.dz_multi_delta_gemm_tiled, base_tiled.data_ptr()
+        rc = fn(x2.data_ptr(), wptr, qweight_stacked.data_ptr(), meta_stacked.data_ptr(), scales_stacked.data_ptr(),
+                S, bits, group_size, blocks.tiles.data_ptr(), blocks.max_tiles, blocks.perm.data_ptr(),
+                out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), stream)
+        _lib.check(rc, "dz_multi_delta_gemm")
+    if blocks.short is not None:
+        rc = lib.dz_multi_delta_gemm_rows(
+            x2.data_ptr(), base_tiled.data_ptr() if base_tiled is not None else row_major,
+            1 if base_tiled is not None else 0, qweight_stacked.data_ptr(), meta_stacked.data_ptr(),
+            scales_stacked.data_ptr(), S, bits, group_size, blocks.short.data_ptr(), blocks.max_short,
+            blocks.perm.data_ptr(), out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), stream)
+        _lib.check(rc, "dz_multi_delta_gemm_rows")
     return out

@@ -48,6 +48,7 @@ extern "C" {
 #define DZ_MAX_BATCH_CALLS 4      /* layer calls dz_multi_delta_linear_batch takes at once    */
 #define DZ_STATIC_MAX_N 16384      /* largest N dz_multi_delta_linear_static takes             */
 #define DZ_MAX_SLOTS_SEGMENT 768   /* largest S dz_segment takes (its tables live in LDS)      */
+#define DZ_SHORT_ROWS 128         /* rows of a block of dz_multi_delta_gemm_rows */
 #define DZ_MAX_SLOTS_MAP 4096      /* largest S dz_map_ids takes (the slot table lives in LDS) */
 
 /* Library version (major*10000 + minor*100 + patch). */
@@ -326,6 +327,25 @@ int dz_gemm_f16_select(const uint16_t* x, const uint16_t* w_base, const uint16_t
  * in use are marked empty.  max_tiles >= (T + 255) / 256 + min(S + 1, T) always suffices, so the
  * host never needs to read the offsets back.  S <= DZ_MAX_SLOTS_SEGMENT. */
 int dz_build_tiles(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles, void* stream);
+
+/* dz_build_tiles with blocks of at most `rows` rows: max_tiles >= (T + rows - 1) / rows +
+ * min(S + 1, T) always suffices. */
+int dz_build_tiles_rows(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, void* stream);
+
+/* Both tables at once: on the device, all rows go either into blocks of at most 256 (`tiles`, for
+ * dz_multi_delta_gemm) or into blocks of at most DZ_SHORT_ROWS (`short_tiles`, for
+ * dz_multi_delta_gemm_rows), whichever suits the lengths of the segments; the other table is left
+ * empty.  A caller launches both products. */
+int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles,
+                          dz_gemm_tile* short_tiles, int max_short, void* stream);
+
+/* dz_multi_delta_gemm for row blocks of up to DZ_SHORT_ROWS rows (longer ones are taken that many rows at a time):
+ * the faster one where most blocks are that short.  w_base is row-major [N, K] (w_tiled = 0), the
+ * tiles dz_tile_base writes (w_tiled != 0), or NULL. */
+int dz_multi_delta_gemm_rows(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                             const void* meta_stacked, const void* scales_stacked, int S, int bits, int group_size,
+                             const dz_gemm_tile* tiles, int ntiles, const int32_t* perm, uint16_t* y, int T, int K,
+                             int N, int accumulate, int ldy, void* stream);
 
 /* The layer at prefill sizes, deltas in packed form: for every row block b of `tiles` and every
  * position p in [row_lo, row_hi), with t = perm ? perm[p] : p,

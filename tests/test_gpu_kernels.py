@@ -312,6 +312,76 @@ def test_row_blocks_made_once_per_batch(dev):
                                order=blocks)
 
 
+@pytest.mark.parametrize("n,k,bits,gs,nd", [(32, 256, 2, -1, 3), (96, 512, 4, -1, 2), (160, 768, 2, 64, 4),
+                                            (288, 1024, 4, 128, 3), (128, 512, 2, -1, 1)])
+def test_short_row_blocks(dev, n, k, bits, gs, nd):
+    """dz_multi_delta_gemm_rows over blocks at the edges of its token tiles (1, 15, 16, 17 .. 127, 128 tokens
+    and one of 200, taken in two parts), unsorted rows, row-major and tiled base weight, in place and
+    without a base weight, against the kernel for long blocks and the oracle.  2-bit deltas: the same
+    products in the same order, so equal bits; 4-bit: the long kernel adds all base products first."""
+    from deltazip_amd import _lib
+    L = _lib.lib()
+    sizes = [1, 15, 16, 17, 32, 33, 48, 49, 64, 65, 96, 97, 127, 128, 200]
+    t = sum(sizes)
+    p = make_problem(n, k, bits, gs, nd, t, "uniform", 900 + n, dev)
+    perm = np.random.default_rng(n).permutation(t).astype(np.int32)
+    rows, ids, r = [], np.empty(t, dtype=np.int64), 0
+    for i, c in enumerate(sizes):
+        slot = i % (nd + 1) - 1
+        rows.append([r, r + c, slot, 0])
+        ids[perm[r:r + c]] = slot
+        r += c
+    rows += [[0, 0, -1, 0]] * 2                       # unused entries
+    tiles = torch.tensor(rows, dtype=torch.int32, device=dev)
+    pd, st = torch.from_numpy(perm).to(dev), torch.cuda.current_stream().cuda_stream
+    wt = ops.tile_base(p["wb"])
+
+    def call(short, w, tiled, y, acc):
+        args = (p["q"].data_ptr(), p["m"].data_ptr(), p["s"].data_ptr(), nd, bits, gs, tiles.data_ptr(), len(rows),
+                pd.data_ptr(), y.data_ptr(), t, k, n, acc, y.stride(0), st)
+        wp = None if w is None else w.data_ptr()
+        assert (L.dz_multi_delta_gemm_rows(p["x"].data_ptr(), wp, tiled, *args) if short
+                else L.dz_multi_delta_gemm(p["x"].data_ptr(), wp, *args)) == 0
+        torch.cuda.synchronize()
+        return y
+    new = lambda: torch.zeros(t, n + 8, device=dev, dtype=torch.float16)[:, :n]
+    for w, tiled in ((p["wb"], 0), (wt, 1), (None, 0)):
+        for acc in (0, 1):
+            y, y0 = new(), new()
+            if acc:
+                y += 0.5
+                y0 += 0.5
+            call(True, w, tiled, y, acc)
+            # (the long kernel takes at most 256 rows a block: all of these)
+            call(False, None if w is None else p["wb"], 0, y0, acc)
+            if bits == 2:
+                assert torch.equal(y, y0)
+            ref = o.forward_ref(p["x_np"], None if w is None else p["wb_np"], p["dts"], ids) + 0.5 * acc
+            assert o.rel_err(y.float().cpu().numpy(), ref) <= TOL
+            assert o.rel_err(y0.float().cpu().numpy(), ref) <= TOL
+
+
+@pytest.mark.parametrize("lens,short", [([0, 300, 20, 5], True), ([0, 512, 250, 0], False), ([10, 0, 0, 0], True),
+                                        ([192, 192, 192, 192], False), ([191, 192, 192, 192], True)])
+def test_build_tiles_either(dev, lens, short):
+    """All rows go into the table whose blocks suit them -- long blocks from three quarters full on --
+    and the other table is empty."""
+    from deltazip_amd import _lib
+    L = _lib.lib()
+    off = np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)
+    seg = torch.from_numpy(off).to(dev)
+    tabs = [torch.full((16, 4), 77, dtype=torch.int32, device=dev) for _ in range(2)]
+    assert L.dz_build_tiles_either(seg.data_ptr(), len(lens) - 1, tabs[0].data_ptr(), 16, tabs[1].data_ptr(), 16,
+                                   torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    step = 128 if short else 256
+    want = [[a, min(a + step, int(off[s + 1])), s - 1, 0] for s in range(len(lens))
+            for a in range(int(off[s]), int(off[s + 1]), step)]
+    want += [[0, 0, -1, 0]] * (16 - len(want))
+    assert tabs[short].cpu().tolist() == want and tabs[not short].cpu().tolist() == [[0, 0, -1, 0]] * 16
+    assert L.dz_build_tiles_either(seg.data_ptr(), len(lens) - 1, tabs[0].data_ptr(), 16, None, 16, None) == -1
+
+
 @pytest.mark.parametrize("t,nd", [(129, 3), (256, 40), (300, 4), (512, 17)])
 def test_mid_size_batches_go_through_the_fused_kernel_in_chunks(dev, t, nd):
     """Between 129 tokens and a few hundred the matrix-core kernel would leave most of the GPU idle:
