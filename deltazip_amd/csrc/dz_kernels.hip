@@ -229,39 +229,96 @@ __global__ __launch_bounds__(256) void dz_embedding_select_kernel(const long lon
 // ---------------------------------------------------------------------------------------------
 // compressor: fp32 delta [N, K] -> symmetric scales, 2:4 magnitude pruning, codes, native layout
 // ---------------------------------------------------------------------------------------------
-// One wavefront per (row, scale group): min / max of the group, then the symmetric parameters of
-// deltazip/core/quant.py:69-83 (perchannel, sym): the range is widened to [-m, m] when the group
-// has a negative value, an all-zero group gets [-1, 1], scale = (xmax - xmin) / maxq.
+// Min / max of a scale group, then the symmetric parameters of deltazip/core/quant.py:69-83
+// (perchannel, sym): the range is widened to [-m, m] when the group has a negative value, an
+// all-zero group gets [-1, 1], scale = (xmax - xmin) / maxq.
+__device__ __forceinline__ void minmax4(float& mn, float& mx, f4_t v) {
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    mn = fminf(mn, v[e]);
+    mx = fmaxf(mx, v[e]);
+  }
+}
+
+__device__ __forceinline__ float symmetric_scale(float mn, float mx, float maxq) {
+  float xmin = mn, xmax = fmaxf(fabsf(mn), mx);
+  if (xmin < 0.f) xmin = -xmax;
+  if (xmin == 0.f && xmax == 0.f) {
+    xmin = -1.f;
+    xmax = 1.f;
+  }
+  return (xmax - xmin) / maxq;
+}
+
+// Long groups: one wavefront per (row, group), four requests in flight per lane.
 __global__ __launch_bounds__(64) void dz_scales_kernel(const float* __restrict__ delta, int K, int N, int gs,
                                                        int G, float maxq, float* __restrict__ scale32,
                                                        _Float16* __restrict__ scale16) {
   const int row = blockIdx.x / G, g = blockIdx.x % G, lane = threadIdx.x;
   const float* p = delta + (size_t)row * K + (size_t)g * gs;
   float mn = 0.f, mx = 0.f;
-  for (int c = lane * 4; c < gs; c += 256) {
-    const f4_t v = *(const f4_t*)(p + c);
+  int c = lane * 4;
+  for (; c + 768 < gs; c += 1024) {
+    f4_t v[4];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      mn = fminf(mn, v[e]);
-      mx = fmaxf(mx, v[e]);
-    }
+    for (int u = 0; u < 4; ++u) v[u] = *(const f4_t*)(p + c + 256 * u);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) minmax4(mn, mx, v[u]);
   }
+  for (; c < gs; c += 256) minmax4(mn, mx, *(const f4_t*)(p + c));
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
     mn = fminf(mn, __shfl_xor(mn, o));
     mx = fmaxf(mx, __shfl_xor(mx, o));
   }
   if (lane == 0) {
-    float xmin = mn, xmax = fmaxf(fabsf(mn), mx);
-    if (xmin < 0.f) xmin = -xmax;
-    if (xmin == 0.f && xmax == 0.f) {
-      xmin = -1.f;
-      xmax = 1.f;
-    }
-    const float sc = (xmax - xmin) / maxq;
+    const float sc = symmetric_scale(mn, mx, maxq);
     scale32[(size_t)g * N + row] = sc;
     scale16[(size_t)g * N + row] = (_Float16)sc;
   }
+}
+
+// Groups of 64, 128 or 256 columns: a wavefront takes the groups of 256 columns of a row at once, GS / 4
+// lanes each, for up to four such stretches (one wavefront per group leaves half or three quarters
+// of its lanes idle, and starts N * G wavefronts).
+template <int GS>
+__global__ __launch_bounds__(64) void dz_scales_short_kernel(const float* __restrict__ delta, int K, int N, float maxq,
+                                                             float* __restrict__ scale32, _Float16* __restrict__ scale16) {
+  const int lane = threadIdx.x, nc = K / 256, per_row = (nc + 3) / 4;
+  const int row = blockIdx.x / per_row, c0 = (blockIdx.x % per_row) * 4;
+  const float* p = delta + (size_t)row * K + lane * 4;
+  f4_t v[4];
+#pragma unroll
+  for (int u = 0; u < 4; ++u) v[u] = *(const f4_t*)(p + min(c0 + u, nc - 1) * 256);
+#pragma unroll
+  for (int u = 0; u < 4; ++u) {
+    if (c0 + u >= nc) break;
+    float mn = 0.f, mx = 0.f;
+    minmax4(mn, mx, v[u]);
+#pragma unroll
+    for (int o = GS / 8; o > 0; o >>= 1) {
+      mn = fminf(mn, __shfl_xor(mn, o));
+      mx = fmaxf(mx, __shfl_xor(mx, o));
+    }
+    if ((lane & (GS / 4 - 1)) == 0) {
+      const float sc = symmetric_scale(mn, mx, maxq);
+      const size_t at = (size_t)((c0 + u) * (256 / GS) + lane / (GS / 4)) * N + row;
+      scale32[at] = sc;
+      scale16[at] = (_Float16)sc;
+    }
+  }
+}
+
+void launch_scales(const float* delta, int K, int N, int bits, int gs, float* scale32, uint16_t* scale16, hipStream_t st) {
+  const float maxq = (float)((1 << bits) - 1);
+  const unsigned grid = (unsigned)N * ((K / 256 + 3) / 4);
+  auto go = [&](auto kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(64), 0, st, delta, K, N, maxq, scale32, (_Float16*)scale16); };
+  if (gs == 64) go(dz_scales_short_kernel<64>);
+  else if (gs == 128) go(dz_scales_short_kernel<128>);
+  else if (gs == 256) go(dz_scales_short_kernel<256>);
+  else
+    hipLaunchKernelGGL(dz_scales_kernel, dim3((unsigned)N * (K / gs)), dim3(64), 0, st, delta, K, N, gs, K / gs, maxq,
+                       scale32, (_Float16*)scale16);
 }
 
 // The same with the reference's grid search over the clipping range (deltazip/core/quant.py:85-101,
@@ -323,79 +380,198 @@ __global__ __launch_bounds__(64) void dz_scales_mse_kernel(const float* __restri
   }
 }
 
-// One wavefront per (n-pair, k-block) tile; lane 16*ga + i produces its own four words of the
-// native arrays from rows i and 16 + i, columns 64*j + 16*ga .. + 15 of the k-block.
+// One wavefront per (n-pair, k-block) tile; the words of lane 16*ga + i of the native arrays hold
+// rows i and 16 + i, columns 64*j + 16*ga .. + 15 of the k-block (word j).
 //   pruning   in every aligned group of 4 columns the 2 values of largest magnitude stay (ties:
 //             the lower column), the others become 0 -- deltazip/core/sparsegpt.py:123-135 with an
 //             identity Hessian
 //   codes     q = clamp(rint(x / scale) + zero, 0, maxq), fp32, zero = 2^(bits-1) -- quant.py:9-18
 //   positions the columns whose code differs from the zero-point, completed with the lowest
 //             remaining columns: what the repacker stores for the same codes
+// Bound by memory at 2 bits (4096 x 11008 packed in 41 us, 4.9 TB/s, from 85; compressed, the pass for
+// the scales included, in 70 us from 113) and by its arithmetic where the scales are found here too.
+//
+// The work of a group of four: six comparisons (a value stays if at least two of its three
+// comparisons go its way), four quotients as products with 1 / scale, and two table lookups on
+// 4-bit masks.  A quotient's rounding is that of the division unless it lies within 1e-5 of half
+// way between two codes (the product is off by 1.5 units in the last place, 1e-6 below 8.5; beyond
+// that both are clamped alike); such a group, one with a NaN, or a scale outside [2^-100, 2^100] goes
+// the plain way: compress_group_plain.
 template <int BITS>
-__global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict__ delta,
-                                                         const float* __restrict__ scale32, int K, int N,
-                                                         int gs, uint32_t* __restrict__ codes,
-                                                         uint32_t* __restrict__ meta) {
-  const int nkb = K / DZ_KBLOCK;
-  const int np = blockIdx.x / nkb, kb = blockIdx.x % nkb;
-  const int la = threadIdx.x, ga = la >> 4, i = la & 15;
+__device__ __forceinline__ void compress_group_plain(const f4_t v, float sc, uint32_t& pos, uint32_t& clo, uint32_t& chi) {
   constexpr int zp = 1 << (BITS - 1);
   constexpr float maxq = (float)((1 << BITS) - 1);
-  uint32_t mword[4] = {0u, 0u, 0u, 0u};
-  uint32_t cword[2][4] = {{0u, 0u, 0u, 0u}, {0u, 0u, 0u, 0u}};
+  int c[4];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int col0 = kb * DZ_KBLOCK + 64 * j + 16 * ga;
+  for (int a = 0; a < 4; ++a) {
+    int rank = 0;   // entries ahead of a: larger magnitude, or equal magnitude at a lower column
 #pragma unroll
-    for (int s = 0; s < 2; ++s) {
-      const int row = np * DZ_NPAIR + 16 * s + i;
-      const float sc = scale32[(size_t)(col0 / gs) * N + row];
-      const float* src = delta + (size_t)row * K + col0;
+    for (int b = 0; b < 4; ++b)
+      if (b != a) rank += (b > a) ? (fabsf(v[b]) > fabsf(v[a])) : (fabsf(v[b]) >= fabsf(v[a]));
+    const float x = rank < 2 ? v[a] : 0.f;
+    const float qf = fminf(fmaxf(rintf(x / sc) + (float)zp, 0.f), maxq);
+    c[a] = (int)qf;
+  }
+  int pa = -1, pb = -1;
 #pragma unroll
-      for (int p = 0; p < 4; ++p) {
-        const f4_t v = *(const f4_t*)(src + 4 * p);
-        int c[4];
+  for (int a = 0; a < 4; ++a)
+    if (c[a] != zp) {
+      if (pa < 0) pa = a;
+      else if (pb < 0) pb = a;
+    }
 #pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          int rank = 0;   // entries ahead of a: larger magnitude, or equal magnitude at a lower column
+  for (int a = 0; a < 4; ++a)
+    if (c[a] == zp) {
+      if (pa < 0) pa = a;
+      else if (pb < 0) pb = a;
+    }
+  const int lo = min(pa, pb), hi = max(pa, pb);
+  pos = (uint32_t)(lo | hi << 2);
+  clo = (uint32_t)(lo == 0 ? c[0] : lo == 1 ? c[1] : c[2]);
+  chi = (uint32_t)(hi == 1 ? c[1] : hi == 2 ? c[2] : c[3]);
+}
+
+// lo | hi << 2 of a mask of at most two columns, completed with the lowest others: entry `mask` of
+// a table of 4-bit entries (0, 1, 2, 4, 8: (0,1) (0,1) (0,1) (0,2) (0,3); 3, 5, 9, 6, 10, 12: themselves)
+constexpr unsigned long long kept_table() {
+  unsigned long long t = 0;
+  for (int m = 0; m < 16; ++m) {
+    int p[4] = {0, 0, 0, 0}, n = 0;
+    for (int a = 0; a < 4; ++a)
+      if (m >> a & 1) p[n++] = a;
+    if (n > 2) continue;
+    for (int a = 0; a < 4 && n < 2; ++a)
+      if (!(m >> a & 1)) p[n++] = a;
+    const int lo = p[0] < p[1] ? p[0] : p[1], hi = p[0] < p[1] ? p[1] : p[0];
+    t |= (unsigned long long)(lo | hi << 2) << (4 * m);
+  }
+  return t;
+}
+
+template <int BITS>
+__device__ __forceinline__ void compress_group(const f4_t v, float sc, float rsc, uint32_t& pos, uint32_t& clo, uint32_t& chi) {
+  constexpr int zp = 1 << (BITS - 1);
+  constexpr float maxq = (float)((1 << BITS) - 1);
+  constexpr unsigned long long TABLE = kept_table();
+  float r[4], far = 0.f, sum = 0.f;
 #pragma unroll
-          for (int b = 0; b < 4; ++b)
-            if (b != a) rank += (b > a) ? (fabsf(v[b]) > fabsf(v[a])) : (fabsf(v[b]) >= fabsf(v[a]));
-          const float x = rank < 2 ? v[a] : 0.f;
-          const float qf = fminf(fmaxf(rintf(x / sc) + (float)zp, 0.f), maxq);
-          c[a] = (int)qf;
-        }
-        int pa = -1, pb = -1;
+  for (int a = 0; a < 4; ++a) {
+    const float q = v[a] * rsc;
+    r[a] = rintf(q);
+    far = fmaxf(far, fabsf(q - r[a]));
+    sum += fabsf(q);
+  }
+  if (!(far < 0.49999f && sum == sum)) {
+    compress_group_plain<BITS>(v, sc, pos, clo, chi);
+    return;
+  }
+  const float m0 = fabsf(v[0]), m1 = fabsf(v[1]), m2 = fabsf(v[2]), m3 = fabsf(v[3]);
+  const bool b01 = m0 >= m1, b02 = m0 >= m2, b03 = m0 >= m3, b12 = m1 >= m2, b13 = m1 >= m3, b23 = m2 >= m3;
+  auto two_of = [](bool a, bool b, bool c) { return (a && b) || (c && (a || b)); };
+  const bool keep[4] = {two_of(b01, b02, b03), two_of(!b01, b12, b13), two_of(!b02, !b12, b23), two_of(!b03, !b13, !b23)};
+  uint32_t mask = 0, c = 0;
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-          if (c[a] != zp) {
-            if (pa < 0) pa = a;
-            else if (pb < 0) pb = a;
-          }
+  for (int a = 0; a < 4; ++a) {
+    const float x = keep[a] ? r[a] : 0.f;
+    mask |= x != 0.f ? 1u << a : 0u;
+    c |= (uint32_t)fminf(fmaxf(x + (float)zp, 0.f), maxq) << (4 * a);
+  }
+  const uint32_t half = mask & 8u ? (uint32_t)(TABLE >> 32) : (uint32_t)TABLE;
+  pos = (half >> (4 * (mask & 7u))) & 15u;
+  clo = (c >> (4 * (pos & 3u))) & 15u;
+  chi = (c >> (4 * (pos >> 2))) & 15u;
+}
+
+// A lane reads one group of four of a row, the wavefront 1 KiB of a row at a time (with the lane of
+// the native layout reading its own 64 bytes of a row, every lane's request falls on a line of its
+// own: 4096 x 11008 at 2 bits 76 us at any amount of arithmetic).  The four lanes that share a word
+// of the layout or their bits together, and the words meet in LDS.
+__device__ __forceinline__ uint32_t or_quad(uint32_t v) {
+  v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xB1, 0xf, 0xf, true);          // lane ^ 1
+  return v | (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4E, 0xf, 0xf, true);    // lane ^ 2
+}
+
+//
+// GS = 0: scales from memory.  GS = 64, 128, 256: the tile holds whole scale groups, so their scales are
+// found here from the values just read (and written out) rather than in a pass of their own
+// (4096 x 11008, 4-bit, groups of 128: 104 -> 90 us, of 64 107 -> 88).
+template <int BITS, int GS>
+__global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict__ delta,
+                                                         float* __restrict__ scale32, _Float16* __restrict__ scale16,
+                                                         int K, int N, int gs, uint32_t* __restrict__ codes,
+                                                         uint32_t* __restrict__ meta) {
+  constexpr int GL = GS ? GS / 4 : 64;             // lanes per scale group
+  constexpr int NW = 1 + BITS / 2;                 // words per (lane of the layout, step): positions, codes
+  __shared__ __attribute__((aligned(16))) uint32_t words[NW * 256];   // as in memory: meta, then codes
+  __shared__ float2 sct[DZ_NPAIR * 4];             // (scale, 1 / scale or NaN) of (row, step)
+  const int nkb = K / DZ_KBLOCK;
+  const int np = blockIdx.x / nkb, kb = blockIdx.x % nkb;
+  const int lane = threadIdx.x, j = lane >> 4, ga = (lane >> 2) & 3, p = lane & 3;
 #pragma unroll
-        for (int a = 0; a < 4; ++a)
-          if (c[a] == zp) {
-            if (pa < 0) pa = a;
-            else if (pb < 0) pb = a;
-          }
-        const int lo = min(pa, pb), hi = max(pa, pb);
-        const uint32_t clo = (uint32_t)(lo == 0 ? c[0] : lo == 1 ? c[1] : c[2]);
-        const uint32_t chi = (uint32_t)(hi == 1 ? c[1] : hi == 2 ? c[2] : c[3]);
-        mword[j] |= ((uint32_t)lo << dz_meta_shift(s, 2 * p)) | ((uint32_t)hi << dz_meta_shift(s, 2 * p + 1));
-        if (BITS == 2) {
-          cword[0][j] |= (clo << dz_code2_shift(s, 2 * p)) | (chi << dz_code2_shift(s, 2 * p + 1));
+  for (int h = 0; h < (GS ? 0 : 2); ++h) {
+    const int at = h * 64 + lane, row = at & 31, step = at >> 5;      // (a scale group spans whole steps)
+    const float sc = scale32[(size_t)((kb * DZ_KBLOCK + step * 64) / gs) * N + np * DZ_NPAIR + row];
+    sct[step * DZ_NPAIR + row] = make_float2(sc, sc >= 0x1p-100f && sc <= 0x1p100f ? 1.f / sc : __builtin_nanf(""));
+  }
+  const float* src = delta + (size_t)np * DZ_NPAIR * K + kb * DZ_KBLOCK + lane * 4;
+  // lane p of four stores the positions (0), the codes (1), or the codes of row 16 + i at 4 bits (2)
+  const int hold = p == 0 ? j : BITS == 2 ? 256 + j : 256 + (j >> 1) * 256 + 2 * (j & 1) + (p - 1);
+  __syncthreads();
+#pragma unroll
+  for (int i0 = 0; i0 < 16; i0 += 4) {
+    f4_t v[2][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int s = 0; s < 2; ++s) v[s][u] = *(const f4_t*)(src + (size_t)(16 * s + i0 + u) * K);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      uint32_t mw = 0, cw[2] = {0, 0};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        float2 sc;
+        if constexpr (GS != 0) {
+          const f4_t w = v[s][u];
+          float top = fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])), fmaxf(fabsf(w[2]), fabsf(w[3])));
+#pragma unroll
+          for (int o = GL / 2; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+          const unsigned long long neg = __ballot(w[0] < 0.f || w[1] < 0.f || w[2] < 0.f || w[3] < 0.f);
+          const bool any_neg = ((neg >> (lane & ~(GL - 1))) & (~0ull >> (64 - GL))) != 0;
+          top = fmaxf(top, 0.f);                   // (all NaN: as a group without a value)
+          sc.x = symmetric_scale(any_neg ? -top : 0.f, top, (float)((1 << BITS) - 1));
+          sc.y = sc.x >= 0x1p-100f && sc.x <= 0x1p100f ? 1.f / sc.x : __builtin_nanf("");
+          if ((lane & (GL - 1)) == 0) sct[lane / GL * DZ_NPAIR + 16 * s + i0 + u].x = sc.x;
         } else {
-          cword[j >> 1][2 * (j & 1) + s] |= (clo << dz_code4_shift(2 * p)) | (chi << dz_code4_shift(2 * p + 1));
+          sc = sct[j * DZ_NPAIR + 16 * s + i0 + u];
         }
+        uint32_t pos, clo, chi;
+        compress_group<BITS>(v[s][u], sc.x, sc.y, pos, clo, chi);
+        mw |= pos << dz_meta_shift(s, 2 * p);      // elements 2p and 2p + 1 are neighbours
+        if (BITS == 2) cw[0] |= (clo << dz_code2_shift(s, 2 * p)) | (chi << dz_code2_shift(s, 2 * p + 1));
+        else cw[s] = (clo << dz_code4_shift(2 * p)) | (chi << dz_code4_shift(2 * p + 1));
       }
+      mw = or_quad(mw);
+      cw[0] = or_quad(cw[0]);
+      if (BITS == 4) cw[1] = or_quad(cw[1]);
+      if (p < NW) words[hold + (16 * ga + i0 + u) * 4] = p == 0 ? mw : p == 1 ? cw[0] : cw[1];
     }
   }
-  *(u4_t*)(meta + dz_meta_word(np, kb, la, 0, nkb)) = (u4_t){mword[0], mword[1], mword[2], mword[3]};
+  __syncthreads();
+  if constexpr (GS != 0) {
+    constexpr int NG = DZ_KBLOCK / (GS ? GS : 1);
+#pragma unroll
+    for (int at = lane; at < NG * DZ_NPAIR; at += 64) {
+      const size_t o = (size_t)(kb * NG + at / DZ_NPAIR) * N + np * DZ_NPAIR + (at & 31);
+      scale32[o] = sct[at].x;
+      scale16[o] = (_Float16)sct[at].x;
+    }
+  }
+  *(u4_t*)(meta + dz_meta_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + lane * 4);
   if (BITS == 2) {
-    *(u4_t*)(codes + dz_code2_word(np, kb, la, 0, nkb)) = (u4_t){cword[0][0], cword[0][1], cword[0][2], cword[0][3]};
+    *(u4_t*)(codes + dz_code2_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
   } else {
-    *(u4_t*)(codes + dz_code4_word(np, kb, la, 0, 0, nkb)) = (u4_t){cword[0][0], cword[0][1], cword[0][2], cword[0][3]};
-    *(u4_t*)(codes + dz_code4_word(np, kb, la, 2, 0, nkb)) = (u4_t){cword[1][0], cword[1][1], cword[1][2], cword[1][3]};
+    *(u4_t*)(codes + dz_code4_word(np, kb, lane, 0, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
+    *(u4_t*)(codes + dz_code4_word(np, kb, lane, 2, 0, nkb)) = *(const u4_t*)(words + (BITS == 2 ? 256 : 512) + lane * 4);
   }
 }
 
@@ -654,17 +830,20 @@ int dz_compress_2of4(const float* delta, int K, int N, int bits, int group_size,
   int gs;
   if ((rc = check_group(K, group_size, &gs))) return rc;
   if ((uintptr_t)delta & 15) return DZ_EALIGN;
-  const int G = K / gs;
   hipStream_t st = (hipStream_t)stream;
-  hipLaunchKernelGGL(dz_scales_kernel, dim3((unsigned)N * G), dim3(64), 0, st, delta, K, N, gs, G,
-                     (float)((1 << bits) - 1), scale_workspace, (_Float16*)out_scales);
   const unsigned tiles = (unsigned)(N / DZ_NPAIR) * (K / DZ_KBLOCK);
-  if (bits == 2)
-    hipLaunchKernelGGL(dz_compress_kernel<2>, dim3(tiles), dim3(64), 0, st, delta, scale_workspace, K, N, gs,
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64), 0, st, delta, scale_workspace, (_Float16*)out_scales, K, N, gs,
                        (uint32_t*)out_codes, (uint32_t*)out_meta);
-  else
-    hipLaunchKernelGGL(dz_compress_kernel<4>, dim3(tiles), dim3(64), 0, st, delta, scale_workspace, K, N, gs,
-                       (uint32_t*)out_codes, (uint32_t*)out_meta);
+  };
+  switch (gs) {
+    case 64: bits == 2 ? go(dz_compress_kernel<2, 64>) : go(dz_compress_kernel<4, 64>); break;
+    case 128: bits == 2 ? go(dz_compress_kernel<2, 128>) : go(dz_compress_kernel<4, 128>); break;
+    case 256: bits == 2 ? go(dz_compress_kernel<2, 256>) : go(dz_compress_kernel<4, 256>); break;
+    default:
+      launch_scales(delta, K, N, bits, gs, scale_workspace, out_scales, st);
+      bits == 2 ? go(dz_compress_kernel<2, 0>) : go(dz_compress_kernel<4, 0>);
+  }
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
@@ -676,9 +855,7 @@ int dz_quant_scales(const float* delta, int K, int N, int bits, int group_size, 
   int gs;
   if ((rc = check_group(K, group_size, &gs))) return rc;
   if ((uintptr_t)delta & 15) return DZ_EALIGN;
-  const int G = K / gs;
-  hipLaunchKernelGGL(dz_scales_kernel, dim3((unsigned)N * G), dim3(64), 0, (hipStream_t)stream, delta, K, N, gs, G,
-                     (float)((1 << bits) - 1), scale32, (_Float16*)scale16);
+  launch_scales(delta, K, N, bits, gs, scale32, scale16, (hipStream_t)stream);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
@@ -708,12 +885,11 @@ int dz_pack_2of4(const float* w, const float* scale32, int K, int N, int bits, i
   if ((uintptr_t)w & 15) return DZ_EALIGN;
   const unsigned tiles = (unsigned)(N / DZ_NPAIR) * (K / DZ_KBLOCK);
   hipStream_t st = (hipStream_t)stream;
-  if (bits == 2)
-    hipLaunchKernelGGL(dz_compress_kernel<2>, dim3(tiles), dim3(64), 0, st, w, scale32, K, N, gs,
+  auto go = [&](auto kern) {                       // (scales are read only)
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64), 0, st, w, const_cast<float*>(scale32), (_Float16*)nullptr, K, N, gs,
                        (uint32_t*)out_codes, (uint32_t*)out_meta);
-  else
-    hipLaunchKernelGGL(dz_compress_kernel<4>, dim3(tiles), dim3(64), 0, st, w, scale32, K, N, gs,
-                       (uint32_t*)out_codes, (uint32_t*)out_meta);
+  };
+  bits == 2 ? go(dz_compress_kernel<2, 0>) : go(dz_compress_kernel<4, 0>);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 

@@ -660,6 +660,37 @@ def test_compressor_matches_reference_pipeline(dev, n, k, bits, gs):
     assert np.array_equal(got.view(np.uint16), np.ascontiguousarray(o.dequant_gptq(qw, qz, sc, gi, bits).T).view(np.uint16))
 
 
+@pytest.mark.parametrize("bits,gs,k", [(2, -1, 1280), (4, -1, 5632), (4, 64, 1280), (2, 128, 256), (4, 256, 768),
+                                       (2, 192, 768)])
+def test_compressor_at_code_boundaries(dev, bits, gs, k):
+    """Byte for byte the oracle's result where a product with the scale's reciprocal could round another way
+    than the quotient: values at and one unit beside every half code, for scales over the whole range
+    of fp32, and rows whose scale is below or above what the reciprocal is used for."""
+    n, maxq, rng = 64, 2**bits - 1, np.random.default_rng(bits + k)
+    g = k if gs == -1 else gs
+    d = np.empty((n, k), np.float32)
+    for r in range(n):
+        top = np.float32(rng.uniform(0.5, 1) * 10.0 ** rng.uniform(-30, 30))
+        if r == 1:
+            top = np.float32(1e-39)
+        if r == 2:
+            top = np.float32(2e37)
+        sc = np.float32(np.float32(2) * top / np.float32(maxq))
+        v = ((rng.integers(-maxq - 1, maxq + 1, k) / 2.0).astype(np.float32) * sc).astype(np.float32)
+        v = np.where(rng.random(k) < 0.5, np.nextafter(v, np.float32(rng.choice([-np.inf, np.inf]))), v)
+        v = np.clip(v, -top, top)
+        v[::g] = -top
+        d[r] = v
+    codes, scales16, zeros, _ = o.compress_delta(d, bits, gs)
+    qw, qz, sc16, gi = o.pack_codes_gptq(codes, zeros, scales16, bits)
+    want_c, want_m, want_s = o.repack_native(qw, qz, sc16, gi, bits)
+    q, m, s = ops.compress_delta(torch.from_numpy(d).to(dev), bits, gs)
+    torch.cuda.synchronize()
+    assert np.array_equal(s.cpu().numpy().view(np.uint16), want_s.view(np.uint16))
+    assert q.cpu().numpy().view(np.uint32).tobytes() == want_c.tobytes()
+    assert m.cpu().numpy().view(np.uint32).tobytes() == want_m.tobytes()
+
+
 def test_compressor_argument_checks(dev):
     with pytest.raises(ValueError):
         ops.compress_delta(torch.zeros(32, 256, device=dev, dtype=torch.float16), 4)
