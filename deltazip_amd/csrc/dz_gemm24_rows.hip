@@ -1,7 +1,9 @@
 // Multi-delta linear layer for batches between decode and prefill, and for prefill batches whose
 // tokens are spread over many deltas:
 //   y[t, :] (+)= x[t, :] @ w_base^T + x[t, :] @ dequant(delta[slot(t)])^T
-// over a table of row blocks of at most 128 tokens, each with one slot.  Same products and the same
+// over a table of row blocks of at most 128 tokens, each with one slot.  The same kernel without
+// deltas, each block with its own full weight (a few rows of the output projection per delta's own
+// table), is dz_gemm_f16_select_rows.  Same products and the same
 // summation order as dz_gemm24.hip (2-bit deltas: bit for bit), on a smaller tile.
 //
 // One workgroup (4 wavefronts) computes 128 output features x one row block; a wavefront owns one
@@ -32,6 +34,8 @@ constexpr int STAGE = 2 * SLAB;
 struct RowsParams {
   const _Float16* x;
   const _Float16* w;             // base weight: [N, K], or in tiles (w_tiled), or nullptr
+  const _Float16* w_stack;       // or nullptr; else a block with a slot takes w_stack[slot] in w's place
+  long long w_stride;
   const u4_t* codes;
   const u4_t* meta;
   const _Float16* scales;
@@ -50,7 +54,8 @@ __device__ __forceinline__ void row_block(const RowsParams& P, unsigned char* sm
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int li = lane & 15, lg = lane >> 4;
   const uint32_t MAGIC = magic_vgpr();
-  const bool do_w = P.w != nullptr, do_d = slot >= 0 && slot < P.S;
+  const _Float16* const w = P.w_stack && slot >= 0 ? P.w_stack + (size_t)slot * P.w_stride : P.w;
+  const bool do_w = w != nullptr, do_d = slot >= 0 && slot < P.S;
   const int np_own = n0 / DZ_NPAIR + wave;
   const int np = min(np_own, P.NP - 1);          // beyond N: the last n-pair again, never stored
   const unsigned Kb = (unsigned)P.K * 2u;
@@ -60,11 +65,11 @@ __device__ __forceinline__ void row_block(const RowsParams& P, unsigned char* sm
   const char* wp;
   unsigned wl, w_a, w_j, w_h, w_kb;
   if (P.w_tiled) {
-    wp = (const char*)P.w + (size_t)np * P.NKB * 16384;
+    wp = (const char*)w + (size_t)np * P.NKB * 16384;
     wl = (unsigned)((lg & 1) * 1024 + ((lg >> 1) * 16 + li) * 16);
     w_a = 8192; w_j = 2048; w_h = 512; w_kb = 16384;
   } else {
-    wp = (const char*)P.w + (size_t)np * DZ_NPAIR * Kb;
+    wp = (const char*)w + (size_t)np * DZ_NPAIR * Kb;
     wl = (unsigned)li * Kb + (unsigned)lg * 16u;
     w_a = 16 * Kb; w_j = 128; w_h = 64; w_kb = 512;
   }
@@ -252,7 +257,17 @@ __global__ __launch_bounds__(256, 2) void dz_gemm24_rows_kernel(const RowsParams
   // The row blocks of one feature tile run next to each other on one XCD: they read the same base
   // weight, which only the first of them fetches from beyond that XCD's L2.
   const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
-  const int tn = (q / P.tiles_m) * 8 + xcd, tm = q % P.tiles_m;
+  // Only the entries in use are counted for that: workgroups of unused ones between the others would
+  // each hold a place on a CU until they have read their entry (32000 x 4096, 32 tokens without a
+  // delta among 8 slots: 111 -> 57 us).
+  int used = 0;
+  for (int e = 0; e < P.tiles_m; e += 64) {
+    const dz_gemm_tile t = P.tiles[min(e + (int)(threadIdx.x & 63), P.tiles_m - 1)];
+    const unsigned long long has = __ballot(t.row_hi > t.row_lo && e + (int)(threadIdx.x & 63) < P.tiles_m);
+    if (has) used = e + 64 - __clzll((long long)has);
+  }
+  if (used == 0) return;
+  const int tn = (q / used) * 8 + xcd, tm = q % used;
   if (tn >= P.tiles_n) return;
   const int row_lo = P.tiles[tm].row_lo, row_hi = P.tiles[tm].row_hi, slot = P.tiles[tm].group;
   // (a block of more than RB rows is taken RB rows at a time; the loop's last barrier is behind the
@@ -269,6 +284,21 @@ __global__ __launch_bounds__(256, 2) void dz_gemm24_rows_kernel(const RowsParams
 }
 
 }  // namespace
+
+static int launch(RowsParams P, int bits, int ntiles, hipStream_t st) {
+  P.tiles_m = ntiles; P.tiles_n = (P.N + BN - 1) / BN;
+  P.NKB = P.K / DZ_KBLOCK; P.NP = P.N / DZ_NPAIR;
+  const unsigned long long grid = (unsigned long long)((P.tiles_n + 7) / 8) * 8ull * (unsigned)ntiles;
+  if (grid > 0x7fffffffull) return DZ_ESHAPE;
+  const int lds = 2 * STAGE;
+  static std::atomic<unsigned long long> attr_done[2];
+  auto go = [&](auto kern, int which) -> int {
+    if (!dz_lds_limit_once(attr_done[which], (const void*)kern, lds)) return DZ_ELAUNCH;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, st, P);
+    return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
+  };
+  return bits == 2 ? go(dz_gemm24_rows_kernel<2>, 0) : go(dz_gemm24_rows_kernel<4>, 1);
+}
 
 extern "C" int dz_multi_delta_gemm_rows(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
                                         const void* meta_stacked, const void* scales_stacked, int S, int bits,
@@ -289,17 +319,24 @@ extern "C" int dz_multi_delta_gemm_rows(const uint16_t* x, const uint16_t* w_bas
   P.codes_slot_u4 = (long long)(cb / 16); P.meta_slot_u4 = (long long)(mb / 16); P.scales_slot = (long long)(sb / 2);
   P.tiles = tiles; P.perm = perm;
   P.K = K; P.N = N; P.S = S; P.G = K / gs; P.gslabs = gs / 64; P.accumulate = accumulate; P.ldy = ldy;
-  P.tiles_m = ntiles; P.tiles_n = (N + BN - 1) / BN;
-  P.NKB = K / DZ_KBLOCK; P.NP = N / DZ_NPAIR;
   P.w_tiled = (w_tiled && w_base) ? 1 : 0;
-  const unsigned long long grid = (unsigned long long)((P.tiles_n + 7) / 8) * 8ull * (unsigned)ntiles;
-  if (grid > 0x7fffffffull) return DZ_ESHAPE;
-  const int lds = 2 * STAGE;
-  static std::atomic<unsigned long long> attr_done[2];
-  auto go = [&](auto kern, int which) -> int {
-    if (!dz_lds_limit_once(attr_done[which], (const void*)kern, lds)) return DZ_ELAUNCH;
-    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), lds, (hipStream_t)stream, P);
-    return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
-  };
-  return bits == 2 ? go(dz_gemm24_rows_kernel<2>, 0) : go(dz_gemm24_rows_kernel<4>, 1);
+  return launch(P, bits, ntiles, (hipStream_t)stream);
+}
+
+extern "C" int dz_gemm_f16_select_rows(const uint16_t* x, const uint16_t* w_base, const uint16_t* w_stack,
+                                       long long w_stride, const dz_gemm_tile* tiles, int ntiles, const int32_t* perm,
+                                       uint16_t* y, int T, int K, int N, int accumulate, int ldy, void* stream) {
+  if (!x || !y || !tiles || ntiles < 1 || !w_base || !w_stack) return DZ_EINVAL;
+  if (T < 1 || K < DZ_KBLOCK || K % DZ_KBLOCK || N < DZ_NPAIR || N % DZ_NPAIR || ldy < N || ldy % 4) return DZ_ESHAPE;
+  if (((uintptr_t)x & 15) || ((uintptr_t)w_base & 15) || ((uintptr_t)w_stack & 15) || ((uintptr_t)y & 7) || (w_stride & 7))
+    return DZ_EALIGN;
+  if ((unsigned long long)T * (unsigned)K * 2ull >= (1ull << 31) ||
+      (unsigned long long)N * (unsigned)K * 2ull >= (1ull << 31))
+    return DZ_ESHAPE;
+  RowsParams P{};
+  P.x = (const _Float16*)x; P.w = (const _Float16*)w_base; P.y = (_Float16*)y;
+  P.w_stack = (const _Float16*)w_stack; P.w_stride = w_stride;
+  P.tiles = tiles; P.perm = perm;
+  P.K = K; P.N = N; P.G = 1; P.gslabs = K / 64; P.accumulate = accumulate; P.ldy = ldy;   // (S = 0: no deltas)
+  return launch(P, 2, ntiles, (hipStream_t)stream);
 }

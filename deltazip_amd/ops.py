@@ -261,11 +261,18 @@ def apply_delta_uncompressed(x: torch.Tensor, delta_weights: torch.Tensor, indic
         raise ValueError("shapes: x [T, K], delta_weights [S, N, K], base_embedding [N, K], indices [T]")
     if not (delta_weights.is_contiguous() and base_embedding.is_contiguous() and x.is_contiguous()):
         raise ValueError("x and the weights must be contiguous")
-    blocks = row_blocks(indices, S, long_only=True)
+    # The kernel whose weights go straight into registers is the faster one up to 600 rows, whatever the
+    # number of tables (32000 x 4096, 32 / 256 / 600 rows of 8 tables: 421 / 464 / 523 against 368 / 389 /
+    # 423 us, of one: 102 / 156 / 286 against 56 / 104 / 244); at 1024 tiles of 256 x 256 are (582 against
+    # 691), unless there are too few of them to fill the GPU (4096 x 1024: 46 against 32).
+    short = K % 256 == 0 and N % 32 == 0 and (
+        T <= 600 or (T <= 1024 and ((N + 255) // 256) * ((T + 255) // 256) <= 64))
+    blocks = row_blocks(indices, S, long_only=not short)
+    tiles, ntiles = (blocks.short, blocks.max_short) if short else (blocks.tiles, blocks.max_tiles)
     out = torch.empty((T, N), dtype=torch.float16, device=x.device)
-    _lib.check(_lib.lib().dz_gemm_f16_select(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K,
-                                             blocks.tiles.data_ptr(), blocks.max_tiles, blocks.perm.data_ptr(),
-                                             out.data_ptr(), T, K, N, 0, N, _stream()), "dz_gemm_f16_select")
+    fn = _lib.lib().dz_gemm_f16_select_rows if short else _lib.lib().dz_gemm_f16_select
+    _lib.check(fn(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K, tiles.data_ptr(), ntiles,
+                  blocks.perm.data_ptr(), out.data_ptr(), T, K, N, 0, N, _stream()), "dz_gemm_f16_select")
     return out
 
 

@@ -321,6 +321,13 @@ int dz_gemm_f16_select(const uint16_t* x, const uint16_t* w_base, const uint16_t
                        long long w_stride, const dz_gemm_tile* tiles, int ntiles, const int32_t* perm,
                        uint16_t* y, int T, int K, int N, int accumulate, int ldy, void* stream);
 
+/* dz_gemm_f16_select for row blocks of up to DZ_SHORT_ROWS rows (longer ones are taken that many rows
+ * at a time), K a multiple of 256 and N of 32: weights go straight into registers, which is the
+ * faster way where a weight meets few rows. */
+int dz_gemm_f16_select_rows(const uint16_t* x, const uint16_t* w_base, const uint16_t* w_stack,
+                            long long w_stride, const dz_gemm_tile* tiles, int ntiles, const int32_t* perm,
+                            uint16_t* y, int T, int K, int N, int accumulate, int ldy, void* stream);
+
 /* Row blocks for dz_multi_delta_gemm from the segment offsets dz_segment wrote (device memory,
  * S + 2 entries): every segment is cut into blocks of at most 256 rows, group = slot (-1 for the
  * tokens without a delta); entries of `tiles` (device memory, max_tiles of them) beyond the blocks

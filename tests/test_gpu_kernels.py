@@ -361,6 +361,31 @@ def test_short_row_blocks(dev, n, k, bits, gs, nd):
             assert o.rel_err(y0.float().cpu().numpy(), ref) <= TOL
 
 
+@pytest.mark.parametrize("n,k,s,t", [(32, 256, 3, 1), (96, 512, 8, 33), (160, 768, 2, 128), (4128, 256, 5, 129),
+                                     (288, 1024, 1, 300), (64, 512, 20, 1024)])
+def test_select_over_short_blocks(dev, n, k, s, t):
+    """apply_delta_uncompressed where its row blocks are short: every row against its own table in 64 bits
+    (fp32 sums rounded once to fp16: half a unit of 2^-11, and as much again for the sums), and the
+    kernel for long blocks on the same rows."""
+    from deltazip_amd import _lib
+    g = torch.Generator().manual_seed(n + t)
+    x = torch.randn(t, k, generator=g).half()
+    stack, base = (torch.randn(s, n, k, generator=g) * 0.02).half(), (torch.randn(n, k, generator=g) * 0.02).half()
+    ids = torch.randint(-1, s, (t,), generator=g)
+    tables = torch.cat([base[None], stack]).double()
+    want = torch.stack([x[i].double() @ tables[int(ids[i]) + 1].t() for i in range(t)])
+    xd, sd, bd, idd = x.to(dev), stack.to(dev), base.to(dev), ids.to(dev)
+    got = ops.apply_delta_uncompressed(xd, sd, idd, bd)
+    blocks = ops.row_blocks(idd, s, long_only=True)
+    other = torch.empty_like(got)
+    assert _lib.lib().dz_gemm_f16_select(xd.data_ptr(), bd.data_ptr(), sd.data_ptr(), n * k, blocks.tiles.data_ptr(),
+                                         blocks.max_tiles, blocks.perm.data_ptr(), other.data_ptr(), t, k, n, 0, n,
+                                         torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    for y in (got, other):
+        assert ((y.cpu().double() - want).abs() <= 2.0**-10 * want.abs() + 1e-4).all()
+
+
 @pytest.mark.parametrize("lens,short", [([0, 300, 20, 5], True), ([0, 512, 250, 0], False), ([10, 0, 0, 0], True),
                                         ([192, 192, 192, 192], False), ([191, 192, 192, 192], True)])
 def test_build_tiles_either(dev, lens, short):
