@@ -22,6 +22,7 @@ SIGNATURES = {
     "dz_unrepack_2of4": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp]),
     "dz_dequant": (_i, [_vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]),
     "dz_merge": (_i, [_vp, _vp, _vp, _vp, _i, _i, _i, _i, _vp, _vp]),
+    "dz_segment_status": (_i, [_vp, _i, _i, _vp, _vp, _vp, _vp]),
     "dz_segment": (_i, [_vp, _i, _i, _vp, _vp, _vp]),
     "dz_embedding_select": (_i, [_vp, _vp, _vp, _vp, C.c_longlong, _i, _vp, _i, _i, _i, _i, _vp]),
     "dz_build_tiles": (_i, [_vp, _i, _vp, _i, _vp]),

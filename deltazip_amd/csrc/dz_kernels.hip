@@ -96,7 +96,7 @@ __global__ __launch_bounds__(64) void dz_dequant_kernel(const uint32_t* __restri
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(1024) void dz_segment_kernel(const long long* __restrict__ idx, int T,
                                                           int S, int* __restrict__ perm,
-                                                          int* __restrict__ seg_off) {
+                                                          int* __restrict__ seg_off, unsigned* status) {
   // hist[S+2] (exclusive offsets after the scan), running[S+1] (tokens of a key placed by earlier
   // chunks), cnt[16][S+1] (tokens of a key per wavefront of the current chunk)
   extern __shared__ int sm[];
@@ -108,11 +108,14 @@ __global__ __launch_bounds__(1024) void dz_segment_kernel(const long long* __res
   for (int s = tid; s < S + 2; s += 1024) hist[s] = 0;
   for (int s = tid; s < nk; s += 1024) running[s] = 0;
   __syncthreads();
+  bool bad = false;
   for (int t = tid; t < T; t += 1024) {
     long long id = idx[t];
     int key = (id < 0 || id >= S) ? 0 : (int)id + 1;
+    bad |= id < -1 || id >= S;
     atomicAdd(&hist[key + 1], 1);
   }
+  if (bad && status) atomicOr(status, 1u);
   __syncthreads();
   if (tid == 0) {
     for (int s = 1; s < S + 2; ++s) hist[s] += hist[s - 1];
@@ -782,11 +785,16 @@ int dz_merge(const uint16_t* w_base, const void* codes, const void* meta, const 
 }
 
 int dz_segment(const int64_t* indices, int T, int S, int32_t* perm, int32_t* seg_off, void* stream) {
+  return dz_segment_status(indices, T, S, perm, seg_off, nullptr, stream);
+}
+
+int dz_segment_status(const int64_t* indices, int T, int S, int32_t* perm, int32_t* seg_off, uint32_t* status,
+                      void* stream) {
   if (!indices || !perm || !seg_off) return DZ_EINVAL;
   if (T < 1 || S < 0 || S > DZ_MAX_SLOTS_SEGMENT) return DZ_ESHAPE;
   const size_t lds = (size_t)((S + 2) + (S + 1) + 16 * (S + 1)) * 4;   // < 64 KiB
   hipLaunchKernelGGL(dz_segment_kernel, dim3(1), dim3(1024), lds, (hipStream_t)stream,
-                     (const long long*)indices, T, S, perm, seg_off);
+                     (const long long*)indices, T, S, perm, seg_off, status);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 

@@ -145,16 +145,18 @@ def merge(base_weight: torch.Tensor, qweight, meta, scales, bits: int) -> torch.
     return out
 
 
-def segment(indices: torch.Tensor, num_slots: int):
-    """(perm [T] int32, seg_off [S+2] int32): tokens grouped by delta id, id -1 first."""
+def segment(indices: torch.Tensor, num_slots: int, report: bool = False):
+    """(perm [T] int32, seg_off [S+2] int32): tokens grouped by delta id, id -1 first.  `report`: an id
+    outside [-1, S) sets bit 0 of the status word of this stream's workspace."""
     _need_cuda(indices)
     if indices.dtype != torch.int64:
         raise ValueError("indices must be int64")
     T = indices.numel()
     perm = torch.empty(T, dtype=torch.int32, device=indices.device)
     off = torch.empty(num_slots + 2, dtype=torch.int32, device=indices.device)
-    _lib.check(_lib.lib().dz_segment(indices.data_ptr(), T, num_slots, perm.data_ptr(), off.data_ptr(),
-                                     _stream()), "dz_segment")
+    status = _workspace(indices.device, 1, 256, 32).data_ptr() if report else None
+    _lib.check(_lib.lib().dz_segment_status(indices.data_ptr(), T, num_slots, perm.data_ptr(), off.data_ptr(), status,
+                                            _stream()), "dz_segment")
     return perm, off
 
 
@@ -200,7 +202,8 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False) -
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
     T = indices.numel()
-    perm, seg_off = segment(indices, num_slots)
+    # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
+    perm, seg_off = segment(indices, num_slots, not long_only and T > MAX_TOKENS_FUSED and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
     if not long_only and T <= 1024:
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)

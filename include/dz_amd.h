@@ -99,6 +99,10 @@ int dz_merge(const uint16_t* w_base, const void* codes, const void* meta, const 
  * id, serving/vllm/core/scheduler.py:101-104; this makes the op independent of that.) */
 int dz_segment(const int64_t* indices, int T, int S, int32_t* perm, int32_t* seg_off, void* stream);
 
+/* dz_segment that sets bit 0 of *status (device memory, or NULL) where an id outside [-1, S) is met. */
+int dz_segment_status(const int64_t* indices, int T, int S, int32_t* perm, int32_t* seg_off, uint32_t* status,
+                      void* stream);
+
 /* Delta id -> slot index for a batch, on the device: the index tensors the reference's manager
  * builds in a Python loop over tokens (convert_mapping, serving/vllm/delta/models.py:69-145).
  * token_ids [T] and prompt_ids [P] hold delta ids (<= 0: base model); slot_ids [S] holds the id

@@ -361,6 +361,22 @@ def test_short_row_blocks(dev, n, k, bits, gs, nd):
             assert o.rel_err(y0.float().cpu().numpy(), ref) <= TOL
 
 
+def test_bad_ids_of_mid_size_batches_are_reported(dev):
+    """An id outside [-1, S) is served as -1 and sets bit 0 of the status word, as at decode sizes."""
+    p = make_problem(64, 256, 2, -1, 3, 200, "uniform", 5, dev)
+    run_layer(p)
+    ops.poll_status(wait=True)
+    assert ops.workspace_status() == 0
+    good = run_layer(dict(p, ids=torch.where(p["ids"] == 1, torch.full_like(p["ids"], -1), p["ids"])))
+    assert ops.workspace_status() == 0
+    bad = run_layer(dict(p, ids=torch.where(p["ids"] == 1, torch.full_like(p["ids"], 7), p["ids"])))
+    assert torch.equal(good, bad) and ops.workspace_status() == ops.STATUS_BAD_ID
+    warned, ops._warned_bad_id = ops._warned_bad_id, True
+    ops.poll_status(wait=True)                        # clears it
+    ops._warned_bad_id = warned
+    assert ops.workspace_status() == 0
+
+
 @pytest.mark.parametrize("n,k,s,t", [(32, 256, 3, 1), (96, 512, 8, 33), (160, 768, 2, 128), (4128, 256, 5, 129),
                                      (288, 1024, 1, 300), (64, 512, 20, 1024)])
 def test_select_over_short_blocks(dev, n, k, s, t):
