@@ -168,12 +168,28 @@ class RowBlocks:
     """A batch of more than 128 tokens ordered by delta id and cut into row blocks of one delta each
     (what dz_segment and dz_build_tiles write): depends on the indices only, so it can be made once
     per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
-    256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short")
+    256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None.
+    They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`."""
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured")
 
     def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
         self.short, self.max_short = short, max_short
+        self.captured = torch.cuda.is_current_stream_capturing()
+
+
+def _usable_blocks(order, T: int, S: int) -> Optional[RowBlocks]:
+    """`order` if it holds row blocks this call can use, else None: the call then makes its own from the
+    indices.  A captured call does so unless the blocks were made under capture too: a replay must
+    read the indices as they are then, and the tables of a batch that is over may have been given
+    back.  (Blocks made under capture hold nothing before the first replay: no eager call takes them.)"""
+    if not isinstance(order, RowBlocks) or order.captured != torch.cuda.is_current_stream_capturing():
+        return None
+    if order.T == T and order.S == S:
+        return order
+    if takes_fused_chunks(T, S):
+        return None                                   # (at these sizes a stale order was never an error)
+    raise ValueError("row blocks were made for another batch size or number of slots")
 
 
 def _block_table(T: int, num_slots: int, rows: int, device):
@@ -679,14 +695,9 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
                                    out=out[r:r + MAX_TOKENS_FUSED], accumulate=accumulate, base_tiled=base_tiled)
             return out
         from .prefill import multi_delta_linear_prefill
-        blocks = order if isinstance(order, RowBlocks) else None
-        if blocks is not None and (blocks.T != T or blocks.S != S) and takes_fused_chunks(T, S):
-            blocks = None                             # (at these sizes a stale order was never an error)
-        if blocks is not None and (blocks.T != T or blocks.S != S):
-            raise ValueError("row blocks were made for another batch size or number of slots")
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
-                                          indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
-                                          base_tiled=base_tiled)
+                                          indices, bits=bits, out=out, accumulate=accumulate,
+                                          blocks=_usable_blocks(order, T, S), base_tiled=base_tiled)
     ws = _workspace(x.device, T, K, N)
     optr = _order_ptr(order, T, x.device)
     if base_tiled is not None:

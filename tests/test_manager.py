@@ -109,6 +109,27 @@ def make_delta_model(delta_id, bits, seed):
 # ---------------------------------------------------------------------------------------------
 # CPU
 # ---------------------------------------------------------------------------------------------
+def test_row_blocks_stay_on_their_side_of_a_capture(monkeypatch):
+    """Tables made outside a graph capture are gone when the graph is replayed after the next mapping
+    (their row numbers would address whatever took their place), and tables made under capture
+    hold nothing before a replay: a call on the other side makes its own from the indices."""
+    now = [False]
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now[0])
+    perm = torch.arange(200, dtype=torch.int32)
+    made = {}
+    for now[0] in (False, True):
+        made[now[0]] = ops.RowBlocks(perm, None, 0, 200, 3, perm, 1)
+    for now[0] in (False, True):
+        assert ops._usable_blocks(made[now[0]], 200, 3) is made[now[0]]
+        assert ops._usable_blocks(made[not now[0]], 200, 3) is None
+        assert ops._usable_blocks(perm, 200, 3) is None and ops._usable_blocks(None, 200, 3) is None
+        assert ops._usable_blocks(made[now[0]], 201, 3) is None
+    now[0] = False
+    late = ops.RowBlocks(perm, None, 0, 600, 3, perm, 1)
+    with pytest.raises(ValueError):
+        ops._usable_blocks(late, 601, 3)
+
+
 def test_oracle_convert_mapping_known_answers():
     # slots: [id 7, free, id 3]; manager passes max_deltas = slots + 1 = 4
     base, samp, padded, emb = o.convert_mapping_ref((3, 3, 0, 7, 0), (3, 0, 7), [7, None, 3], 4, 100, 10)
@@ -427,6 +448,48 @@ def test_manager_makes_row_blocks_once_for_a_large_batch(dev):
     assert mgr.row_blocks[0] is blocks          # made once, not per layer call
     mgr.set_delta_mapping(DeltaMapping(ids[:9], ids[:2]))
     assert mgr.row_blocks[0] is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T", [200, 400, 1100])
+def test_wrapped_layers_replay_from_a_graph_with_the_mapping_of_the_day(dev, T):
+    """Layers captured above the fused kernel's sizes and replayed after further set_delta_mapping calls,
+    with tensors of other sizes made and dropped in between: every replay reads the ids as they are
+    then, and equals the eager call of the same mapping bit for bit."""
+    model = ToyModel(dev)
+    mgr = create_delta_manager(model, 8, 2048, V, DeltaConfig(max_deltas=6, max_bitwidth=4, max_cpu_deltas=6))
+    for did in (11, 12, 13):
+        mgr.add_delta(make_delta_model(did, 4, 100 * did)[0])
+        mgr.activate_delta(did)
+    layers = [model.get_submodule("model.layers.0." + n) for n in ("self_attn.qkv_proj", "self_attn.o_proj")]
+    x = torch.from_numpy(o.make_x(T, H, 3)).to(dev)
+    step = lambda: [layer(x)[0] for layer in layers]
+    rng = np.random.default_rng(T)
+
+    def mapping(t):
+        ids = tuple(int(i) for i in np.sort(rng.choice([0, 11, 12, 13], size=t, p=rng.dirichlet(np.ones(4)))))
+        mgr.set_delta_mapping(DeltaMapping(ids, ids[:2]))
+    mapping(T)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        step()                                       # this stream's workspace is made outside the capture
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            outs = step()
+    torch.cuda.current_stream().wait_stream(side)
+    for rep in range(4):
+        mapping(9 + 200 * rep)                       # batches of other sizes in between, their tables dropped
+        junk = [torch.full((n, 4), 1 << 20, dtype=torch.int32, device=dev) for n in (5, 9, 17, T)]
+        mapping(T)
+        want = step()
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(outs, want):
+            assert torch.equal(a, b), rep
+        del junk
 
 
 @pytest.mark.gpu
