@@ -347,8 +347,9 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
         const float diff = w[r] - qv;
         float e;
         if (FAST) {
-          // without rounding a column that stays has no error
-          e = QUANT || pr ? div_by(diff, d[r], y[r]) : 0.f;
+          // without rounding a column that stays has no error (diff is 0, and NaN where w is: the range
+          // check's minimum and maximum pass over a NaN)
+          e = QUANT || pr ? div_by(diff, d[r], y[r]) : diff;
           xmin = fminf(fminf(xmin, fabsf(w[r])), QUANT ? fabsf(diff) : X_MAX);
           xmax = fmaxf(xmax, fabsf(w[r]));
         } else {

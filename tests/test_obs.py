@@ -104,6 +104,27 @@ def test_obs_sweep_values_outside_the_fast_range(dev, n, k, quant, prune):
     assert np.array_equal(loss.cpu().numpy(), want_loss, equal_nan=True)
 
 
+@pytest.mark.parametrize("prune", [(0, 0), (1, 2), (2, 4), (3, 8)])
+def test_obs_sweep_without_rounding_carries_nan_and_infinity(dev, prune):
+    """A weight that is no finite number spoils its row from its column on, and no other row: in the
+    places the oracle's sweep has it, the rest bit for bit."""
+    n, k = 20, 384
+    W, X = _inputs(n, k, 1024, 321)
+    H, _ = o.hessian_add_batch_ref(np.zeros((k, k), np.float32), 0, X)
+    hinv, W0 = o.hinv_upper_ref(H, W)
+    W0[2, 5], W0[4, 130], W0[17, 383] = np.nan, np.nan, np.nan
+    W0[6, 64], W0[9, 257] = np.inf, -np.inf
+    W0[11, 200], W0[11, 201] = np.nan, np.inf
+    with np.errstate(invalid="ignore"):
+        want, want_loss = o.obs_sweep_ref(W0.copy(), hinv, None, 4, *prune)
+    Wd = torch.from_numpy(W0.copy()).to(dev)
+    loss = ops.obs_sweep(Wd, torch.from_numpy(hinv).to(dev), None, 4, *prune)
+    torch.cuda.synchronize()
+    assert np.isnan(want[2, 200:]).any() and np.isfinite(want[[0, 1, 3, 19]]).all()
+    assert np.array_equal(Wd.cpu().numpy(), want, equal_nan=True)
+    assert np.array_equal(loss.cpu().numpy(), want_loss, equal_nan=True)
+
+
 @pytest.mark.parametrize("n,k,bits,gs", [(64, 512, 4, -1), (96, 1024, 2, -1), (32, 512, 4, 128), (64, 256, 2, 64)])
 def test_scales_with_the_search_over_the_clipping_range(dev, n, k, bits, gs):
     """dz_quant_scales_mse against the oracle's restatement of quant.py:85-101.  The candidates'
