@@ -118,7 +118,7 @@ __global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ 
     __syncthreads();
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
-      const float sv = t0 + lt + l * TSTEP < T ? s1 : 0.f;
+      const bool in = t0 + lt + l * TSTEP < T;
 #pragma unroll
       for (int side = 0; side < 2; ++side)
 #pragma unroll
@@ -126,7 +126,7 @@ __global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ 
           const xv_t& q = next[side][l];
           f4_t f = {(float)q[v], (float)q[v + 1], (float)q[v + 2], (float)q[v + 3]};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) f[e] = sv == 0.f ? 0.f : sv * f[e];
+          for (int e = 0; e < 4; ++e) f[e] = in ? s1 * f[e] : 0.f;
           *(f4_t*)&st[side][lt + l * TSTEP][lc + v] = f;
         }
     }

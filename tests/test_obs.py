@@ -72,6 +72,23 @@ def test_hessian_tiles_bit_exact(dev, k, tokens, half):
         assert np.array_equal(H.cpu().numpy(), want)
 
 
+def test_hessian_factor_zero_is_still_a_product(dev):
+    """scale_x = 0: 0 times an infinite or NaN input is NaN, in the input's rows and columns; only the
+    places beyond the last token are filled with zeros."""
+    from deltazip_amd import _lib
+    k, tokens = 128, 33
+    x = torch.ones(tokens, k, dtype=torch.float16, device=dev)
+    x[32, 3], x[5, 100] = float("inf"), float("nan")
+    H = torch.ones(k, k, device=dev)
+    assert _lib.lib().dz_hessian_add(H.data_ptr(), x.data_ptr(), 1, tokens, k, 0.5, 0.0,
+                                     torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    want = torch.full((k, k), 0.5)
+    for c in (3, 100):
+        want[c], want[:, c] = float("nan"), float("nan")
+    assert np.array_equal(H.cpu().numpy(), want.numpy(), equal_nan=True)
+
+
 @pytest.mark.parametrize("n,k,quant,prune", [(1, 128, True, (2, 4)), (17, 256, True, (2, 4)), (17, 256, False, (2, 4)),
                                              (50, 384, True, (1, 8)), (50, 384, False, (3, 8)), (16, 128, True, (1, 2)),
                                              (65, 256, False, (0, 0))])
