@@ -777,11 +777,13 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     G = scales_stacked[0][0].numel() // base_weight[0].shape[0]
     S = qweight_stacked[0].shape[0]
     if T > MAX_TOKENS_FUSED:
-        if not isinstance(order, RowBlocks) and n > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
+        blocks = order if isinstance(order, RowBlocks) else None
+        if blocks is None and n > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
-            order = row_blocks(indices, S)            # once for all projections
+            blocks = row_blocks(indices, S)           # once for all projections with as many slots as the first
+        fits = lambda q: blocks is not None and blocks.T == T and blocks.S == q.shape[0]
         return [apply_delta(xs[j], qweight_stacked[j], scales_stacked[j], meta_stacked[j], indices, base_weight[j],
-                            order=order if isinstance(order, RowBlocks) and order.S == S and order.T == T else None,
+                            order=blocks if fits(qweight_stacked[j]) else None,
                             base_tiled=None if base_tiled is None else base_tiled[j])
                 for j in range(n)]
     _need_cuda(indices, *xs, *qweight_stacked, *scales_stacked, *meta_stacked, *base_weight)

@@ -796,6 +796,25 @@ def _batched_equal_separate(dev, bits, gs, t, ns, k, nd):
         ops.apply_delta_batch(x, [ps[0]["q"]] * 5, [ps[0]["s"]] * 5, [ps[0]["m"]] * 5, ids, [ps[0]["wb"]] * 5)
 
 
+@pytest.mark.parametrize("t", [200, 700])
+def test_batched_calls_over_stacks_of_different_slot_counts(dev, t):
+    """Above the fused kernel's sizes every projection is served by its own number of slots: an id that is
+    in the first stack and beyond the second counts as -1 there, as in the separate call."""
+    ps = [make_problem(96, 512, 2, -1, nd, t, "uniform", 60 + nd, dev) for nd in (5, 3)]
+    x, ids = ps[0]["x"], ps[0]["ids"]
+    args = [[p[key] for p in ps] for key in ("q", "s", "m")]
+    for order in (None, ops.row_blocks(ids, 5), ops.row_blocks(ids, 3)):
+        ys = ops.apply_delta_batch(x, *args, ids, [p["wb"] for p in ps], order=order)
+        torch.cuda.synchronize()
+        for p, y, nd in zip(ps, ys, (5, 3)):
+            assert torch.equal(y, ops.apply_delta(x, p["q"], p["s"], p["m"], ids, p["wb"]))
+            seen = np.where(ps[0]["ids_np"] < nd, ps[0]["ids_np"], -1)
+            assert o.rel_err(y.cpu().numpy(), o.forward_ref(ps[0]["x_np"], p["wb_np"], p["dts"], seen)) <= TOL
+    warned, ops._warned_bad_id = ops._warned_bad_id, True
+    ops.poll_status(wait=True)                            # clears what ids beyond three slots have set
+    ops._warned_bad_id = warned
+
+
 @pytest.mark.parametrize("t,kind", [(33, "uniform"), (64, "zipf"), (128, "uniform"), (20, "uniform")])
 def test_token_order_is_a_permutation_and_reusable(dev, t, kind):
     """dz_token_order: a permutation of the tokens in which every delta's tokens are contiguous; passing
