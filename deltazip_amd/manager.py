@@ -360,7 +360,9 @@ class DeltaModelManager:
             ops.token_order(self.base_indices[:T], self.delta_slots, out=self.token_order)
         self.row_blocks[0] = None
         if T > ops.MAX_TOKENS_FUSED and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
-            self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots)
+            # (the mix decides at sizes where other routes than row blocks may be the faster one)
+            self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
+                                                mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None)
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 

@@ -14,7 +14,8 @@ from __future__ import annotations
 
 import ctypes as C
 import math
-from typing import Dict, Optional, Sequence, Tuple
+from collections import Counter
+from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 
 import torch
 
@@ -169,13 +170,66 @@ class RowBlocks:
     (what dz_segment and dz_build_tiles write): depends on the indices only, so it can be made once
     per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
     256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None.
-    They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured")
+    They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`.
+    `mix`: what the maker knew of the batch on the host, or None."""
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix")
 
-    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0):
+    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
-        self.short, self.max_short = short, max_short
+        self.short, self.max_short, self.mix = short, max_short, mix
         self.captured = torch.cuda.is_current_stream_capturing()
+
+
+class BatchMix(NamedTuple):
+    """What the choice between the kernels looks at: deltas in the batch (the base model counts as
+    one), row blocks of 128 tokens, tokens of the most popular delta, and the deltas met by each chunk
+    of 128 tokens, summed."""
+    deltas: int
+    blocks: int
+    longest: int
+    met: int
+
+
+def batch_mix(ids: Sequence[int]) -> BatchMix:
+    """The mix of a batch whose delta ids the host has (ids below 1: the base model)."""
+    ids = [max(i, 0) for i in ids]
+    counts = Counter(ids).values()
+    return BatchMix(len(counts), sum(-(-c // SHORT_ROWS) for c in counts), max(counts),
+                    sum(len(set(ids[r:r + MAX_TOKENS_FUSED])) for r in range(0, len(ids), MAX_TOKENS_FUSED)))
+
+
+def _even_mix(T: int, S: int) -> BatchMix:
+    """Stands in for a mix that only the device knows: every slot in use, sorted by delta."""
+    d = min(S, T)
+    return BatchMix(d, d * -(-T // (SHORT_ROWS * d)), T // d, d + -(-T // MAX_TOKENS_FUSED) - 1)
+
+
+def _chunks_faster(T: int, K: int, N: int, bits: int, mix: BatchMix) -> bool:
+    """Whether a batch that chunks of the fused kernel can serve (takes_fused_chunks) is faster there
+    than in row blocks of 128 tokens.  A row block costs much the same whether it holds 2 tokens or 60,
+    because it reads the base weight again; a chunk of 128 reads it once for all its deltas.
+
+    The estimates below are in us; they were fitted to 2400 timed calls over tiles (129 to 512 tokens
+    of 1 to 64 deltas, sorted, shuffled and in requests; 4096 x 4096 to 5120 x 27648; 2 bits and 4) and
+    are within a sixth of 90 % of them.  What they choose is 0.3 % slower in the mean than the faster
+    route, where row blocks throughout were 5 % slower and up to 2.0 times.  Chunks / row blocks, sorted:
+      5120 x 27648, 2-bit, 129 tokens of 4 / 16 / 64 deltas   251 / 307 / 557 against 138 / 376 / 1103 us
+                           256                                388 / 433 / 698 against 177 / 386 / 1224
+                           512                                769 / 798 / 1064 against 297 / 425 / 1356
+      5120 x 5120, 4-bit,  129 tokens of 4 / 16 / 64 deltas   79 / 99 / 178 against 65 / 115 / 281
+                           512                                220 / 243 / 352 against 86 / 126 / 315
+    Row blocks come in waves of 512 workgroups (two per CU), and a single wave is the faster route but
+    for one delta's long blocks over few features, where the fused kernel splits K and fills the GPU
+    (129 tokens of one delta: 4096 x 4096 48 against 58, 13824 x 5120 160 against 184; 5120 x 5120 72 / 70)."""
+    waves = -(-mix.blocks * -(-N // 128) // 512)
+    if waves == 1:
+        return T <= 160 and mix.longest > 64 and (N <= 4096 or (N <= 5120 and K >= 2 * N))
+    k, weight = K / 5120, K * N / 5120**2
+    chunks, turns = -(-T // MAX_TOKENS_FUSED), -(-T // 32)
+    per_block, per_turn, per_delta = (45.3, 0.65, 1.17) if bits == 2 else (57.8, 1.6, 1.93)
+    rows_us = k * waves * (per_block + 62 * T / (SHORT_ROWS * mix.blocks))
+    chunks_us = k * (11.5 * chunks + per_turn * turns) + weight * (7.2 * turns + per_delta * mix.met)
+    return chunks_us < rows_us
 
 
 def _usable_blocks(order, T: int, S: int) -> Optional[RowBlocks]:
@@ -197,23 +251,25 @@ def _block_table(T: int, num_slots: int, rows: int, device):
     return torch.empty((n, 4), dtype=torch.int32, device=device), n
 
 
-def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False) -> RowBlocks:
+def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
-    (serving/vllm/delta/models.py:421-435).  Two small launches, nothing read back to the host.
+    (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
     Which of the two kernels serves the batch.  Tiles of 256 features x 256 tokens want full
     blocks and some 256 of them; tiles of 128 x 128 read the weights twice as often but fill the GPU
     with a quarter of the tokens and multiply few rows that are not there.
       up to 1024 tokens   short blocks: even with a single delta there are too few long ones to fill
-                          the GPU (5120 x 5120, 2-bit, 1024 tokens, 1 / 16 / 64 deltas: 103 / 147 / 266
-                          against 187 / 241 / 640 us; 5120 x 27648: 437 / 602 / 1382 against 757 / 959 /
-                          3251; the exception, one delta and many features at 512 tokens, 232 against
-                          204, stays within the launches it saves)
+                          the GPU (5120 x 5120, 2-bit, 1024 tokens, 1 / 16 / 64 deltas: 116 / 153 / 276
+                          against 192 / 246 / 649 us; 5120 x 27648: 435 / 630 / 1443 against 810 / 1000 /
+                          3468)
       above, 256 tokens   long blocks: they are at least half full, and at 8192 tokens of 16 deltas
-      per slot and more   the larger tile is the faster one
+      per slot and more   or fewer the larger tile is the faster one at 2 bits (5120 x 27648: 3113
+                          against 3499; 4096 x 12288: 1133 against 1243; 4 bits: equal)
       between             the number of deltas in the batch is known on the device only: it picks
                           (dz_build_tiles_either), and both products are launched, one of them empty
-    `long_only`: the table of 256-token blocks alone, whatever the batch."""
+    `long_only`: the table of 256-token blocks alone, whatever the batch.  `mix`: batch_mix() of the
+    same ids, if the host has them: calls of a few hundred tokens then choose between these blocks and
+    chunks of the fused kernel by it."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
@@ -221,19 +277,20 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False) -
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
     perm, seg_off = segment(indices, num_slots, not long_only and T > MAX_TOKENS_FUSED and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
-    if not long_only and T <= 1024:
+    tiles, n, short, ns = None, 0, None, 0
+    if long_only or T > 1024:
+        tiles, n = _block_table(T, num_slots, 256, dev)
+    if not long_only and (T <= 1024 or T < 256 * (num_slots + 1)):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
-        _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
-                   "dz_build_tiles_rows")
-        return RowBlocks(perm, None, 0, T, num_slots, short, ns)
-    tiles, n = _block_table(T, num_slots, 256, dev)
-    if not long_only and T < 256 * (num_slots + 1):
-        short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
+    if tiles is not None and short is not None:
         _lib.check(L.dz_build_tiles_either(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, short.data_ptr(), ns, st),
                    "dz_build_tiles_either")
-        return RowBlocks(perm, tiles, n, T, num_slots, short, ns)
-    _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
-    return RowBlocks(perm, tiles, n, T, num_slots)
+    elif tiles is not None:
+        _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
+    else:
+        _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
+                   "dz_build_tiles_rows")
+    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,
@@ -629,11 +686,18 @@ def _check_tiled(base_tiled, base_weight, N: int, K: int, device) -> None:
 
 
 def takes_fused_chunks(T: int, S: int) -> bool:
-    """Whether a batch above the fused kernel's 128 tokens can go through it in chunks of 128 (sizes at
-    which that costs no more than row blocks of 256 tokens).  Row blocks of 128 tokens are faster at
-    every one of them (5120 x 5120, 2-bit, 192 / 333 / 512 tokens of 16 deltas: 84 / 58 / 95 us against
-    132 / 153 / 262), so chunks serve only what `segment` cannot order: more than 768 slots."""
+    """Whether a batch above the fused kernel's 128 tokens may go through it in chunks of 128: sizes at
+    which that can be faster than row blocks (`_chunks_faster`; always where there are more than 768
+    slots, which `segment` cannot order)."""
     return T <= 3 * MAX_TOKENS_FUSED or (T <= 4 * MAX_TOKENS_FUSED and S >= 16)
+
+
+def _goes_in_chunks(T: int, K: int, N: int, bits: int, S: int, blocks: Optional[RowBlocks]) -> bool:
+    """A caller's own row blocks without a mix are taken as they are."""
+    if not takes_fused_chunks(T, S):
+        return False
+    mix = _even_mix(T, S) if blocks is None else blocks.mix
+    return S > MAX_SLOTS_SEGMENT or (mix is not None and _chunks_faster(T, K, N, bits, mix))
 
 
 def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qweight_stacked,
@@ -688,7 +752,8 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             raise ValueError("out must be float16 [T, N] with unit column stride")
     ldy = out.stride(0)
     if T > MAX_TOKENS_FUSED:
-        if S > MAX_SLOTS_SEGMENT and takes_fused_chunks(T, S):
+        blocks = _usable_blocks(order, T, S)
+        if _goes_in_chunks(T, K, N, bits, S, blocks):
             for r in range(0, T, MAX_TOKENS_FUSED):
                 multi_delta_linear(x2[r:r + MAX_TOKENS_FUSED], base_weight, qweight_stacked, scales_stacked,
                                    meta_stacked, indices[r:r + MAX_TOKENS_FUSED], bits=bits,
@@ -696,8 +761,8 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             return out
         from .prefill import multi_delta_linear_prefill
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
-                                          indices, bits=bits, out=out, accumulate=accumulate,
-                                          blocks=_usable_blocks(order, T, S), base_tiled=base_tiled)
+                                          indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
+                                          base_tiled=base_tiled)
     ws = _workspace(x.device, T, K, N)
     optr = _order_ptr(order, T, x.device)
     if base_tiled is not None:
@@ -778,12 +843,16 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     S = qweight_stacked[0].shape[0]
     if T > MAX_TOKENS_FUSED:
         blocks = order if isinstance(order, RowBlocks) else None
-        if blocks is None and n > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
+        # row blocks made once serve the projections that would make the same ones
+        shared = [q.shape[0] == S and (blocks is not None or not _goes_in_chunks(T, K, w.shape[0], bits, S, None))
+                  for q, w in zip(qweight_stacked, base_weight)]
+        if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
-            blocks = row_blocks(indices, S)           # once for all projections with as many slots as the first
-        fits = lambda q: blocks is not None and blocks.T == T and blocks.S == q.shape[0]
+            blocks = row_blocks(indices, S)
+        if blocks is not None and (blocks.T != T or blocks.S != S):
+            blocks = None
         return [apply_delta(xs[j], qweight_stacked[j], scales_stacked[j], meta_stacked[j], indices, base_weight[j],
-                            order=blocks if fits(qweight_stacked[j]) else None,
+                            order=blocks if shared[j] else None,
                             base_tiled=None if base_tiled is None else base_tiled[j])
                 for j in range(n)]
     _need_cuda(indices, *xs, *qweight_stacked, *scales_stacked, *meta_stacked, *base_weight)

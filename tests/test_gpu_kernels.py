@@ -796,6 +796,31 @@ def _batched_equal_separate(dev, bits, gs, t, ns, k, nd):
         ops.apply_delta_batch(x, [ps[0]["q"]] * 5, [ps[0]["s"]] * 5, [ps[0]["m"]] * 5, ids, [ps[0]["wb"]] * 5)
 
 
+@pytest.mark.parametrize("n,k,bits,gs,nd,t,present", [
+    (4096, 256, 2, -1, 24, 129, None), (4096, 256, 4, 128, 24, 130, None), (256, 256, 2, -1, 2, 140, None),   # chunks
+    (256, 512, 4, 64, 2, 150, 1), (4096, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None)])            # row blocks
+def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
+    """129 to 512 tokens through the routes the sizes, the slots and -- where the host knows it -- the mix
+    choose: the direct call, the call with the manager's row blocks, and several projections at once."""
+    p = make_problem(n, k, bits, gs, nd, t, "uniform", n + t, dev)
+    if present is not None:
+        p["ids_np"] = np.where(p["ids_np"] >= present, present - 1, p["ids_np"])
+    else:
+        p["ids_np"] = p["ids_np"].copy()
+    p["ids_np"][7:9] = nd - 1 if present is None else present - 1
+    p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
+    ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
+    tiled = ops.tile_base(p["wb"])
+    known = ops.row_blocks(p["ids"], nd, mix=ops.batch_mix((p["ids_np"] + 1).tolist()))
+    for order in (None, known, ops.row_blocks(p["ids"], nd)):
+        for base in (None, tiled):
+            y = ops.apply_delta(p["x"], p["q"], p["s"], p["m"], p["ids"], p["wb"], order=order, base_tiled=base)
+            torch.cuda.synchronize()
+            assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+    for y in ops.apply_delta_batch(p["x"], [p["q"]] * 2, [p["s"]] * 2, [p["m"]] * 2, p["ids"], [p["wb"]] * 2):
+        assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+
+
 @pytest.mark.parametrize("t", [200, 700])
 def test_batched_calls_over_stacks_of_different_slot_counts(dev, t):
     """Above the fused kernel's sizes every projection is served by its own number of slots: an id that is

@@ -130,6 +130,31 @@ def test_row_blocks_stay_on_their_side_of_a_capture(monkeypatch):
         ops._usable_blocks(late, 601, 3)
 
 
+def test_batch_mix_counts_what_the_routes_meet():
+    ids = [0] * 3 + [-1] * 2 + [7] * 130 + [9] * 128 + [7] * 1                 # 264 tokens, three chunks
+    assert ops.batch_mix(ids) == ops.BatchMix(3, 1 + 2 + 1, 131, 2 + 2 + 2)
+    assert ops.batch_mix(tuple(reversed(ids))) == ops.BatchMix(3, 4, 131, 2 + 2 + 2)
+    for t, s, want in ((129, 1, (1, 2, 129, 2)), (512, 16, (16, 16, 32, 19)), (300, 2, (2, 4, 150, 4)),
+                       (130, 700, (130, 130, 1, 131))):
+        assert ops._even_mix(t, s) == ops.BatchMix(*want)
+
+
+@pytest.mark.parametrize("k,n,bits,t,deltas,chunks,rows", [
+    (5120, 27648, 2, 129, 4, 251, 138), (5120, 27648, 2, 129, 16, 307, 376), (5120, 27648, 2, 129, 64, 557, 1103),
+    (5120, 27648, 2, 256, 16, 433, 386), (5120, 27648, 2, 256, 24, 478, 540), (5120, 27648, 2, 384, 48, 798, 1016),
+    (5120, 27648, 2, 512, 64, 1064, 1356), (5120, 27648, 2, 512, 1, 741, 238), (5120, 5120, 2, 129, 12, 81, 54),
+    (5120, 5120, 2, 160, 32, 108, 140), (5120, 5120, 2, 320, 16, 151, 103), (13824, 5120, 2, 129, 1, 160, 184),
+    (13824, 5120, 2, 192, 48, 324, 507), (4096, 4096, 2, 129, 1, 48, 58), (4096, 4096, 2, 129, 64, 86, 150),
+    (4096, 4096, 2, 512, 48, 143, 119), (5120, 27648, 4, 192, 32, 596, 891), (5120, 27648, 4, 448, 8, 761, 337),
+    (4096, 12288, 4, 129, 24, 185, 242), (4096, 12288, 4, 384, 16, 267, 173)])
+def test_the_faster_route_is_taken(k, n, bits, t, deltas, chunks, rows):
+    """Measured times (us, sorted batches) of both routes on a few hundred tokens: the rule takes the
+    faster one wherever they differ by a tenth or more."""
+    ids = np.sort(np.random.RandomState(deltas + t).randint(1, deltas + 1, t)).tolist()
+    for mix in (ops.batch_mix(ids), ops._even_mix(t, deltas)):
+        assert ops._chunks_faster(t, k, n, bits, mix) == (chunks < rows)
+
+
 def test_oracle_convert_mapping_known_answers():
     # slots: [id 7, free, id 3]; manager passes max_deltas = slots + 1 = 4
     base, samp, padded, emb = o.convert_mapping_ref((3, 3, 0, 7, 0), (3, 0, 7), [7, None, 3], 4, 100, 10)
