@@ -171,12 +171,12 @@ class RowBlocks:
     per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
     256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None.
     They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`.
-    `mix`: what the maker knew of the batch on the host, or None."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix")
+    `mix`: what the maker knew of the batch on the host, or None; `host_picks`: both tables hold all rows."""
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix", "host_picks")
 
-    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None):
+    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None, host_picks=False):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
-        self.short, self.max_short, self.mix = short, max_short, mix
+        self.short, self.max_short, self.mix, self.host_picks = short, max_short, mix, host_picks
         self.captured = torch.cuda.is_current_stream_capturing()
 
 
@@ -232,6 +232,14 @@ def _chunks_faster(T: int, K: int, N: int, bits: int, mix: BatchMix) -> bool:
     return chunks_us < rows_us
 
 
+def _one_wave_of_long_blocks(T: int, N: int, bits: int) -> bool:
+    """Where a single delta's two blocks of 256 tokens beat its four of 128: their tiles of 256 features
+    then fill the 256 CUs once, nearly (512 tokens, 2-bit, 5120 x 27648 223 against 257 us, 8192 x
+    28672 361 / 395, 4096 x 32768 194 / 221; with fewer tiles, 5120 x 24576, 222 / 204; 448 tokens 235 /
+    242; at 4 bits never: 257 / 249)."""
+    return bits == 2 and 448 < T <= 512 and 208 < 2 * -(-N // 256) <= 256
+
+
 def _usable_blocks(order, T: int, S: int) -> Optional[RowBlocks]:
     """`order` if it holds row blocks this call can use, else None: the call then makes its own from the
     indices.  A captured call does so unless the blocks were made under capture too: a replay must
@@ -251,7 +259,8 @@ def _block_table(T: int, num_slots: int, rows: int, device):
     return torch.empty((n, 4), dtype=torch.int32, device=device), n
 
 
-def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None) -> RowBlocks:
+def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
+               device_picks: bool = False) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
     (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
@@ -261,7 +270,7 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
       up to 1024 tokens   short blocks: even with a single delta there are too few long ones to fill
                           the GPU (5120 x 5120, 2-bit, 1024 tokens, 1 / 16 / 64 deltas: 116 / 153 / 276
                           against 192 / 246 / 649 us; 5120 x 27648: 435 / 630 / 1443 against 810 / 1000 /
-                          3468)
+                          3468), but for `_one_wave_of_long_blocks`
       above, 256 tokens   long blocks: they are at least half full, and at 8192 tokens of 16 deltas
       per slot and more   or fewer the larger tile is the faster one at 2 bits (5120 x 27648: 3113
                           against 3499; 4096 x 12288: 1133 against 1243; 4 bits: equal)
@@ -269,7 +278,7 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
                           (dz_build_tiles_either), and both products are launched, one of them empty
     `long_only`: the table of 256-token blocks alone, whatever the batch.  `mix`: batch_mix() of the
     same ids, if the host has them: calls of a few hundred tokens then choose between these blocks and
-    chunks of the fused kernel by it."""
+    chunks of the fused kernel by it.  `device_picks`: as between, whatever the batch."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
@@ -277,20 +286,23 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
     perm, seg_off = segment(indices, num_slots, not long_only and T > MAX_TOKENS_FUSED and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
+    small = not long_only and not device_picks and T <= 1024
     tiles, n, short, ns = None, 0, None, 0
-    if long_only or T > 1024:
+    host_picks = small and mix is not None and mix.deltas == 1 and 448 < T <= 512
+    if not small or host_picks:
         tiles, n = _block_table(T, num_slots, 256, dev)
-    if not long_only and (T <= 1024 or T < 256 * (num_slots + 1)):
+    if small or device_picks or (not long_only and T < 256 * (num_slots + 1)):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
-    if tiles is not None and short is not None:
+    if tiles is not None and short is not None and not host_picks:
         _lib.check(L.dz_build_tiles_either(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, short.data_ptr(), ns, st),
                    "dz_build_tiles_either")
-    elif tiles is not None:
-        _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
     else:
-        _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
-                   "dz_build_tiles_rows")
-    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix)
+        if tiles is not None:
+            _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
+        if short is not None:
+            _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
+                       "dz_build_tiles_rows")
+    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,
@@ -844,7 +856,9 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     if T > MAX_TOKENS_FUSED:
         blocks = order if isinstance(order, RowBlocks) else None
         # row blocks made once serve the projections that would make the same ones
-        shared = [q.shape[0] == S and (blocks is not None or not _goes_in_chunks(T, K, w.shape[0], bits, S, None))
+        shared = [q.shape[0] == S and (blocks is not None or (
+                      not _goes_in_chunks(T, K, w.shape[0], bits, S, None)
+                      and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():

@@ -43,7 +43,7 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
     host, gathered, scattered or dequantised to memory.  `blocks`: ops.row_blocks(indices, S) when
     the caller made it once for the batch (else made here, per call).  `base_tiled`: the base weight
     in tiles (ops.tile_base), read instead of base_weight when given."""
-    from .ops import row_blocks
+    from .ops import _one_wave_of_long_blocks, row_blocks
     T, K = x2.shape
     N = scales_stacked.shape[-1]
     S = qweight_stacked.shape[0]
@@ -60,10 +60,14 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
         return out
     lib = _lib.lib()
     stream = torch.cuda.current_stream().cuda_stream
+    one_wave = _one_wave_of_long_blocks(T, N, bits)
     if blocks is None:
-        blocks = row_blocks(indices, S)
+        blocks = row_blocks(indices, S, device_picks=S == 1 and one_wave)
+    take_long, take_short = blocks.tiles is not None, blocks.short is not None
+    if blocks.host_picks:
+        take_long, take_short = one_wave, not one_wave
     row_major = base_weight.data_ptr() if base_weight is not None else None
-    if blocks.tiles is not None:
+    if take_long:
         fn, wptr = lib.dz_multi_delta_gemm, row_major
         if base_tiled is not None:
             fn, wptr = lib.dz_multi_delta_gemm_tiled, base_tiled.data_ptr()
@@ -71,7 +75,7 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
                 S, bits, group_size, blocks.tiles.data_ptr(), blocks.max_tiles, blocks.perm.data_ptr(),
                 out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), stream)
         _lib.check(rc, "dz_multi_delta_gemm")
-    if blocks.short is not None:
+    if take_short:
         rc = lib.dz_multi_delta_gemm_rows(
             x2.data_ptr(), base_tiled.data_ptr() if base_tiled is not None else row_major,
             1 if base_tiled is not None else 0, qweight_stacked.data_ptr(), meta_stacked.data_ptr(),

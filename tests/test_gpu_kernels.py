@@ -798,7 +798,9 @@ def _batched_equal_separate(dev, bits, gs, t, ns, k, nd):
 
 @pytest.mark.parametrize("n,k,bits,gs,nd,t,present", [
     (4096, 256, 2, -1, 24, 129, None), (4096, 256, 4, 128, 24, 130, None), (256, 256, 2, -1, 2, 140, None),   # chunks
-    (256, 512, 4, 64, 2, 150, 1), (4096, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None)])            # row blocks
+    (256, 512, 4, 64, 2, 150, 1), (4096, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None),             # row blocks
+    (27648, 256, 2, -1, 1, 512, None), (27648, 256, 2, -1, 1, 449, None), (27648, 256, 2, -1, 3, 512, 1),     # 256-token blocks
+    (27648, 256, 2, -1, 1, 512, 0)])
 def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
     """129 to 512 tokens through the routes the sizes, the slots and -- where the host knows it -- the mix
     choose: the direct call, the call with the manager's row blocks, and several projections at once."""
@@ -807,7 +809,9 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
         p["ids_np"] = np.where(p["ids_np"] >= present, present - 1, p["ids_np"])
     else:
         p["ids_np"] = p["ids_np"].copy()
-    p["ids_np"][7:9] = nd - 1 if present is None else present - 1
+    p["ids_np"][7:9] = nd - 1 if present is None else max(present - 1, 0)
+    if present == 0:                                  # one slot, a third of the tokens
+        p["ids_np"][::3] = 0
     p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
     ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
     tiled = ops.tile_base(p["wb"])

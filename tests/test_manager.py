@@ -155,6 +155,14 @@ def test_the_faster_route_is_taken(k, n, bits, t, deltas, chunks, rows):
         assert ops._chunks_faster(t, k, n, bits, mix) == (chunks < rows)
 
 
+@pytest.mark.parametrize("n,bits,t,short,long", [
+    (27648, 2, 512, 257, 223), (28672, 2, 512, 395, 361), (32768, 2, 512, 221, 194), (24576, 2, 512, 204, 222),
+    (22016, 2, 512, 157, 169), (27648, 2, 640, 320, 585), (15360, 2, 1024, 237, 391), (27648, 4, 512, 249, 257)])
+def test_one_delta_takes_long_blocks_where_they_fill_one_wave(n, bits, t, short, long):
+    """Measured times (us) of one delta's tokens in blocks of 128 and of 256."""
+    assert ops._one_wave_of_long_blocks(t, n, bits) == (long < short)
+
+
 def test_oracle_convert_mapping_known_answers():
     # slots: [id 7, free, id 3]; manager passes max_deltas = slots + 1 = 4
     base, samp, padded, emb = o.convert_mapping_ref((3, 3, 0, 7, 0), (3, 0, 7), [7, None, 3], 4, 100, 10)
