@@ -15,6 +15,8 @@ from __future__ import annotations
 import ctypes as C
 import math
 from collections import Counter
+from functools import lru_cache
+from operator import lt
 from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 
 import torch
@@ -191,45 +193,51 @@ class BatchMix(NamedTuple):
 
 
 def batch_mix(ids: Sequence[int]) -> BatchMix:
-    """The mix of a batch whose delta ids the host has (ids below 1: the base model)."""
-    ids = [max(i, 0) for i in ids]
+    """The mix of a batch whose delta ids the host has (any ids: one per delta, one for the base model)."""
     counts = Counter(ids).values()
-    return BatchMix(len(counts), sum(-(-c // SHORT_ROWS) for c in counts), max(counts),
-                    sum(len(set(ids[r:r + MAX_TOKENS_FUSED])) for r in range(0, len(ids), MAX_TOKENS_FUSED)))
+    return BatchMix(len(counts), sum([-(-c // SHORT_ROWS) for c in counts]), max(counts),
+                    sum([len(set(ids[r:r + MAX_TOKENS_FUSED])) for r in range(0, len(ids), MAX_TOKENS_FUSED)]))
 
 
-def _even_mix(T: int, S: int) -> BatchMix:
-    """Stands in for a mix that only the device knows: every slot in use, sorted by delta."""
-    d = min(S, T)
+def _even_mix(T: int, deltas: int) -> BatchMix:
+    """That many deltas (or one per token), as many tokens of each, sorted."""
+    d = min(deltas, T)
     return BatchMix(d, d * -(-T // (SHORT_ROWS * d)), T // d, d + -(-T // MAX_TOKENS_FUSED) - 1)
 
 
-def _chunks_faster(T: int, K: int, N: int, bits: int, mix: BatchMix) -> bool:
-    """Whether a batch that chunks of the fused kernel can serve (takes_fused_chunks) is faster there
-    than in row blocks of 128 tokens.  A row block costs much the same whether it holds 2 tokens or 60,
-    because it reads the base weight again; a chunk of 128 reads it once for all its deltas.
+@lru_cache(maxsize=4096)
+def _route_us(T: int, K: int, N: int, bits: int, mix: BatchMix) -> Tuple[float, float]:
+    """What a batch of a few hundred tokens takes in chunks of the fused kernel, and in row blocks of 128
+    tokens.  A row block costs much the same whether it holds 2 tokens or 60,
+    because it reads the base weight again, and walks all of K; a chunk of 128 reads the base weight once
+    for all its deltas and splits K where there are few features.
 
-    The estimates below are in us; they were fitted to 2400 timed calls over tiles (129 to 512 tokens
-    of 1 to 64 deltas, sorted, shuffled and in requests; 4096 x 4096 to 5120 x 27648; 2 bits and 4) and
-    are within a sixth of 90 % of them.  What they choose is 0.3 % slower in the mean than the faster
-    route, where row blocks throughout were 5 % slower and up to 2.0 times.  Chunks / row blocks, sorted:
-      5120 x 27648, 2-bit, 129 tokens of 4 / 16 / 64 deltas   251 / 307 / 557 against 138 / 376 / 1103 us
-                           256                                388 / 433 / 698 against 177 / 386 / 1224
-                           512                                769 / 798 / 1064 against 297 / 425 / 1356
-      5120 x 5120, 4-bit,  129 tokens of 4 / 16 / 64 deltas   79 / 99 / 178 against 65 / 115 / 281
-                           512                                220 / 243 / 352 against 86 / 126 / 315
-    Row blocks come in waves of 512 workgroups (two per CU), and a single wave is the faster route but
-    for one delta's long blocks over few features, where the fused kernel splits K and fills the GPU
-    (129 tokens of one delta: 4096 x 4096 48 against 58, 13824 x 5120 160 against 184; 5120 x 5120 72 / 70)."""
-    waves = -(-mix.blocks * -(-N // 128) // 512)
+    Estimates in us, fitted to 10464 timed calls over tiles (129 to 512 tokens of 1 to 64 deltas, sorted,
+    shuffled and in requests; K and N from 512 to 27648; 2 bits and 4) and within a fifth of 90 % of
+    them.  What they choose is 0.3 % slower in the mean than the faster route, where row blocks
+    throughout were 11 % slower and up to 4.3 times.  Chunks / row blocks, sorted, 2-bit:
+      5120 x 27648, 129 tokens of 4 / 16 / 64 deltas   251 / 307 / 557 against 138 / 376 / 1103 us
+                    256                                388 / 433 / 698 against 177 / 386 / 1224
+                    512                                769 / 798 / 1064 against 297 / 425 / 1356
+      4096 x 4096,  129 tokens of 1 / 4 / 16 deltas    47 / 47 / 54 against 57 / 39 / 44
+      13824 x 1024, 129 tokens of 1 / 4 / 16 deltas    48 / 49 / 53 against 173 / 119 / 110
+                    512                                119 / 123 / 127 against 178 / 176 / 108
+    Row blocks come in waves of 512 workgroups, two per CU: a single wave's time is that of its longest
+    block's walk, and of sharing a CU; several are bound by their products.  A chunk's launches take
+    the host 24 us."""
+    k, weight = K / 1024, K * N / 2**20
+    groups = mix.blocks * -(-N // 128)
+    waves, chunks, turns = -(-groups // 512), -(-T // MAX_TOKENS_FUSED), -(-T // 32)
     if waves == 1:
-        return T <= 160 and mix.longest > 64 and (N <= 4096 or (N <= 5120 and K >= 2 * N))
-    k, weight = K / 5120, K * N / 5120**2
-    chunks, turns = -(-T // MAX_TOKENS_FUSED), -(-T // 32)
-    per_block, per_turn, per_delta = (45.3, 0.65, 1.17) if bits == 2 else (57.8, 1.6, 1.93)
-    rows_us = k * waves * (per_block + 62 * T / (SHORT_ROWS * mix.blocks))
-    chunks_us = k * (11.5 * chunks + per_turn * turns) + weight * (7.2 * turns + per_delta * mix.met)
-    return chunks_us < rows_us
+        start, walk, full, shared = (7.2, 7.25, 5.85, 3.8) if bits == 2 else (6.7, 9.2, 5.4, 4.9)
+        rows_us = start + k * (walk + full * (min(mix.longest, SHORT_ROWS) / SHORT_ROWS)**2
+                               + shared * max(0, groups - 256) / 256)
+    else:
+        block, token = (9.4, 12.3) if bits == 2 else (11.9, 11.2)
+        rows_us = k * waves * (block + token * T / (SHORT_ROWS * mix.blocks))
+    launch, walk, turn, delta = (13.5, 0.12, 0.286, 0.0463) if bits == 2 else (13.0, 0.15, 0.288, 0.0812)
+    chunks_us = max(24 * chunks, chunks * (launch + walk * k) + weight * (turn * turns + delta * mix.met))
+    return chunks_us, rows_us
 
 
 def _one_wave_of_long_blocks(T: int, N: int, bits: int) -> bool:
@@ -699,17 +707,26 @@ def _check_tiled(base_tiled, base_weight, N: int, K: int, device) -> None:
 
 def takes_fused_chunks(T: int, S: int) -> bool:
     """Whether a batch above the fused kernel's 128 tokens may go through it in chunks of 128: sizes at
-    which that can be faster than row blocks (`_chunks_faster`; always where there are more than 768
+    which that can be faster than row blocks (`_route_us`; always where there are more than 768
     slots, which `segment` cannot order)."""
     return T <= 3 * MAX_TOKENS_FUSED or (T <= 4 * MAX_TOKENS_FUSED and S >= 16)
 
 
 def _goes_in_chunks(T: int, K: int, N: int, bits: int, S: int, blocks: Optional[RowBlocks]) -> bool:
-    """A caller's own row blocks without a mix are taken as they are."""
+    """The faster route by the mix of the batch.  Where only the device knows it, the route that loses
+    less between two mixes: all slots in use, which favours the chunks, and prompts of some 64 tokens,
+    which favours the row blocks (5120 x 27648, 2-bit, 129 tokens of 64 slots: 557 against 1103 us
+    and 251 against 135; 256 tokens of 32: 534 / 728 and 392 / 196).  A caller that has the ids on the
+    host says more with order=row_blocks(..., mix=batch_mix(ids)), or takes row blocks whatever the
+    batch without the mix."""
     if not takes_fused_chunks(T, S):
         return False
-    mix = _even_mix(T, S) if blocks is None else blocks.mix
-    return S > MAX_SLOTS_SEGMENT or (mix is not None and _chunks_faster(T, K, N, bits, mix))
+    if S > MAX_SLOTS_SEGMENT:
+        return True
+    if blocks is not None:
+        return blocks.mix is not None and lt(*_route_us(T, K, N, bits, blocks.mix))
+    many, few = (_route_us(T, K, N, bits, _even_mix(T, d)) for d in (S, min(S, 1 + T // 64)))
+    return many[0] * few[0] < many[1] * few[1]
 
 
 def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qweight_stacked,

@@ -797,8 +797,8 @@ def _batched_equal_separate(dev, bits, gs, t, ns, k, nd):
 
 
 @pytest.mark.parametrize("n,k,bits,gs,nd,t,present", [
-    (4096, 256, 2, -1, 24, 129, None), (4096, 256, 4, 128, 24, 130, None), (256, 256, 2, -1, 2, 140, None),   # chunks
-    (256, 512, 4, 64, 2, 150, 1), (4096, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None),             # row blocks
+    (256, 8192, 2, -1, 9, 129, None), (96, 8192, 4, 128, 3, 300, None), (128, 8192, 2, 64, 17, 256, None),   # chunks
+    (256, 512, 4, 64, 2, 150, 1), (2048, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None),            # row blocks
     (27648, 256, 2, -1, 1, 512, None), (27648, 256, 2, -1, 1, 449, None), (27648, 256, 2, -1, 3, 512, 1),     # 256-token blocks
     (27648, 256, 2, -1, 1, 512, 0)])
 def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
@@ -815,6 +815,7 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
     p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
     ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
     tiled = ops.tile_base(p["wb"])
+    assert ops._goes_in_chunks(t, k, n, bits, nd, None) == (k == 8192)
     known = ops.row_blocks(p["ids"], nd, mix=ops.batch_mix((p["ids_np"] + 1).tolist()))
     for order in (None, known, ops.row_blocks(p["ids"], nd)):
         for base in (None, tiled):

@@ -131,7 +131,7 @@ def test_row_blocks_stay_on_their_side_of_a_capture(monkeypatch):
 
 
 def test_batch_mix_counts_what_the_routes_meet():
-    ids = [0] * 3 + [-1] * 2 + [7] * 130 + [9] * 128 + [7] * 1                 # 264 tokens, three chunks
+    ids = [0] * 5 + [7] * 130 + [9] * 128 + [7] * 1                            # 264 tokens, three chunks
     assert ops.batch_mix(ids) == ops.BatchMix(3, 1 + 2 + 1, 131, 2 + 2 + 2)
     assert ops.batch_mix(tuple(reversed(ids))) == ops.BatchMix(3, 4, 131, 2 + 2 + 2)
     for t, s, want in ((129, 1, (1, 2, 129, 2)), (512, 16, (16, 16, 32, 19)), (300, 2, (2, 4, 150, 4)),
@@ -146,13 +146,28 @@ def test_batch_mix_counts_what_the_routes_meet():
     (5120, 5120, 2, 160, 32, 108, 140), (5120, 5120, 2, 320, 16, 151, 103), (13824, 5120, 2, 129, 1, 160, 184),
     (13824, 5120, 2, 192, 48, 324, 507), (4096, 4096, 2, 129, 1, 48, 58), (4096, 4096, 2, 129, 64, 86, 150),
     (4096, 4096, 2, 512, 48, 143, 119), (5120, 27648, 4, 192, 32, 596, 891), (5120, 27648, 4, 448, 8, 761, 337),
-    (4096, 12288, 4, 129, 24, 185, 242), (4096, 12288, 4, 384, 16, 267, 173)])
+    (4096, 12288, 4, 129, 24, 185, 242), (4096, 12288, 4, 384, 16, 267, 173),
+    # few features: the walk over K is one workgroup's, where a chunk splits it
+    (13824, 512, 2, 129, 1, 46, 172), (13824, 1024, 2, 512, 4, 123, 176), (13824, 2048, 2, 256, 4, 95, 151),
+    (13824, 2048, 2, 512, 16, 188, 131), (13824, 4096, 2, 384, 8, 240, 144), (8192, 1024, 4, 256, 1, 63, 137),
+    (4096, 1024, 2, 256, 16, 50, 34), (1024, 4096, 2, 129, 4, 45, 14), (512, 512, 4, 300, 2, 72, 12)])
 def test_the_faster_route_is_taken(k, n, bits, t, deltas, chunks, rows):
     """Measured times (us, sorted batches) of both routes on a few hundred tokens: the rule takes the
-    faster one wherever they differ by a tenth or more."""
+    faster one where it knows the mix."""
     ids = np.sort(np.random.RandomState(deltas + t).randint(1, deltas + 1, t)).tolist()
     for mix in (ops.batch_mix(ids), ops._even_mix(t, deltas)):
-        assert ops._chunks_faster(t, k, n, bits, mix) == (chunks < rows)
+        a, b = ops._route_us(t, k, n, bits, mix)
+        assert (a < b) == (chunks < rows)
+
+
+@pytest.mark.parametrize("k,n,t,slots,chunks", [(5120, 27648, 129, 64, True), (5120, 27648, 256, 32, False),
+                                                (5120, 27648, 129, 16, False), (13824, 1024, 256, 8, True),
+                                                (512, 512, 300, 2, False), (512, 512, 512, 1000, True),
+                                                (13824, 512, 400, 4, False), (13824, 512, 400, 16, True)])
+def test_route_of_a_batch_whose_mix_the_host_does_not_know(k, n, t, slots, chunks):
+    """Wide layers go in chunks only where their many slots could cost far more than a few prompts
+    would; narrow ones whatever the mix; above 384 tokens only with 16 slots or more."""
+    assert ops._goes_in_chunks(t, k, n, 2, slots, None) == chunks
 
 
 @pytest.mark.parametrize("n,bits,t,short,long", [
