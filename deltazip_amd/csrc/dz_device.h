@@ -104,6 +104,7 @@ struct MdlParams {
   int accumulate, ldy, nsplit, cb;
   int NP, NKB, NPG;
   int base_tiled;    // wb holds the base weight in tiles (dz_layout.h) instead of row-major [N, K]
+  const int* only_if;   // or nullptr; else the launch does nothing where it points to 0 (single calls only)
 };
 
 // Up to DZ_MAX_BATCH layer calls in one launch; np_end[j] = n-pairs of calls 0..j (entries beyond

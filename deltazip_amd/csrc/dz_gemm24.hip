@@ -472,10 +472,12 @@ __global__ __launch_bounds__(512, 2) void dz_gemm24_kernel(const Gemm24Params P)
 // second one where the first one's blocks would be less than three quarters full.  There the short
 // blocks' kernel is the faster one although it reads the weights more often (5120 x 27648, 2-bit,
 // 256 against 128 rows: 4096 tokens of 16 deltas, 65 % full: 2064 against 1837 us; 2000 tokens of 8,
-// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).
+// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).  With `over` the table is left empty
+// and *over is 1 where there are more than `limit` blocks (0 otherwise).
 __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S, int rows,
                                                               dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
-                                                              dz_gemm_tile* __restrict__ tiles2, int max_tiles2) {
+                                                              dz_gemm_tile* __restrict__ tiles2, int max_tiles2, int limit,
+                                                              int* __restrict__ over) {
   extern __shared__ int first[];    // first[k]: index of segment k's first block; first[S + 1]: total
   const int tid = threadIdx.x, nseg = S + 1;
   auto count = [&](int r) {
@@ -497,6 +499,14 @@ __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restr
     for (int b = tid; b < max_t; b += 1024) t[b] = dz_gemm_tile{0, 0, -1, 0};
   };
   count(rows);
+  if (over) {
+    const bool many = first[nseg] > limit;
+    if (tid == 0) *over = many;
+    if (many) {
+      empty(tiles, max_tiles);
+      return;
+    }
+  }
   if (!tiles2) {
     fill(tiles, max_tiles, rows);
     return;
@@ -516,11 +526,11 @@ __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restr
 }  // namespace
 
 static int build_tiles(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, int rows2,
-                       dz_gemm_tile* tiles2, int max_tiles2, void* stream) {
+                       dz_gemm_tile* tiles2, int max_tiles2, void* stream, int limit = 0, int32_t* over = nullptr) {
   if (!seg_off || !tiles) return DZ_EINVAL;
   if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || max_tiles < 1 || rows < 1) return DZ_ESHAPE;
   hipLaunchKernelGGL(dz_build_tiles_kernel, dim3(1), dim3(1024), (size_t)(S + 2) * 4, (hipStream_t)stream,
-                     seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2);
+                     seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2, limit, over);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
@@ -531,6 +541,13 @@ extern "C" int dz_build_tiles(const int32_t* seg_off, int S, dz_gemm_tile* tiles
 extern "C" int dz_build_tiles_rows(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles,
                                    void* stream) {
   return build_tiles(seg_off, S, rows, tiles, max_tiles, 0, nullptr, 0, stream);
+}
+
+extern "C" int dz_build_tiles_rows_upto(const int32_t* seg_off, int S, int rows, int limit, dz_gemm_tile* tiles,
+                                        int max_tiles, int32_t* over, void* stream) {
+  if (!over) return DZ_EINVAL;
+  if (limit < 0 || max_tiles < limit) return DZ_ESHAPE;
+  return build_tiles(seg_off, S, rows, tiles, max_tiles, 0, nullptr, 0, stream, limit, over);
 }
 
 extern "C" int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles,

@@ -915,7 +915,8 @@ static int multi_delta_linear_batch(int ncalls, const uint16_t* const* x, const 
                                     const void* const* scales_stacked, const int64_t* indices,
                                     uint16_t* const* y, const int* N, const int* ldy, int T, int K, int S,
                                     int bits, int group_size, int accumulate, const int32_t* order,
-                                    void* workspace, size_t workspace_bytes, void* stream, int base_tiled) {
+                                    void* workspace, size_t workspace_bytes, void* stream, int base_tiled,
+                                    const int32_t* only_if = nullptr) {
   if (ncalls < 1 || ncalls > DZ_MAX_BATCH_CALLS) return DZ_ESHAPE;
   if (!x || !w_base || !indices || !y || !N || !ldy) return DZ_EINVAL;
   if (S > 0 && (!codes_stacked || !meta_stacked || !scales_stacked)) return DZ_EINVAL;
@@ -967,6 +968,7 @@ static int multi_delta_linear_batch(int ncalls, const uint16_t* const* x, const 
     Q.NP = N[j] / DZ_NPAIR; Q.NKB = K / DZ_KBLOCK;
     Q.nsplit = 1; Q.cb = Q.NKB; Q.NPG = 0;
     Q.base_tiled = (base_tiled && w_base[j]) ? 1 : 0;
+    Q.only_if = only_if;
     Q.perm = T <= 32 ? nullptr : (order ? order : perm);
     Q.tok0 = 0;
     Q.nchunk = 1;
@@ -1000,6 +1002,25 @@ int dz_multi_delta_linear_batch_tiled(int ncalls, const uint16_t* const* x, cons
   return multi_delta_linear_batch(ncalls, x, w_base_tiled, codes_stacked, meta_stacked, scales_stacked, indices, y, N,
                                   ldy, T, K, S, bits, group_size, accumulate, order, workspace, workspace_bytes,
                                   stream, 1);
+}
+
+int dz_multi_delta_linear_chunks(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                                 const void* meta_stacked, const void* scales_stacked, const int64_t* indices,
+                                 uint16_t* y, int T, int K, int N, int S, int bits, int group_size, int accumulate,
+                                 int ldy, const int32_t* only_if, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!x || !indices || !y) return DZ_EINVAL;
+  if (T < 1) return DZ_ESHAPE;
+  // (a first chunk that fails its checks has launched nothing; the others differ in T alone)
+  for (int t0 = 0; t0 < T; t0 += DZ_MAX_TOKENS_FUSED) {
+    const uint16_t* xc = x + (size_t)t0 * K;
+    uint16_t* yc = y + (size_t)t0 * ldy;
+    const int t = T - t0 < DZ_MAX_TOKENS_FUSED ? T - t0 : DZ_MAX_TOKENS_FUSED;
+    const int rc = multi_delta_linear_batch(1, &xc, &w_base, &codes_stacked, &meta_stacked, &scales_stacked, indices + t0,
+                                            &yc, &N, &ldy, t, K, S, bits, group_size, accumulate, nullptr, workspace,
+                                            workspace_bytes, stream, w_tiled, only_if);
+    if (rc) return rc;
+  }
+  return DZ_OK;
 }
 
 int dz_tile_base(const uint16_t* w, int K, int N, uint16_t* out, void* stream) {

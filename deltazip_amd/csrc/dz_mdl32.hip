@@ -587,7 +587,7 @@ __global__ __launch_bounds__(64 * WK32, 2) void dz_mdl32_kernel(const MdlParams 
   const int xcd = blockIdx.x & 7, q = blockIdx.x >> 3;
   const int per = P.nsplit * P.nchunk, rem = q % per;
   const int np = (q / per) * 8 + xcd, kc = rem / P.nchunk, ch = rem % P.nchunk;
-  if (np >= P.NP) return;
+  if (np >= P.NP || (P.only_if && *P.only_if == 0)) return;
   mdl32_body<BITS, TT, PRE, BASE, EARLY, true>(P, np, kc, ch, smem);
 }
 

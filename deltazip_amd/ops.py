@@ -233,8 +233,8 @@ def _route_us(T: int, K: int, N: int, bits: int, mix: BatchMix) -> Tuple[float, 
         rows_us = start + k * (walk + full * (min(mix.longest, SHORT_ROWS) / SHORT_ROWS)**2
                                + shared * max(0, groups - 256) / 256)
     else:
-        block, token = (9.4, 12.3) if bits == 2 else (11.9, 11.2)
-        rows_us = k * waves * (block + token * T / (SHORT_ROWS * mix.blocks))
+        start, walk, token = (3.4, 8.5, 12.0) if bits == 2 else (3.2, 11.0, 11.1)
+        rows_us = waves * (start + k * (walk + token * T / (SHORT_ROWS * mix.blocks)))
     launch, walk, turn, delta = (13.5, 0.12, 0.286, 0.0463) if bits == 2 else (13.0, 0.15, 0.288, 0.0812)
     chunks_us = max(24 * chunks, chunks * (launch + walk * k) + weight * (turn * turns + delta * mix.met))
     return chunks_us, rows_us
@@ -712,21 +712,39 @@ def takes_fused_chunks(T: int, S: int) -> bool:
     return T <= 3 * MAX_TOKENS_FUSED or (T <= 4 * MAX_TOKENS_FUSED and S >= 16)
 
 
-def _goes_in_chunks(T: int, K: int, N: int, bits: int, S: int, blocks: Optional[RowBlocks]) -> bool:
-    """The faster route by the mix of the batch.  Where only the device knows it, the route that loses
-    less between two mixes: all slots in use, which favours the chunks, and prompts of some 64 tokens,
-    which favours the row blocks (5120 x 27648, 2-bit, 129 tokens of 64 slots: 557 against 1103 us
-    and 251 against 135; 256 tokens of 32: 534 / 728 and 392 / 196).  A caller that has the ids on the
-    host says more with order=row_blocks(..., mix=batch_mix(ids)), or takes row blocks whatever the
-    batch without the mix."""
+@lru_cache(maxsize=4096)
+def _most_blocks_unknown(T: int, K: int, N: int, bits: int, S: int) -> Optional[int]:
+    """`_most_row_blocks` where only the device knows the mix.  Over wide layers all slots in use favour
+    the chunks, a few prompts of some 64 tokens the row blocks (5120 x 27648, 2-bit, 129 tokens of 64 slots: 557
+    against 1103 us and 251 against 135; 256 tokens of 32: 534 / 728 and 392 / 196).  Where that differs, and
+    by more than the 8 to 15 us that launching both costs, the device takes the row blocks up to the
+    number with which they are the faster route; it does not look at their lengths, so they count as
+    full.  Otherwise the route that loses less between the two."""
+    def costs(deltas, longest=None):
+        mix = _even_mix(T, deltas)
+        return _route_us(T, K, N, bits, mix if longest is None else mix._replace(longest=longest, blocks=deltas))
+    many, few = costs(S), costs(min(S, 1 + T // 64), SHORT_ROWS)
+    if few[0] < few[1] or many[1] - many[0] < 30:
+        return 0 if many[0] * few[0] < many[1] * few[1] else None
+    lo, hi = -(-T // SHORT_ROWS), min(S, T)
+    while lo < hi:
+        mid = (lo + hi + 1) // 2
+        chunks, rows = costs(mid, SHORT_ROWS)
+        lo, hi = (mid, hi) if rows <= chunks else (lo, mid - 1)
+    return lo
+
+
+def _most_row_blocks(T: int, K: int, N: int, bits: int, S: int, blocks: Optional[RowBlocks]) -> Optional[int]:
+    """The faster route: None stands for row blocks, 0 for chunks, a number for the row blocks if there
+    are no more of them, by the device's count.  A caller that has the ids on the host says so with
+    order=row_blocks(..., mix=batch_mix(ids)); its row blocks without a mix are taken as they are."""
     if not takes_fused_chunks(T, S):
-        return False
+        return None
     if S > MAX_SLOTS_SEGMENT:
-        return True
+        return 0
     if blocks is not None:
-        return blocks.mix is not None and lt(*_route_us(T, K, N, bits, blocks.mix))
-    many, few = (_route_us(T, K, N, bits, _even_mix(T, d)) for d in (S, min(S, 1 + T // 64)))
-    return many[0] * few[0] < many[1] * few[1]
+        return 0 if blocks.mix is not None and lt(*_route_us(T, K, N, bits, blocks.mix)) else None
+    return _most_blocks_unknown(T, K, N, bits, S)
 
 
 def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qweight_stacked,
@@ -782,11 +800,25 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
     ldy = out.stride(0)
     if T > MAX_TOKENS_FUSED:
         blocks = _usable_blocks(order, T, S)
-        if _goes_in_chunks(T, K, N, bits, S, blocks):
-            for r in range(0, T, MAX_TOKENS_FUSED):
-                multi_delta_linear(x2[r:r + MAX_TOKENS_FUSED], base_weight, qweight_stacked, scales_stacked,
-                                   meta_stacked, indices[r:r + MAX_TOKENS_FUSED], bits=bits,
-                                   out=out[r:r + MAX_TOKENS_FUSED], accumulate=accumulate, base_tiled=base_tiled)
+        most = _most_row_blocks(T, K, N, bits, S, blocks)
+        if most is not None:
+            ws = _workspace(x.device, MAX_TOKENS_FUSED, K, N)
+            w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
+            delta = (qweight_stacked.data_ptr(), meta_stacked.data_ptr(), scales_stacked.data_ptr())
+            shape = (T, K, N, 1 if accumulate else 0, ldy)
+            wptr, over, L, st = w.data_ptr() if w is not None else None, None, _lib.lib(), _stream()
+            if most:                                  # the row blocks if there are few, else the chunks
+                perm, seg_off = segment(indices, S, True)
+                table = torch.empty(4 * most + 1, dtype=torch.int32, device=x.device)
+                over = table[4 * most:].data_ptr()
+                _lib.check(L.dz_build_tiles_rows_upto(seg_off.data_ptr(), S, SHORT_ROWS, most, table.data_ptr(), most,
+                                                      over, st), "dz_build_tiles_rows_upto")
+                _lib.check(L.dz_multi_delta_gemm_rows(x2.data_ptr(), wptr, tiled, *delta, S, bits, group_size,
+                                                      table.data_ptr(), most, perm.data_ptr(), out.data_ptr(), *shape, st),
+                           "dz_multi_delta_gemm_rows")
+            _lib.check(L.dz_multi_delta_linear_chunks(x2.data_ptr(), wptr, tiled, *delta, indices.data_ptr(),
+                                                      out.data_ptr(), T, K, N, S, bits, group_size, *shape[3:], over,
+                                                      ws.data_ptr(), ws.numel(), st), "dz_multi_delta_linear_chunks")
             return out
         from .prefill import multi_delta_linear_prefill
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
@@ -874,7 +906,7 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
         blocks = order if isinstance(order, RowBlocks) else None
         # row blocks made once serve the projections that would make the same ones
         shared = [q.shape[0] == S and (blocks is not None or (
-                      not _goes_in_chunks(T, K, w.shape[0], bits, S, None)
+                      _most_row_blocks(T, K, w.shape[0], bits, S, None) is None
                       and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \

@@ -274,6 +274,14 @@ int dz_multi_delta_linear_batch_tiled(int ncalls, const uint16_t* const* x,
                                       const int32_t* order, void* workspace, size_t workspace_bytes,
                                       void* stream);
 
+/* dz_multi_delta_linear for any T >= 1, DZ_MAX_TOKENS_FUSED tokens at a time (workspace as for that many).
+ * w_base is row-major [N, K] (w_tiled = 0), the tiles dz_tile_base writes (w_tiled != 0), or NULL.
+ * only_if: NULL, or device memory read when the kernels run: 0 there leaves y as it is. */
+int dz_multi_delta_linear_chunks(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                                 const void* meta_stacked, const void* scales_stacked, const int64_t* indices,
+                                 uint16_t* y, int T, int K, int N, int S, int bits, int group_size, int accumulate,
+                                 int ldy, const int32_t* only_if, void* workspace, size_t workspace_bytes, void* stream);
+
 /* The order in which the fused kernel takes the tokens of a batch of up to DZ_MAX_TOKENS_FUSED
  * tokens, 32 per chunk: order[T], a permutation of 0..T-1 in which the tokens of one delta stay
  * together and every chunk of 32 meets about the same number of distinct deltas.  Depends on the
@@ -342,6 +350,12 @@ int dz_build_tiles(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_t
 /* dz_build_tiles with blocks of at most `rows` rows: max_tiles >= (T + rows - 1) / rows +
  * min(S + 1, T) always suffices. */
 int dz_build_tiles_rows(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, void* stream);
+
+/* dz_build_tiles_rows that leaves the table empty and sets *over (device memory) to 1 where there are
+ * more than `limit` blocks, and to 0 otherwise: with dz_multi_delta_linear_chunks(only_if = over) the
+ * device chooses between two ways of one call.  max_tiles >= limit. */
+int dz_build_tiles_rows_upto(const int32_t* seg_off, int S, int rows, int limit, dz_gemm_tile* tiles, int max_tiles,
+                             int32_t* over, void* stream);
 
 /* Both tables at once: on the device, all rows go either into blocks of at most 256 (`tiles`, for
  * dz_multi_delta_gemm) or into blocks of at most DZ_SHORT_ROWS (`short_tiles`, for

@@ -77,6 +77,14 @@ def test_argument_checks_happen_on_the_host(dzlib):
     assert gt(one, None, one, one, one, 2, 4, -1, one, 4, None, one, 300, 512, 64, 0, 64, None) == -1
     assert gt(one, one, one, one, one, 2, 3, -1, one, 4, None, one, 300, 512, 64, 0, 64, None) == -3
     assert gt(one, one, one, one, one, 2, 4, -1, one, 4, None, one, 300, 500, 64, 0, 64, None) == -2
+    # chunks of any length, and the choice made on the device
+    ck = lambda x=one, w=one, T=300, ldy=64, ws=one, wsb=1 << 30: dzlib.dz_multi_delta_linear_chunks(
+        x, w, 1, one, one, one, one, one, T, 512, 64, 2, 4, -1, 0, ldy, None, ws, wsb, None)
+    assert ck(x=None) == -1 and ck(T=0) == -2 and ck(ldy=32) == -2 and ck(wsb=16) == -8
+    assert ck(x=C.c_void_p(0x1004)) == -10 and ck(w=C.c_void_p(0x1004)) == -10
+    up = dzlib.dz_build_tiles_rows_upto
+    assert up(one, 2, 128, 4, one, 4, None, None) == -1 and up(None, 2, 128, 4, one, 4, one, None) == -1
+    assert up(one, 2, 128, 4, one, 3, one, None) == -2 and up(one, 2, 128, -1, one, 3, one, None) == -2
     # the read-only yardstick validates like the launch it stands beside
     arr = lambda v: (C.c_void_p * 1)(v)
     pr = dzlib.dz_probe_read

@@ -815,7 +815,7 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
     p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
     ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
     tiled = ops.tile_base(p["wb"])
-    assert ops._goes_in_chunks(t, k, n, bits, nd, None) == (k == 8192)
+    assert (ops._most_row_blocks(t, k, n, bits, nd, None) == 0) == (k == 8192)
     known = ops.row_blocks(p["ids"], nd, mix=ops.batch_mix((p["ids_np"] + 1).tolist()))
     for order in (None, known, ops.row_blocks(p["ids"], nd)):
         for base in (None, tiled):
@@ -824,6 +824,33 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
             assert o.rel_err(y.cpu().numpy(), ref) <= TOL
     for y in ops.apply_delta_batch(p["x"], [p["q"]] * 2, [p["s"]] * 2, [p["m"]] * 2, p["ids"], [p["wb"]] * 2):
         assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+
+
+@pytest.mark.parametrize("n,k,bits,gs,t", [(96, 512, 2, -1, 200), (160, 1024, 4, 128, 129), (32, 256, 2, 64, 384)])
+@pytest.mark.parametrize("spare", [0, 3, -1])
+def test_device_chooses_between_row_blocks_and_chunks(dev, monkeypatch, n, k, bits, gs, t, spare):
+    """One launch of each is made and one of them does nothing, by the number of row blocks: exactly as many
+    as the limit, fewer, and one more (`spare`: the limit over the number); every token is written once."""
+    p = make_problem(n, k, bits, gs, 6, t, "uniform", 40 + n + t, dev)
+    p["ids_np"][::9] = -1
+    p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
+    limit = ops.batch_mix((p["ids_np"] + 1).tolist()).blocks + spare
+    called = []
+    monkeypatch.setattr(ops, "_most_row_blocks", lambda *a: called.append(a) or limit)
+    base = o.make_x(t, n, 5)
+    for w, tiled in ((p["wb"], None), (p["wb"], ops.tile_base(p["wb"])), (None, None)):
+        ref = o.forward_ref(p["x_np"], None if w is None else p["wb_np"], p["dts"], p["ids_np"])
+        for accumulate in (False, True):
+            wide = torch.zeros(t, n + 32, dtype=torch.float16, device=dev)
+            y = wide[:, 16:16 + n]
+            y.copy_(torch.from_numpy(base) if accumulate else torch.full((t, n), float("nan")))
+            ops.multi_delta_linear(p["x"], w, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y, accumulate=accumulate,
+                                   base_tiled=tiled)
+            torch.cuda.synchronize()
+            want = ref + (base.astype(np.float32) if accumulate else 0)
+            assert o.rel_err(y.float().cpu().numpy(), want) <= TOL
+            assert not wide[:, :16].any() and not wide[:, 16 + n:].any()
+    assert len(called) == 6
 
 
 @pytest.mark.parametrize("t", [200, 700])
