@@ -363,12 +363,17 @@ def apply_delta_uncompressed(x: torch.Tensor, delta_weights: torch.Tensor, indic
     # 691), unless there are too few of them to fill the GPU (4096 x 1024: 46 against 32).
     short = K % 256 == 0 and N % 32 == 0 and (
         T <= 600 or (T <= 1024 and ((N + 255) // 256) * ((T + 255) // 256) <= 64))
-    blocks = row_blocks(indices, S, long_only=not short)
-    tiles, ntiles = (blocks.short, blocks.max_short) if short else (blocks.tiles, blocks.max_tiles)
+    indices = indices.reshape(-1)
+    if not indices.is_contiguous():
+        raise ValueError("indices must be contiguous")
+    L, st, rows = _lib.lib(), _stream(), SHORT_ROWS if short else 256
+    perm, seg_off = segment(indices, S)               # (ids without a table take the base table, unreported)
+    tiles, ntiles = _block_table(T, S, rows, x.device)
+    _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), S, rows, tiles.data_ptr(), ntiles, st), "dz_build_tiles_rows")
     out = torch.empty((T, N), dtype=torch.float16, device=x.device)
-    fn = _lib.lib().dz_gemm_f16_select_rows if short else _lib.lib().dz_gemm_f16_select
+    fn = L.dz_gemm_f16_select_rows if short else L.dz_gemm_f16_select
     _lib.check(fn(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K, tiles.data_ptr(), ntiles,
-                  blocks.perm.data_ptr(), out.data_ptr(), T, K, N, 0, N, _stream()), "dz_gemm_f16_select")
+                  perm.data_ptr(), out.data_ptr(), T, K, N, 0, N, st), "dz_gemm_f16_select")
     return out
 
 

@@ -377,6 +377,20 @@ def test_bad_ids_of_mid_size_batches_are_reported(dev):
     assert ops.workspace_status() == 0
 
 
+def test_output_projection_does_not_report_ids(dev):
+    """apply_delta_uncompressed serves an id without a table from the base table and leaves the fused
+    kernel's status word alone, at every size."""
+    stack, base = torch.randn(2, 64, 256, device=dev).half(), torch.randn(64, 256, device=dev).half()
+    ops.poll_status(wait=True)
+    for t in (40, 200, 700):
+        x = torch.randn(t, 256, device=dev).half()
+        ids = torch.arange(t, device=dev) % 4 - 1          # 2 has no table
+        y = ops.apply_delta_uncompressed(x, stack, ids, base)
+        assert torch.equal(y, ops.apply_delta_uncompressed(x, stack, torch.where(ids == 2, -1, ids), base))
+        torch.cuda.synchronize()
+        assert ops.workspace_status() == 0, t
+
+
 @pytest.mark.parametrize("n,k,s,t", [(32, 256, 3, 1), (96, 512, 8, 33), (160, 768, 2, 128), (4128, 256, 5, 129),
                                      (288, 1024, 1, 300), (64, 512, 20, 1024)])
 def test_select_over_short_blocks(dev, n, k, s, t):
