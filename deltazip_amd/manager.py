@@ -205,6 +205,7 @@ class DeltaModelManager:
                                               {"embed_tokens": "input_embeddings", "lm_head": "output_embeddings"}))
         self.packed_modules: Dict[str, List[str]] = {}
         self.modules: Dict[str, BaseLayerWithDelta] = {}
+        self._widest = 0                 # output features of the widest linear layer
         self._last_mapping: Optional[DeltaMapping] = None
         self._wrap_modules()
         self.model.delta_manager = self
@@ -362,7 +363,8 @@ class DeltaModelManager:
         if T > ops.MAX_TOKENS_FUSED and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
             # (the mix decides at sizes where other routes than row blocks may be the faster one)
             self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
-                                                mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None)
+                                                mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
+                                                features=self._widest or None)
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 
@@ -423,6 +425,8 @@ class DeltaModelManager:
         if not isinstance(module, BaseLayerWithDelta):
             raise TypeError("only delta-carrying layers are registered")
         self.modules[module_name] = module
+        if isinstance(module, LinearWithDelta):
+            self._widest = max(self._widest, getattr(module, "base_shape", (0, 0))[0])
         # a fused layer also answers for the projections it is made of (q/k/v, gate/up)
         parent, _, leaf = module_name.rpartition(".")
         parts = self.packed_modules_mapping.get(leaf)

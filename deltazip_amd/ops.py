@@ -268,7 +268,7 @@ def _block_table(T: int, num_slots: int, rows: int, device):
 
 
 def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
-               device_picks: bool = False) -> RowBlocks:
+               device_picks: bool = False, features: Optional[int] = None) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
     (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
@@ -283,10 +283,14 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
       per slot and more   or fewer the larger tile is the faster one at 2 bits (5120 x 27648: 3113
                           against 3499; 4096 x 12288: 1133 against 1243; 4 bits: equal)
       between             the number of deltas in the batch is known on the device only: it picks
-                          (dz_build_tiles_either), and both products are launched, one of them empty
+                          (dz_build_tiles_either), and both products are launched, one of them empty --
+                          but for layers so narrow that long blocks would fill at most half the GPU,
+                          where short ones win and a second launch is felt (512 x 2048, 1500 tokens
+                          of 12 slots: 57 against 50 us)
     `long_only`: the table of 256-token blocks alone, whatever the batch.  `mix`: batch_mix() of the
     same ids, if the host has them: calls of a few hundred tokens then choose between these blocks and
-    chunks of the fused kernel by it.  `device_picks`: as between, whatever the batch."""
+    chunks of the fused kernel by it.  `device_picks`: as between, whatever the batch.  `features`: of the
+    widest layer they are for, if known."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
@@ -294,7 +298,8 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
     perm, seg_off = segment(indices, num_slots, not long_only and T > MAX_TOKENS_FUSED and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
-    small = not long_only and not device_picks and T <= 1024
+    narrow = features is not None and -(-features // 256) * -(-T // 256) <= 128 and T < 256 * (num_slots + 1)
+    small = not long_only and not device_picks and (T <= 1024 or narrow)
     tiles, n, short, ns = None, 0, None, 0
     host_picks = small and mix is not None and mix.deltas == 1 and 448 < T <= 512
     if not small or host_picks:
@@ -916,7 +921,7 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
-            blocks = row_blocks(indices, S)
+            blocks = row_blocks(indices, S, features=max(w.shape[0] for w in base_weight))
         if blocks is not None and (blocks.T != T or blocks.S != S):
             blocks = None
         return [apply_delta(xs[j], qweight_stacked[j], scales_stacked[j], meta_stacked[j], indices, base_weight[j],

@@ -840,6 +840,40 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
         assert o.rel_err(y.cpu().numpy(), ref) <= TOL
 
 
+@pytest.mark.parametrize("n,k,bits,gs", [(352, 512, 2, -1), (96, 768, 4, 128)])
+@pytest.mark.parametrize("t,nd,long", [(1025, 7, False), (1300, 16, False), (1025, 6, True), (1300, 5, True)])
+def test_either_table_above_1024_tokens(dev, n, k, bits, gs, t, nd, long):
+    """The device puts all rows into long or into short blocks and both products are launched, one over an
+    empty table (`long`: ids that fill long blocks); a call that knows how narrow its layer is launches
+    the short blocks alone.  Tiles, rows and no base weight, plain and added into a column slice."""
+    p = make_problem(n, k, bits, gs, nd, t, "uniform", 17 * t + nd, dev)
+    if long:                                              # two deltas of 256 * m tokens, the rest with another
+        p["ids_np"] = np.where(np.arange(t) < 256, 1, np.where(np.arange(t) < 768, 4, 0))
+    p["ids_np"] = np.random.default_rng(t).permutation(p["ids_np"])
+    p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
+    either = ops.row_blocks(p["ids"], nd)
+    torch.cuda.synchronize()
+    used = [bool((tab[:, 1] > tab[:, 0]).any()) for tab in (either.tiles, either.short)]
+    assert used == [long, not long]
+    narrow = ops.row_blocks(p["ids"], nd, features=n)
+    assert narrow.tiles is None and narrow.short is not None
+    assert ops.row_blocks(p["ids"], nd, features=1 << 16).tiles is not None
+    base = o.make_x(t, n, 5)
+    for w, tiled in ((p["wb"], None), (None, ops.tile_base(p["wb"])), (None, None)):
+        ref = o.forward_ref(p["x_np"], None if w is None and tiled is None else p["wb_np"], p["dts"], p["ids_np"])
+        for order in (either, narrow, None):
+            for accumulate in (False, True):
+                wide = torch.zeros(t, n + 32, dtype=torch.float16, device=dev)
+                y = wide[:, 16:16 + n]
+                y.copy_(torch.from_numpy(base) if accumulate else torch.full((t, n), float("nan")))
+                ops.multi_delta_linear(p["x"], w, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y,
+                                       accumulate=accumulate, order=order, base_tiled=tiled)
+                torch.cuda.synchronize()
+                want = ref + (base.astype(np.float32) if accumulate else 0)
+                assert o.rel_err(y.float().cpu().numpy(), want) <= TOL
+                assert not wide[:, :16].any() and not wide[:, 16 + n:].any()
+
+
 @pytest.mark.parametrize("n,k,bits,gs,t", [(96, 512, 2, -1, 200), (160, 1024, 4, 128, 129), (32, 256, 2, 64, 384)])
 @pytest.mark.parametrize("spare", [0, 3, -1])
 def test_device_chooses_between_row_blocks_and_chunks(dev, monkeypatch, n, k, bits, gs, t, spare):
