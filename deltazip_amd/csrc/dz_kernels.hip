@@ -383,7 +383,7 @@ __global__ __launch_bounds__(64) void dz_scales_mse_kernel(const float* __restri
   }
 }
 
-// One wavefront per (n-pair, k-block) tile; the words of lane 16*ga + i of the native arrays hold
+// One workgroup per (n-pair, k-block) tile; the words of lane 16*ga + i of the native arrays hold
 // rows i and 16 + i, columns 64*j + 16*ga .. + 15 of the k-block (word j).
 //   pruning   in every aligned group of 4 columns the 2 values of largest magnitude stay (ties:
 //             the lower column), the others become 0 -- deltazip/core/sparsegpt.py:123-135 with an
@@ -391,8 +391,11 @@ __global__ __launch_bounds__(64) void dz_scales_mse_kernel(const float* __restri
 //   codes     q = clamp(rint(x / scale) + zero, 0, maxq), fp32, zero = 2^(bits-1) -- quant.py:9-18
 //   positions the columns whose code differs from the zero-point, completed with the lowest
 //             remaining columns: what the repacker stores for the same codes
-// Bound by memory at 2 bits (4096 x 11008 packed in 41 us, 4.9 TB/s, from 85; compressed, the pass for
-// the scales included, in 70 us from 113) and by its arithmetic where the scales are found here too.
+// Bound by memory (4096 x 11008, per channel, the pass for the scales included: 96 us with a lane reading
+// its own 64 bytes of a row, 64 with the reads below and one wavefront per tile, 60 now), and at a few
+// hundred tiles by the chain of one wavefront's rows: with all 32 rows in one, 768 x 640 in groups of 128
+// took 33 us, where the separate passes for scales and codes before it took 21; four wavefronts of
+// 8 rows 17.
 //
 // The work of a group of four: six comparisons (a value stays if at least two of its three
 // comparisons go its way), four quotients as products with 1 / scale, and two table lookups on
@@ -497,9 +500,11 @@ __device__ __forceinline__ uint32_t or_quad(uint32_t v) {
 //
 // GS = 0: scales from memory.  GS = 64, 128, 256: the tile holds whole scale groups, so their scales are
 // found here from the values just read (and written out) rather than in a pass of their own
-// (4096 x 11008, 4-bit, groups of 128: 104 -> 90 us, of 64 107 -> 88).
+// (4096 x 11008, 4-bit, groups of 128: 90 us with one wavefront per tile, now 75, of 64 88 and 74).
+constexpr int COMPRESS_WAVES = 4;   // per tile: rows 4w .. 4w + 3 and 16 + 4w .. of wavefront w
+
 template <int BITS, int GS>
-__global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict__ delta,
+__global__ __launch_bounds__(64 * COMPRESS_WAVES) void dz_compress_kernel(const float* __restrict__ delta,
                                                          float* __restrict__ scale32, _Float16* __restrict__ scale16,
                                                          int K, int N, int gs, uint32_t* __restrict__ codes,
                                                          uint32_t* __restrict__ meta) {
@@ -509,10 +514,10 @@ __global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict
   __shared__ float2 sct[DZ_NPAIR * 4];             // (scale, 1 / scale or NaN) of (row, step)
   const int nkb = K / DZ_KBLOCK;
   const int np = blockIdx.x / nkb, kb = blockIdx.x % nkb;
-  const int lane = threadIdx.x, j = lane >> 4, ga = (lane >> 2) & 3, p = lane & 3;
-#pragma unroll
-  for (int h = 0; h < (GS ? 0 : 2); ++h) {
-    const int at = h * 64 + lane, row = at & 31, step = at >> 5;      // (a scale group spans whole steps)
+  const int tid = threadIdx.x, lane = tid & 63, j = lane >> 4, ga = (lane >> 2) & 3, p = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  if (GS == 0 && tid < 4 * DZ_NPAIR) {
+    const int row = tid & 31, step = tid >> 5;      // (a scale group spans whole steps)
     const float sc = scale32[(size_t)((kb * DZ_KBLOCK + step * 64) / gs) * N + np * DZ_NPAIR + row];
     sct[step * DZ_NPAIR + row] = make_float2(sc, sc >= 0x1p-100f && sc <= 0x1p100f ? 1.f / sc : __builtin_nanf(""));
   }
@@ -520,8 +525,8 @@ __global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict
   // lane p of four stores the positions (0), the codes (1), or the codes of row 16 + i at 4 bits (2)
   const int hold = p == 0 ? j : BITS == 2 ? 256 + j : 256 + (j >> 1) * 256 + 2 * (j & 1) + (p - 1);
   __syncthreads();
-#pragma unroll
-  for (int i0 = 0; i0 < 16; i0 += 4) {
+  {
+    const int i0 = 4 * wave;
     f4_t v[2][4];
 #pragma unroll
     for (int u = 0; u < 4; ++u)
@@ -562,18 +567,18 @@ __global__ __launch_bounds__(64) void dz_compress_kernel(const float* __restrict
   __syncthreads();
   if constexpr (GS != 0) {
     constexpr int NG = DZ_KBLOCK / (GS ? GS : 1);
-#pragma unroll
-    for (int at = lane; at < NG * DZ_NPAIR; at += 64) {
-      const size_t o = (size_t)(kb * NG + at / DZ_NPAIR) * N + np * DZ_NPAIR + (at & 31);
-      scale32[o] = sct[at].x;
-      scale16[o] = (_Float16)sct[at].x;
+    if (tid < NG * DZ_NPAIR) {
+      const size_t o = (size_t)(kb * NG + tid / DZ_NPAIR) * N + np * DZ_NPAIR + (tid & 31);
+      scale32[o] = sct[tid].x;
+      scale16[o] = (_Float16)sct[tid].x;
     }
   }
-  *(u4_t*)(meta + dz_meta_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + lane * 4);
+  if (wave == 3) *(u4_t*)(meta + dz_meta_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + lane * 4);
   if (BITS == 2) {
-    *(u4_t*)(codes + dz_code2_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
-  } else {
+    if (wave == 2) *(u4_t*)(codes + dz_code2_word(np, kb, lane, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
+  } else if (wave == 2) {
     *(u4_t*)(codes + dz_code4_word(np, kb, lane, 0, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
+  } else if (wave == 1) {
     *(u4_t*)(codes + dz_code4_word(np, kb, lane, 2, 0, nkb)) = *(const u4_t*)(words + (BITS == 2 ? 256 : 512) + lane * 4);
   }
 }
@@ -841,7 +846,7 @@ int dz_compress_2of4(const float* delta, int K, int N, int bits, int group_size,
   hipStream_t st = (hipStream_t)stream;
   const unsigned tiles = (unsigned)(N / DZ_NPAIR) * (K / DZ_KBLOCK);
   auto go = [&](auto kern) {
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64), 0, st, delta, scale_workspace, (_Float16*)out_scales, K, N, gs,
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64 * COMPRESS_WAVES), 0, st, delta, scale_workspace, (_Float16*)out_scales, K, N, gs,
                        (uint32_t*)out_codes, (uint32_t*)out_meta);
   };
   switch (gs) {
@@ -894,7 +899,7 @@ int dz_pack_2of4(const float* w, const float* scale32, int K, int N, int bits, i
   const unsigned tiles = (unsigned)(N / DZ_NPAIR) * (K / DZ_KBLOCK);
   hipStream_t st = (hipStream_t)stream;
   auto go = [&](auto kern) {                       // (scales are read only)
-    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64), 0, st, w, const_cast<float*>(scale32), (_Float16*)nullptr, K, N, gs,
+    hipLaunchKernelGGL(kern, dim3(tiles), dim3(64 * COMPRESS_WAVES), 0, st, w, const_cast<float*>(scale32), (_Float16*)nullptr, K, N, gs,
                        (uint32_t*)out_codes, (uint32_t*)out_meta);
   };
   bits == 2 ? go(dz_compress_kernel<2, 0>) : go(dz_compress_kernel<4, 0>);
