@@ -27,6 +27,7 @@ SIGNATURES = {
     "dz_embedding_select": (_i, [_vp, _vp, _vp, _vp, C.c_longlong, _i, _vp, _i, _i, _i, _i, _vp]),
     "dz_build_tiles": (_i, [_vp, _i, _vp, _i, _vp]),
     "dz_build_tiles_either": (_i, [_vp, _i, _vp, _i, _vp, _i, _vp]),
+    "dz_build_tiles_either_for": (_i, [_vp, _i, _i, _vp, _i, _vp, _i, _vp]),
     "dz_build_tiles_rows_upto": (_i, [_vp, _i, _i, _i, _vp, _i, _vp, _vp]),
     "dz_multi_delta_linear_chunks": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _vp,
                                           C.c_size_t, _vp]),

@@ -472,12 +472,14 @@ __global__ __launch_bounds__(512, 2) void dz_gemm24_kernel(const Gemm24Params P)
 // second one where the first one's blocks would be less than three quarters full.  There the short
 // blocks' kernel is the faster one although it reads the weights more often (5120 x 27648, 2-bit,
 // 256 against 128 rows: 4096 tokens of 16 deltas, 65 % full: 2064 against 1837 us; 2000 tokens of 8,
-// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).  With `over` the table is left empty
-// and *over is 1 where there are more than `limit` blocks (0 otherwise).
+// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).  With `features` the first one gets the
+// rows only where its blocks fill one wave of workgroups (one per CU) by four fifths or more and those
+// of the second one do not fit theirs (two per CU).  With `over` the table is left empty and *over is 1 where there are
+// more than `limit` blocks (0 otherwise).
 __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S, int rows,
                                                               dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
                                                               dz_gemm_tile* __restrict__ tiles2, int max_tiles2, int limit,
-                                                              int* __restrict__ over) {
+                                                              int* __restrict__ over, int features) {
   extern __shared__ int first[];    // first[k]: index of segment k's first block; first[S + 1]: total
   const int tid = threadIdx.x, nseg = S + 1;
   auto count = [&](int r) {
@@ -511,8 +513,17 @@ __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restr
     fill(tiles, max_tiles, rows);
     return;
   }
-  const long long held = seg_off[nseg] - seg_off[0], room = (long long)first[nseg] * rows;
-  if (4 * held >= 3 * room) {
+  const long long held = seg_off[nseg] - seg_off[0], longs = first[nseg];
+  bool take_first = 4 * held >= 3 * longs * rows;
+  if (features) {
+    __syncthreads();
+    count(rows2);
+    const long long groups = longs * ((features + 255) / 256);
+    take_first = groups > 208 && groups <= 256 && (long long)first[nseg] * ((features + 127) / 128) > 512;
+    __syncthreads();                // everyone has read both totals
+    count(rows);
+  }
+  if (take_first) {
     fill(tiles, max_tiles, rows);
     empty(tiles2, max_tiles2);
   } else {
@@ -526,11 +537,11 @@ __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restr
 }  // namespace
 
 static int build_tiles(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, int rows2,
-                       dz_gemm_tile* tiles2, int max_tiles2, void* stream, int limit = 0, int32_t* over = nullptr) {
+                       dz_gemm_tile* tiles2, int max_tiles2, void* stream, int limit = 0, int32_t* over = nullptr, int features = 0) {
   if (!seg_off || !tiles) return DZ_EINVAL;
   if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || max_tiles < 1 || rows < 1) return DZ_ESHAPE;
   hipLaunchKernelGGL(dz_build_tiles_kernel, dim3(1), dim3(1024), (size_t)(S + 2) * 4, (hipStream_t)stream,
-                     seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2, limit, over);
+                     seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2, limit, over, features);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
@@ -555,6 +566,13 @@ extern "C" int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile
   if (!short_tiles) return DZ_EINVAL;
   if (max_short < 1) return DZ_ESHAPE;
   return build_tiles(seg_off, S, BM, tiles, max_tiles, DZ_SHORT_ROWS, short_tiles, max_short, stream);
+}
+
+extern "C" int dz_build_tiles_either_for(const int32_t* seg_off, int S, int N, dz_gemm_tile* tiles, int max_tiles,
+                                         dz_gemm_tile* short_tiles, int max_short, void* stream) {
+  if (!short_tiles) return DZ_EINVAL;
+  if (max_short < 1 || N < 1) return DZ_ESHAPE;
+  return build_tiles(seg_off, S, BM, tiles, max_tiles, DZ_SHORT_ROWS, short_tiles, max_short, stream, 0, nullptr, N);
 }
 
 static int multi_delta_gemm(const uint16_t* x, const uint16_t* w_base, bool w_tiled, const void* codes_stacked,

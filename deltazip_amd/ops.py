@@ -371,14 +371,31 @@ def apply_delta_uncompressed(x: torch.Tensor, delta_weights: torch.Tensor, indic
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
-    L, st, rows = _lib.lib(), _stream(), SHORT_ROWS if short else 256
+    L, st = _lib.lib(), _stream()
     perm, seg_off = segment(indices, S)               # (ids without a table take the base table, unreported)
-    tiles, ntiles = _block_table(T, S, rows, x.device)
-    _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), S, rows, tiles.data_ptr(), ntiles, st), "dz_build_tiles_rows")
     out = torch.empty((T, N), dtype=torch.float16, device=x.device)
-    fn = L.dz_gemm_f16_select_rows if short else L.dz_gemm_f16_select
-    _lib.check(fn(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K, tiles.data_ptr(), ntiles,
-                  perm.data_ptr(), out.data_ptr(), T, K, N, 0, N, st), "dz_gemm_f16_select")
+    # A segment of more than 128 rows puts a second, short block over the whole table.  From 225 rows on,
+    # where that is likely, and where two, three or four long blocks fill a wave of workgroups by four
+    # fifths or more, the device picks them if short ones overflow theirs (256 rows, 32000 x 4096, two
+    # tables: long 170, short 203 us; a table and the base table 172 / 204 at 300; one table 168 / 119);
+    # the launch that does nothing costs 4 us.
+    wide = (N + 255) // 256
+    either = short and 224 < T <= 512 and 52 <= wide <= 128 and 256 // wide * wide > 208
+    tables = []
+    for rows, used in ((256, either or not short), (SHORT_ROWS, short)):
+        tables.append(_block_table(T, S, rows, x.device) if used else (None, 0))
+    (tiles, n), (few, nf) = tables
+    if either:
+        _lib.check(L.dz_build_tiles_either_for(seg_off.data_ptr(), S, N, tiles.data_ptr(), n, few.data_ptr(), nf, st),
+                   "dz_build_tiles_either_for")
+    elif short:
+        _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), S, SHORT_ROWS, few.data_ptr(), nf, st), "dz_build_tiles_rows")
+    else:
+        _lib.check(L.dz_build_tiles(seg_off.data_ptr(), S, tiles.data_ptr(), n, st), "dz_build_tiles")
+    for table, rows, fn in ((tiles, n, L.dz_gemm_f16_select), (few, nf, L.dz_gemm_f16_select_rows)):
+        if table is not None:
+            _lib.check(fn(x.data_ptr(), base_embedding.data_ptr(), delta_weights.data_ptr(), N * K, table.data_ptr(), rows,
+                          perm.data_ptr(), out.data_ptr(), T, K, N, 0, N, st), "dz_gemm_f16_select")
     return out
 
 

@@ -364,6 +364,10 @@ int dz_build_tiles_rows_upto(const int32_t* seg_off, int S, int rows, int limit,
 int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile* tiles, int max_tiles,
                           dz_gemm_tile* short_tiles, int max_short, void* stream);
 
+/* The same choice for dz_gemm_f16_select and dz_gemm_f16_select_rows over tables of N features. */
+int dz_build_tiles_either_for(const int32_t* seg_off, int S, int N, dz_gemm_tile* tiles, int max_tiles,
+                              dz_gemm_tile* short_tiles, int max_short, void* stream);
+
 /* dz_multi_delta_gemm for row blocks of up to DZ_SHORT_ROWS rows (longer ones are taken that many rows at a time):
  * the faster one where most blocks are that short.  w_base is row-major [N, K] (w_tiled = 0), the
  * tiles dz_tile_base writes (w_tiled != 0), or NULL. */

@@ -377,6 +377,36 @@ def test_bad_ids_of_mid_size_batches_are_reported(dev):
     assert ops.workspace_status() == 0
 
 
+@pytest.mark.parametrize("n,lens,long", [(32000, [0, 126, 130], True), (32000, [0, 120, 128], False), (32000, [0, 256, 0], False),
+                                         (32000, [13, 243, 0], True), (16384, [64, 0, 192], False), (16384, [60, 130, 300], True),
+                                         (24576, [0, 126, 130], False), (32000, [100, 100, 100], False)])
+def test_projection_picks_blocks_by_waves(dev, n, lens, long):
+    """Long blocks where they fill one wave of workgroups and short ones overflow theirs; the rows' results
+    are those of each row's own table (fp32 sums rounded once to fp16, as for the short blocks)."""
+    from deltazip_amd import _lib
+    k, t, L = 256, sum(lens), _lib.lib()
+    seg = torch.from_numpy(np.concatenate([[0], np.cumsum(lens)]).astype(np.int32)).to(dev)
+    tabs = [torch.full((8, 4), 77, dtype=torch.int32, device=dev) for _ in range(2)]
+    assert L.dz_build_tiles_either_for(seg.data_ptr(), 2, n, tabs[0].data_ptr(), 8, tabs[1].data_ptr(), 8,
+                                       torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    step, at = (256 if long else 128), np.concatenate([[0], np.cumsum(lens)])
+    want = [[a, min(a + step, int(at[s + 1])), s - 1, 0] for s in range(3) for a in range(int(at[s]), int(at[s + 1]), step)]
+    want += [[0, 0, -1, 0]] * (8 - len(want))
+    assert tabs[not long].cpu().tolist() == want and tabs[long].cpu().tolist() == [[0, 0, -1, 0]] * 8
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(t, k, generator=g).half()
+    tables = (torch.randn(3, n, k, generator=g) * 0.02).half()
+    ids = torch.from_numpy(np.random.default_rng(t).permutation(np.repeat(np.arange(3) - 1, lens)))
+    xd, td = x.to(dev), tables.to(dev)
+    got = ops.apply_delta_uncompressed(xd, td[1:].contiguous(), ids.to(dev), td[0].contiguous()).cpu().double()
+    for i in range(0, t, 7):
+        ref = x[i].double() @ tables[int(ids[i]) + 1].double().t()
+        assert ((got[i] - ref).abs() <= 2.0**-10 * ref.abs() + 1e-4).all()
+    assert L.dz_build_tiles_either_for(seg.data_ptr(), 2, 0, tabs[0].data_ptr(), 8, tabs[1].data_ptr(), 8, None) == -2
+    assert L.dz_build_tiles_either_for(seg.data_ptr(), 2, n, tabs[0].data_ptr(), 8, None, 8, None) == -1
+
+
 def test_output_projection_does_not_report_ids(dev):
     """apply_delta_uncompressed serves an id without a table from the base table and leaves the fused
     kernel's status word alone, at every size."""
