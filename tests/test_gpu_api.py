@@ -152,18 +152,21 @@ def test_layer_with_only_the_tiled_base_weight(dev, t):
 
 @pytest.mark.parametrize("bits,gs", [(2, -1), (4, 128)])
 def test_matrix_core_kernel_reads_tiles_or_rows_alike(dev, bits, gs):
-    """dz_multi_delta_gemm_tiled against dz_multi_delta_gemm on the same problem: equal bits, also
-    with fewer features than a tile and with an output slice."""
+    """The kernels for long blocks (dz_multi_delta_gemm_tiled against dz_multi_delta_gemm) and for short
+    ones over tiles and over rows: equal bits, also with fewer features than a tile and with an output
+    slice."""
     from deltazip_amd.prefill import multi_delta_linear_prefill
-    for n, k, t in ((96, 768, 400), (544, 1024, 1000)):
+    for n, k, t, long in ((96, 768, 400, True), (544, 1024, 1000, True), (96, 768, 400, False), (544, 1024, 1000, False)):
         p = make_problem(n, k, bits, gs, 5, t, "uniform", 3 * n + bits, dev)
         wt = ops.tile_base(p["wb"])
+        blocks = ops.row_blocks(p["ids"], 5, long_only=long)
+        assert (blocks.tiles is not None) == long and (blocks.short is not None) != long
         y0 = torch.zeros(t, n + 32, dtype=torch.float16, device=dev)
         y1 = torch.zeros_like(y0)
         multi_delta_linear_prefill(p["x"], p["wb"], p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y0[:, 16:16 + n],
-                                   accumulate=False)
+                                   accumulate=False, blocks=blocks)
         multi_delta_linear_prefill(p["x"], None, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y1[:, 16:16 + n],
-                                   accumulate=False, base_tiled=wt)
+                                   accumulate=False, blocks=blocks, base_tiled=wt)
         torch.cuda.synchronize()
         assert torch.equal(y0, y1)
         ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])

@@ -468,9 +468,10 @@ def test_build_tiles_either(dev, lens, short):
 
 
 @pytest.mark.parametrize("t,nd", [(129, 3), (256, 40), (300, 4), (512, 17)])
-def test_mid_size_batches_go_through_the_fused_kernel_in_chunks(dev, t, nd):
-    """Between 129 tokens and a few hundred the matrix-core kernel would leave most of the GPU idle:
-    the call is made of chunks of 128 tokens through the fused kernel.  Both routes match the oracle."""
+def test_mid_size_batches_over_few_slots_and_many(dev, t, nd):
+    """Between 129 tokens and a few hundred: the call's own choice, row blocks, and -- the same deltas
+    scattered over more slots than the token sort can take -- chunks of 128 tokens through the fused
+    kernel, also into a column slice.  All match the oracle."""
     from deltazip_amd.prefill import multi_delta_linear_prefill
     assert ops.takes_fused_chunks(t, nd) and not ops.takes_fused_chunks(513, 64) and not ops.takes_fused_chunks(400, 4)
     p = make_problem(96, 512, 2, -1, nd, t, "uniform", 77 + t, dev)
@@ -481,7 +482,22 @@ def test_mid_size_batches_go_through_the_fused_kernel_in_chunks(dev, t, nd):
     multi_delta_linear_prefill(p["x"], p["wb"], p["q"], p["s"], p["m"], p["ids"], bits=2, out=y2, accumulate=False)
     torch.cuda.synchronize()
     assert o.rel_err(y2.cpu().numpy(), ref) <= TOL
-    # in place, delta only, into a column slice: the chunks write their rows of the slice
+    # 1000 slots, in arbitrary order
+    S, rng = 1000, np.random.default_rng(t)
+    where, mixed = rng.choice(S, nd, replace=False), rng.permutation(t)
+    stacks = {}
+    for key in ("q", "m", "s"):
+        stacks[key] = torch.zeros((S,) + tuple(p[key].shape[1:]), dtype=p[key].dtype, device=dev)
+        stacks[key][torch.from_numpy(where).to(dev)] = p[key]
+    slots = np.where(p["ids_np"] >= 0, where[np.maximum(p["ids_np"], 0)], -1)
+    assert ops._most_row_blocks(t, 512, 96, 2, S, None) == 0
+    wide = torch.zeros(t, 96 + 64, device=dev, dtype=torch.float16)
+    ops.multi_delta_linear(p["x"][torch.from_numpy(mixed).to(dev)], p["wb"], stacks["q"], stacks["s"], stacks["m"],
+                           torch.from_numpy(slots[mixed]).to(dev), bits=2, out=wide[:, 32:128])
+    torch.cuda.synchronize()
+    assert not wide[:, :32].any() and not wide[:, 128:].any()
+    assert o.rel_err(wide[:, 32:128].cpu().numpy(), ref[mixed]) <= TOL
+    # in place, delta only, into a column slice
     wide = torch.zeros(t, 96 + 64, device=dev, dtype=torch.float16)
     ops.add_delta_slice(wide, p["x"], p["q"], None, p["s"], None, p["ids"], 1.0, 32, 96, meta=p["m"])
     torch.cuda.synchronize()
@@ -492,7 +508,7 @@ def test_mid_size_batches_go_through_the_fused_kernel_in_chunks(dev, t, nd):
 
 @pytest.mark.parametrize("n,k,bits,gs,nd,t", [(64, 512, 2, -1, 3, 1), (96, 768, 4, 128, 5, 16), (256, 4096, 2, -1, 8, 32),
                                               (160, 1024, 2, 64, 7, 33), (128, 2048, 4, -1, 12, 100), (512, 4096, 2, -1, 9, 128),
-                                              (256, 1024, 2, -1, 6, 200)])   # 200 tokens: two chunks through the fused kernel
+                                              (256, 1024, 2, -1, 6, 200)])   # 200 tokens: row blocks
 def test_tiled_base_weight_gives_the_same_bits(dev, n, k, bits, gs, nd, t):
     """The base weight converted to tiles (dz_tile_base) feeds the fused kernel the same operands in the
     same order: outputs equal the row-major call bit for bit, single and batched, and match the oracle.
@@ -679,27 +695,30 @@ PREFILL_CASES = [
 
 @pytest.mark.parametrize("n,k,bits,gs,nd,t,kind", PREFILL_CASES)
 def test_packed_delta_gemm_parity(dev, n, k, bits, gs, nd, t, kind):
-    """T > 128 through dz_segment + dz_build_tiles + dz_multi_delta_gemm: unsorted ids, tokens
-    without a delta, N that is not a multiple of the 256-wide tile, grouped scales, then the
-    delta-only and accumulate forms."""
+    """T > 128 over row blocks, long ones (dz_multi_delta_gemm) and whatever the call chooses: unsorted
+    ids, tokens without a delta, N that is not a multiple of the 256-wide tile, grouped scales, then
+    the delta-only and accumulate forms."""
     p = make_problem(n, k, bits, gs, nd, t, kind, 4000 + n + k + t, dev)
     p["ids_np"][::7] = -1
     p["ids"] = torch.from_numpy(p["ids_np"]).to(dev)
-    y = run_layer(p)
-    ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
-    assert o.rel_err(y.cpu().numpy(), ref) <= TOL
-    # delta only, accumulated onto an existing output (the add_delta form)
-    y0 = torch.from_numpy(o.make_x(t, n, 5)).to(dev)
-    y1 = y0.clone()
-    ops.multi_delta_linear(p["x"], None, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y1, accumulate=True)
-    torch.cuda.synchronize()
-    ref_d = o.forward_ref(p["x_np"], None, p["dts"], p["ids_np"]) + y0.float().cpu().numpy()
-    assert o.rel_err(y1.cpu().numpy(), ref_d) <= TOL
-    # delta only, not accumulated: rows without a delta are zero
-    y2 = ops.multi_delta_linear(p["x"], None, p["q"], p["s"], p["m"], p["ids"], bits=bits)
-    torch.cuda.synchronize()
-    assert (y2[torch.from_numpy(p["ids_np"] < 0).to(dev)] == 0).all()
-    assert o.rel_err(y2.cpu().numpy(), o.forward_ref(p["x_np"], None, p["dts"], p["ids_np"])) <= TOL
+    for order in (ops.row_blocks(p["ids"], nd, long_only=True), None):
+        y = ops.apply_delta(p["x"], p["q"], p["s"], p["m"], p["ids"], p["wb"], order=order)
+        torch.cuda.synchronize()
+        ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
+        assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+        # delta only, accumulated onto an existing output (the add_delta form)
+        y0 = torch.from_numpy(o.make_x(t, n, 5)).to(dev)
+        y1 = y0.clone()
+        ops.multi_delta_linear(p["x"], None, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=y1, accumulate=True,
+                               order=order)
+        torch.cuda.synchronize()
+        ref_d = o.forward_ref(p["x_np"], None, p["dts"], p["ids_np"]) + y0.float().cpu().numpy()
+        assert o.rel_err(y1.cpu().numpy(), ref_d) <= TOL
+        # delta only, not accumulated: rows without a delta are zero
+        y2 = ops.multi_delta_linear(p["x"], None, p["q"], p["s"], p["m"], p["ids"], bits=bits, order=order)
+        torch.cuda.synchronize()
+        assert (y2[torch.from_numpy(p["ids_np"] < 0).to(dev)] == 0).all()
+        assert o.rel_err(y2.cpu().numpy(), o.forward_ref(p["x_np"], None, p["dts"], p["ids_np"])) <= TOL
 
 
 def test_build_tiles(dev):

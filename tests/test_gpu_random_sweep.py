@@ -61,6 +61,21 @@ def _check(dev, rng, n, k, bits, gs, nd, t, mode):
     torch.cuda.synchronize()
     err = o.rel_err(y.float().cpu().numpy(), ref)
     assert err <= tol, (case, err)
+    if t > 128:       # the kernel for long row blocks, which batches of these sizes reach only by their tables
+        long = ops.row_blocks(p["ids"], nd, long_only=True)
+        w, acc = (None, True) if mode == 1 else (p["wb"], False)
+        ys = []
+        for bt in (None, tiled) if w is not None else (None,):
+            wide = torch.zeros(t, n + 64, device=dev, dtype=torch.float16)
+            if acc:
+                wide[:, 32:32 + n] = torch.from_numpy(base16).to(dev)
+            ops.multi_delta_linear(p["x"], w, p["q"], p["s"], p["m"], p["ids"], bits=bits, out=wide[:, 32:32 + n],
+                                   accumulate=acc, order=long, base_tiled=bt)
+            ys.append(wide)
+        assert torch.equal(ys[0], ys[-1]), case
+        assert not ys[0][:, :32].any() and not ys[0][:, 32 + n:].any(), case
+        err = o.rel_err(ys[0][:, 32:32 + n].float().cpu().numpy(), ref)
+        assert err <= tol, (case, err)
 
 
 @pytest.mark.parametrize("seed", [11, 12])

@@ -54,6 +54,16 @@ def test_obs_sweep_bit_exact(dev, n, k, bits, quant, prune):
     torch.cuda.synchronize()
     assert np.array_equal(Wd.cpu().numpy(), want)
     assert np.array_equal(loss.cpu().numpy(), want_loss)
+    # with errors of one block in the workspace instead of two: block after block
+    from deltazip_amd import _lib
+    Wd, hd = torch.from_numpy(W0.copy()).to(dev), torch.from_numpy(hinv).to(dev)
+    scd = torch.from_numpy(sc).to(dev) if quant else None
+    err, loss = torch.empty(n, 128, device=dev), torch.zeros(n, device=dev)
+    assert _lib.lib().dz_obs_sweep(Wd.data_ptr(), hd.data_ptr(), scd.data_ptr() if quant else None, n, k, bits, pn, pm,
+                                   err.data_ptr(), loss.data_ptr(), torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    assert np.array_equal(Wd.cpu().numpy(), want)
+    assert np.array_equal(loss.cpu().numpy(), want_loss)
 
 
 @pytest.mark.parametrize("k,tokens,half", [(64, 1, True), (128, 31, True), (192, 33, False), (320, 64, True), (320, 95, False)])
@@ -173,6 +183,21 @@ def test_scales_with_the_search_over_the_clipping_range(dev, n, k, bits, gs):
     qz.find_params(torch.from_numpy(W).to(dev), weight=True)
     if gs == -1:
         assert torch.equal(qz.scale[:, 0], s32[0]) and float(qz.zero[0, 0]) == 2 ** (bits - 1)
+
+
+@pytest.mark.parametrize("n,k,bits,gs", [(32, 256, 4, 64), (64, 1280, 2, 128), (96, 256, 2, 256), (32, 1280, 4, 256),
+                                         (32, 768, 4, 192), (64, 1024, 2, 64), (32, 3072, 4, 1024), (32, 5120, 2, -1)])
+def test_scales_of_grouped_columns(dev, n, k, bits, gs):
+    """Plain scales for every group length, K / 256 a multiple of four and not: the oracle's, bit for bit,
+    with an all-zero row, one without a negative value and one with an outlier."""
+    W, _ = _inputs(n, k, 8, 60 + n + bits)
+    W[0] = 0
+    W[2] = np.abs(W[2])
+    W[4, 3] = 30 * np.abs(W).max()
+    s32, s16 = ops.quant_scales(torch.from_numpy(W).to(dev), bits, gs)
+    scale, _ = o.find_params_sym(W, bits, gs)
+    assert np.array_equal(s32.cpu().numpy().T, scale)
+    assert np.array_equal(s16.cpu().numpy().T.view(np.uint16), scale.astype(np.float16).view(np.uint16))
 
 
 def test_scales_and_pack_match_the_reference_pipeline(dev):
