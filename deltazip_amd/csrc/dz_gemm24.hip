@@ -471,8 +471,10 @@ __global__ __launch_bounds__(512, 2) void dz_gemm24_kernel(const Gemm24Params P)
 // second table (blocks of rows2 < rows) one of the two gets all rows and the other stays empty: the
 // second one where the first one's blocks would be less than three quarters full.  There the short
 // blocks' kernel is the faster one although it reads the weights more often (5120 x 27648, 2-bit,
-// 256 against 128 rows: 4096 tokens of 16 deltas, 65 % full: 2064 against 1837 us; 2000 tokens of 8,
-// 75 %: 829 against 815; 2048 of one, 100 %: 766 against 833).  With `features` the first one gets the
+// 256 against 128 rows: 4096 tokens of 16 deltas, 64 % full: 2338 against 2019 us; of 32, 50 %: 2606 /
+// 2167).  The line is on the safe side: up to 4096 tokens the short blocks win at any fill by now
+// (1536 of 4, 75 %: 819 / 725; 4096 of 8, 80 %: 2054 / 1900), the long ones at 8192 tokens from 80 % on
+// (16 deltas 3689 / 3715, 4 deltas, 94 %: 3227 / 3528).  With `features` the first one gets the
 // rows only where its blocks fill one wave of workgroups (one per CU) by four fifths or more and those
 // of the second one do not fit theirs (two per CU).  With `over` the table is left empty and *over is 1 where there are
 // more than `limit` blocks (0 otherwise).

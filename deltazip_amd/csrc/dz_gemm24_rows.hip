@@ -14,10 +14,13 @@
 // 256 registers leave room for two workgroups per CU.  The loop is instantiated per number of
 // 16-token tiles: a block of 5 tokens does the work of 16, not of 256.
 //
-// Bound by L2: a block of 128 tokens reads 36 KB per slab for 770 cycles of matrix work, a shorter one
-// nearly as much for less.  5120 x 27648, 2-bit, against the 256 x 256 tiles: 512 tokens of 64 deltas
-// 3239 -> 1338 us, 1024 of 16 959 -> 602, 2048 of 16 1310 -> 1027, 8192 of 64 4892 -> 4129.  (Eight
-// token tiles' operands read two at a time: four at a time spilled 40 bytes per lane.)
+// What bounds it is the way of the weights through the caches, at no one unit's rate: every row block
+// reads the base weight and its delta again, 3.85 GB through L2 for 333 tokens of 7 deltas over 5120 x
+// 27648 (271 us: 14 TB/s, 28 % of it from beyond L2, 0.52 GB from HBM, matrix cores 30 % busy), 7.8 GB
+// for 1999 tokens over 4096 x 22016 (703 us: 11 TB/s, half from beyond L2, matrix cores 35 % busy).
+// 5120 x 27648, 2-bit, against the 256 x 256 tiles: 512 tokens of 64 deltas 3470 -> 1369 us, 1024 of 16
+// 1000 -> 630, 2048 of 16 1502 -> 1121, 8192 of 64 4993 -> 4299.  (Eight token tiles' operands read two
+// at a time: four at a time spilled 40 bytes per lane.)
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
