@@ -16,7 +16,6 @@ import ctypes as C
 import math
 from collections import Counter
 from functools import lru_cache
-from operator import lt
 from typing import Dict, NamedTuple, Optional, Sequence, Tuple
 
 import torch
@@ -212,10 +211,11 @@ def _route_us(T: int, K: int, N: int, bits: int, mix: BatchMix) -> Tuple[float, 
     because it reads the base weight again, and walks all of K; a chunk of 128 reads the base weight once
     for all its deltas and splits K where there are few features.
 
-    Estimates in us, fitted to 10464 timed calls over tiles (129 to 512 tokens of 1 to 64 deltas, sorted,
-    shuffled and in requests; K and N from 512 to 27648; 2 bits and 4) and within a fifth of 90 % of
-    them.  What they choose is 0.3 % slower in the mean than the faster route, where row blocks
-    throughout were 11 % slower and up to 4.3 times.  Chunks / row blocks, sorted, 2-bit:
+    Estimates in us, fitted to 10597 timed calls over tiles (129 to 512 tokens of 1 to 64 deltas, sorted and
+    in requests; K from 512 to 13824, N to 27648; 2 bits and 4) and within a fifth of 90 % of them.  What
+    they choose is 0.5 % slower in the mean than the faster route; row blocks throughout were 14 % and up
+    to 5.4 times, chunks throughout 77 % and 5.7 times.  Chunks / row blocks,
+    sorted, 2-bit:
       5120 x 27648, 129 tokens of 4 / 16 / 64 deltas   251 / 307 / 557 against 138 / 376 / 1103 us
                     256                                388 / 433 / 698 against 177 / 386 / 1224
                     512                                769 / 798 / 1064 against 297 / 425 / 1356
@@ -223,21 +223,26 @@ def _route_us(T: int, K: int, N: int, bits: int, mix: BatchMix) -> Tuple[float, 
       13824 x 1024, 129 tokens of 1 / 4 / 16 deltas    48 / 49 / 53 against 173 / 119 / 110
                     512                                119 / 123 / 127 against 178 / 176 / 108
     Row blocks come in waves of 512 workgroups, two per CU: a single wave's time is that of its longest
-    block's walk, and of sharing a CU; several are bound by their products.  A chunk's launches take
-    the host 24 us."""
+    block's walk, and of sharing a CU; several are bound by their products.  Chunks: two launches each,
+    the products of every 32 tokens, the deltas' words, and the start of each workgroup."""
     k, weight = K / 1024, K * N / 2**20
     groups = mix.blocks * -(-N // 128)
     waves, chunks, turns = -(-groups // 512), -(-T // MAX_TOKENS_FUSED), -(-T // 32)
     if waves == 1:
-        start, walk, full, shared = (7.2, 7.25, 5.85, 3.8) if bits == 2 else (6.7, 9.2, 5.4, 4.9)
+        start, walk, full, shared = (7.3, 7.7, 5.6, 6.1) if bits == 2 else (6.5, 9.9, 5.0, 6.7)
         rows_us = start + k * (walk + full * (min(mix.longest, SHORT_ROWS) / SHORT_ROWS)**2
                                + shared * max(0, groups - 256) / 256)
     else:
-        start, walk, token = (3.4, 8.5, 12.0) if bits == 2 else (3.2, 11.0, 11.1)
+        start, walk, token = (2.8, 8.5, 14.1) if bits == 2 else (2.6, 11.0, 13.1)
         rows_us = waves * (start + k * (walk + token * T / (SHORT_ROWS * mix.blocks)))
-    launch, walk, turn, delta = (13.5, 0.12, 0.286, 0.0463) if bits == 2 else (13.0, 0.15, 0.288, 0.0812)
-    chunks_us = max(24 * chunks, chunks * (launch + walk * k) + weight * (turn * turns + delta * mix.met))
+    walk, turn, delta, shared = (0.63, 0.287, 0.0416, 0.07) if bits == 2 else (0.69, 0.300, 0.0770, 0.119)
+    chunks_us = (chunks * (11.3 + walk * k) + weight * (turn * turns + delta * mix.met - shared * chunks)
+                 + 0.153 * N / 1024 * turns)
     return chunks_us, rows_us
+
+
+def _in_chunks(costs: Tuple[float, float]) -> bool:
+    return costs[0] < 0.98 * costs[1]                 # (closer estimates say nothing: row blocks)
 
 
 def _one_wave_of_long_blocks(T: int, N: int, bits: int) -> bool:
@@ -770,7 +775,7 @@ def _most_row_blocks(T: int, K: int, N: int, bits: int, S: int, blocks: Optional
     if S > MAX_SLOTS_SEGMENT:
         return 0
     if blocks is not None:
-        return 0 if blocks.mix is not None and lt(*_route_us(T, K, N, bits, blocks.mix)) else None
+        return 0 if blocks.mix is not None and _in_chunks(_route_us(T, K, N, bits, blocks.mix)) else None
     return _most_blocks_unknown(T, K, N, bits, S)
 
 

@@ -160,16 +160,18 @@ def test_the_faster_route_is_taken(k, n, bits, t, deltas, chunks, rows):
         assert (a < b) == (chunks < rows)
 
 
-@pytest.mark.parametrize("k,n,t,slots,most", [(5120, 27648, 129, 64, 14), (5120, 27648, 256, 32, 21), (4096, 12288, 129, 64, 16),
+@pytest.mark.parametrize("k,n,t,slots,most", [(5120, 27648, 129, 64, "device"), (5120, 27648, 256, 32, "device"),
+                                              (4096, 12288, 129, 64, "device"),
                                               (5120, 27648, 129, 8, None), (13824, 1024, 256, 8, 0), (4096, 3072, 256, 2, 0),
                                               (512, 512, 300, 2, None), (512, 512, 512, 1000, 0), (1024, 13824, 129, 32, None),
                                               (13824, 512, 400, 4, None), (5120, 27648, 513, 64, None)])
 def test_route_of_a_batch_whose_mix_the_host_does_not_know(k, n, t, slots, most):
     """Narrow layers go in chunks whatever the mix, small ones in row blocks; for wide ones over many
     slots the device chooses, and the limit it is given lies where the two estimates meet."""
-    assert ops._most_row_blocks(t, k, n, 2, slots, None) == most
-    if most:
-        for d, rows in ((most, True), (most + 1, False)):
+    got = ops._most_row_blocks(t, k, n, 2, slots, None)
+    assert got == most if most != "device" else 2 <= got < slots
+    if got:
+        for d, rows in ((got, True), (got + 1, False)):
             a, b = ops._route_us(t, k, n, 2, ops._even_mix(t, d)._replace(blocks=d, longest=128))
             assert (b <= a) == rows
 
