@@ -356,8 +356,8 @@ def apply_delta_uncompressed(x: torch.Tensor, delta_weights: torch.Tensor, indic
     Where the reference loops over torch.unique(indices) on the host, the rows are grouped by id
     and cut into row blocks on the device (dz_segment, dz_build_tiles) and one launch multiplies
     every block by its own table (dz_gemm_f16_select), reading and writing the rows in place
-    through the token order: three launches, nothing gathered, scattered or read back to the
-    host, so the call can be captured in a HIP graph."""
+    through the token order: three launches (four where the device picks the block length), nothing
+    gathered, scattered or read back to the host, so the call can be captured in a HIP graph."""
     _need_cuda(x, delta_weights, indices, base_embedding)
     if x.dtype != torch.float16 or delta_weights.dtype != torch.float16 or base_embedding.dtype != torch.float16:
         raise ValueError("x and the weights must be float16")
