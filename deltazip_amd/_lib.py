@@ -33,6 +33,11 @@ SIGNATURES = {
                                           C.c_size_t, _vp]),
     "dz_build_tiles_rows": (_i, [_vp, _i, _i, _vp, _i, _vp]),
     "dz_multi_delta_gemm_rows": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
+    "dz_mixed_blocks": (_i, [_i, _i, _i, _i]),
+    "dz_build_mixed": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _vp]),
+    "dz_build_tables": (_i, [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
+    "dz_multi_delta_gemm_mixed": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _vp,
+                                       _vp]),
     "dz_multi_delta_gemm": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_multi_delta_gemm_tiled": (_i, [_vp, _vp, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_compress_2of4": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _vp]),

@@ -28,6 +28,7 @@
 
 #include "../../include/dz_amd.h"
 #include "dz_device.h"
+#include "dz_tables.h"
 
 namespace {
 
@@ -478,11 +479,11 @@ __global__ __launch_bounds__(512, 2) void dz_gemm24_kernel(const Gemm24Params P)
 // rows only where its blocks fill one wave of workgroups (one per CU) by four fifths or more and those
 // of the second one do not fit theirs (two per CU).  With `over` the table is left empty and *over is 1 where there are
 // more than `limit` blocks (0 otherwise).
-__global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S, int rows,
-                                                              dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
-                                                              dz_gemm_tile* __restrict__ tiles2, int max_tiles2, int limit,
-                                                              int* __restrict__ over, int features) {
-  extern __shared__ int first[];    // first[k]: index of segment k's first block; first[S + 1]: total
+__device__ __forceinline__ void build_tiles_body(const int* __restrict__ seg_off, int S, int rows,
+                                                 dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
+                                                 dz_gemm_tile* __restrict__ tiles2, int max_tiles2, int limit,
+                                                 int* __restrict__ over, int features, int* first) {
+  // first[k]: index of segment k's first block; first[S + 1]: total
   const int tid = threadIdx.x, nseg = S + 1;
   auto count = [&](int r) {
     for (int k = tid; k < nseg; k += 1024) first[k + 1] = (seg_off[k + 1] - seg_off[k] + r - 1) / r;
@@ -536,6 +537,39 @@ __global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restr
   }
 }
 
+__global__ __launch_bounds__(1024) void dz_build_tiles_kernel(const int* __restrict__ seg_off, int S, int rows,
+                                                              dz_gemm_tile* __restrict__ tiles, int max_tiles, int rows2,
+                                                              dz_gemm_tile* __restrict__ tiles2, int max_tiles2, int limit,
+                                                              int* __restrict__ over, int features) {
+  extern __shared__ int first[];
+  build_tiles_body(seg_off, S, rows, tiles, max_tiles, rows2, tiles2, max_tiles2, limit, over, features, first);
+}
+
+// All tables of a batch, one workgroup each.
+struct BatchTables {
+  dz_gemm_tile *tiles, *short_tiles;
+  dz_mixed_block* mixed[2];
+  int* count[2];
+  int max_tiles, max_short, max_mixed[2], either, deltas;
+};
+__global__ __launch_bounds__(1024) void dz_build_tables_kernel(const int* __restrict__ seg_off, const int* __restrict__ perm,
+                                                               int S, const BatchTables B) {
+  extern __shared__ int first[];
+  const int which = blockIdx.x;
+  if (which >= 2) {
+    if (B.mixed[which - 2])
+      dz_build_mixed_blocks(seg_off, perm, S, which == 2 ? DZ_MIXED_ROWS / 16 : DZ_MIXED_SMALL_TILES,
+                            which == 2 ? B.deltas : DZ_MIXED_SMALL_DELTAS, B.count[which - 2], B.mixed[which - 2],
+                            B.max_mixed[which - 2], first);
+  } else if (which == 0) {
+    if (B.tiles)
+      build_tiles_body(seg_off, S, BM, B.tiles, B.max_tiles, DZ_SHORT_ROWS, B.either ? B.short_tiles : nullptr, B.max_short, 0,
+                       nullptr, 0, first);
+  } else if (B.short_tiles && !B.either) {
+    build_tiles_body(seg_off, S, DZ_SHORT_ROWS, B.short_tiles, B.max_short, 0, nullptr, 0, 0, nullptr, 0, first);
+  }
+}
+
 }  // namespace
 
 static int build_tiles(const int32_t* seg_off, int S, int rows, dz_gemm_tile* tiles, int max_tiles, int rows2,
@@ -575,6 +609,22 @@ extern "C" int dz_build_tiles_either_for(const int32_t* seg_off, int S, int N, d
   if (!short_tiles) return DZ_EINVAL;
   if (max_short < 1 || N < 1) return DZ_ESHAPE;
   return build_tiles(seg_off, S, BM, tiles, max_tiles, DZ_SHORT_ROWS, short_tiles, max_short, stream, 0, nullptr, N);
+}
+
+extern "C" int dz_build_tables(const int32_t* seg_off, const int32_t* perm, int S, int T, dz_gemm_tile* tiles, int max_tiles,
+                               dz_gemm_tile* short_tiles, int max_short, int either, int deltas, int32_t* mixed, int max_mixed,
+                               int32_t* small, int max_small, void* stream) {
+  if (!seg_off || !perm || !mixed || !small) return DZ_EINVAL;
+  if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || T < 1) return DZ_ESHAPE;
+  if ((tiles && max_tiles < 1) || (short_tiles && max_short < 1) || (either && !(tiles && short_tiles))) return DZ_ESHAPE;
+  const int need = dz_mixed_blocks(T, S, DZ_MIXED_ROWS / 16, deltas);
+  if (need < 1 || max_mixed < need ||
+      max_small < dz_mixed_blocks(T, S, DZ_MIXED_SMALL_TILES, DZ_MIXED_SMALL_DELTAS))
+    return DZ_ESHAPE;
+  const BatchTables B{tiles, short_tiles, {(dz_mixed_block*)(mixed + DZ_MIXED_HEADER), (dz_mixed_block*)(small + DZ_MIXED_HEADER)},
+                      {mixed, small}, max_tiles, max_short, {max_mixed, max_small}, either, deltas};
+  hipLaunchKernelGGL(dz_build_tables_kernel, dim3(4), dim3(1024), (size_t)(S + 2) * 4, (hipStream_t)stream, seg_off, perm, S, B);
+  return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 
 static int multi_delta_gemm(const uint16_t* x, const uint16_t* w_base, bool w_tiled, const void* codes_stacked,

@@ -364,7 +364,9 @@ class DeltaModelManager:
             # (the mix decides at sizes where other routes than row blocks may be the faster one)
             self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
                                                 mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
-                                                features=self._widest or None)
+                                                features=self._widest or None,
+                                                deltas=ops.mixed_deltas(self.delta_config.max_bitwidth,
+                                                                        self.delta_config.group_size != -1))
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 

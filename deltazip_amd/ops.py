@@ -171,14 +171,85 @@ class RowBlocks:
     (what dz_segment and dz_build_tiles write): depends on the indices only, so it can be made once
     per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
     256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None.
+    `mixed`: tables of blocks of several deltas (MixedTable), full and small ones, or None.
     They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`.
     `mix`: what the maker knew of the batch on the host, or None; `host_picks`: both tables hold all rows."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix", "host_picks")
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix", "host_picks", "mixed")
 
-    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None, host_picks=False):
+    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None, host_picks=False, mixed=None):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
         self.short, self.max_short, self.mix, self.host_picks = short, max_short, mix, host_picks
+        self.mixed = mixed
         self.captured = torch.cuda.is_current_stream_capturing()
+
+
+class MixedTable(NamedTuple):
+    """What dz_build_mixed writes: the table, how many blocks it has room for, and the most deltas of one."""
+    table: torch.Tensor
+    max_blocks: int
+    deltas: int
+
+
+MIXED_BLOCKS = ((8, 4), (4, 2))   # (tiles of 16 tokens, deltas) of a block: full, small (DZ_MIXED_*)
+
+
+def mixed_deltas(bits: int, grouped: bool) -> int:
+    """Most deltas of a full block: a delta's words stay in registers while its block is multiplied, and at 4 bits
+    and with scales that change along K three deltas' fit beside the sums."""
+    return 4 if bits == 2 and not grouped else 3
+
+
+@lru_cache(maxsize=4096)
+def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
+    """How a batch of more than 128 tokens takes blocks of several deltas: (0 for full blocks, 1 for small
+    ones; parts K is cut into), or None where they do not pay.  By the sizes alone, so that a token's result
+    depends on neither the mix nor its place in the batch.
+
+    Fitted to 2240 timed batches of 129 to 1700 tokens and 3780 of 129 to 8192 (1 to 64 slots, sorted ids and
+    requests, both bit widths, K from 512 to 13824, N to 27648): the choice takes 6.6 % longer in the mean than
+    the best of two to five sizes of blocks and five of parts.  Against the faster of the other kernels (one delta
+    per block; chunks of the decode kernel), in the mean: 129 tokens 1.28 times as fast, 333 1.33, 1000 1.29,
+    2000 1.22, 8192 1.11.
+      small blocks   where the full ones' workgroups would leave most of the 256 CUs idle: a block of half as
+                     many tiles walks K in less time (2048 x 2048, 230 tokens: in the mean 1.42 against
+                     1.23 times as fast as before; 4096 x 12288 of 333: 1.12 against 1.27)
+      parts          each a walk over its share of K, and one more pass over the sums at 3 TB/s (13824 x 5120,
+                     333 tokens of 10 deltas: 1 / 2 / 3 / 4 / 6 parts 220 / 128 / 100 / 122 / 110 us)
+      K <= 1024      the walk is too short to pay for a workgroup's start unless there are several waves of them
+                     (1024 x 8192: 129 tokens 14 / 19 us, 640 tokens 1.24 times as fast)"""
+    if T <= MAX_TOKENS_FUSED or 2 * T * K >= 1 << 31:
+        return None                                   # (32-bit offsets)
+    if K <= 1024 and -(-T // 128) * -(-N // 128) <= 384:
+        return None
+    wide, steps = -(-N // 256), K // 256
+    small = wide * T / 128 < (140 if K <= 3072 else 25)
+    blocks = -(-T // (64 if small else 128))
+    best = None
+    for parts in (1, 2, 3, 4, 6):
+        if parts > steps:
+            break
+        groups = wide * blocks * parts
+        waves = -(-groups // 256) if groups <= 1024 else groups / 256
+        cost = waves * (8 + -(-steps // parts) * 4 * (1.0 if small else 1.7) * (0.6 + 0.4 * min(1.0, groups / 256)))
+        if parts > 1:
+            cost += 3 + 8 * T * N * parts / 3e6
+        if best is None or cost < best[0]:
+            best = (cost, parts)
+    return int(small), best[1]
+
+
+def _in_mixed_blocks(T: int, K: int, N: int, S: int, mix: Optional["BatchMix"]) -> Optional[Tuple[int, int]]:
+    """`_mixed_plan` but for batches whose mix the host knows to suit another kernel: a few tokens of each of many
+    deltas over a long and narrow layer go in chunks (11008 x 4096, 129 tokens of 55 deltas: 180 against 261 us),
+    and over a short one, where the row blocks are one wave of workgroups, in row blocks (1536 x 3072, 170 tokens
+    of 20 deltas: 18 / 27)."""
+    plan = _mixed_plan(T, K, N) if 0 < S <= MAX_SLOTS_SEGMENT else None
+    if plan is not None and mix is not None:
+        if takes_fused_chunks(T, S) and 3 * mix.deltas > T and K >= 2 * N:
+            return None
+        if K <= 2560 and 20 * mix.blocks >= T and mix.blocks * -(-N // 128) <= 512:
+            return None
+    return plan
 
 
 class BatchMix(NamedTuple):
@@ -272,8 +343,16 @@ def _block_table(T: int, num_slots: int, rows: int, device):
     return torch.empty((n, 4), dtype=torch.int32, device=device), n
 
 
+def _mixed_table(T: int, S: int, small: int, deltas: int, device) -> MixedTable:
+    tiles, most = MIXED_BLOCKS[small]
+    deltas = min(deltas, most)
+    n = _lib.lib().dz_mixed_blocks(T, S, tiles, deltas)
+    # DZ_MIXED_HEADER words and n times sizeof(dz_mixed_block)
+    return MixedTable(torch.empty(4 + n * (2 + 4 * 4 + 128), dtype=torch.int32, device=device), n, deltas)
+
+
 def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
-               device_picks: bool = False, features: Optional[int] = None) -> RowBlocks:
+               device_picks: bool = False, features: Optional[int] = None, deltas: int = 3) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
     (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
@@ -295,7 +374,10 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     `long_only`: the table of 256-token blocks alone, whatever the batch.  `mix`: batch_mix() of the
     same ids, if the host has them: calls of a few hundred tokens then choose between these blocks and
     chunks of the fused kernel by it.  `device_picks`: as between, whatever the batch.  `features`: of the
-    widest layer they are for, if known."""
+    widest layer they are for, if known.
+
+    Layers with a base weight take the batch in blocks of several deltas where those pay (`_mixed_plan`): their
+    tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
@@ -311,16 +393,16 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
         tiles, n = _block_table(T, num_slots, 256, dev)
     if small or device_picks or (not long_only and T < 256 * (num_slots + 1)):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
-    if tiles is not None and short is not None and not host_picks:
-        _lib.check(L.dz_build_tiles_either(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, short.data_ptr(), ns, st),
-                   "dz_build_tiles_either")
-    else:
-        if tiles is not None:
-            _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
-        if short is not None:
-            _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
-                       "dz_build_tiles_rows")
-    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks)
+    if long_only:
+        _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
+        return RowBlocks(perm, tiles, n, T, num_slots)
+    mixed = [_mixed_table(T, num_slots, small_ones, deltas, dev) for small_ones in (0, 1)]
+    ptr = lambda t: None if t is None else t.data_ptr()
+    _lib.check(L.dz_build_tables(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, ptr(tiles), n, ptr(short), ns,
+                                 int(tiles is not None and short is not None and not host_picks), mixed[0].deltas,
+                                 mixed[0].table.data_ptr(), mixed[0].max_blocks, mixed[1].table.data_ptr(),
+                                 mixed[1].max_blocks, st), "dz_build_tables")
+    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks, mixed)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,
@@ -833,6 +915,14 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
     if T > MAX_TOKENS_FUSED:
         blocks = _usable_blocks(order, T, S)
         most = _most_row_blocks(T, K, N, bits, S, blocks)
+        plan = None
+        if (base_weight is not None or base_tiled is not None) and (blocks is None or blocks.mixed is not None):
+            plan = _in_mixed_blocks(T, K, N, S, blocks.mix if blocks is not None else None)
+        if plan is not None:
+            from .prefill import multi_delta_linear_mixed
+            return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
+                                            bits=bits, out=out, accumulate=accumulate, plan=plan, blocks=blocks,
+                                            base_tiled=base_tiled)
         if most is not None:
             ws = _workspace(x.device, MAX_TOKENS_FUSED, K, N)
             w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
@@ -937,13 +1027,13 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     if T > MAX_TOKENS_FUSED:
         blocks = order if isinstance(order, RowBlocks) else None
         # row blocks made once serve the projections that would make the same ones
-        shared = [q.shape[0] == S and (blocks is not None or (
+        shared = [q.shape[0] == S and (blocks is not None or _in_mixed_blocks(T, K, w.shape[0], S, None) is not None or (
                       _most_row_blocks(T, K, w.shape[0], bits, S, None) is None
                       and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
-            blocks = row_blocks(indices, S, features=max(w.shape[0] for w in base_weight))
+            blocks = row_blocks(indices, S, features=max(w.shape[0] for w in base_weight), deltas=mixed_deltas(bits, G > 1))
         if blocks is not None and (blocks.T != T or blocks.S != S):
             blocks = None
         return [apply_delta(xs[j], qweight_stacked[j], scales_stacked[j], meta_stacked[j], indices, base_weight[j],

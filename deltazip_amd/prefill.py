@@ -83,3 +83,32 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
             blocks.perm.data_ptr(), out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), stream)
         _lib.check(rc, "dz_multi_delta_gemm_rows")
     return out
+
+
+def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices, *, bits: int,
+                             out: torch.Tensor, accumulate: bool, plan, blocks=None, base_tiled=None) -> torch.Tensor:
+    """The layer over blocks that hold the tokens of several deltas (dz_multi_delta_gemm_mixed), with a base weight.
+    `plan`: ops._mixed_plan(T, K, N).  `blocks`: as for multi_delta_linear_prefill; without them, or where they
+    were made for more deltas than this layer's block can hold, the call makes the table it needs."""
+    from .ops import _mixed_table, mixed_deltas, segment, takes_fused_chunks
+    small, parts = plan
+    T, K = x2.shape
+    N, S = scales_stacked.shape[-1], qweight_stacked.shape[0]
+    G = scales_stacked[0].numel() // N
+    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    deltas = mixed_deltas(bits, G > 1)
+    table = blocks.mixed[small] if blocks is not None else None
+    if table is None or table.deltas > deltas:
+        perm, seg_off = segment(indices, S, takes_fused_chunks(T, S))
+        table = _mixed_table(T, S, small, deltas, x2.device)
+        _lib.check(L.dz_build_mixed(seg_off.data_ptr(), perm.data_ptr(), S, T, 4 if small else 8, table.deltas,
+                                    table.table.data_ptr(), table.max_blocks, stream), "dz_build_mixed")
+    sums = torch.empty(parts * T * N, dtype=torch.float32, device=x2.device) if parts > 1 else None
+    w = base_tiled if base_tiled is not None else base_weight
+    rc = L.dz_multi_delta_gemm_mixed(
+        x2.data_ptr(), w.data_ptr(), 1 if base_tiled is not None else 0, qweight_stacked.data_ptr(),
+        meta_stacked.data_ptr(), scales_stacked.data_ptr(), S, bits, -1 if G == 1 else K // G, table.table.data_ptr(),
+        table.max_blocks, table.deltas, out.data_ptr(), T, K, N, 1 if accumulate else 0, out.stride(0), parts,
+        sums.data_ptr() if sums is not None else None, stream)
+    _lib.check(rc, "dz_multi_delta_gemm_mixed")
+    return out

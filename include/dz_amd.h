@@ -49,6 +49,11 @@ extern "C" {
 #define DZ_STATIC_MAX_N 16384      /* largest N dz_multi_delta_linear_static takes             */
 #define DZ_MAX_SLOTS_SEGMENT 768   /* largest S dz_segment takes (its tables live in LDS)      */
 #define DZ_SHORT_ROWS 128         /* rows of a block of dz_multi_delta_gemm_rows */
+#define DZ_MIXED_ROWS 128         /* rows of a block of dz_multi_delta_gemm_mixed */
+#define DZ_MIXED_DELTAS 4         /* most deltas in such a block (2-bit deltas with one scale per row; else 3) */
+#define DZ_MIXED_SMALL_TILES 4    /* the smaller blocks of dz_build_tables: tiles of 16 rows, */
+#define DZ_MIXED_SMALL_DELTAS 2   /* deltas */
+#define DZ_MIXED_HEADER 4         /* words in front of the blocks of a table; the first: how many there are */
 #define DZ_MAX_SLOTS_MAP 4096      /* largest S dz_map_ids takes (the slot table lives in LDS) */
 
 /* Library version (major*10000 + minor*100 + patch). */
@@ -367,6 +372,42 @@ int dz_build_tiles_either(const int32_t* seg_off, int S, dz_gemm_tile* tiles, in
 /* The same choice for dz_gemm_f16_select and dz_gemm_f16_select_rows over tables of N features. */
 int dz_build_tiles_either_for(const int32_t* seg_off, int S, int N, dz_gemm_tile* tiles, int max_tiles,
                               dz_gemm_tile* short_tiles, int max_short, void* stream);
+
+/* A block of up to DZ_MIXED_ROWS rows that holds the tokens of several deltas, in nt tiles of 16 rows, each
+ * of one delta: delta e < nd, slot[e], takes positions lo[e] .. hi[e] - 1 of the token order, in tiles
+ * that begin behind those of delta e - 1 and end in front of tend[e].  nd = 0: tokens lo[0] .. hi[0] - 1
+ * without a delta.  row[r]: the row of x and y of row r, or for a row that is there to fill a tile ~(row
+ * whose values it repeats). */
+typedef struct dz_mixed_block {
+  int32_t nt, nd;
+  int32_t slot[DZ_MIXED_DELTAS], lo[DZ_MIXED_DELTAS], hi[DZ_MIXED_DELTAS], tend[DZ_MIXED_DELTAS];
+  int32_t row[DZ_MIXED_ROWS];
+} dz_mixed_block;
+
+/* Most blocks of up to `tiles` tiles and `deltas` deltas dz_build_mixed makes of T tokens over S slots. */
+int dz_mixed_blocks(int T, int S, int tiles, int deltas);
+
+/* Cuts the token order of dz_segment (perm NULL: the tokens are in order) into such blocks, tiles <=
+ * DZ_MIXED_ROWS / 16, deltas <= DZ_MIXED_DELTAS.  table: DZ_MIXED_HEADER words, then max_blocks blocks, at
+ * least dz_mixed_blocks(T, S, tiles, deltas). */
+int dz_build_mixed(const int32_t* seg_off, const int32_t* perm, int S, int T, int tiles, int deltas, int32_t* table,
+                   int max_blocks, void* stream);
+
+/* The tables of a batch in one launch: those of dz_build_tiles (tiles, or NULL) and dz_build_tiles_rows with
+ * DZ_SHORT_ROWS rows (short_tiles, or NULL), or of dz_build_tiles_either (either != 0); those of dz_build_mixed with
+ * DZ_MIXED_ROWS / 16 tiles and `deltas` deltas (mixed) and with the smaller blocks (small). */
+int dz_build_tables(const int32_t* seg_off, const int32_t* perm, int S, int T, dz_gemm_tile* tiles, int max_tiles,
+                    dz_gemm_tile* short_tiles, int max_short, int either, int deltas, int32_t* mixed, int max_mixed,
+                    int32_t* small, int max_small, void* stream);
+
+/* dz_multi_delta_gemm over blocks of several deltas: every block reads the base weight once, whatever
+ * deltas it holds.  deltas: what the table was made with (DZ_MIXED_DELTAS for 2-bit deltas with one scale per
+ * row only).  w_base is row-major [N, K] (w_tiled = 0) or the tiles dz_tile_base writes.  ksplit > 1: K is cut
+ * into that many parts (1 .. K / 256), computed side by side; partials then holds ksplit * T * N floats. */
+int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                              const void* meta_stacked, const void* scales_stacked, int S, int bits, int group_size,
+                              const int32_t* table, int max_blocks, int deltas, uint16_t* y, int T, int K, int N,
+                              int accumulate, int ldy, int ksplit, float* partials, void* stream);
 
 /* dz_multi_delta_gemm for row blocks of up to DZ_SHORT_ROWS rows (longer ones are taken that many rows at a time):
  * the faster one where most blocks are that short.  w_base is row-major [N, K] (w_tiled = 0), the

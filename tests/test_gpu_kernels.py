@@ -1014,3 +1014,133 @@ def test_batched_calls_after_a_wide_single_call(dev):
             assert o.rel_err(y.cpu().numpy(), ref) <= TOL
     finally:
         ops.set_ksplit(0)
+
+
+def _mixed_call(p, w, tiled, table, bits, gs, y, acc, parts, deltas):
+    from deltazip_amd import _lib
+    t, n, k = y.shape[0], y.shape[1], p["x"].shape[1]
+    sums = torch.full((parts * t * n,), float("nan"), dtype=torch.float32, device=y.device) if parts > 1 else None
+    rc = _lib.lib().dz_multi_delta_gemm_mixed(
+        p["x"].data_ptr(), w.data_ptr(), tiled, p["q"].data_ptr(), p["m"].data_ptr(), p["s"].data_ptr(), p["q"].shape[0], bits,
+        gs, table.table.data_ptr(), table.max_blocks, deltas, y.data_ptr(), t, k, n, acc, y.stride(0), parts,
+        None if sums is None else sums.data_ptr(), torch.cuda.current_stream().cuda_stream)
+    assert rc == 0
+    torch.cuda.synchronize()
+    return y
+
+
+@pytest.mark.parametrize("n,k,bits,gs,nd,t,tiles,most", [
+    (32, 256, 2, -1, 4, 129, 8, 4), (288, 512, 2, -1, 9, 300, 8, 4), (544, 768, 2, 64, 5, 517, 8, 3),
+    (256, 1280, 4, 128, 7, 130, 8, 3), (96, 1536, 4, 192, 40, 257, 8, 3), (320, 512, 4, -1, 3, 400, 8, 3),
+    (160, 768, 2, 192, 17, 140, 4, 2), (512, 1024, 4, 64, 20, 333, 4, 2), (64, 512, 2, -1, 1, 1000, 8, 4),
+    (96, 512, 2, -1, 60, 150, 2, 1)])
+def test_blocks_of_several_deltas(dev, n, k, bits, gs, nd, t, tiles, most):
+    """dz_build_mixed and dz_multi_delta_gemm_mixed: every token in one row of one block, tiles of one delta,
+    blocks within their limits; unsorted ids with base-only tokens, N that is no multiple of 256, whole and split K,
+    rows and tiles, plain and added into a column slice.  Unsplit sums are those of the kernel with one delta
+    per block, in the same order: equal bits.  Split: fp32 partial sums added once more, within one
+    fp16 rounding of the unsplit result and a few fp32 ones."""
+    from deltazip_amd import _lib
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    p = make_problem(n, k, bits, gs, nd, t, "uniform", 77 + n + t, dev)
+    p["ids_np"] = p["ids_np"].copy()
+    p["ids_np"][::11] = -1
+    ids = torch.from_numpy(p["ids_np"]).to(dev)
+    perm, off = ops.segment(ids, nd)
+    room = L.dz_mixed_blocks(t, nd, tiles, most)
+    table = ops.MixedTable(torch.full((4 + room * 146,), 77, dtype=torch.int32, device=dev), room, most)
+    assert L.dz_build_mixed(off.data_ptr(), perm.data_ptr(), nd, t, tiles, most, table.table.data_ptr(), room, st) == 0
+    torch.cuda.synchronize()
+    tab = table.table.cpu().numpy()
+    blocks, seen = tab[4:].reshape(room, 146)[:tab[0]], []
+    assert 0 < tab[0] <= room
+    for b in blocks:
+        bt, bd, slot, tend, rows = b[0], b[1], b[2:6], b[14:18], b[18:]
+        assert 1 <= bt <= tiles and 0 <= bd <= most
+        for tile in range(bt):
+            e = int(np.searchsorted(tend[:max(bd, 1)], tile, side="right")) if bd else 0
+            held = rows[16 * tile:16 * tile + 16]
+            seen += [r for r in held if r >= 0]
+            want = slot[e] if bd else -1
+            assert all(p["ids_np"][r if r >= 0 else ~r] == want for r in held) and held[0] >= 0
+        assert all(r < 0 for r in rows[16 * bt:])
+    assert sorted(seen) == list(range(t))
+
+    short = ops._block_table(t, nd, 128, dev)
+    assert L.dz_build_tiles_rows(off.data_ptr(), nd, 128, short[0].data_ptr(), short[1], st) == 0
+    one = torch.empty(t, n, dtype=torch.float16, device=dev)
+    assert L.dz_multi_delta_gemm_rows(p["x"].data_ptr(), p["wb"].data_ptr(), 0, p["q"].data_ptr(), p["m"].data_ptr(),
+                                      p["s"].data_ptr(), nd, bits, gs, short[0].data_ptr(), short[1], perm.data_ptr(),
+                                      one.data_ptr(), t, k, n, 0, n, st) == 0
+    ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
+    base = torch.from_numpy(o.make_x(t, n, 5)).to(dev)
+    for w, tiled in ((p["wb"], 0), (ops.tile_base(p["wb"]), 1)):
+        for parts in sorted({1, min(2, k // 256), min(3, k // 256), k // 256}):
+            wide = torch.zeros(t, n + 32, dtype=torch.float16, device=dev)
+            y = _mixed_call(p, w, tiled, table, bits, gs, torch.full((t, n), float("nan"), dtype=torch.float16, device=dev), 0,
+                            parts, most)
+            assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+            if parts == 1:
+                assert torch.equal(y, one)
+            else:
+                # |sum of parts - sum| <= (parts + K / 8) fp32 roundings of a value below 64, then half a unit each
+                assert ((y.float() - one.float()).abs() <= 2.0**-10 * one.float().abs() + 2e-3).all()
+            y = wide[:, 16:16 + n]
+            y.copy_(base)
+            _mixed_call(p, w, tiled, table, bits, gs, y, 1, parts, most)
+            assert o.rel_err(y.float().cpu().numpy(), ref + base.float().cpu().numpy()) <= TOL
+            assert not wide[:, :16].any() and not wide[:, 16 + n:].any()
+    if most == 4:                                         # three deltas at most elsewhere
+        assert L.dz_multi_delta_gemm_mixed(p["x"].data_ptr(), p["wb"].data_ptr(), 0, p["q"].data_ptr(), p["m"].data_ptr(),
+                                           p["s"].data_ptr(), nd, 4, -1, table.table.data_ptr(), room, 4, one.data_ptr(), t, k,
+                                           n, 0, n, 1, None, st) == -2
+
+
+def test_blocks_of_several_deltas_keep_tokens_apart(dev):
+    """A block's tokens share tiles of activations and nothing else: an infinite scale reaches its own delta's
+    tokens only, an infinite or NaN activation its own token only."""
+    p = make_problem(256, 1280, 2, -1, 6, 300, "uniform", 9, dev)
+    plan = ops._mixed_plan(300, 1280, 256)
+    assert plan is not None
+    clean = run_layer(p)
+    s = p["s"].clone()
+    s[2] = float("inf")
+    x = p["x"].clone()
+    x[17, 5], x[44, 1000] = float("inf"), float("nan")
+    y = run_layer(dict(p, s=s, x=x))
+    touched = torch.from_numpy(p["ids_np"] == 2).to(dev)
+    touched[[17, 44]] = True
+    assert torch.equal(y[~touched], clean[~touched])
+    assert not torch.isfinite(y[17]).all() and torch.isnan(y[44]).all()
+
+
+@pytest.mark.parametrize("t,n,k,parts", [(200, 1280, 2560, 2), (700, 12288, 1280, 1)])
+def test_blocks_of_several_deltas_under_capture(dev, t, n, k, parts):
+    """A captured call over blocks of several deltas reads the ids of the replay, and gives the eager call's bits,
+    with tensors of other sizes made and dropped in between."""
+    p = make_problem(n, k, 2, -1, 5, t, "uniform", 3, dev)
+    assert ops._mixed_plan(t, k, n)[1] >= parts
+    ids = p["ids"].clone()
+    tiled = ops.tile_base(p["wb"])
+    call = lambda: ops.apply_delta(p["x"], p["q"], p["s"], p["m"], ids, p["wb"], base_tiled=tiled)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        call()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph, stream=side):
+            y = call()
+    torch.cuda.current_stream().wait_stream(side)
+    rng = np.random.default_rng(t)
+    for rep in range(4):
+        ids.copy_(torch.from_numpy(rng.integers(-1, 5, t) if rep else np.zeros(t, dtype=np.int64)))
+        want = call()
+        blocks = ops.row_blocks(ids, 5, deltas=ops.mixed_deltas(2, False))
+        known = ops.apply_delta(p["x"], p["q"], p["s"], p["m"], ids, p["wb"], order=blocks, base_tiled=tiled)
+        junk = torch.full((1 + rep, t), 1 << 20, dtype=torch.int32, device=dev)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y, want) and torch.equal(known, want), rep
+        del junk

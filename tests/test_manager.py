@@ -577,3 +577,18 @@ def test_manager_with_one_copy_of_the_base_weights(dev):
         torch.cuda.synchronize()
         for a, b in zip(*outs):
             assert torch.equal(a, b), T
+
+
+@pytest.mark.parametrize("t,k,n,plan", [
+    (128, 4096, 4096, None), (129, 1024, 8192, None), (2000, 1024, 8192, (0, 1)),        # a short walk
+    (129, 5120, 27648, (0, 1)), (8192, 5120, 27648, (0, 1)), (333, 4096, 12288, (0, 1)),  # enough workgroups
+    (230, 2048, 2048, (1, 4)), (333, 13824, 5120, (0, 4)), (333, 5120, 5120, (0, 4)),     # few: K in parts
+    (300000, 4096, 4096, None)])                                                          # 32-bit offsets
+def test_plan_of_blocks_of_several_deltas(t, k, n, plan):
+    """By the sizes alone; where the host knows the mix, a few tokens of each of many deltas go elsewhere."""
+    assert ops._mixed_plan(t, k, n) == plan
+    assert ops._in_mixed_blocks(t, k, n, 769, None) is None
+    many = ops._even_mix(t, t)
+    assert ops._in_mixed_blocks(t, k, n, 64, None) == plan
+    if plan is not None and (k >= 2 * n and t <= 512):
+        assert ops._in_mixed_blocks(t, k, n, 64, many) is None
