@@ -178,7 +178,7 @@ class LinearWithDelta(BaseLayerWithDelta):
     def apply_weights(self, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         T = self.indices_len[0]
         order = self.token_order[:T] if self.token_order is not None and 32 < T <= ops.MAX_TOKENS_FUSED else None
-        if T > ops.MAX_TOKENS_FUSED and self.row_blocks is not None:
+        if T > 32 and self.row_blocks is not None and (T > ops.MAX_TOKENS_FUSED or self.row_blocks[0] is not None):
             order = self.row_blocks[0]
         w = self.base_layer.weight
         if self._row_major_dropped:

@@ -206,6 +206,7 @@ class DeltaModelManager:
         self.packed_modules: Dict[str, List[str]] = {}
         self.modules: Dict[str, BaseLayerWithDelta] = {}
         self._widest = 0                 # output features of the widest linear layer
+        self._largest = (0, 0)           # K, N of the one with the most weights
         self._last_mapping: Optional[DeltaMapping] = None
         self._wrap_modules()
         self.model.delta_manager = self
@@ -360,13 +361,16 @@ class DeltaModelManager:
         if 32 < T <= ops.MAX_TOKENS_FUSED:
             ops.token_order(self.base_indices[:T], self.delta_slots, out=self.token_order)
         self.row_blocks[0] = None
-        if T > ops.MAX_TOKENS_FUSED and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
+        decode = 32 < T <= ops.MAX_TOKENS_FUSED
+        wanted = T > ops.MAX_TOKENS_FUSED or (decode and ops.mixes_at_decode(T, *self._largest, len(set(mapping.index_mapping))))
+        if wanted and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
             # (the mix decides at sizes where other routes than row blocks may be the faster one)
             self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
                                                 mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
                                                 features=self._widest or None,
                                                 deltas=ops.mixed_deltas(self.delta_config.max_bitwidth,
-                                                                        self.delta_config.group_size != -1))
+                                                                        self.delta_config.group_size != -1),
+                                                order=self.token_order[:T] if decode else None)
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 
@@ -428,7 +432,9 @@ class DeltaModelManager:
             raise TypeError("only delta-carrying layers are registered")
         self.modules[module_name] = module
         if isinstance(module, LinearWithDelta):
-            self._widest = max(self._widest, getattr(module, "base_shape", (0, 0))[0])
+            n, k = getattr(module, "base_shape", (0, 0))
+            self._widest = max(self._widest, n)
+            self._largest = max(self._largest, (k, n), key=lambda kn: kn[0] * kn[1])
         # a fused layer also answers for the projections it is made of (q/k/v, gate/up)
         parent, _, leaf = module_name.rpartition(".")
         parts = self.packed_modules_mapping.get(leaf)

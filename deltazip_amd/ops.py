@@ -171,15 +171,17 @@ class RowBlocks:
     (what dz_segment and dz_build_tiles write): depends on the indices only, so it can be made once
     per batch and passed to every layer call of the step (`order=`).  `tiles` are blocks of up to
     256 tokens, `short` blocks of up to 128 for the kernel with the smaller tile; either may be None.
-    `mixed`: tables of blocks of several deltas (MixedTable), full and small ones, or None.
+    `mixed`: tables of blocks of several deltas (MixedTable), full and small ones, or None.  Up to 128 tokens these
+    are all there is, and `order` is the token order for layers that go another way.
     They serve the side of a graph capture they were made on (`captured`), see `_usable_blocks`.
     `mix`: what the maker knew of the batch on the host, or None; `host_picks`: both tables hold all rows."""
-    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix", "host_picks", "mixed")
+    __slots__ = ("perm", "tiles", "max_tiles", "T", "S", "short", "max_short", "captured", "mix", "host_picks", "mixed", "order")
 
-    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None, host_picks=False, mixed=None):
+    def __init__(self, perm, tiles, max_tiles, T, S, short=None, max_short=0, mix=None, host_picks=False, mixed=None,
+                 order=None):
         self.perm, self.tiles, self.max_tiles, self.T, self.S = perm, tiles, max_tiles, T, S
         self.short, self.max_short, self.mix, self.host_picks = short, max_short, mix, host_picks
-        self.mixed = mixed
+        self.mixed, self.order = mixed, order
         self.captured = torch.cuda.is_current_stream_capturing()
 
 
@@ -221,21 +223,46 @@ def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
         return None                                   # (32-bit offsets)
     if K <= 1024 and -(-T // 128) * -(-N // 128) <= 384:
         return None
-    wide, steps = -(-N // 256), K // 256
-    small = wide * T / 128 < (140 if K <= 3072 else 25)
-    blocks = -(-T // (64 if small else 128))
-    best = None
+    small = -(-N // 256) * T / 128 < (140 if K <= 3072 else 25)
+    return int(small), _parts(T, K, N, -(-T // (64 if small else 128)), 1.0 if small else 1.7)
+
+
+def _parts(T: int, K: int, N: int, blocks: int, slab_us: float) -> int:
+    """Parts of K for so many blocks: what a wave of workgroups takes to start and to walk its part of K, alone
+    and with all CUs busy, and the pass over the partial sums."""
+    wide, steps, best = -(-N // 256), K // 256, None
     for parts in (1, 2, 3, 4, 6):
         if parts > steps:
             break
         groups = wide * blocks * parts
         waves = -(-groups // 256) if groups <= 1024 else groups / 256
-        cost = waves * (8 + -(-steps // parts) * 4 * (1.0 if small else 1.7) * (0.6 + 0.4 * min(1.0, groups / 256)))
+        cost = waves * (8 + -(-steps // parts) * 4 * slab_us * (0.6 + 0.4 * min(1.0, groups / 256)))
         if parts > 1:
             cost += 3 + 8 * T * N * parts / 3e6
         if best is None or cost < best[0]:
             best = (cost, parts)
-    return int(small), best[1]
+    return best[1]
+
+
+def mixes_at_decode(T: int, K: int, N: int, deltas: int) -> bool:
+    """Whether a batch of 33 to 128 tokens of so many deltas (the base model counts as one) goes in blocks of several
+    deltas: the decode kernel makes its products once per 32 tokens and delta, a block once per 16 tokens and never
+    twice for a weight it has in registers; with many deltas the blocks are many and short.  By 840 timed calls over
+    layers of 20 M weights and more, in the mean and at worst: 33 tokens of up to 8 deltas 1.37 / 0.96 times as
+    fast, 48 and 64 tokens of 1 or 2 1.34 / 0.92 (of 7 or 8 1.14 / 0.81: left as they are), 96 tokens of up to 8
+    1.41 / 0.97, 128 of up to 8 1.66 / 1.14 and of 13 to 16 1.33 / 0.97 (of more 1.01 / 0.77).  5120 x 27648,
+    2-bit, 128 tokens of 4 / 8 / 16 deltas: 194 -> 102, 209 -> 132, 253 -> 230 us; 13824 x 5120: 122 -> 51, 129 -> 67, 151 ->
+    104.  Smaller layers take about the time of their calls' host half either way (a layer of 2048/5632, 100 tokens of
+    4 deltas: 116 / 125 us)."""
+    if not 32 < T <= MAX_TOKENS_FUSED or K * N < 24 << 20:
+        return False
+    return deltas <= (16 if T > 112 else 8 if T > 64 or T <= 40 else 2)
+
+
+@lru_cache(maxsize=4096)
+def _decode_plan(T: int, K: int, N: int, deltas: int) -> Tuple[int, int]:
+    """`_mixed_plan` of such a batch, whose number of blocks is that of its deltas."""
+    return 0, _parts(T, K, N, max(1, -(-deltas // 4)), 1.7)
 
 
 def _in_mixed_blocks(T: int, K: int, N: int, S: int, mix: Optional["BatchMix"]) -> Optional[Tuple[int, int]]:
@@ -352,7 +379,8 @@ def _mixed_table(T: int, S: int, small: int, deltas: int, device) -> MixedTable:
 
 
 def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
-               device_picks: bool = False, features: Optional[int] = None, deltas: int = 3) -> RowBlocks:
+               device_picks: bool = False, features: Optional[int] = None, deltas: int = 3,
+               order: Optional[torch.Tensor] = None) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
     (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
@@ -377,13 +405,14 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     widest layer they are for, if known.
 
     Layers with a base weight take the batch in blocks of several deltas where those pay (`_mixed_plan`): their
-    tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers."""
+    tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers.  `order`: token_order() of the same
+    indices, for a batch of up to 128 tokens (mixes_at_decode)."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
     T = indices.numel()
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
-    perm, seg_off = segment(indices, num_slots, not long_only and T > MAX_TOKENS_FUSED and takes_fused_chunks(T, num_slots))
+    perm, seg_off = segment(indices, num_slots, not long_only and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
     narrow = features is not None and -(-features // 256) * -(-T // 256) <= 128 and T < 256 * (num_slots + 1)
     small = not long_only and not device_picks and (T <= 1024 or narrow)
@@ -391,7 +420,7 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     host_picks = small and mix is not None and mix.deltas == 1 and 448 < T <= 512
     if not small or host_picks:
         tiles, n = _block_table(T, num_slots, 256, dev)
-    if small or device_picks or (not long_only and T < 256 * (num_slots + 1)):
+    if T > MAX_TOKENS_FUSED and (small or device_picks or (not long_only and T < 256 * (num_slots + 1))):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
     if long_only:
         _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
@@ -402,7 +431,7 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
                                  int(tiles is not None and short is not None and not host_picks), mixed[0].deltas,
                                  mixed[0].table.data_ptr(), mixed[0].max_blocks, mixed[1].table.data_ptr(),
                                  mixed[1].max_blocks, st), "dz_build_tables")
-    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks, mixed)
+    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks, mixed, order)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,
@@ -946,6 +975,19 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
                                           indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
                                           base_tiled=base_tiled)
+    if T > 32 and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT:
+        blocks = order if isinstance(order, RowBlocks) and order.order is not None else None
+        if blocks is not None and (blocks.T != T or blocks.S != S
+                                   or blocks.captured != torch.cuda.is_current_stream_capturing()):
+            blocks = None
+        # A call that has to make its own table takes 8 us for it: large layers over few slots only (5120 x 13824, 100
+        # tokens of 4 slots 104 -> 70 us; 4096 x 12288, 4-bit, 128 tokens of 8 106 / 111).
+        met = blocks.mix.deltas if blocks is not None else S if order is None and T > 64 and S <= 4 and K * N >= 40 << 20 else T
+        if mixes_at_decode(T, K, N, met):
+            from .prefill import multi_delta_linear_mixed
+            return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
+                                            bits=bits, out=out, accumulate=accumulate, plan=_decode_plan(T, K, N, met),
+                                            blocks=blocks, base_tiled=base_tiled)
     ws = _workspace(x.device, T, K, N)
     optr = _order_ptr(order, T, x.device)
     if base_tiled is not None:
@@ -997,7 +1039,10 @@ def apply_delta(x: torch.Tensor, qweight_stacked: torch.Tensor, scales_stacked: 
 
 def _order_ptr(order: Optional[torch.Tensor], T: int, device) -> Optional[int]:
     if isinstance(order, RowBlocks):
-        raise ValueError("row blocks are for batches above %d tokens; pass token_order() here" % MAX_TOKENS_FUSED)
+        if order.order is None or order.T != T:
+            raise ValueError("row blocks are for batches above %d tokens; pass token_order() here" % MAX_TOKENS_FUSED)
+        # (a captured call makes its own from the indices, as it makes its own row blocks)
+        order = order.order if order.captured == torch.cuda.is_current_stream_capturing() else None
     if order is None or T <= 32:
         return None
     if (not order.is_cuda or order.device != device or order.dtype != torch.int32 or order.numel() < T

@@ -1144,3 +1144,42 @@ def test_blocks_of_several_deltas_under_capture(dev, t, n, k, parts):
         torch.cuda.synchronize()
         assert torch.equal(y, want) and torch.equal(known, want), rep
         del junk
+
+
+@pytest.mark.parametrize("bits,gs,t,met", [(2, -1, 33, 3), (2, -1, 128, 16), (4, 128, 96, 8), (4, -1, 70, 1)])
+def test_decode_batches_of_few_deltas(dev, bits, gs, t, met):
+    """33 to 128 tokens of few deltas over a layer of 25 M weights: with the blocks its maker hands on the call
+    goes in blocks of several deltas, without them through the decode kernel; the two differ by the order of fp32
+    sums (as between parts of K) and one rounding.  Bad ids are reported either way; blocks of another batch
+    are refused."""
+    from deltazip_amd.synthetic import gaussian_native_stack
+    n, k, S = 10240, 2560, 20
+    gen = torch.Generator(device=dev).manual_seed(t)
+    q, m, s = gaussian_native_stack(k, n, bits, k if gs == -1 else gs, 4, dev, gen)
+    q, m, s = (v.repeat((5,) + (1,) * (v.dim() - 1)).contiguous() for v in (q, m, s))
+    w, x = (torch.randn(n, k, device=dev, generator=gen) * 0.02).half(), torch.randn(t, k, device=dev, generator=gen).half()
+    tiled, ids_np = ops.tile_base(w), np.random.default_rng(t).integers(0, met, t)
+    ids_np[:met] = np.arange(met)
+    ids_np[t // 2] = -1 if met < 8 else 0
+    ids = torch.from_numpy(ids_np).to(dev)
+    mix = ops.batch_mix(ids_np.tolist())
+    assert ops.mixes_at_decode(t, k, n, mix.deltas)
+    order = ops.token_order(ids, S)
+    blocks = ops.row_blocks(ids, S, mix=mix, deltas=ops.mixed_deltas(bits, gs != -1), order=order)
+    call = lambda o_, i=ids: ops.apply_delta(x, q, s, m, i, w, order=o_, base_tiled=tiled)
+    y, y0 = call(blocks), call(order)
+    torch.cuda.synchronize()
+    assert ((y.float() - y0.float()).abs() <= 2.0**-10 * y0.float().abs() + 2e-3).all()
+    assert not torch.equal(y, y0)                          # (it did go the other way)
+    with pytest.raises(ValueError):
+        ops.apply_delta(x[:32 + 1], q, s, m, ids[:33].contiguous() if t != 33 else torch.cat([ids, ids])[:40], w, order=blocks)
+    ops.poll_status(wait=True)
+    bad = torch.where(ids == 0, torch.full_like(ids, S + 3), ids)
+    base = torch.where(ids == 0, torch.full_like(ids, -1), ids)
+    made = [ops.row_blocks(i, S, mix=mix, deltas=3, order=ops.token_order(i, S)) for i in (bad, base)]
+    yb, yg = call(made[0], bad), call(made[1], base)
+    torch.cuda.synchronize()
+    assert torch.equal(yb, yg) and ops.workspace_status() == ops.STATUS_BAD_ID
+    warned, ops._warned_bad_id = ops._warned_bad_id, True
+    ops.poll_status(wait=True)
+    ops._warned_bad_id = warned
