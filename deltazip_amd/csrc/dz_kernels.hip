@@ -498,7 +498,7 @@ __device__ __forceinline__ uint32_t or_quad(uint32_t v) {
 }
 
 //
-// GS = 0: scales from memory.  GS = 64, 128, 256: the tile holds whole scale groups, so their scales are
+// GS = 0: scales from memory (groups of another length, and whole rows of more than 16384 columns).  GS = 64, 128, 256: the tile holds whole scale groups, so their scales are
 // found here from the values just read (and written out) rather than in a pass of their own
 // (4096 x 11008, 4-bit, groups of 128: 90 us with one wavefront per tile, now 75, of 64 88 and 74).
 constexpr int COMPRESS_WAVES = 4;   // per tile: rows 4w .. 4w + 3 and 16 + 4w .. of wavefront w
@@ -580,6 +580,105 @@ __global__ __launch_bounds__(64 * COMPRESS_WAVES) void dz_compress_kernel(const 
     *(u4_t*)(codes + dz_code4_word(np, kb, lane, 0, 0, nkb)) = *(const u4_t*)(words + 256 + lane * 4);
   } else if (wave == 1) {
     *(u4_t*)(codes + dz_code4_word(np, kb, lane, 2, 0, nkb)) = *(const u4_t*)(words + (BITS == 2 ? 256 : 512) + lane * 4);
+  }
+}
+
+// One scale per row: the values are read once.  A workgroup of eight wavefronts holds R rows of either half
+// of an n-pair (rows i0 .. i0 + R - 1 and 16 + i0 ..) whole, in registers, CH k-blocks per wavefront; the
+// rows' extremes meet in LDS, and the codes are made from the registers.  The words of R neighbouring rows
+// are 16 * R bytes of the native arrays, written from LDS.  Bound by memory: with a pass for the scales and a
+// second reading 4096 x 11008, 2 bits, 65 us, now 40 (192 MB, 4.8 TB/s); 5120 x 13824 97 -> 59, 11008 x 4096 69 -> 41,
+// 2048 x 2048 18 -> 16.  R is such that a lane holds 32 values (64 where a row has more than 8192): with
+// 64 values 4096 x 11008 took 48 us, with 128 5120 x 13824 110: one workgroup per CU then loads, and
+// the next computes nothing beside it.
+template <int BITS, int CH, int R>
+__global__ __launch_bounds__(512, 2) void dz_compress_rows_kernel(const float* __restrict__ delta,
+                                                                  float* __restrict__ scale32, _Float16* __restrict__ scale16,
+                                                                  int K, int N, uint32_t* __restrict__ codes,
+                                                                  uint32_t* __restrict__ meta) {
+  constexpr int WAVES = 8, SETS = 1 + BITS / 2;    // 16-byte chunks per (row pair, 16 columns): positions, codes
+  __shared__ float tops[WAVES][2 * R];             // largest magnitude; its sign: whether a value is negative
+  __shared__ float2 sct[2 * R];                    // scale, 1 / scale or NaN
+  __shared__ __attribute__((aligned(16))) uint32_t words[WAVES][SETS * R * 16];
+  const int nkb = K / DZ_KBLOCK, per = 16 / R;
+  // (the rows of an n-pair on one XCD: their words share the lines of its L2)
+  const int np = (int)(blockIdx.x / (8 * per)) * 8 + (int)(blockIdx.x & 7), i0 = (int)(blockIdx.x >> 3) % per * R;
+  if (np >= N / DZ_NPAIR) return;
+  const int tid = threadIdx.x, lane = tid & 63, j = lane >> 4, ga = (lane >> 2) & 3, p = lane & 3;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const float* src = delta + ((size_t)np * DZ_NPAIR + i0) * K + lane * 4;
+  f4_t v[CH][2 * R];
+#pragma unroll
+  for (int c = 0; c < CH; ++c)
+#pragma unroll
+    for (int r = 0; r < 2 * R; ++r)                // (beyond the row: its last k-block again, not stored)
+      v[c][r] = *(const f4_t*)(src + (size_t)(r < R ? r : 16 + r - R) * K + min(wave + WAVES * c, nkb - 1) * DZ_KBLOCK);
+#pragma unroll
+  for (int r = 0; r < 2 * R; ++r) {
+    float top = 0.f;
+    bool neg = false;
+#pragma unroll
+    for (int c = 0; c < CH; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        top = fmaxf(top, fabsf(v[c][r][e]));       // (a NaN has no say)
+        neg = neg || v[c][r][e] < 0.f;
+      }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) top = fmaxf(top, __shfl_xor(top, o));
+    const bool any = __ballot(neg) != 0;
+    if (lane == 0) tops[wave][r] = any ? -top : top;   // (negative: top > 0)
+  }
+  __syncthreads();
+  if (tid < 2 * R) {
+    float top = 0.f;
+    bool any = false;
+#pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+      const float t = tops[w][tid];
+      top = fmaxf(top, fabsf(t));
+      any = any || t < 0.f;
+    }
+    const float sc = symmetric_scale(any ? -top : 0.f, top, (float)((1 << BITS) - 1));
+    sct[tid] = make_float2(sc, sc >= 0x1p-100f && sc <= 0x1p100f ? 1.f / sc : __builtin_nanf(""));
+    const int row = np * DZ_NPAIR + i0 + (tid < R ? tid : 16 + tid - R);
+    scale32[row] = sc;
+    scale16[row] = (_Float16)sc;
+  }
+  __syncthreads();
+  uint32_t* const mine = words[wave];
+  // lane p of four keeps the positions (0), the codes (1), or the codes of row 16 + i at 4 bits (2)
+  const int set = p == 0 ? 0 : BITS == 2 ? 1 : 1 + (j >> 1), at = p == 0 || BITS == 2 ? j : 2 * (j & 1) + (p - 1);
+#pragma unroll
+  for (int c = 0; c < CH; ++c) {
+    const int kb = wave + WAVES * c;
+    if (kb >= nkb) break;
+#pragma unroll
+    for (int u = 0; u < R; ++u) {
+      uint32_t mw = 0, cw[2] = {0, 0};
+#pragma unroll
+      for (int s = 0; s < 2; ++s) {
+        const float2 sc = sct[s * R + u];
+        uint32_t pos, clo, chi;
+        compress_group<BITS>(v[c][s * R + u], sc.x, sc.y, pos, clo, chi);
+        mw |= pos << dz_meta_shift(s, 2 * p);
+        if (BITS == 2) cw[0] |= (clo << dz_code2_shift(s, 2 * p)) | (chi << dz_code2_shift(s, 2 * p + 1));
+        else cw[s] = (clo << dz_code4_shift(2 * p)) | (chi << dz_code4_shift(2 * p + 1));
+      }
+      mw = or_quad(mw);
+      cw[0] = or_quad(cw[0]);
+      if (BITS == 4) cw[1] = or_quad(cw[1]);
+      if (p < (BITS == 2 ? 2 : 3)) mine[(set * 4 * R + ga * R + u) * 4 + at] = p == 0 ? mw : p == 1 ? cw[0] : cw[1];
+    }
+    __builtin_amdgcn_wave_barrier();               // (one wavefront's own words: LDS keeps its order)
+    if (lane < SETS * 4 * R) {
+      const int which = lane / (4 * R), q = lane % (4 * R), la = 16 * (q / R) + i0 + q % R;
+      uint32_t* dst = which == 0 ? meta + dz_meta_word(np, kb, la, 0, nkb)
+                                 : codes + (BITS == 2 ? dz_code2_word(np, kb, la, 0, nkb)
+                                                      : dz_code4_word(np, kb, la, 2 * (which - 1), 0, nkb));
+      *(u4_t*)dst = *(const u4_t*)(mine + lane * 4);
+    }
+    __builtin_amdgcn_wave_barrier();
   }
 }
 
@@ -854,6 +953,20 @@ int dz_compress_2of4(const float* delta, int K, int N, int bits, int group_size,
     case 128: bits == 2 ? go(dz_compress_kernel<2, 128>) : go(dz_compress_kernel<4, 128>); break;
     case 256: bits == 2 ? go(dz_compress_kernel<2, 256>) : go(dz_compress_kernel<4, 256>); break;
     default:
+      if (gs == K && K <= 64 * DZ_KBLOCK) {
+        // a row's k-blocks over eight wavefronts, at most eight each; the pass for the scales and the tiles are
+        // left to longer rows, of which a lane would hold 128 values and more
+        const int nkb = K / DZ_KBLOCK;
+        auto rows = [&](auto kern, int r) {
+          hipLaunchKernelGGL(kern, dim3((unsigned)((N / DZ_NPAIR + 7) / 8 * 8) * (16 / r)), dim3(512), 0, st, delta, scale_workspace,
+                             (_Float16*)out_scales, K, N, (uint32_t*)out_codes, (uint32_t*)out_meta);
+        };
+        if (nkb <= 8) bits == 2 ? rows(dz_compress_rows_kernel<2, 1, 4>, 4) : rows(dz_compress_rows_kernel<4, 1, 4>, 4);
+        else if (nkb <= 16) bits == 2 ? rows(dz_compress_rows_kernel<2, 2, 2>, 2) : rows(dz_compress_rows_kernel<4, 2, 2>, 2);
+        else if (nkb <= 32) bits == 2 ? rows(dz_compress_rows_kernel<2, 4, 1>, 1) : rows(dz_compress_rows_kernel<4, 4, 1>, 1);
+        else bits == 2 ? rows(dz_compress_rows_kernel<2, 8, 1>, 1) : rows(dz_compress_rows_kernel<4, 8, 1>, 1);
+        break;
+      }
       launch_scales(delta, K, N, bits, gs, scale_workspace, out_scales, st);
       bits == 2 ? go(dz_compress_kernel<2, 0>) : go(dz_compress_kernel<4, 0>);
   }

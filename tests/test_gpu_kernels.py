@@ -1183,3 +1183,26 @@ def test_decode_batches_of_few_deltas(dev, bits, gs, t, met):
     warned, ops._warned_bad_id = ops._warned_bad_id, True
     ops.poll_status(wait=True)
     ops._warned_bad_id = warned
+
+
+@pytest.mark.parametrize("n,k", [(32, 512), (288, 2048), (64, 2304), (96, 4096), (32, 4352), (288, 8192), (32, 8448), (64, 16384),
+                                 (32, 16640)])
+@pytest.mark.parametrize("bits", [2, 4])
+def test_compressor_of_whole_rows(dev, n, k, bits):
+    """One scale per row, at the edges of the k-blocks a wavefront holds and beyond the longest row held whole: the
+    bytes of the separate passes (dz_quant_scales, dz_pack_2of4), for ordinary rows and for rows of zeros, of one
+    sign, with a single value, with infinities and NaNs."""
+    gen = torch.Generator(device=dev).manual_seed(n + k)
+    d = torch.randn(n, k, device=dev, generator=gen) * 1e-3
+    d[0] = 0
+    d[1] = d[1].abs()
+    d[2, :] = -0.0
+    d[3] = 0
+    d[3, k - 1] = -7.0
+    d[17, 5], d[18, 256], d[19] = float("inf"), float("nan"), float("nan")
+    d[20] = d[20].sign() * 1e-40
+    q, m, s = ops.compress_delta(d, bits)
+    s32, s16 = ops.quant_scales(d, bits)
+    q0, m0 = ops.pack_2of4(d, s32, bits)
+    torch.cuda.synchronize()
+    assert torch.equal(s.view(torch.int16), s16.view(torch.int16)) and torch.equal(q, q0) and torch.equal(m, m0)
