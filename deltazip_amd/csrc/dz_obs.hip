@@ -46,59 +46,84 @@ __device__ __forceinline__ void outer_add(float (&acc)[NI][NJ], const float (&va
   }
 }
 
-// N steps of acc += a b^T over operands staged in LDS: a 4 values at pa + k * lda, b 4 values each at
-// pb + k * ldb and pb + k * ldb + second.  The operands of a step are read while the step before is summed.
-template <int N>
-__device__ __forceinline__ void outer_steps(float (&acc)[4][8], const float* pa, int lda, const float* pb, int ldb,
-                                            int second) {
-  f4_t a = *(const f4_t*)pa, b = *(const f4_t*)pb, c = *(const f4_t*)(pb + second);
-#pragma unroll 4
-  for (int k = 0; k < N; ++k) {
-    // (the read behind the last step repeats the first)
-    pa = k + 1 < N ? pa + lda : pa - (N - 1) * lda;
-    pb = k + 1 < N ? pb + ldb : pb - (N - 1) * ldb;
-    const f4_t an = *(const f4_t*)pa, bn = *(const f4_t*)pb, cn = *(const f4_t*)(pb + second);
-    __builtin_amdgcn_sched_barrier(0);
-    const float va[4] = {a[0], a[1], a[2], a[3]}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
-    outer_add(acc, va, vb);
-    a = an;
-    b = bn;
-    c = cn;
+template <int NV>
+struct vec_of {
+  typedef float t __attribute__((ext_vector_type(NV)));
+  typedef float u __attribute__((ext_vector_type(NV), aligned(4)));   // of an array that is aligned to its elements only
+};
+
+// n steps of acc += a b^T over operands staged in LDS: NI values at pa + k * lda, and NJ at pb + k * ldb, or
+// for NJ = 8 four of them there and four at pb + k * ldb + second.  The operands of a step are read while the
+// step before is summed.  N: a multiple of 8, or 0 for n, which is one.
+template <int N, int NI, int NJ>
+__device__ __forceinline__ void outer_steps(float (&acc)[NI][NJ], const float* pa, int lda, const float* pb, int ldb,
+                                            int second, int n = N) {
+  constexpr int NB = NJ == 8 ? 4 : NJ;
+  typedef typename vec_of<NI>::t a_t;
+  typedef typename vec_of<NB>::t b_t;
+  a_t a = *(const a_t*)pa;
+  b_t b = *(const b_t*)pb, c;
+  if constexpr (NJ == 8) c = *(const b_t*)(pb + second);
+  if (N) n = N;
+  for (int k0 = 0; k0 < n; k0 += 8) {
+#pragma unroll
+    for (int k = k0; k < k0 + 8; ++k) {
+      // (the read behind the last step repeats the first)
+      pa = k + 1 < n ? pa + lda : pa - (n - 1) * lda;
+      pb = k + 1 < n ? pb + ldb : pb - (n - 1) * ldb;
+      const a_t an = *(const a_t*)pa;
+      const b_t bn = *(const b_t*)pb;
+      b_t cn;
+      if constexpr (NJ == 8) cn = *(const b_t*)(pb + second);
+      __builtin_amdgcn_sched_barrier(0);
+      float va[NI], vb[NJ];
+#pragma unroll
+      for (int i = 0; i < NI; ++i) va[i] = a[i];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) vb[j] = j < NB ? b[j] : c[j - NB];
+      outer_add(acc, va, vb);
+      a = an;
+      b = bn;
+      if constexpr (NJ == 8) c = cn;
+    }
   }
 }
 
 // ---- H <- H * s0 + sum_t (s1 x[t, a]) * (s1 x[t, b]), t ascending.
 // Bound by the multiply-add rate.  The product of columns a and b has the same bits as that of b
 // and a, so only the tiles on and above the diagonal are summed and each is written to both places
-// (H itself need not be symmetric: either place scales its own old value).  64 x 64 outputs per
-// workgroup of two wavefronts, 4 x 8 per thread (three 16-byte LDS reads per 64 instructions; with
-// 4 x 4 per thread the LDS is the bound), 32 tokens staged at a time and the next 32 on their way
-// in registers.  The tile is this small because the tiles of a launch are equal and all run at
-// once: 2080 of them at K = 4096 are 8.1 per CU, a loss of a tenth where 64 x 128 would lose a fifth.
-// K = 4096, 2048 tokens: 1.38 -> 0.79 ms.
-template <typename XT>
-__global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ H, const XT* __restrict__ x, int T,
-                                                         int K, float s0, float s1) {
+// (H itself need not be symmetric: either place scales its own old value).  A tile of 64 x 64 is summed
+// by four wavefronts, 4 x 4 outputs per thread, 32 tokens of both sides staged at a time and the next 32 on
+// their way in registers.  With 4 x 8 per thread there is less to read from LDS (at full occupancy either
+// takes 82 us per 2048 tokens and tile of a CU), but two wavefronts per tile leave half the SIMDs
+// of a last tile idle and the others at half their rate: 2080 tiles at K = 4096 took 790 us for
+// 2048 tokens, now 665, 1128 tiles (K = 3072) 520, now 400.  A tile of 32 x 32 in four wavefronts, 2 x 2 per thread, is
+// for the tiles that do not go round the CUs: alone on a CU it takes 76 us where one of 64 x 64 takes 190 (290
+// with 4 x 8 per thread), but LDS bounds a CU full of them at 125 us for the outputs of one of 64 x 64.
+template <typename XT, int TILE, int NI, int NJ>
+__device__ __forceinline__ void hessian_tile(float* __restrict__ H, const XT* __restrict__ x, int T, int K, float s0, float s1,
+                                             int ta, int tb, float* sm) {
 #pragma clang fp contract(off)
-  constexpr int TC = sizeof(XT) == 2 ? 32 : 16;   // tokens per stage
+  constexpr int NT = TILE * TILE / (NI * NJ);
+  constexpr int STAGE = 2048 / TILE;                    // tokens that 16 KiB hold of both sides
+  constexpr int TC = sizeof(XT) == 2 ? STAGE : STAGE / 2;   // tokens per stage
   constexpr int PER = 16 / sizeof(XT);         // elements per 16-byte load
-  constexpr int ROWL = 64 / PER;               // loads per (token, 64 columns)
-  constexpr int NL = TC * ROWL / 128;          // loads per thread, stage and side
-  constexpr int TSTEP = 128 / ROWL;            // tokens between a thread's loads
-  __shared__ __attribute__((aligned(16))) float st[2][32][64];   // [a | b][token][column]; the mirrored tile at the end
-  // tile number -> (ta <= tb): number = tb (tb + 1) / 2 + ta
-  const int n = blockIdx.x;
-  int tb = (int)((sqrtf(8.f * (float)n + 1.f) - 1.f) * 0.5f);
-  while (tb * (tb + 1) / 2 > n) --tb;
-  while ((tb + 1) * (tb + 2) / 2 <= n) ++tb;
-  const int ta = n - tb * (tb + 1) / 2;
-  const int a0 = ta * 64, b0 = tb * 64;
-  const int tid = threadIdx.x, tr = tid >> 3, tc = tid & 7;   // rows 4 tr .. + 3, columns 4 tc .. + 3 and 32 + 4 tc .. + 3
-  float acc[4][8];
+  constexpr int ROWL = TILE / PER;             // loads per (token, TILE columns)
+  constexpr int NL = TC * ROWL / NT;           // loads per thread, stage and side
+  constexpr int TSTEP = NT / ROWL;             // tokens between a thread's loads
+  constexpr int CN = TILE / NJ;
+  static_assert(NL >= 1 && TC * ROWL % NT == 0, "");
+  typedef typename vec_of<NJ>::t b_t;
+  typedef typename vec_of<NJ>::u bu_t;
+  typedef typename vec_of<NI>::t a_t;
+  float(*st)[STAGE][TILE] = (float(*)[STAGE][TILE])sm;   // [a | b][token][column]; the mirrored tile at the end
+  const int a0 = ta * TILE, b0 = tb * TILE;
+  const int tid = threadIdx.x, tr = tid / CN, tc = tid % CN;   // rows NI tr .. + NI - 1, columns NJ tc .. + NJ - 1
+  float acc[NI][NJ];
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+    for (int j = 0; j < NJ; ++j) acc[i][j] = 0.f;
 
   typedef XT xv_t __attribute__((ext_vector_type(PER), aligned(sizeof(XT))));
   const int lt = tid / ROWL, lc = (tid % ROWL) * PER;
@@ -113,12 +138,10 @@ __global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ 
       next[1][l] = *(const xv_t*)(base + b0 + off);
     }
   };
-  fetch(0);
-  for (int t0 = 0; t0 < T; t0 += TC) {
-    __syncthreads();
+  auto place = [&](int tokens) {
 #pragma unroll
     for (int l = 0; l < NL; ++l) {
-      const bool in = t0 + lt + l * TSTEP < T;
+      const bool in = lt + l * TSTEP < tokens;
 #pragma unroll
       for (int side = 0; side < 2; ++side)
 #pragma unroll
@@ -130,38 +153,53 @@ __global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ 
           *(f4_t*)&st[side][lt + l * TSTEP][lc + v] = f;
         }
     }
+  };
+  const float *pa = &st[0][0][NI * tr], *pb = &st[1][0][NJ * tc];
+  fetch(0);
+  int t0 = 0;
+  for (; t0 + TC <= T; t0 += TC) {
+    __syncthreads();
+    place(TC);
     __syncthreads();
     if (t0 + TC < T) fetch(t0 + TC);
-    outer_steps<TC>(acc, &st[0][0][4 * tr], 64, &st[1][0][4 * tc], 64, 32);
+    outer_steps<TC>(acc, pa, TILE, pb, TILE, 0);
+  }
+  if (t0 < T) {
+    __syncthreads();
+    place(T - t0);
+    __syncthreads();
+    outer_steps<0>(acc, pa, TILE, pb, TILE, 0, (T - t0 + 7) & ~7);
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+  for (int i = 0; i < NI; ++i) {
+    bu_t* h = (bu_t*)(H + (size_t)(a0 + NI * tr + i) * K + b0 + NJ * tc);
+    const b_t old = *h;
+    b_t v;
 #pragma unroll
-    for (int j = 0; j < 8; j += 4) {
-      f4u_t* h = (f4u_t*)(H + (size_t)(a0 + 4 * tr + i) * K + b0 + 8 * j + 4 * tc);
-      const f4_t old = *h;
-      f4_t v;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float scaled = old[e] * s0;
-        v[e] = scaled + acc[i][j + e];
-      }
-      *h = v;
+    for (int e = 0; e < NJ; ++e) {
+      const float scaled = old[e] * s0;
+      v[e] = scaled + acc[i][e];
     }
+    *h = v;
+  }
   if (ta == tb) return;
   // the mirrored tile, turned in LDS (16-byte chunks of a row rotated by the row: no shared banks)
   float* turn = &st[0][0][0];
+  constexpr int NCH = TILE / 4;
+  auto chunk = [&](int b, int ch) { return turn + b * TILE + (((ch + b + (b >> 4)) & (NCH - 1)) << 2); };
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    const int b = (j < 4 ? 0 : 28) + 4 * tc + j;
-    *(f4_t*)(turn + b * 64 + (((tr + b + (b >> 4)) & 15) << 2)) = (f4_t){acc[0][j], acc[1][j], acc[2][j], acc[3][j]};
+  for (int j = 0; j < NJ; ++j) {
+    a_t v;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) v[i] = acc[i][j];
+    *(a_t*)(chunk(NJ * tc + j, NI * tr >> 2) + (NI * tr & 3)) = v;
   }
   __syncthreads();
 #pragma unroll
-  for (int l = 0; l < 8; ++l) {
-    const int b = l * 8 + (tid >> 4), ch = tid & 15;
-    const f4_t s = *(const f4_t*)(turn + b * 64 + (((ch + b + (b >> 4)) & 15) << 2));
+  for (int l = 0; l < TILE * NCH / NT; ++l) {
+    const int b = (l * NT + tid) / NCH, ch = tid % NCH;
+    const f4_t s = *(const f4_t*)chunk(b, ch);
     f4u_t* h = (f4u_t*)(H + (size_t)(b0 + b) * K + a0 + 4 * ch);
     const f4_t old = *h;
     f4_t v;
@@ -172,6 +210,24 @@ __global__ __launch_bounds__(128, 4) void dz_hessian_kernel(float* __restrict__ 
     }
     *h = v;
   }
+}
+
+// The first `whole` tiles of 64 x 64 as they are, the others in quarters.
+template <typename XT>
+__global__ __launch_bounds__(256, 4) void dz_hessian_kernel(float* __restrict__ H, const XT* __restrict__ x, int T, int K,
+                                                          float s0, float s1, int whole) {
+  __shared__ __attribute__((aligned(16))) float sm[4096];
+  const int wg = blockIdx.x;
+  const bool quarter = wg >= whole;
+  // tile number -> (ta <= tb): number = tb (tb + 1) / 2 + ta
+  const int n = quarter ? whole + ((wg - whole) >> 2) : wg;
+  int tb = (int)((sqrtf(8.f * (float)n + 1.f) - 1.f) * 0.5f);
+  while (tb * (tb + 1) / 2 > n) --tb;
+  while ((tb + 1) * (tb + 2) / 2 <= n) ++tb;
+  const int ta = n - tb * (tb + 1) / 2;
+  if (!quarter) return hessian_tile<XT, 64, 4, 4>(H, x, T, K, s0, s1, ta, tb, sm);
+  const int qa = 2 * ta + ((wg - whole) & 1), qb = 2 * tb + ((wg - whole) >> 1 & 1);
+  if (qa <= qb) hessian_tile<XT, 32, 2, 2>(H, x, T, K, s0, s1, qa, qb, sm);
 }
 
 // ---- one block of 128 columns (sparsegpt.py:98-142)
@@ -420,7 +476,7 @@ constexpr size_t OBS_LDS = (size_t)(OBS_TRI + 4 * OBS_BLOCK + 16 * (OBS_BLOCK + 
 
 // ---- W[:, c0 .. c0 + 127] -= Err @ hinv[i1 .. i1 + 127, c0 ..] for 64 rows, the sum over the block's
 // 128 columns in ascending order (sparsegpt.py:146).  Bound by the multiply-add rate: 4 x 8 values
-// per thread as in dz_hessian_kernel; the errors are staged with the row index innermost (with the
+// per thread; the errors are staged with the row index innermost (with the
 // column innermost the four rows of a thread fell on one bank) and in stages of 32 columns, so that
 // several workgroups fit a CU.
 __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const float* __restrict__ err,
@@ -505,14 +561,20 @@ int dz_hessian_add(float* H, const void* x, int x_is_fp16, int T, int K, float s
   if (!H || !x) return DZ_EINVAL;
   if (T < 1 || K < 64 || K % 64) return DZ_ESHAPE;
   hipStream_t st = (hipStream_t)stream;
-  const int nt = K / 64;
-  const dim3 grid((unsigned)(nt * (nt + 1) / 2));
+  const int nt = K / 64, n = nt * (nt + 1) / 2;
+  // Tiles that do not fill a round of the 256 CUs go in quarters, over all of them (2048 tokens: K = 4096, 32 tiles beyond
+  // eight rounds, 731 -> 665 us; K = 2560, 52 beyond three, 350 -> 309; 3968, 161 beyond seven, 660 -> 620), unless
+  // they nearly fill it (2816, 222 beyond three, 352 us in quarters and 341 whole).  Below 448 tiles all go in
+  // quarters: one round of whole tiles takes as long as two (K = 1600, 325 tiles, 207 us and 169 in
+  // quarters; 1856, 435 tiles, 204 and 199; 1984, 496 tiles, 203 and 217).
+  const int rest = n % 256, whole = n < 448 ? 0 : rest > 208 ? n : n - rest;
+  const dim3 grid((unsigned)(whole + 4 * (n - whole)));
   if (x_is_fp16)
-    hipLaunchKernelGGL(dz_hessian_kernel<_Float16>, grid, dim3(128), 0, st, H, (const _Float16*)x, T, K, scale_h,
-                       scale_x);
+    hipLaunchKernelGGL(dz_hessian_kernel<_Float16>, grid, dim3(256), 0, st, H, (const _Float16*)x, T, K, scale_h,
+                       scale_x, whole);
   else
-    hipLaunchKernelGGL(dz_hessian_kernel<float>, grid, dim3(128), 0, st, H, (const float*)x, T, K, scale_h,
-                       scale_x);
+    hipLaunchKernelGGL(dz_hessian_kernel<float>, grid, dim3(256), 0, st, H, (const float*)x, T, K, scale_h,
+                       scale_x, whole);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 

@@ -82,6 +82,20 @@ def test_hessian_tiles_bit_exact(dev, k, tokens, half):
         assert np.array_equal(H.cpu().numpy(), want)
 
 
+@pytest.mark.parametrize("k,tokens,half", [(64, 66, True), (576, 129, False), (1856, 17, True), (1920, 40, True), (2048, 37, False),
+                                           (2112, 5, True)])
+def test_hessian_rounds_of_tiles_bit_exact(dev, k, tokens, half):
+    """Quarter tiles alone (64 to 1856 columns), whole ones alone (1920), whole ones and a few quartered ones (2048,
+    2112), at the edges of their 32- and 64-token stages."""
+    rng = np.random.default_rng(k + tokens)
+    x = rng.standard_normal((tokens, k)).astype(np.float16 if half else np.float32)
+    H0 = rng.standard_normal((k, k)).astype(np.float32)
+    H = torch.from_numpy(H0.copy()).to(dev)
+    assert ops.hessian_add(H, torch.from_numpy(x).to(dev), 2, 1) == 3
+    want, _ = o.hessian_add_batch_ref(H0.copy(), 2, x.reshape(1, tokens, k))
+    assert np.array_equal(H.cpu().numpy(), want)
+
+
 def test_hessian_factor_zero_is_still_a_product(dev):
     """scale_x = 0: 0 times an infinite or NaN input is NaN, in the input's rows and columns; only the
     places beyond the last token are filled with zeros."""
