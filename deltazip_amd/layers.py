@@ -178,8 +178,12 @@ class LinearWithDelta(BaseLayerWithDelta):
     def apply_weights(self, x: torch.Tensor, bias: Optional[torch.Tensor] = None) -> torch.Tensor:
         T = self.indices_len[0]
         order = self.token_order[:T] if self.token_order is not None and 32 < T <= ops.MAX_TOKENS_FUSED else None
-        if T > 32 and self.row_blocks is not None and (T > ops.MAX_TOKENS_FUSED or self.row_blocks[0] is not None):
-            order = self.row_blocks[0]
+        if T > 32 and self.row_blocks is not None:
+            blocks = self.row_blocks[0]
+            # (a decode step that is captured keeps the token order, whose buffer stays: blocks serve eager calls only)
+            if T > ops.MAX_TOKENS_FUSED or (blocks is not None
+                                            and blocks.captured == torch.cuda.is_current_stream_capturing()):
+                order = blocks
         w = self.base_layer.weight
         if self._row_major_dropped:
             w = None

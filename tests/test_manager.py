@@ -1,6 +1,8 @@
 """Slot manager: bookkeeping on the CPU (no kernels), the oracle's convert_mapping restatement
 against hand-computed answers, and on the GPU the device-side mapping and a checkpoint -> manager
 -> layer forward pass checked against the oracle."""
+from types import SimpleNamespace
+
 import numpy as np
 import pytest
 import torch
@@ -9,7 +11,7 @@ import torch.nn as nn
 from oracle import dz_oracle as o
 from deltazip_amd import (DeltaConfig, DeltaMapping, DeltaModel, CompressionConfig, LRUCacheDeltaModelManager,
                           DeltaModelManager, create_delta_manager, convert_model)
-from deltazip_amd.layers import (MergedQKVParallelLinearWithDelta, MergedColumnParallelLinearWithDelta,
+from deltazip_amd.layers import (LinearWithDelta, MergedQKVParallelLinearWithDelta, MergedColumnParallelLinearWithDelta,
                                  RowParallelLinearWithDelta, VocabParallelEmbeddingWithDelta,
                                  LogitsProcessorWithDelta)
 from deltazip_amd.manager import LRUCache
@@ -592,3 +594,21 @@ def test_plan_of_blocks_of_several_deltas(t, k, n, plan):
     assert ops._in_mixed_blocks(t, k, n, 64, None) == plan
     if plan is not None and (k >= 2 * n and t <= 512):
         assert ops._in_mixed_blocks(t, k, n, 64, many) is None
+
+
+@pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
+def test_captured_decode_step_keeps_the_token_order(monkeypatch, made_captured, capturing, blocks_go):
+    """A decode batch whose blocks were made outside a capture goes into it with the manager's token order, as a
+    batch without blocks does; a prefill batch hands its blocks on either way."""
+    seen = []
+    monkeypatch.setattr(ops, "apply_delta", lambda *a, order, base_tiled: seen.append(order))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: capturing)
+    blocks, token_order = SimpleNamespace(captured=made_captured), torch.arange(256)
+    layer = SimpleNamespace(token_order=token_order, row_blocks=[blocks], base_layer=SimpleNamespace(weight=None),
+                            _row_major_dropped=False, base_tiled=None, qweight_stacked=None, scales_stacked=None,
+                            meta_stacked=None, indices=token_order)
+    for t in (64, 200):
+        layer.indices_len = [t]
+        LinearWithDelta.apply_weights(layer, None)
+    assert (seen[0] is blocks) == blocks_go and (blocks_go or torch.equal(seen[0], token_order[:64]))
+    assert seen[1] is blocks
