@@ -943,7 +943,6 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
     ldy = out.stride(0)
     if T > MAX_TOKENS_FUSED:
         blocks = _usable_blocks(order, T, S)
-        most = _most_row_blocks(T, K, N, bits, S, blocks)
         plan = None
         if (base_weight is not None or base_tiled is not None) and (blocks is None or blocks.mixed is not None):
             plan = _in_mixed_blocks(T, K, N, S, blocks.mix if blocks is not None else None)
@@ -952,6 +951,7 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
                                             bits=bits, out=out, accumulate=accumulate, plan=plan, blocks=blocks,
                                             base_tiled=base_tiled)
+        most = _most_row_blocks(T, K, N, bits, S, blocks)
         if most is not None:
             ws = _workspace(x.device, MAX_TOKENS_FUSED, K, N)
             w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
@@ -977,7 +977,7 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
                                           base_tiled=base_tiled)
     if T > 32 and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT:
         blocks = order if isinstance(order, RowBlocks) and order.order is not None else None
-        if blocks is not None and (blocks.T != T or blocks.S != S
+        if blocks is not None and (blocks.T != T or blocks.S != S or blocks.mix is None
                                    or blocks.captured != torch.cuda.is_current_stream_capturing()):
             blocks = None
         # A call that has to make its own table takes 8 us for it: large layers over few slots only (5120 x 13824, 100

@@ -1171,6 +1171,7 @@ def test_decode_batches_of_few_deltas(dev, bits, gs, t, met):
     torch.cuda.synchronize()
     assert ((y.float() - y0.float()).abs() <= 2.0**-10 * y0.float().abs() + 2e-3).all()
     assert not torch.equal(y, y0)                          # (it did go the other way)
+    assert torch.equal(call(ops.row_blocks(ids, S, order=order)), y0)   # (their maker did not count the deltas)
     with pytest.raises(ValueError):
         ops.apply_delta(x[:32 + 1], q, s, m, ids[:33].contiguous() if t != 33 else torch.cat([ids, ids])[:40], w, order=blocks)
     ops.poll_status(wait=True)
