@@ -420,7 +420,9 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     host_picks = small and mix is not None and mix.deltas == 1 and 448 < T <= 512
     if not small or host_picks:
         tiles, n = _block_table(T, num_slots, 256, dev)
-    if T > MAX_TOKENS_FUSED and (small or device_picks or (not long_only and T < 256 * (num_slots + 1))):
+    # (a decode batch that has its token order takes no blocks of one delta; the last piece of a very long batch, which
+    # may be as short, has nothing else)
+    if (order is None or T > MAX_TOKENS_FUSED) and (small or device_picks or (not long_only and T < 256 * (num_slots + 1))):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
     if long_only:
         _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")

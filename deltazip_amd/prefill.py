@@ -66,6 +66,8 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
     take_long, take_short = blocks.tiles is not None, blocks.short is not None
     if blocks.host_picks:
         take_long, take_short = one_wave, not one_wave
+    if not (take_long or take_short):
+        raise ValueError("these row blocks hold no blocks of one delta")
     row_major = base_weight.data_ptr() if base_weight is not None else None
     if take_long:
         fn, wptr = lib.dz_multi_delta_gemm, row_major

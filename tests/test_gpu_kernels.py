@@ -312,6 +312,21 @@ def test_row_blocks_made_once_per_batch(dev):
                                order=blocks)
 
 
+@pytest.mark.parametrize("t", [1, 100, 128])
+def test_prefill_call_of_decode_size(dev, t):
+    """The product over blocks of one delta called directly with up to 128 rows, the size of the last piece of a very
+    long batch: every row is written, or added to."""
+    from deltazip_amd.prefill import multi_delta_linear_prefill
+    p = make_problem(96, 512, 2, -1, 3, t, "uniform", t, dev)
+    ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
+    base = o.make_x(t, 96, 5)
+    for accumulate in (False, True):
+        y = torch.from_numpy(base).to(dev) if accumulate else torch.full((t, 96), float("nan"), dtype=torch.float16, device=dev)
+        multi_delta_linear_prefill(p["x"], p["wb"], p["q"], p["s"], p["m"], p["ids"], bits=2, out=y, accumulate=accumulate)
+        torch.cuda.synchronize()
+        assert o.rel_err(y.cpu().numpy(), ref + (base.astype(np.float32) if accumulate else 0)) <= TOL
+
+
 @pytest.mark.parametrize("n,k,bits,gs,nd", [(32, 256, 2, -1, 3), (96, 512, 4, -1, 2), (160, 768, 2, 64, 4),
                                             (288, 1024, 4, 128, 3), (128, 512, 2, -1, 1)])
 def test_short_row_blocks(dev, n, k, bits, gs, nd):

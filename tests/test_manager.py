@@ -596,6 +596,64 @@ def test_plan_of_blocks_of_several_deltas(t, k, n, plan):
         assert ops._in_mixed_blocks(t, k, n, 64, many) is None
 
 
+class _Calls:
+    """The library with its launches written down instead of made."""
+
+    def __init__(self, lib):
+        self.lib, self.names = lib, []
+
+    def __getattr__(self, name):
+        if not name.startswith(("dz_build", "dz_multi_delta")):
+            return getattr(self.lib, name)
+        return lambda *a: self.names.append(name) or 0
+
+
+@pytest.fixture
+def launches(monkeypatch):
+    from deltazip_amd import _lib
+    calls = _Calls(_lib.lib())
+    monkeypatch.setattr(_lib, "lib", lambda: calls)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=0))
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "segment", lambda ids, s, report=False: (torch.empty(ids.numel(), dtype=torch.int32),
+                                                                      torch.empty(s + 2, dtype=torch.int32)))
+    return calls.names
+
+
+@pytest.mark.parametrize("t,order,tables", [(1, False, "short"), (100, False, "short"), (128, False, "short"), (100, True, ""),
+                                            (129, False, "short"), (1024, False, "short"), (1025, False, "both"), (9000, False, "long")])
+def test_row_blocks_hold_blocks_of_one_delta(launches, t, order, tables):
+    """Every batch has them, also one that is as short as a decode step: the last piece of a very long one.  Only blocks
+    that come with a token order have none, and the product over blocks of one delta refuses those."""
+    from deltazip_amd.prefill import multi_delta_linear_prefill
+    ids, s = torch.zeros(t, dtype=torch.int64), 8
+    blocks = ops.row_blocks(ids, s, order=torch.zeros(t, dtype=torch.int32) if order else None)
+    assert ((blocks.tiles is not None) + 2 * (blocks.short is not None)) == ("", "long", "short", "both").index(tables)
+    args = (torch.empty(t, 256, dtype=torch.float16), None, torch.empty(s, 4), torch.empty(s, 1, 32), torch.empty(s, 4), ids)
+    out = torch.empty(t, 32, dtype=torch.float16)
+    if not tables:
+        with pytest.raises(ValueError):
+            multi_delta_linear_prefill(*args, bits=2, out=out, accumulate=False, blocks=blocks)
+    else:
+        multi_delta_linear_prefill(*args, bits=2, out=out, accumulate=False, blocks=blocks)
+        assert [n for n in launches if "gemm" in n] == ["dz_multi_delta_gemm"] * (tables != "short") + \
+            ["dz_multi_delta_gemm_rows"] * (tables != "long")
+
+
+@pytest.mark.parametrize("k,t", [(13824, 77673), (13824, 77696), (11008, 97542), (5120, 209792)])
+def test_last_piece_of_a_very_long_batch(launches, k, t):
+    """A call beyond the kernels' 31-bit offsets goes in pieces, each of them multiplied, also a last one of 1 to 128 rows."""
+    from deltazip_amd.prefill import multi_delta_linear_prefill
+    assert ops._mixed_plan(t, k, 32) is None
+    x = torch.empty(1, k, dtype=torch.float16).expand(t, k)
+    multi_delta_linear_prefill(x, None, torch.empty(2, 4), torch.empty(2, 1, 32), torch.empty(2, 4),
+                               torch.zeros(1, dtype=torch.int64).expand(t), bits=2, out=torch.empty(t, 32, dtype=torch.float16),
+                               accumulate=False)
+    tables = [i for i, n in enumerate(launches) if n.startswith("dz_build")]
+    assert len(tables) >= 2 and all("gemm" in launches[i + 1] for i in tables[:-1]) and "gemm" in launches[-1]
+
+
 @pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
 def test_captured_decode_step_keeps_the_token_order(monkeypatch, made_captured, capturing, blocks_go):
     """A decode batch whose blocks were made outside a capture goes into it with the manager's token order, as a
