@@ -19,7 +19,7 @@ it has one).
 """
 from __future__ import annotations
 
-from typing import Any, Dict, Hashable, List, Optional, Type
+from typing import Any, Dict, Hashable, List, Optional, Tuple, Type
 
 import torch
 import torch.nn as nn
@@ -206,7 +206,7 @@ class DeltaModelManager:
         self.packed_modules: Dict[str, List[str]] = {}
         self.modules: Dict[str, BaseLayerWithDelta] = {}
         self._widest = 0                 # output features of the widest linear layer
-        self._largest = (0, 0)           # K, N of the one with the most weights
+        self._projections: Dict[Tuple[int, int], int] = {}   # how many there are of every K, N
         self._last_mapping: Optional[DeltaMapping] = None
         self._wrap_modules()
         self.model.delta_manager = self
@@ -362,7 +362,8 @@ class DeltaModelManager:
             ops.token_order(self.base_indices[:T], self.delta_slots, out=self.token_order)
         self.row_blocks[0] = None
         decode = 32 < T <= ops.MAX_TOKENS_FUSED
-        wanted = T > ops.MAX_TOKENS_FUSED or (decode and ops.mixes_at_decode(T, *self._largest, len(set(mapping.index_mapping))))
+        wanted = T > ops.MAX_TOKENS_FUSED or (decode and ops.decode_step_mixes(
+            T, self.delta_config.max_bitwidth, len(set(mapping.index_mapping)), self._projections))
         if wanted and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
             # (the mix decides at sizes where other routes than row blocks may be the faster one)
             self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
@@ -434,7 +435,8 @@ class DeltaModelManager:
         if isinstance(module, LinearWithDelta):
             n, k = getattr(module, "base_shape", (0, 0))
             self._widest = max(self._widest, n)
-            self._largest = max(self._largest, (k, n), key=lambda kn: kn[0] * kn[1])
+            if k and n:
+                self._projections[k, n] = self._projections.get((k, n), 0) + 1
         # a fused layer also answers for the projections it is made of (q/k/v, gate/up)
         parent, _, leaf = module_name.rpartition(".")
         parts = self.packed_modules_mapping.get(leaf)

@@ -259,6 +259,20 @@ def mixes_at_decode(T: int, K: int, N: int, deltas: int) -> bool:
     return deltas <= (16 if T > 112 else 8 if T > 64 or T <= 40 else 2)
 
 
+def decode_step_mixes(T: int, bits: int, deltas: int, projections: Dict[Tuple[int, int], int]) -> bool:
+    """Whether a decode step over so many `projections` of (K, N) makes tables for blocks of several deltas: where
+    one of them would take such blocks, and the decode kernel keeps the GPU busy for longer than the host needs to
+    launch the step.  A layer call takes the host some 30 us, 3 more over blocks (a second launch, the sums' tensor),
+    and the blocks are looked up by the projections that do not take them, too.  By 190 timed layers of four projections
+    that went in blocks: below 160 us of the decode kernel, as `_route_us` has it, 120 us became 130
+    (2048/8448, 81 tokens of 4 deltas, 4-bit), at 160 and above 1.22 times as fast in the mean, 0.94 at worst."""
+    if not any(mixes_at_decode(T, k, n, deltas) for k, n in projections):
+        return False
+    mix = _even_mix(T, deltas)
+    return (sum(count * _route_us(T, k, n, bits, mix)[0] for (k, n), count in projections.items())
+            >= 40 * sum(projections.values()))
+
+
 @lru_cache(maxsize=4096)
 def _decode_plan(T: int, K: int, N: int, deltas: int) -> Tuple[int, int]:
     """`_mixed_plan` of such a batch, whose number of blocks is that of its deltas."""

@@ -654,6 +654,32 @@ def test_last_piece_of_a_very_long_batch(launches, k, t):
     assert len(tables) >= 2 and all("gemm" in launches[i + 1] for i in tables[:-1]) and "gemm" in launches[-1]
 
 
+def _mapped(monkeypatch, layers):
+    """A manager on the CPU whose kernels are left out, and which counts projections of these sizes."""
+    for name in ("map_ids", "token_order", "poll_status"):
+        monkeypatch.setattr(ops, name, lambda *a, **kw: None)
+    mgr = create_delta_manager(ToyModel(), 128, 256, V, DeltaConfig(max_deltas=8, max_bitwidth=4, group_size=-1))
+    assert mgr._projections == {(H, H + 128): 1, (H, H): 1, (H, 2 * I): 1, (I, H): 1}
+    mgr.delta_index_to_id = list(range(1, 9))
+    mgr._projections = {(k, n): 32 for h, i in layers for k, n in ((h, 3 * h), (h, h), (h, 2 * i), (i, h))}
+    return mgr
+
+
+@pytest.mark.parametrize("t,deltas,layers,makes", [
+    (81, 4, [(2048, 8448)], False), (52, 2, [(2048, 6144)], False), (51, 2, [(4096, 3584)], False),   # over before the host
+    (36, 1, [(1536, 10752)], False), (128, 4, [(256, 512)], False), (128, 8, [(4096, 5000)], True),
+    (128, 4, [(4096, 11008)], True), (33, 8, [(5120, 13824)], True), (64, 7, [(5120, 13824)], False)])
+def test_decode_step_makes_blocks_where_the_whole_step_gains(monkeypatch, t, deltas, layers, makes):
+    """One projection that would take blocks of several deltas is not enough: a step the decode kernel is through with
+    before the host has launched it makes none."""
+    made = []
+    monkeypatch.setattr(ops, "row_blocks", lambda *a, **kw: made.append(a) or SimpleNamespace())
+    mgr = _mapped(monkeypatch, layers)
+    ids = tuple(1 + i * deltas // t for i in range(t))
+    mgr.set_delta_mapping(DeltaMapping(ids, ids[:1]))
+    assert bool(made) == makes and (mgr.row_blocks[0] is not None) == makes
+
+
 @pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
 def test_captured_decode_step_keeps_the_token_order(monkeypatch, made_captured, capturing, blocks_go):
     """A decode batch whose blocks were made outside a capture goes into it with the manager's token order, as a
