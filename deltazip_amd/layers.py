@@ -171,7 +171,7 @@ class LinearWithDelta(BaseLayerWithDelta):
         # 33..128-token batch (the manager refreshes it with the mapping; None: computed per call)
         self.token_order = token_order
         # optional: the manager's one-element list holding ops.row_blocks() of the current batch when
-        # it has more than 128 tokens (None inside: made per call)
+        # it has more than 128 tokens (None inside: made per call), ops.DecodeBlocks of some smaller ones
         self.row_blocks = row_blocks
 
     # -- compute -------------------------------------------------------------------------------
@@ -181,8 +181,10 @@ class LinearWithDelta(BaseLayerWithDelta):
         if T > 32 and self.row_blocks is not None:
             blocks = self.row_blocks[0]
             # (a decode step that is captured keeps the token order, whose buffer stays: blocks serve eager calls only)
-            if T > ops.MAX_TOKENS_FUSED or (blocks is not None
-                                            and blocks.captured == torch.cuda.is_current_stream_capturing()):
+            if isinstance(blocks, ops.DecodeBlocks):
+                order = blocks.for_layer(*self.base_shape)
+            elif T > ops.MAX_TOKENS_FUSED or (blocks is not None
+                                              and blocks.captured == torch.cuda.is_current_stream_capturing()):
                 order = blocks
         w = self.base_layer.weight
         if self._row_major_dropped:

@@ -183,8 +183,8 @@ class DeltaModelManager:
         # order in which the fused kernel takes the tokens of a 33..128-token batch; refreshed with
         # the mapping, shared by every linear layer
         self.token_order = torch.zeros(ops.MAX_TOKENS_FUSED, dtype=torch.int32, device=self.device)
-        # larger batches: the tokens ordered by delta and cut into row blocks, made once per batch
-        # (the layers keep a reference to this list)
+        # larger batches: the tokens ordered by delta and cut into row blocks, made once per batch; decode batches
+        # that gain by blocks of several deltas: ops.DecodeBlocks (the layers keep a reference to this list)
         self.row_blocks = [None]
         # raw delta ids of the batch ([tokens | sampled rows]) and the id resident in each slot:
         # staged in pinned host memory, copied with one transfer each
@@ -361,17 +361,17 @@ class DeltaModelManager:
         if 32 < T <= ops.MAX_TOKENS_FUSED:
             ops.token_order(self.base_indices[:T], self.delta_slots, out=self.token_order)
         self.row_blocks[0] = None
-        decode = 32 < T <= ops.MAX_TOKENS_FUSED
-        wanted = T > ops.MAX_TOKENS_FUSED or (decode and ops.decode_step_mixes(
-            T, self.delta_config.max_bitwidth, len(set(mapping.index_mapping)), self._projections))
-        if wanted and self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
-            # (the mix decides at sizes where other routes than row blocks may be the faster one)
-            self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
-                                                mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
-                                                features=self._widest or None,
-                                                deltas=ops.mixed_deltas(self.delta_config.max_bitwidth,
-                                                                        self.delta_config.group_size != -1),
-                                                order=self.token_order[:T] if decode else None)
+        cfg = self.delta_config
+        if self.delta_slots <= ops.MAX_SLOTS_SEGMENT:
+            deltas = ops.mixed_deltas(cfg.max_bitwidth, cfg.group_size != -1)
+            if T > ops.MAX_TOKENS_FUSED:
+                # (the mix decides at sizes where other routes than row blocks may be the faster one)
+                self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
+                                                    mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
+                                                    features=self._widest or None, deltas=deltas)
+            elif T > 32 and ops.decode_step_mixes(T, cfg.max_bitwidth, len(set(mapping.index_mapping)), self._projections):
+                self.row_blocks[0] = ops.DecodeBlocks(self.base_indices[:T], self.delta_slots, mapping.index_mapping, deltas,
+                                                      self.token_order[:T])
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 

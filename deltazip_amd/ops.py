@@ -192,6 +192,26 @@ class MixedTable(NamedTuple):
     deltas: int
 
 
+class DecodeBlocks:
+    """The blocks of several deltas of a decode step, made by the first eager call on each stream of a layer that takes
+    them: a step that is replayed from a graph reads the token order and never asks, and the tables belong to the stream
+    whose calls read them.  `ids`: of the tokens, any, one per delta and one for the base model."""
+    __slots__ = ("indices", "S", "ids", "met", "deltas", "order", "made")
+
+    def __init__(self, indices, S, ids, deltas, order):
+        self.indices, self.S, self.ids, self.met, self.deltas = indices, S, ids, len(set(ids)), deltas
+        self.order, self.made = order, {}
+
+    def for_layer(self, N: int, K: int):
+        """What a layer of that size passes on as `order`."""
+        if not mixes_at_decode(len(self.ids), K, N, self.met) or torch.cuda.is_current_stream_capturing():
+            return self.order
+        stream = _stream()
+        if stream not in self.made:
+            self.made[stream] = row_blocks(self.indices, self.S, mix=batch_mix(self.ids), deltas=self.deltas, order=self.order)
+        return self.made[stream]
+
+
 MIXED_BLOCKS = ((8, 4), (4, 2))   # (tiles of 16 tokens, deltas) of a block: full, small (DZ_MIXED_*)
 
 
@@ -441,6 +461,11 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     if long_only:
         _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
         return RowBlocks(perm, tiles, n, T, num_slots)
+    if tiles is None and short is None:               # (a decode step takes full blocks only)
+        full = _mixed_table(T, num_slots, 0, deltas, dev)
+        _lib.check(L.dz_build_mixed(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, MIXED_BLOCKS[0][0], full.deltas,
+                                    full.table.data_ptr(), full.max_blocks, st), "dz_build_mixed")
+        return RowBlocks(perm, None, 0, T, num_slots, mix=mix, mixed=[full, None], order=order)
     mixed = [_mixed_table(T, num_slots, small_ones, deltas, dev) for small_ones in (0, 1)]
     ptr = lambda t: None if t is None else t.data_ptr()
     _lib.check(L.dz_build_tables(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, ptr(tiles), n, ptr(short), ns,

@@ -1201,6 +1201,37 @@ def test_decode_batches_of_few_deltas(dev, bits, gs, t, met):
     ops._warned_bad_id = warned
 
 
+def test_decode_blocks_of_each_stream(dev):
+    """The tables a decode step's layers make for themselves: one set per stream, equal bits from each and from tables
+    handed over, and the token order for a layer that takes no blocks and for a captured call."""
+    from deltazip_amd.synthetic import gaussian_native_stack
+    n, k, S, t = 10240, 2560, 4, 100
+    gen = torch.Generator(device=dev).manual_seed(t)
+    q, m, s = gaussian_native_stack(k, n, 4, k, S, dev, gen)
+    w, x = (torch.randn(n, k, device=dev, generator=gen) * 0.02).half(), torch.randn(t, k, device=dev, generator=gen).half()
+    ids_np = np.random.default_rng(t).integers(-1, S, t)
+    ids = torch.from_numpy(ids_np).to(dev)
+    order = ops.token_order(ids, S)
+    made = ops.DecodeBlocks(ids, S, ids_np.tolist(), 3, order)
+    want = ops.apply_delta(x, q, s, m, ids, w, order=ops.row_blocks(ids, S, mix=ops.batch_mix(ids_np.tolist()), order=order))
+    assert made.for_layer(1024, 1024) is order
+    streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
+    streams[1].wait_stream(streams[0])
+    for turn in range(2):
+        for stream in streams:
+            with torch.cuda.stream(stream):
+                blocks = made.for_layer(n, k)
+                y = ops.apply_delta(x, q, s, m, ids, w, order=blocks)
+            torch.cuda.synchronize()
+            assert torch.equal(y, want) and blocks.mixed[1] is None
+    assert len(made.made) == 2
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(streams[1]), torch.cuda.graph(graph, stream=streams[1]):
+        assert made.for_layer(n, k) is order
+        y.add_(0)
+    torch.cuda.synchronize()
+
+
 @pytest.mark.parametrize("n,k", [(32, 512), (288, 2048), (64, 2304), (96, 4096), (32, 4352), (288, 8192), (32, 8448), (64, 16384),
                                  (32, 16640)])
 @pytest.mark.parametrize("bits", [2, 4])

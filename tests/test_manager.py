@@ -672,12 +672,44 @@ def _mapped(monkeypatch, layers):
 def test_decode_step_makes_blocks_where_the_whole_step_gains(monkeypatch, t, deltas, layers, makes):
     """One projection that would take blocks of several deltas is not enough: a step the decode kernel is through with
     before the host has launched it makes none."""
-    made = []
-    monkeypatch.setattr(ops, "row_blocks", lambda *a, **kw: made.append(a) or SimpleNamespace())
     mgr = _mapped(monkeypatch, layers)
     ids = tuple(1 + i * deltas // t for i in range(t))
     mgr.set_delta_mapping(DeltaMapping(ids, ids[:1]))
-    assert bool(made) == makes and (mgr.row_blocks[0] is not None) == makes
+    assert (mgr.row_blocks[0] is not None) == makes
+
+
+def test_decode_blocks_are_made_by_the_layers_that_take_them(monkeypatch, launches):
+    """set_delta_mapping itself launches nothing for them (a step that is replayed from a graph reads the token order
+    alone); the first eager call of a layer that takes them does, once for every stream, and makes one table."""
+    mgr = _mapped(monkeypatch, [(4096, 11008)])
+    ids, now, seen = tuple(1 + i // 32 for i in range(128)), SimpleNamespace(stream=7, capturing=False), []
+    monkeypatch.setattr(ops, "_stream", lambda: now.stream)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: now.capturing)
+    monkeypatch.setattr(ops, "apply_delta", lambda *a, order, base_tiled: seen.append(order))
+    mgr.set_delta_mapping(DeltaMapping(ids, ids[:1]))
+    assert launches == []
+    layer = mgr.model.model.layers[0].mlp.down_proj
+    layer.base_tiled = None
+
+    def call(n, k):
+        layer.base_shape = (n, k)
+        layer.apply_weights(None)
+        return seen[-1]
+    small = call(4096, 4096)                           # under 24 M weights
+    now.capturing = True
+    captured = call(4096, 11008)
+    now.capturing = False
+    assert launches == [] and small.data_ptr() == captured.data_ptr() == mgr.token_order.data_ptr() and small.numel() == 128
+    first, again = call(4096, 11008), call(22016, 4096)
+    assert first is again and isinstance(first, ops.RowBlocks) and first.mix.deltas == 4
+    assert first.order.data_ptr() == mgr.token_order.data_ptr() and first.mixed[0].deltas == 4 - 1 and first.mixed[1] is None
+    now.stream = 8
+    other = call(4096, 11008)
+    assert other is not first and launches == ["dz_build_mixed"] * 2
+    now.stream = 7
+    assert call(4096, 11008) is first and len(launches) == 2
+    mgr.set_delta_mapping(DeltaMapping(ids[:20], ids[:1]))
+    assert mgr.row_blocks[0] is None
 
 
 @pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
