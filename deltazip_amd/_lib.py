@@ -35,6 +35,7 @@ SIGNATURES = {
     "dz_multi_delta_gemm_rows": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_mixed_blocks": (_i, [_i, _i, _i, _i]),
     "dz_build_mixed": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _vp]),
+    "dz_order_mixed": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp]),
     "dz_build_tables": (_i, [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _i, _vp, _i, _vp]),
     "dz_multi_delta_gemm_mixed": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _i, _vp, _i, _i, _i, _i, _i, _i, _vp,
                                        _vp]),

@@ -557,10 +557,11 @@ __global__ __launch_bounds__(1024) void dz_build_tables_kernel(const int* __rest
   extern __shared__ int first[];
   const int which = blockIdx.x;
   if (which >= 2) {
+    for (int k = threadIdx.x; k < S + 2; k += 1024) first[k] = seg_off[k];
     if (B.mixed[which - 2])
-      dz_build_mixed_blocks(seg_off, perm, S, which == 2 ? DZ_MIXED_ROWS / 16 : DZ_MIXED_SMALL_TILES,
+      dz_build_mixed_blocks(first, perm, S, which == 2 ? DZ_MIXED_ROWS / 16 : DZ_MIXED_SMALL_TILES,
                             which == 2 ? B.deltas : DZ_MIXED_SMALL_DELTAS, B.count[which - 2], B.mixed[which - 2],
-                            B.max_mixed[which - 2], first);
+                            B.max_mixed[which - 2]);
   } else if (which == 0) {
     if (B.tiles)
       build_tiles_body(seg_off, S, BM, B.tiles, B.max_tiles, DZ_SHORT_ROWS, B.either ? B.short_tiles : nullptr, B.max_short, 0,

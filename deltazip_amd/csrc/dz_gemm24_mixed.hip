@@ -418,7 +418,17 @@ __global__ __launch_bounds__(1024) void dz_build_mixed_kernel(const int* __restr
                                                               int S, int most, int deltas, int* __restrict__ count,
                                                               dz_mixed_block* __restrict__ blocks, int max_blocks) {
   extern __shared__ int off[];
-  dz_build_mixed_blocks(seg_off, perm, S, most, deltas, count, blocks, max_blocks, off);
+  for (int k = threadIdx.x; k < S + 2; k += 1024) off[k] = seg_off[k];
+  dz_build_mixed_blocks(off, perm, S, most, deltas, count, blocks, max_blocks);
+}
+
+// The order and the table in one launch, for a call that has to make its own: on a few hundred tokens two kernels are over
+// long before the host has launched them (a call over a small layer 44 -> 37 us, bound by the host's half either way).
+__global__ __launch_bounds__(1024) void dz_order_mixed_kernel(const long long* idx, int T, int S, int most, int deltas, int* perm,
+                                                              int* count, dz_mixed_block* blocks, int max_blocks, unsigned* status) {
+  extern __shared__ int sm[];
+  dz_segment_tokens(idx, T, S, perm, status, sm);
+  dz_build_mixed_blocks(sm, perm, S, most, deltas, count, blocks, max_blocks);
 }
 
 }  // namespace
@@ -439,6 +449,17 @@ extern "C" int dz_build_mixed(const int32_t* seg_off, const int32_t* perm, int S
   if (need < 1 || max_blocks < need) return DZ_ESHAPE;
   hipLaunchKernelGGL(dz_build_mixed_kernel, dim3(1), dim3(1024), (size_t)(S + 2) * 4, (hipStream_t)stream, seg_off,
                      perm, S, tiles, deltas, table, (dz_mixed_block*)(table + DZ_MIXED_HEADER), max_blocks);
+  return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
+}
+
+extern "C" int dz_order_mixed(const int64_t* indices, int T, int S, int tiles, int deltas, int32_t* perm, int32_t* table,
+                              int max_blocks, uint32_t* status, void* stream) {
+  if (!indices || !perm || !table) return DZ_EINVAL;
+  if (S < 0 || S > DZ_MAX_SLOTS_SEGMENT || T < 1) return DZ_ESHAPE;
+  const int need = dz_mixed_blocks(T, S, tiles, deltas);
+  if (need < 1 || max_blocks < need) return DZ_ESHAPE;
+  hipLaunchKernelGGL(dz_order_mixed_kernel, dim3(1), dim3(1024), dz_segment_lds(S), (hipStream_t)stream, (const long long*)indices,
+                     T, S, tiles, deltas, perm, table, (dz_mixed_block*)(table + DZ_MIXED_HEADER), max_blocks, status);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }
 

@@ -404,12 +404,28 @@ def _block_table(T: int, num_slots: int, rows: int, device):
     return torch.empty((n, 4), dtype=torch.int32, device=device), n
 
 
-def _mixed_table(T: int, S: int, small: int, deltas: int, device) -> MixedTable:
+def _mixed_table(T: int, S: int, small: int, deltas: int, device, behind: int = 0) -> MixedTable:
     tiles, most = MIXED_BLOCKS[small]
     deltas = min(deltas, most)
     n = _lib.lib().dz_mixed_blocks(T, S, tiles, deltas)
     # DZ_MIXED_HEADER words and n times sizeof(dz_mixed_block)
-    return MixedTable(torch.empty(4 + n * (2 + 4 * 4 + 128), dtype=torch.int32, device=device), n, deltas)
+    return MixedTable(torch.empty(4 + n * (2 + 4 * 4 + 128) + behind, dtype=torch.int32, device=device), n, deltas)
+
+
+def own_mixed_table(indices: torch.Tensor, S: int, small: int, deltas: int) -> MixedTable:
+    """The one table a call needs, from the ids, in one launch; the token order is left behind its blocks.  Bad ids are
+    reported at the sizes that chunks of the decode kernel can serve, as that kernel does."""
+    _need_cuda(indices)
+    if indices.dtype != torch.int64:
+        raise ValueError("indices must be int64")
+    T = indices.numel()
+    made = _mixed_table(T, S, small, deltas, indices.device, T)
+    table = made.table.data_ptr()
+    status = _workspace(indices.device, 1, 256, 32).data_ptr() if takes_fused_chunks(T, S) else None
+    _lib.check(_lib.lib().dz_order_mixed(indices.data_ptr(), T, S, MIXED_BLOCKS[small][0], made.deltas,
+                                         table + 4 * (made.table.numel() - T), table, made.max_blocks, status, _stream()),
+               "dz_order_mixed")
+    return made
 
 
 def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
@@ -445,6 +461,9 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
     T = indices.numel()
+    if order is not None and T <= MAX_TOKENS_FUSED and not long_only:   # (a decode step takes full blocks only)
+        full = own_mixed_table(indices, num_slots, 0, deltas)
+        return RowBlocks(full.table[-T:], None, 0, T, num_slots, mix=mix, mixed=[full, None], order=order)
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
     perm, seg_off = segment(indices, num_slots, not long_only and takes_fused_chunks(T, num_slots))
     L, dev, st = _lib.lib(), indices.device, _stream()
@@ -454,18 +473,11 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     host_picks = small and mix is not None and mix.deltas == 1 and 448 < T <= 512
     if not small or host_picks:
         tiles, n = _block_table(T, num_slots, 256, dev)
-    # (a decode batch that has its token order takes no blocks of one delta; the last piece of a very long batch, which
-    # may be as short, has nothing else)
-    if (order is None or T > MAX_TOKENS_FUSED) and (small or device_picks or (not long_only and T < 256 * (num_slots + 1))):
+    if small or device_picks or (not long_only and T < 256 * (num_slots + 1)):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
     if long_only:
         _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
         return RowBlocks(perm, tiles, n, T, num_slots)
-    if tiles is None and short is None:               # (a decode step takes full blocks only)
-        full = _mixed_table(T, num_slots, 0, deltas, dev)
-        _lib.check(L.dz_build_mixed(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, MIXED_BLOCKS[0][0], full.deltas,
-                                    full.table.data_ptr(), full.max_blocks, st), "dz_build_mixed")
-        return RowBlocks(perm, None, 0, T, num_slots, mix=mix, mixed=[full, None], order=order)
     mixed = [_mixed_table(T, num_slots, small_ones, deltas, dev) for small_ones in (0, 1)]
     ptr = lambda t: None if t is None else t.data_ptr()
     _lib.check(L.dz_build_tables(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, ptr(tiles), n, ptr(short), ns,

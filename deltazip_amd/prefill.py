@@ -92,7 +92,7 @@ def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, m
     """The layer over blocks that hold the tokens of several deltas (dz_multi_delta_gemm_mixed), with a base weight.
     `plan`: ops._mixed_plan(T, K, N).  `blocks`: as for multi_delta_linear_prefill; without them, or where they
     were made for more deltas than this layer's block can hold, the call makes the table it needs."""
-    from .ops import _mixed_table, mixed_deltas, segment, takes_fused_chunks
+    from .ops import mixed_deltas, own_mixed_table
     small, parts = plan
     T, K = x2.shape
     N, S = scales_stacked.shape[-1], qweight_stacked.shape[0]
@@ -101,10 +101,7 @@ def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, m
     deltas = mixed_deltas(bits, G > 1)
     table = blocks.mixed[small] if blocks is not None else None
     if table is None or table.deltas > deltas:
-        perm, seg_off = segment(indices, S, takes_fused_chunks(T, S))
-        table = _mixed_table(T, S, small, deltas, x2.device)
-        _lib.check(L.dz_build_mixed(seg_off.data_ptr(), perm.data_ptr(), S, T, 4 if small else 8, table.deltas,
-                                    table.table.data_ptr(), table.max_blocks, stream), "dz_build_mixed")
+        table = own_mixed_table(indices, S, small, deltas)
     sums = torch.empty(parts * T * N, dtype=torch.float32, device=x2.device) if parts > 1 else None
     w = base_tiled if base_tiled is not None else base_weight
     rc = L.dz_multi_delta_gemm_mixed(

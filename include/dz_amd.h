@@ -393,6 +393,10 @@ int dz_mixed_blocks(int T, int S, int tiles, int deltas);
 int dz_build_mixed(const int32_t* seg_off, const int32_t* perm, int S, int T, int tiles, int deltas, int32_t* table,
                    int max_blocks, void* stream);
 
+/* dz_segment_status and dz_build_mixed in one launch.  perm: scratch of T words. */
+int dz_order_mixed(const int64_t* indices, int T, int S, int tiles, int deltas, int32_t* perm, int32_t* table, int max_blocks,
+                   uint32_t* status, void* stream);
+
 /* The tables of a batch in one launch: those of dz_build_tiles (tiles, or NULL) and dz_build_tiles_rows with
  * DZ_SHORT_ROWS rows (short_tiles, or NULL), or of dz_build_tiles_either (either != 0); those of dz_build_mixed with
  * DZ_MIXED_ROWS / 16 tiles and `deltas` deltas (mixed) and with the smaller blocks (small). */

@@ -1111,6 +1111,31 @@ def test_blocks_of_several_deltas(dev, n, k, bits, gs, nd, t, tiles, most):
                                            n, 0, n, 1, None, st) == -2
 
 
+@pytest.mark.parametrize("t,nd", [(1, 1), (129, 0), (200, 5), (1024, 17), (1025, 3), (5000, 768)])
+@pytest.mark.parametrize("small", [0, 1])
+def test_order_and_table_in_one_launch(dev, t, nd, small):
+    """dz_order_mixed writes the order and the blocks that dz_segment and dz_build_mixed write, and reports bad ids."""
+    from deltazip_amd import _lib
+    L, st = _lib.lib(), torch.cuda.current_stream().cuda_stream
+    ids_np = np.random.default_rng(t + nd).integers(-1, nd, t)
+    tiles, most = ops.MIXED_BLOCKS[small]
+    room = L.dz_mixed_blocks(t, nd, tiles, most)
+    for bad in (False, True):
+        if bad:
+            ids_np[t // 2] = nd + 3
+        ids = torch.from_numpy(ids_np).to(dev)
+        perm, off = ops.segment(ids, nd)
+        want, got = (torch.zeros(4 + room * 146, dtype=torch.int32, device=dev) for _ in range(2))
+        order, status = torch.zeros(t, dtype=torch.int32, device=dev), torch.zeros(1, dtype=torch.int32, device=dev)
+        assert L.dz_build_mixed(off.data_ptr(), perm.data_ptr(), nd, t, tiles, most, want.data_ptr(), room, st) == 0
+        assert L.dz_order_mixed(ids.data_ptr(), t, nd, tiles, most, order.data_ptr(), got.data_ptr(), room, status.data_ptr(),
+                                st) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(order, perm) and int(status) == int(bad) and torch.equal(got, want)
+    assert L.dz_order_mixed(ids.data_ptr(), t, 769, tiles, most, order.data_ptr(), got.data_ptr(), room, None, st) != 0
+    assert L.dz_order_mixed(ids.data_ptr(), t, nd, tiles, most, order.data_ptr(), got.data_ptr(), room - 1, None, st) != 0
+
+
 def test_blocks_of_several_deltas_keep_tokens_apart(dev):
     """A block's tokens share tiles of activations and nothing else: an infinite scale reaches its own delta's
     tokens only, an infinite or NaN activation its own token only."""

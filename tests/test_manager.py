@@ -603,7 +603,7 @@ class _Calls:
         self.lib, self.names = lib, []
 
     def __getattr__(self, name):
-        if not name.startswith(("dz_build", "dz_multi_delta")):
+        if not name.startswith(("dz_build", "dz_order", "dz_multi_delta")):
             return getattr(self.lib, name)
         return lambda *a: self.names.append(name) or 0
 
@@ -616,6 +616,8 @@ def launches(monkeypatch):
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     monkeypatch.setattr(torch.cuda, "current_stream", lambda *a: SimpleNamespace(cuda_stream=0))
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(ops, "_need_cuda", lambda *a: None)
+    monkeypatch.setattr(ops, "_workspace", lambda *a: torch.empty(4))
     monkeypatch.setattr(ops, "segment", lambda ids, s, report=False: (torch.empty(ids.numel(), dtype=torch.int32),
                                                                       torch.empty(s + 2, dtype=torch.int32)))
     return calls.names
@@ -705,7 +707,7 @@ def test_decode_blocks_are_made_by_the_layers_that_take_them(monkeypatch, launch
     assert first.order.data_ptr() == mgr.token_order.data_ptr() and first.mixed[0].deltas == 4 - 1 and first.mixed[1] is None
     now.stream = 8
     other = call(4096, 11008)
-    assert other is not first and launches == ["dz_build_mixed"] * 2
+    assert other is not first and launches == ["dz_order_mixed"] * 2
     now.stream = 7
     assert call(4096, 11008) is first and len(launches) == 2
     mgr.set_delta_mapping(DeltaMapping(ids[:20], ids[:1]))
