@@ -313,6 +313,18 @@ def _in_mixed_blocks(T: int, K: int, N: int, S: int, mix: Optional["BatchMix"]) 
     return plan
 
 
+@lru_cache(maxsize=4096)
+def _short_chunks(T: int, K: int, N: int, bits: int, S: int) -> bool:
+    """Whether a call that would have to make its own table goes in chunks of the decode kernel, of which there are few
+    and short ones: it takes the host 28 us to launch two of them, and 37 to launch the table, the product and the sum
+    of its parts.  By 300 timed calls of 129 to 512 tokens the two meet at an estimate (`_route_us`) of 36 us: at 28 to
+    32 us chunks take 29.7 us and blocks 37.2 (2304 x 1088, 4-bit, 237 tokens of one slot: 31.6 and 45.2 while the
+    order and the table were two launches), at 40 to 44 us 40.6 and 37.3.  The line lies a tenth below, the estimate being
+    that good."""
+    return (takes_fused_chunks(T, S) and _most_blocks_unknown(T, K, N, bits, S) == 0
+            and _route_us(T, K, N, bits, _even_mix(T, S))[0] < 33)
+
+
 class BatchMix(NamedTuple):
     """What the choice between the kernels looks at: deltas in the batch (the base model counts as
     one), row blocks of 128 tokens, tokens of the most popular delta, and the deltas met by each chunk
@@ -997,7 +1009,8 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
     if T > MAX_TOKENS_FUSED:
         blocks = _usable_blocks(order, T, S)
         plan = None
-        if (base_weight is not None or base_tiled is not None) and (blocks is None or blocks.mixed is not None):
+        if ((base_weight is not None or base_tiled is not None)
+                and (not _short_chunks(T, K, N, bits, S) if blocks is None else blocks.mixed is not None)):
             plan = _in_mixed_blocks(T, K, N, S, blocks.mix if blocks is not None else None)
         if plan is not None:
             from .prefill import multi_delta_linear_mixed
@@ -1125,9 +1138,10 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     if T > MAX_TOKENS_FUSED:
         blocks = order if isinstance(order, RowBlocks) else None
         # row blocks made once serve the projections that would make the same ones
-        shared = [q.shape[0] == S and (blocks is not None or _in_mixed_blocks(T, K, w.shape[0], S, None) is not None or (
-                      _most_row_blocks(T, K, w.shape[0], bits, S, None) is None
-                      and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
+        shared = [q.shape[0] == S and (blocks is not None or (
+                      _in_mixed_blocks(T, K, w.shape[0], S, None) is not None and not _short_chunks(T, K, w.shape[0], bits, S))
+                      or (_most_row_blocks(T, K, w.shape[0], bits, S, None) is None
+                          and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():

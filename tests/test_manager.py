@@ -714,6 +714,28 @@ def test_decode_blocks_are_made_by_the_layers_that_take_them(monkeypatch, launch
     assert mgr.row_blocks[0] is None
 
 
+@pytest.mark.parametrize("t,k,n,bits,slots,route", [
+    (155, 2048, 1408, 2, 1, "chunks"), (144, 2560, 736, 4, 21, "chunks"), (210, 2304, 640, 4, 3, "chunks"),   # the host's half
+    (200, 2560, 1280, 2, 5, "blocks"), (293, 6656, 1728, 2, 2, "blocks"), (333, 13824, 5120, 2, 16, "blocks"),
+    (600, 2560, 1280, 2, 5, "blocks"), (129, 4096, 512, 2, 700, "blocks"), (129, 4096, 512, 2, 769, "chunks")])
+def test_route_of_a_call_that_makes_its_own_table(monkeypatch, launches, t, k, n, bits, slots, route):
+    """Few short chunks are over before the host has launched the table, the product and its sums; a batch whose tables
+    are there goes in blocks of several deltas all the same, and so do projections that share theirs."""
+    def called(make):
+        launches.clear()
+        make()
+        return set(launches)
+    x, w = torch.empty(t, k, dtype=torch.float16), torch.empty(n, k, dtype=torch.float16)
+    ids = torch.zeros(t, dtype=torch.int64)
+    qs, ms, ss = ops.stacked_shapes(k, n, bits, -1)
+    stack = [torch.empty((slots,) + tuple(v), dtype=d) for v, d in ((qs, torch.int32), (ss, torch.float16), (ms, torch.int16))]
+    got = called(lambda: ops.apply_delta(x, *stack, ids, w))
+    assert got == ({"dz_multi_delta_linear_chunks"} if route == "chunks" else {"dz_order_mixed", "dz_multi_delta_gemm_mixed"})
+    if slots <= 768:
+        known = ops.row_blocks(ids, slots, deltas=3)
+        assert called(lambda: ops.apply_delta(x, *stack, ids, w, order=known)) == {"dz_multi_delta_gemm_mixed"}
+
+
 @pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
 def test_captured_decode_step_keeps_the_token_order(monkeypatch, made_captured, capturing, blocks_go):
     """A decode batch whose blocks were made outside a capture goes into it with the manager's token order, as a
