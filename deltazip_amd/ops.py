@@ -234,22 +234,26 @@ def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
     2000 1.22, 8192 1.11.
       small blocks   where the full ones' workgroups would leave most of the 256 CUs idle: a block of half as
                      many tiles walks K in less time (2048 x 2048, 230 tokens: in the mean 1.42 against
-                     1.23 times as fast as before; 4096 x 12288 of 333: 1.12 against 1.27)
+                     1.23 times as fast as before; 4096 x 12288 of 333: 1.12 against 1.27); but a batch has more
+                     blocks than T / 64, and from 224 workgroups by that count they were a second wave (2560
+                     x 10240, 401 tokens of 3 deltas, 4-bit: full 50, small 67 us, one delta per block 60)
       parts          each a walk over its share of K, and one more pass over the sums at 3 TB/s (13824 x 5120,
-                     333 tokens of 10 deltas: 1 / 2 / 3 / 4 / 6 parts 220 / 128 / 100 / 122 / 110 us)
+                     333 tokens of 10 deltas: 1 / 2 / 3 / 4 / 6 parts 220 / 128 / 100 / 122 / 110 us, of which the
+                     estimate takes 4, counting 3 blocks where there are 4); one where the host takes longer to launch
+                     the sums than the walk takes (1536 x 1536, 263 tokens: 26.6 in 3 parts, 21.2 in one)
       K <= 1024      the walk is too short to pay for a workgroup's start unless there are several waves of them
                      (1024 x 8192: 129 tokens 14 / 19 us, 640 tokens 1.24 times as fast)"""
     if T <= MAX_TOKENS_FUSED or 2 * T * K >= 1 << 31:
         return None                                   # (32-bit offsets)
     if K <= 1024 and -(-T // 128) * -(-N // 128) <= 384:
         return None
-    small = -(-N // 256) * T / 128 < (140 if K <= 3072 else 25)
-    return int(small), _parts(T, K, N, -(-T // (64 if small else 128)), 1.0 if small else 1.7)
+    small = -(-N // 256) * T / 128 < (112 if K <= 3072 else 25)
+    return int(small), _parts(T, K, N, -(-T // (64 if small else 128)), 1.0 if small else 1.7, 25)
 
 
-def _parts(T: int, K: int, N: int, blocks: int, slab_us: float) -> int:
+def _parts(T: int, K: int, N: int, blocks: int, slab_us: float, host_us: float = 0) -> int:
     """Parts of K for so many blocks: what a wave of workgroups takes to start and to walk its part of K, alone
-    and with all CUs busy, and the pass over the partial sums."""
+    and with all CUs busy, and the pass over the partial sums.  `host_us`: one part if it takes no longer."""
     wide, steps, best = -(-N // 256), K // 256, None
     for parts in (1, 2, 3, 4, 6):
         if parts > steps:
@@ -261,6 +265,8 @@ def _parts(T: int, K: int, N: int, blocks: int, slab_us: float) -> int:
             cost += 3 + 8 * T * N * parts / 3e6
         if best is None or cost < best[0]:
             best = (cost, parts)
+        if parts == 1 and cost <= host_us:
+            break
     return best[1]
 
 

@@ -132,6 +132,15 @@ def test_row_blocks_stay_on_their_side_of_a_capture(monkeypatch):
         ops._usable_blocks(late, 601, 3)
 
 
+@pytest.mark.parametrize("t,k,n,plan", [
+    (263, 1536, 1536, (1, 1)), (154, 1280, 1280, (1, 1)), (383, 1280, 1280, (1, 1)),      # the host's half: no second launch
+    (401, 2560, 10240, (0, 1)), (329, 1280, 13184, (0, 1)), (479, 2560, 8736, (0, 1)),    # no second wave of small blocks
+    (333, 2560, 8736, (1, 1)), (200, 2560, 1280, (1, 6))])
+def test_plan_of_small_layers(t, k, n, plan):
+    """A walk that is over before the host could launch a sum is not cut; small blocks only where they are one wave."""
+    assert ops._mixed_plan(t, k, n) == plan
+
+
 def test_batch_mix_counts_what_the_routes_meet():
     ids = [0] * 5 + [7] * 130 + [9] * 128 + [7] * 1                            # 264 tokens, three chunks
     assert ops.batch_mix(ids) == ops.BatchMix(3, 1 + 2 + 1, 131, 2 + 2 + 2)
