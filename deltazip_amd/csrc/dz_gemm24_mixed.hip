@@ -1,5 +1,5 @@
-// Multi-delta linear layer for more than 128 tokens over blocks of rows that hold the tokens of several
-// deltas:
+// Multi-delta linear layer for more than 128 tokens, and for decode batches of few deltas over large layers, over blocks of
+// rows that hold the tokens of several deltas:
 //   y[t, :] (+)= x[t, :] @ w_base^T + x[t, :] @ dequant(delta[slot(t)])^T
 // A block (dz_tables.h) is up to 8 tiles of 16 tokens, each tile of one delta, up to 4 deltas: base
 // weight and activations are read once per block, whatever deltas it holds, and a delta of a few
@@ -21,8 +21,8 @@
 // unpacking, 25 vector instructions a delta, which the wavefront's twin on the SIMD covers in part.  With all
 // CUs busy and the base weight of 256 features per CU coming from memory 1.7 us, 4.9 to 5.9 TB/s.  5120 x
 // 27648, 2-bit, against one delta per block and against 256 x 256 tiles: 333 tokens of 10 deltas 250 -> 215 us, 1000
-// of 32 950 -> 700, 8192 of 16 3460 -> 3020; 13824 x 5120, 333 tokens 178 -> 100 (K in three parts).  A layer of
-// 5120/13824, 333 tokens: 770 -> 593 us.
+// of 32 950 -> 700, 8192 of 16 3460 -> 3020; 13824 x 5120, 333 tokens 178 -> 122 (K in four parts; in three, which would fit
+// this batch's four blocks better, 100).  A layer of 5120/13824, 333 tokens: 770 -> 593 us.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -47,12 +47,12 @@ struct MixedParams {
   const u4_t* codes;
   const u4_t* meta;
   const _Float16* scales;
-  long long codes_slot_u4, meta_slot_u4, scales_slot;
+  long long meta_slot_u4, scales_slot;
   const int* count;              // blocks in use
   const dz_mixed_block* blocks;
   _Float16* y;
   float* part;                   // partial sums [ksplit][T][N], or nullptr
-  int T, K, N, S, G, accumulate, ldy, tiles_n, NKB, NP, w_tiled, ksplit;
+  int T, K, N, G, accumulate, ldy, tiles_n, NKB, NP, w_tiled, ksplit;
   unsigned gmagic;               // group of a slab: (slab * gmagic) >> 32
 };
 
@@ -483,9 +483,9 @@ extern "C" int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_ba
   MixedParams P{};
   P.x = (const _Float16*)x; P.w = (const _Float16*)w_base; P.y = (_Float16*)y;
   P.codes = (const u4_t*)codes_stacked; P.meta = (const u4_t*)meta_stacked; P.scales = (const _Float16*)scales_stacked;
-  P.codes_slot_u4 = (long long)(cb / 16); P.meta_slot_u4 = (long long)(mb / 16); P.scales_slot = (long long)(sb / 2);
+  P.meta_slot_u4 = (long long)(mb / 16); P.scales_slot = (long long)(sb / 2);
   P.count = table; P.blocks = (const dz_mixed_block*)(table + DZ_MIXED_HEADER); P.part = ksplit > 1 ? partials : nullptr;
-  P.T = T; P.K = K; P.N = N; P.S = S; P.G = K / gs; P.accumulate = accumulate; P.ldy = ldy;
+  P.T = T; P.K = K; P.N = N; P.G = K / gs; P.accumulate = accumulate; P.ldy = ldy;
   P.NKB = K / DZ_KBLOCK; P.NP = N / DZ_NPAIR; P.w_tiled = w_tiled ? 1 : 0; P.ksplit = ksplit;
   P.tiles_n = (N + MN - 1) / MN;
   const unsigned gslabs = (unsigned)(gs / 64);

@@ -1146,8 +1146,7 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
         # row blocks made once serve the projections that would make the same ones
         shared = [q.shape[0] == S and (blocks is not None or (
                       _in_mixed_blocks(T, K, w.shape[0], S, None) is not None and not _short_chunks(T, K, w.shape[0], bits, S))
-                      or (_most_row_blocks(T, K, w.shape[0], bits, S, None) is None
-                          and not (S == 1 and _one_wave_of_long_blocks(T, w.shape[0], bits))))
+                      or _most_row_blocks(T, K, w.shape[0], bits, S, None) is None)
                   for q, w in zip(qweight_stacked, base_weight)]
         if blocks is None and sum(shared) > 1 and S <= MAX_SLOTS_SEGMENT and indices.is_cuda \
                 and indices.dtype == torch.int64 and indices.numel() == T and indices.is_contiguous():
