@@ -875,13 +875,14 @@ def _batched_equal_separate(dev, bits, gs, t, ns, k, nd):
 
 
 @pytest.mark.parametrize("n,k,bits,gs,nd,t,present", [
-    (256, 8192, 2, -1, 9, 129, None), (96, 8192, 4, 128, 3, 300, None), (128, 8192, 2, 64, 17, 256, None),   # chunks
-    (256, 512, 4, 64, 2, 150, 1), (2048, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None),            # row blocks
-    (27648, 256, 2, -1, 1, 512, None), (27648, 256, 2, -1, 1, 449, None), (27648, 256, 2, -1, 3, 512, 1),     # 256-token blocks
+    (256, 8192, 2, -1, 9, 129, None), (96, 8192, 4, 128, 3, 300, None), (128, 8192, 2, 64, 17, 256, None),   # few features
+    (256, 512, 4, 64, 2, 150, 1), (2048, 256, 2, -1, 24, 200, 3), (96, 256, 2, -1, 5, 384, None),            # short walks
+    (27648, 256, 2, -1, 1, 512, None), (27648, 256, 2, -1, 1, 449, None), (27648, 256, 2, -1, 3, 512, 1),     # wide, one delta
     (27648, 256, 2, -1, 1, 512, 0)])
 def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
-    """129 to 512 tokens through the routes the sizes, the slots and -- where the host knows it -- the mix
-    choose: the direct call, the call with the manager's row blocks, and several projections at once."""
+    """129 to 512 tokens by whatever route the sizes, the slots and -- where the host knows it -- the mix choose
+    (test_route_of_a_mid_size_call names them): the direct call, the call with the manager's row blocks, and several
+    projections at once."""
     p = make_problem(n, k, bits, gs, nd, t, "uniform", n + t, dev)
     if present is not None:
         p["ids_np"] = np.where(p["ids_np"] >= present, present - 1, p["ids_np"])
@@ -902,6 +903,48 @@ def test_every_route_of_a_mid_size_batch(dev, n, k, bits, gs, nd, t, present):
             assert o.rel_err(y.cpu().numpy(), ref) <= TOL
     for y in ops.apply_delta_batch(p["x"], [p["q"]] * 2, [p["s"]] * 2, [p["m"]] * 2, p["ids"], [p["wb"]] * 2):
         assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+
+
+class _Recorded:
+    """The library, with the names of the products it launches written down."""
+
+    def __init__(self, lib, names):
+        self.lib, self.names = lib, names
+
+    def __getattr__(self, name):
+        if name.startswith("dz_multi_delta"):
+            self.names.add(name.removeprefix("dz_multi_delta_"))
+        return getattr(self.lib, name)
+
+
+@pytest.mark.parametrize("n,k,bits,gs,nd,t,present,base,order,route", [
+    # without a base weight: one delta per block, or chunks of the decode kernel
+    (256, 8192, 2, -1, 9, 129, None, False, None, {"linear_chunks"}), (96, 8192, 4, 128, 3, 300, None, False, None, {"linear_chunks"}),
+    (128, 8192, 2, 64, 17, 256, None, False, "known", {"linear_chunks"}), (96, 256, 2, -1, 5, 384, None, False, None, {"gemm_rows"}),
+    (2048, 256, 2, -1, 24, 200, 3, False, "known", {"gemm_rows"}), (27648, 256, 2, -1, 3, 512, 2, False, "known", {"gemm_rows"}),
+    (27648, 256, 2, -1, 3, 512, 1, False, "known", {"gemm"}),                            # 256-token blocks, one wave of them
+    (27648, 256, 2, -1, 1, 512, None, False, None, {"gemm", "gemm_rows"}),               # the device picks
+    # with one: blocks of several deltas ...
+    (256, 8192, 2, -1, 9, 129, None, True, None, {"gemm_mixed"}), (96, 8192, 4, 128, 3, 300, None, True, "known", {"gemm_mixed"}),
+    (27648, 256, 2, -1, 1, 449, None, True, "known", {"gemm_mixed"}), (128, 2560, 2, 64, 3, 160, None, True, "plain", {"gemm_mixed"}),
+    # ... but for a short walk, a few tokens of each of many deltas, short walks in one wave of row blocks, few short chunks
+    (96, 256, 2, -1, 5, 384, None, True, None, {"gemm_rows"}), (96, 8192, 2, -1, 44, 129, None, True, "known", {"linear_chunks"}),
+    (256, 1280, 2, -1, 20, 170, None, True, "known", {"gemm_rows"}), (704, 1792, 4, 64, 1, 213, None, True, None, {"linear_chunks"})])
+def test_route_of_a_mid_size_call(dev, monkeypatch, n, k, bits, gs, nd, t, present, base, order, route):
+    """129 to 512 tokens: the products that are launched, by name, and what they give.  `order`: with row blocks whose
+    maker knew the mix, or did not, or the ids alone."""
+    from deltazip_amd import _lib
+    p = make_problem(n, k, bits, gs, nd, t, np.arange(t) % (present or nd), n + t, dev)
+    blocks = None
+    if order is not None:
+        blocks = ops.row_blocks(p["ids"], nd, mix=ops.batch_mix(p["ids_np"].tolist()) if order == "known" else None,
+                                deltas=ops.mixed_deltas(bits, gs != -1))
+    names, lib = set(), _lib.lib()
+    monkeypatch.setattr(_lib, "lib", lambda: _Recorded(lib, names))
+    y = ops.multi_delta_linear(p["x"], p["wb"] if base else None, p["q"], p["s"], p["m"], p["ids"], bits=bits, order=blocks)
+    torch.cuda.synchronize()
+    assert names == route
+    assert o.rel_err(y.cpu().numpy(), o.forward_ref(p["x_np"], p["wb_np"] if base else None, p["dts"], p["ids_np"])) <= TOL
 
 
 @pytest.mark.parametrize("n,k,bits,gs", [(352, 512, 2, -1), (96, 768, 4, 128)])
