@@ -182,7 +182,7 @@ class LinearWithDelta(BaseLayerWithDelta):
             blocks = self.row_blocks[0]
             # (a decode step that is captured keeps the token order, whose buffer stays: blocks serve eager calls only)
             if isinstance(blocks, ops.DecodeBlocks):
-                order = blocks.for_layer(*self.base_shape)
+                order = blocks.for_layer(*self.base_shape, order)
             elif T > ops.MAX_TOKENS_FUSED or (blocks is not None
                                               and blocks.captured == torch.cuda.is_current_stream_capturing()):
                 order = blocks

@@ -206,7 +206,7 @@ class DeltaModelManager:
         self.packed_modules: Dict[str, List[str]] = {}
         self.modules: Dict[str, BaseLayerWithDelta] = {}
         self._widest = 0                 # output features of the widest linear layer
-        self._projections: Dict[Tuple[int, int], int] = {}   # how many there are of every K, N
+        self._projections: Tuple[Tuple[Tuple[int, int], int], ...] = ()   # ((K, N), how many there are)
         self._last_mapping: Optional[DeltaMapping] = None
         self._wrap_modules()
         self.model.delta_manager = self
@@ -334,8 +334,10 @@ class DeltaModelManager:
         if T < 1 or T > n or P > n:
             raise ValueError(f"batch of {T} tokens / {P} sampled rows does not fit the index buffers ({n})")
         resident = {d for d in self.delta_index_to_id if d is not None}
-        for ids in (mapping.index_mapping, mapping.prompt_mapping):
-            for x in set(ids):
+        present = set(mapping.index_mapping)
+        met = len(present)                  # (the base model counts as one)
+        for ids in (present, set(mapping.prompt_mapping)):
+            for x in ids:
                 if x > 0 and x not in resident:
                     raise ValueError(f"{x} is not in list")     # what list.index raises in the reference
         if self._staged is not None:
@@ -369,9 +371,8 @@ class DeltaModelManager:
                 self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
                                                     mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
                                                     features=self._widest or None, deltas=deltas)
-            elif T > 32 and ops.decode_step_mixes(T, cfg.max_bitwidth, len(set(mapping.index_mapping)), self._projections):
-                self.row_blocks[0] = ops.DecodeBlocks(self.base_indices[:T], self.delta_slots, mapping.index_mapping, deltas,
-                                                      self.token_order[:T])
+            elif T > 32 and ops.decode_step_mixes(T, cfg.max_bitwidth, met, self._projections):
+                self.row_blocks[0] = ops.DecodeBlocks(self.base_indices, self.delta_slots, mapping.index_mapping, met, deltas)
         # the layers keep a reference to this list
         self.indices_len[:] = (T, P, P, T)
 
@@ -436,7 +437,9 @@ class DeltaModelManager:
             n, k = getattr(module, "base_shape", (0, 0))
             self._widest = max(self._widest, n)
             if k and n:
-                self._projections[k, n] = self._projections.get((k, n), 0) + 1
+                count = dict(self._projections)
+                count[k, n] = count.get((k, n), 0) + 1
+                self._projections = tuple(count.items())
         # a fused layer also answers for the projections it is made of (q/k/v, gate/up)
         parent, _, leaf = module_name.rpartition(".")
         parts = self.packed_modules_mapping.get(leaf)

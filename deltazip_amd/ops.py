@@ -195,20 +195,21 @@ class MixedTable(NamedTuple):
 class DecodeBlocks:
     """The blocks of several deltas of a decode step, made by the first eager call on each stream of a layer that takes
     them: a step that is replayed from a graph reads the token order and never asks, and the tables belong to the stream
-    whose calls read them.  `ids`: of the tokens, any, one per delta and one for the base model."""
-    __slots__ = ("indices", "S", "ids", "met", "deltas", "order", "made")
+    whose calls read them.  `ids`: of the tokens, any, one per delta and one for the base model, `met` of them; `indices`
+    may be longer."""
+    __slots__ = ("indices", "S", "ids", "met", "deltas", "made")
 
-    def __init__(self, indices, S, ids, deltas, order):
-        self.indices, self.S, self.ids, self.met, self.deltas = indices, S, ids, len(set(ids)), deltas
-        self.order, self.made = order, {}
+    def __init__(self, indices, S, ids, met, deltas):
+        self.indices, self.S, self.ids, self.met, self.deltas, self.made = indices, S, ids, met, deltas, {}
 
-    def for_layer(self, N: int, K: int):
-        """What a layer of that size passes on as `order`."""
-        if not mixes_at_decode(len(self.ids), K, N, self.met) or torch.cuda.is_current_stream_capturing():
-            return self.order
+    def for_layer(self, N: int, K: int, order: torch.Tensor):
+        """What a layer of that size passes on as `order`, given the token order."""
+        T = len(self.ids)
+        if not mixes_at_decode(T, K, N, self.met) or torch.cuda.is_current_stream_capturing():
+            return order
         stream = _stream()
         if stream not in self.made:
-            self.made[stream] = row_blocks(self.indices, self.S, mix=batch_mix(self.ids), deltas=self.deltas, order=self.order)
+            self.made[stream] = row_blocks(self.indices[:T], self.S, mix=batch_mix(self.ids), deltas=self.deltas, order=order)
         return self.made[stream]
 
 
@@ -285,18 +286,18 @@ def mixes_at_decode(T: int, K: int, N: int, deltas: int) -> bool:
     return deltas <= (16 if T > 112 else 8 if T > 64 or T <= 40 else 2)
 
 
-def decode_step_mixes(T: int, bits: int, deltas: int, projections: Dict[Tuple[int, int], int]) -> bool:
-    """Whether a decode step over so many `projections` of (K, N) makes tables for blocks of several deltas: where
+@lru_cache(maxsize=4096)
+def decode_step_mixes(T: int, bits: int, deltas: int, projections: Tuple[Tuple[Tuple[int, int], int], ...]) -> bool:
+    """Whether a decode step over `projections`, ((K, N), how many), makes tables for blocks of several deltas: where
     one of them would take such blocks, and the decode kernel keeps the GPU busy for longer than the host needs to
     launch the step.  A layer call takes the host some 30 us, 3 more over blocks (a second launch, the sums' tensor),
     and the blocks are looked up by the projections that do not take them, too.  By 190 timed layers of four projections
     that went in blocks: below 160 us of the decode kernel, as `_route_us` has it, 120 us became 130
     (2048/8448, 81 tokens of 4 deltas, 4-bit), at 160 and above 1.22 times as fast in the mean, 0.94 at worst."""
-    if not any(mixes_at_decode(T, k, n, deltas) for k, n in projections):
+    if not any(mixes_at_decode(T, k, n, deltas) for (k, n), _ in projections):
         return False
     mix = _even_mix(T, deltas)
-    return (sum(count * _route_us(T, k, n, bits, mix)[0] for (k, n), count in projections.items())
-            >= 40 * sum(projections.values()))
+    return sum(c * _route_us(T, k, n, bits, mix)[0] for (k, n), c in projections) >= 40 * sum(c for _, c in projections)
 
 
 @lru_cache(maxsize=4096)
@@ -1047,19 +1048,21 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
         return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
                                           indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
                                           base_tiled=base_tiled)
-    if T > 32 and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT:
-        blocks = order if isinstance(order, RowBlocks) and order.order is not None else None
-        if blocks is not None and (blocks.T != T or blocks.S != S or blocks.mix is None
-                                   or blocks.captured != torch.cuda.is_current_stream_capturing()):
-            blocks = None
+    blocks, met = None, T
+    if isinstance(order, RowBlocks):
+        if (order.order is not None and order.T == T and order.S == S and order.mix is not None
+                and order.captured == torch.cuda.is_current_stream_capturing()):
+            blocks, met = order, order.mix.deltas
+    elif order is None and T > 64 and S <= 4 and K * N >= 40 << 20:
         # A call that has to make its own table takes 8 us for it: large layers over few slots only (5120 x 13824, 100
         # tokens of 4 slots 104 -> 70 us; 4096 x 12288, 4-bit, 128 tokens of 8 106 / 111).
-        met = blocks.mix.deltas if blocks is not None else S if order is None and T > 64 and S <= 4 and K * N >= 40 << 20 else T
-        if mixes_at_decode(T, K, N, met):
-            from .prefill import multi_delta_linear_mixed
-            return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
-                                            bits=bits, out=out, accumulate=accumulate, plan=_decode_plan(T, K, N, met),
-                                            blocks=blocks, base_tiled=base_tiled)
+        met = S
+    if (met < T and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT
+            and mixes_at_decode(T, K, N, met)):
+        from .prefill import multi_delta_linear_mixed
+        return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
+                                        bits=bits, out=out, accumulate=accumulate, plan=_decode_plan(T, K, N, met),
+                                        blocks=blocks, base_tiled=base_tiled)
     ws = _workspace(x.device, T, K, N)
     optr = _order_ptr(order, T, x.device)
     if base_tiled is not None:

@@ -1280,22 +1280,22 @@ def test_decode_blocks_of_each_stream(dev):
     ids_np = np.random.default_rng(t).integers(-1, S, t)
     ids = torch.from_numpy(ids_np).to(dev)
     order = ops.token_order(ids, S)
-    made = ops.DecodeBlocks(ids, S, ids_np.tolist(), 3, order)
+    made = ops.DecodeBlocks(ids, S, ids_np.tolist(), len(set(ids_np.tolist())), 3)
     want = ops.apply_delta(x, q, s, m, ids, w, order=ops.row_blocks(ids, S, mix=ops.batch_mix(ids_np.tolist()), order=order))
-    assert made.for_layer(1024, 1024) is order
+    assert made.for_layer(1024, 1024, order) is order
     streams = [torch.cuda.current_stream(), torch.cuda.Stream()]
     streams[1].wait_stream(streams[0])
     for turn in range(2):
         for stream in streams:
             with torch.cuda.stream(stream):
-                blocks = made.for_layer(n, k)
+                blocks = made.for_layer(n, k, order)
                 y = ops.apply_delta(x, q, s, m, ids, w, order=blocks)
             torch.cuda.synchronize()
             assert torch.equal(y, want) and blocks.mixed[1] is None
     assert len(made.made) == 2
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.stream(streams[1]), torch.cuda.graph(graph, stream=streams[1]):
-        assert made.for_layer(n, k) is order
+        assert made.for_layer(n, k, order) is order
         y.add_(0)
     torch.cuda.synchronize()
 

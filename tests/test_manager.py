@@ -670,9 +670,9 @@ def _mapped(monkeypatch, layers):
     for name in ("map_ids", "token_order", "poll_status"):
         monkeypatch.setattr(ops, name, lambda *a, **kw: None)
     mgr = create_delta_manager(ToyModel(), 128, 256, V, DeltaConfig(max_deltas=8, max_bitwidth=4, group_size=-1))
-    assert mgr._projections == {(H, H + 128): 1, (H, H): 1, (H, 2 * I): 1, (I, H): 1}
+    assert dict(mgr._projections) == {(H, H + 128): 1, (H, H): 1, (H, 2 * I): 1, (I, H): 1}
     mgr.delta_index_to_id = list(range(1, 9))
-    mgr._projections = {(k, n): 32 for h, i in layers for k, n in ((h, 3 * h), (h, h), (h, 2 * i), (i, h))}
+    mgr._projections = tuple(((k, n), 32) for h, i in layers for k, n in ((h, 3 * h), (h, h), (h, 2 * i), (i, h)))
     return mgr
 
 
