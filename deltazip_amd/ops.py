@@ -225,8 +225,9 @@ def mixed_deltas(bits: int, grouped: bool) -> int:
 @lru_cache(maxsize=4096)
 def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
     """How a batch of more than 128 tokens takes blocks of several deltas: (0 for full blocks, 1 for small
-    ones; parts K is cut into), or None where they do not pay.  By the sizes alone, so that a token's result
-    depends on neither the mix nor its place in the batch.
+    ones; parts K is cut into), or None where they do not pay.  By the sizes alone, so that above 512 tokens a token's
+    result depends on neither the mix nor its place in the batch (up to 512 `_in_mixed_blocks` and `_short_chunks` may
+    choose another kernel, whose fp32 sums have another order).
 
     Fitted to 2240 timed batches of 129 to 1700 tokens and 3780 of 129 to 8192 (1 to 64 slots, sorted ids and
     requests, both bit widths, K from 512 to 13824, N to 27648): the choice takes 6.6 % longer in the mean than
@@ -239,8 +240,8 @@ def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
                      blocks than T / 64, and from 224 workgroups by that count they were a second wave (2560
                      x 10240, 401 tokens of 3 deltas, 4-bit: full 50, small 67 us, one delta per block 60)
       parts          each a walk over its share of K, and one more pass over the sums at 3 TB/s (13824 x 5120,
-                     333 tokens of 10 deltas: 1 / 2 / 3 / 4 / 6 parts 220 / 128 / 100 / 122 / 110 us, of which the
-                     estimate takes 4, counting 3 blocks where there are 4); one where the host takes longer to launch
+                     333 tokens of 10 deltas: 1 / 2 / 3 / 4 / 6 parts 222 / 135 / 112 / 146 / 124 us, one delta per
+                     block 160; the estimate takes 4, for it counts T / 128 blocks, 3, where there are 4); one where the host takes longer to launch
                      the sums than the walk takes (1536 x 1536, 263 tokens: 26.6 in 3 parts, 21.2 in one)
       K <= 1024      the walk is too short to pay for a workgroup's start unless there are several waves of them
                      (1024 x 8192: 129 tokens 14 / 19 us, 640 tokens 1.24 times as fast)"""
@@ -291,7 +292,7 @@ def decode_step_mixes(T: int, bits: int, deltas: int, projections: Tuple[Tuple[T
     """Whether a decode step over `projections`, ((K, N), how many), makes tables for blocks of several deltas: where
     one of them would take such blocks, and the decode kernel keeps the GPU busy for longer than the host needs to
     launch the step.  A layer call takes the host some 30 us, 3 more over blocks (a second launch, the sums' tensor),
-    and the blocks are looked up by the projections that do not take them, too.  By 190 timed layers of four projections
+    and the blocks are looked up by every projection.  By 190 timed layers of four projections
     that went in blocks: below 160 us of the decode kernel, as `_route_us` has it, 120 us became 130
     (2048/8448, 81 tokens of 4 deltas, 4-bit), at 160 and above 1.22 times as fast in the mean, 0.94 at worst."""
     if not any(mixes_at_decode(T, k, n, deltas) for (k, n), _ in projections):
@@ -302,7 +303,9 @@ def decode_step_mixes(T: int, bits: int, deltas: int, projections: Tuple[Tuple[T
 
 @lru_cache(maxsize=4096)
 def _decode_plan(T: int, K: int, N: int, deltas: int) -> Tuple[int, int]:
-    """`_mixed_plan` of such a batch, whose number of blocks is that of its deltas."""
+    """`_mixed_plan` of such a batch, whose number of blocks is taken to be that of its deltas over four (at 4 bits and with
+    grouped scales there are three to a block, and the base model's tokens have blocks of their own).  A token's result
+    so depends on how many deltas share the batch, by the order of fp32 sums."""
     return 0, _parts(T, K, N, max(1, -(-deltas // 4)), 1.7)
 
 
@@ -474,8 +477,9 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     widest layer they are for, if known.
 
     Layers with a base weight take the batch in blocks of several deltas where those pay (`_mixed_plan`): their
-    tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers.  `order`: token_order() of the same
-    indices, for a batch of up to 128 tokens (mixes_at_decode)."""
+    tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers (a layer that can hold more in a block reads
+    tables made for three all the same, one that can hold fewer makes its own).  `order`: token_order() of the same
+    indices, for a batch of up to 128 tokens: the table of full blocks is then all that is made (mixes_at_decode)."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
