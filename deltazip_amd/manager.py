@@ -370,7 +370,8 @@ class DeltaModelManager:
                 # (the mix decides at sizes where other routes than row blocks may be the faster one)
                 self.row_blocks[0] = ops.row_blocks(self.base_indices[:T], self.delta_slots,
                                                     mix=ops.batch_mix(mapping.index_mapping) if T <= 512 else None,
-                                                    features=self._widest or None, deltas=deltas)
+                                                    features=self._widest or None, deltas=deltas,
+                                                    mixed=any(ops._mixed_plan(T, k, n) for (k, n), _ in self._projections))
             elif T > 32 and ops.decode_step_mixes(T, cfg.max_bitwidth, met, self._projections):
                 self.row_blocks[0] = ops.DecodeBlocks(self.base_indices, self.delta_slots, mapping.index_mapping, met, deltas)
         # the layers keep a reference to this list

@@ -452,7 +452,7 @@ def own_mixed_table(indices: torch.Tensor, S: int, small: int, deltas: int) -> M
 
 def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, mix: Optional[BatchMix] = None,
                device_picks: bool = False, features: Optional[int] = None, deltas: int = 3,
-               order: Optional[torch.Tensor] = None) -> RowBlocks:
+               order: Optional[torch.Tensor] = None, mixed: bool = True) -> RowBlocks:
     """Row blocks of a prefill-sized batch, as the reference converts its mapping once per batch
     (serving/vllm/delta/models.py:421-435).  Small launches, nothing read back to the host.
 
@@ -479,12 +479,13 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
     Layers with a base weight take the batch in blocks of several deltas where those pay (`_mixed_plan`): their
     tables are made in the same launch.  `deltas`: `mixed_deltas` of the layers (a layer that can hold more in a block reads
     tables made for three all the same, one that can hold fewer makes its own).  `order`: token_order() of the same
-    indices, for a batch of up to 128 tokens: the table of full blocks is then all that is made (mixes_at_decode)."""
+    indices, for a batch of up to 128 tokens: the table of full blocks is then all that is made (mixes_at_decode).  `mixed`: False
+    leaves the blocks of several deltas out, for a call that has turned them down."""
     indices = indices.reshape(-1)
     if not indices.is_contiguous():
         raise ValueError("indices must be contiguous")
     T = indices.numel()
-    if order is not None and T <= MAX_TOKENS_FUSED and not long_only:   # (a decode step takes full blocks only)
+    if mixed and order is not None and T <= MAX_TOKENS_FUSED and not long_only:   # (a decode step takes full blocks only)
         full = own_mixed_table(indices, num_slots, 0, deltas)
         return RowBlocks(full.table[-T:], None, 0, T, num_slots, mix=mix, mixed=[full, None], order=order)
     # (at the sizes chunks of the fused kernel can serve, bad ids are reported as that kernel does)
@@ -498,16 +499,24 @@ def row_blocks(indices: torch.Tensor, num_slots: int, long_only: bool = False, m
         tiles, n = _block_table(T, num_slots, 256, dev)
     if small or device_picks or (not long_only and T < 256 * (num_slots + 1)):
         short, ns = _block_table(T, num_slots, SHORT_ROWS, dev)
-    if long_only:
-        _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
-        return RowBlocks(perm, tiles, n, T, num_slots)
-    mixed = [_mixed_table(T, num_slots, small_ones, deltas, dev) for small_ones in (0, 1)]
-    ptr = lambda t: None if t is None else t.data_ptr()
-    _lib.check(L.dz_build_tables(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, ptr(tiles), n, ptr(short), ns,
-                                 int(tiles is not None and short is not None and not host_picks), mixed[0].deltas,
-                                 mixed[0].table.data_ptr(), mixed[0].max_blocks, mixed[1].table.data_ptr(),
-                                 mixed[1].max_blocks, st), "dz_build_tables")
-    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks, mixed, order)
+    either = tiles is not None and short is not None and not host_picks
+    if mixed and not long_only:
+        made = [_mixed_table(T, num_slots, small_ones, deltas, dev) for small_ones in (0, 1)]
+        ptr = lambda t: None if t is None else t.data_ptr()
+        _lib.check(L.dz_build_tables(seg_off.data_ptr(), perm.data_ptr(), num_slots, T, ptr(tiles), n, ptr(short), ns,
+                                     int(either), made[0].deltas, made[0].table.data_ptr(), made[0].max_blocks,
+                                     made[1].table.data_ptr(), made[1].max_blocks, st), "dz_build_tables")
+        return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks, made, order)
+    if either:
+        _lib.check(L.dz_build_tiles_either(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, short.data_ptr(), ns, st),
+                   "dz_build_tiles_either")
+    else:
+        if tiles is not None:
+            _lib.check(L.dz_build_tiles(seg_off.data_ptr(), num_slots, tiles.data_ptr(), n, st), "dz_build_tiles")
+        if short is not None:
+            _lib.check(L.dz_build_tiles_rows(seg_off.data_ptr(), num_slots, SHORT_ROWS, short.data_ptr(), ns, st),
+                       "dz_build_tiles_rows")
+    return RowBlocks(perm, tiles, n, T, num_slots, short, ns, mix, host_picks)
 
 
 def apply_delta_embed(x: torch.Tensor, delta_weights: torch.Tensor, indices: torch.Tensor,

@@ -62,7 +62,7 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
     stream = torch.cuda.current_stream().cuda_stream
     one_wave = _one_wave_of_long_blocks(T, N, bits)
     if blocks is None:
-        blocks = row_blocks(indices, S, device_picks=S == 1 and one_wave, features=N)
+        blocks = row_blocks(indices, S, device_picks=S == 1 and one_wave, features=N, mixed=False)
     take_long, take_short = blocks.tiles is not None, blocks.short is not None
     if blocks.host_picks:
         take_long, take_short = one_wave, not one_wave

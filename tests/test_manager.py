@@ -647,6 +647,13 @@ def test_row_blocks_hold_blocks_of_one_delta(launches, t, order, tables):
         with pytest.raises(ValueError):
             multi_delta_linear_prefill(*args, bits=2, out=out, accumulate=False, blocks=blocks)
     else:
+        assert blocks.mixed is not None and launches == ["dz_build_tables"]
+        launches.clear()
+        multi_delta_linear_prefill(*args, bits=2, out=out, accumulate=False)   # (makes the table it reads and no other)
+        assert [n for n in launches if "build" in n] == ["dz_build_tiles" if tables == "long" else "dz_build_tiles_rows"]
+        ops.row_blocks(ids, s, mixed=False)
+        assert launches[-1] == {"short": "dz_build_tiles_rows", "long": "dz_build_tiles", "both": "dz_build_tiles_either"}[tables]
+        launches.clear()
         multi_delta_linear_prefill(*args, bits=2, out=out, accumulate=False, blocks=blocks)
         assert [n for n in launches if "gemm" in n] == ["dz_multi_delta_gemm"] * (tables != "short") + \
             ["dz_multi_delta_gemm_rows"] * (tables != "long")
@@ -743,6 +750,15 @@ def test_route_of_a_call_that_makes_its_own_table(monkeypatch, launches, t, k, n
     if slots <= 768:
         known = ops.row_blocks(ids, slots, deltas=3)
         assert called(lambda: ops.apply_delta(x, *stack, ids, w, order=known)) == {"dz_multi_delta_gemm_mixed"}
+
+
+@pytest.mark.parametrize("layers,mixed", [([(256, 512)], False), ([(1024, 1024)], False), ([(256, 512), (4096, 11008)], True)])
+def test_mapping_makes_the_tables_its_projections_read(monkeypatch, launches, layers, mixed):
+    mgr = _mapped(monkeypatch, layers)
+    ids = tuple(1 + i // 32 for i in range(200))
+    mgr.set_delta_mapping(DeltaMapping(ids, ids[:1]))
+    assert launches == ["dz_build_tables" if mixed else "dz_build_tiles_rows"]
+    assert (mgr.row_blocks[0].mixed is not None) == mixed and mgr.row_blocks[0].short is not None
 
 
 @pytest.mark.parametrize("made_captured,capturing,blocks_go", [(False, False, True), (False, True, False), (True, True, True)])
