@@ -52,6 +52,8 @@ SIGNATURES = {
                                          _vp, C.c_size_t, _vp]),
     "dz_multi_delta_linear_batch_tiled": (_i, [_i, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i,
                                                _vp, _vp, C.c_size_t, _vp]),
+    "dz_multi_delta_linear_ordered": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _vp, _vp, _i, _i, _i, _i, _i, _i, _i, _i, _vp, _vp,
+                                           C.c_size_t, _vp]),
     "dz_tile_base": (_i, [_vp, _i, _i, _vp, _vp]),
     "dz_token_order": (_i, [_vp, _i, _i, _vp, _vp]),
     "dz_map_ids": (_i, [_vp, _i, _vp, _i, _vp, _i, _i, _i, _i, _vp, _vp, _vp, _vp, _i, _vp, _vp]),

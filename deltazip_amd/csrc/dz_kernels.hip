@@ -1067,6 +1067,15 @@ int dz_multi_delta_linear_batch_tiled(int ncalls, const uint16_t* const* x, cons
                                   stream, 1);
 }
 
+int dz_multi_delta_linear_ordered(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                                  const void* meta_stacked, const void* scales_stacked, const int64_t* indices, uint16_t* y,
+                                  int T, int K, int N, int S, int bits, int group_size, int accumulate, int ldy,
+                                  const int32_t* order, void* workspace, size_t workspace_bytes, void* stream) {
+  if (!x || !indices || !y) return DZ_EINVAL;
+  return multi_delta_linear_batch(1, &x, &w_base, &codes_stacked, &meta_stacked, &scales_stacked, indices, &y, &N, &ldy, T, K, S,
+                                  bits, group_size, accumulate, order, workspace, workspace_bytes, stream, w_tiled);
+}
+
 int dz_multi_delta_linear_chunks(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
                                  const void* meta_stacked, const void* scales_stacked, const int64_t* indices,
                                  uint16_t* y, int T, int K, int N, int S, int bits, int group_size, int accumulate,

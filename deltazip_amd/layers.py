@@ -61,6 +61,12 @@ class BaseLayerWithDelta(nn.Module):
         ...
 
 
+def _base_of(layer):
+    """`layer.base_layer` (a sub-module, or any object with a weight), without nn.Module's search for the name."""
+    base = layer.__dict__.get("_modules", {}).get("base_layer")
+    return layer.base_layer if base is None else base
+
+
 class LinearWithDelta(BaseLayerWithDelta):
     """Shared implementation of the four linear variants."""
 
@@ -186,7 +192,7 @@ class LinearWithDelta(BaseLayerWithDelta):
             elif T > ops.MAX_TOKENS_FUSED or (blocks is not None
                                               and blocks.captured == torch.cuda.is_current_stream_capturing()):
                 order = blocks
-        w = self.base_layer.weight
+        w = _base_of(self).weight
         if self._row_major_dropped:
             w = None
         elif self.base_tiled is not None and self._tiled_of != (w.data_ptr(), w._version):
@@ -196,8 +202,9 @@ class LinearWithDelta(BaseLayerWithDelta):
                                self.indices[:T], w, order=order, base_tiled=self.base_tiled)
 
     def forward(self, input_):
-        skip_bias_add = getattr(self.base_layer, "skip_bias_add", False)
-        base_bias = getattr(self.base_layer, "bias", None)
+        base = _base_of(self)
+        skip_bias_add = getattr(base, "skip_bias_add", False)
+        base_bias = getattr(base, "bias", None)
         bias = base_bias if not skip_bias_add else None
         output = self.apply_weights(input_, bias)
         if bias is not None:
@@ -248,7 +255,7 @@ class RowParallelLinearWithDelta(LinearWithDelta):
     _n_packed = 0
 
     def apply_weights(self, x: torch.Tensor, bias=None) -> torch.Tensor:
-        if getattr(self.base_layer, "bias", None) is not None:
+        if getattr(_base_of(self), "bias", None) is not None:
             raise ValueError("RowParallelLinearWithDelta does not support bias yet.")
         return super().apply_weights(x, None)
 

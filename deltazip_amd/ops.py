@@ -37,6 +37,15 @@ def native_sizes(K: int, N: int, bits: int, group_size: int = -1) -> Tuple[int, 
     return cb.value, mb.value, sb.value
 
 
+_sizes = lru_cache(maxsize=4096)(native_sizes)      # of the calls' path: by the sizes alone
+
+
+def _slot_bytes_differ(q, m, sc, sizes) -> bool:
+    cb, mb, sb = sizes
+    return (_slot_numel(q) * q.element_size() != cb or _slot_numel(m) * m.element_size() != mb
+            or _slot_numel(sc) * sc.element_size() != sb)
+
+
 def stacked_shapes(K: int, N: int, bits: int, group_size: int = -1):
     """Shapes (without the leading slot dimension) of the three stacked tensors, following
     layers_marlin.py:311-333: qweight [K/(pf*4), 2N] int32, meta [N, K/16] int16, scales [G, N]."""
@@ -111,8 +120,22 @@ def unrepack_native_to_gptq(qweight: torch.Tensor, meta: torch.Tensor, scales: t
     return out_q, out_z, out_s, out_g
 
 
+# The host's half of a call over a small layer is longer than the kernel: what it looks up more than once is looked up
+# here.  (The raw handle without the Stream object around it: 0.3 against 3.6 us.)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_current_device = getattr(torch._C, "_cuda_getDevice", None)
+
+
 def _stream() -> int:
-    return torch.cuda.current_stream().cuda_stream
+    if _raw_stream is None or _current_device is None:
+        return torch.cuda.current_stream().cuda_stream
+    return _raw_stream(_current_device())
+
+
+def _slot_numel(stacked: torch.Tensor) -> int:
+    """Values of one slot of a stacked tensor (IndexError where there is none)."""
+    shape = stacked.shape
+    return stacked.numel() // shape[0] if shape and shape[0] else stacked[0].numel()
 
 
 def _need_cuda(*ts):
@@ -426,10 +449,15 @@ def _block_table(T: int, num_slots: int, rows: int, device):
     return torch.empty((n, 4), dtype=torch.int32, device=device), n
 
 
+@lru_cache(maxsize=4096)
+def _most_mixed_blocks(T: int, S: int, tiles: int, deltas: int) -> int:
+    return _lib.lib().dz_mixed_blocks(T, S, tiles, deltas)
+
+
 def _mixed_table(T: int, S: int, small: int, deltas: int, device, behind: int = 0) -> MixedTable:
     tiles, most = MIXED_BLOCKS[small]
     deltas = min(deltas, most)
-    n = _lib.lib().dz_mixed_blocks(T, S, tiles, deltas)
+    n = _most_mixed_blocks(T, S, tiles, deltas)
     # DZ_MIXED_HEADER words and n times sizeof(dz_mixed_block)
     return MixedTable(torch.empty(4 + n * (2 + 4 * 4 + 128) + behind, dtype=torch.int32, device=device), n, deltas)
 
@@ -777,10 +805,15 @@ STATUS_BAD_ID = 1              # a delta id outside [-1, S) was met and treated 
 STATUS_SUM_MISSING = 2         # a partial sum of a K-slice did not arrive: that call's output is invalid
 
 
+@lru_cache(maxsize=4096)
+def _workspace_bytes(T: int, K: int, N: int) -> int:
+    return _lib.lib().dz_workspace_bytes(T, K, N)
+
+
 def _workspace(device: torch.device, T: int, K: int, N: int) -> torch.Tensor:
-    need = _lib.lib().dz_workspace_bytes(T, K, N)
-    idx = device.index if device.index is not None else torch.cuda.current_device()
-    key = (idx, _stream())
+    need = _workspace_bytes(T, K, N)
+    idx = device.index
+    key = (torch.cuda.current_device() if idx is None else idx, _stream())
     ws = _workspaces.get(key)
     if ws is None or ws.numel() < need:
         new = torch.zeros(max(need, 1 << 20), dtype=torch.uint8, device=device)
@@ -927,7 +960,7 @@ def untile_base(tiled: torch.Tensor) -> torch.Tensor:
 
 
 def _check_tiled(base_tiled, base_weight, N: int, K: int, device) -> None:
-    if tuple(base_tiled.shape) != (N, K) or base_tiled.dtype != torch.float16 \
+    if base_tiled.shape != (N, K) or base_tiled.dtype != torch.float16 \
             or not base_tiled.is_contiguous() or base_tiled.device != device \
             or (base_weight is not None and base_weight.numel() and base_tiled.shape != base_weight.shape):
         raise ValueError("base_tiled must be tile_base(base_weight): float16 [N, K], contiguous, on x's device")
@@ -993,39 +1026,41 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
         raise ValueError("indices must be int64")
     if bits not in (2, 4):
         raise NotImplementedError("Only 2 and 4 bits are supported.")
-    K = x.shape[-1]
-    x2 = x.reshape(-1, K)
+    x2 = x if x.dim() == 2 else x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous():
         x2 = x2.contiguous()
-    T = x2.shape[0]
-    indices = indices.reshape(-1)
-    if indices.numel() != T or not indices.is_contiguous():
+    T, K = x2.shape
+    if indices.dim() != 1:
+        indices = indices.reshape(-1)
+    if indices.shape[0] != T or not indices.is_contiguous():
         raise ValueError("indices must be a contiguous vector with one entry per token")
     S = qweight_stacked.shape[0]
     N = scales_stacked.shape[-1]
+    device = x.device
     if base_tiled is not None:
-        _check_tiled(base_tiled, base_weight, N, K, x.device)
+        _check_tiled(base_tiled, base_weight, N, K, device)
         if base_weight is not None and base_weight.numel() == 0:
             base_weight = None
     if base_weight is not None:
-        if base_weight.dtype != torch.float16 or tuple(base_weight.shape) != (N, K) or not base_weight.is_contiguous():
+        if base_weight.dtype != torch.float16 or base_weight.shape != (N, K) or not base_weight.is_contiguous():
             raise ValueError("base_weight must be a contiguous float16 [N, K] tensor")
-    G = scales_stacked[0].numel() // N
+    G = _slot_numel(scales_stacked) // N
     group_size = -1 if G == 1 else K // G
-    cb, mb, sb = native_sizes(K, N, bits, group_size)
-    if (qweight_stacked[0].numel() * qweight_stacked.element_size() != cb
-            or meta_stacked[0].numel() * meta_stacked.element_size() != mb
+    cb, mb, _ = _sizes(K, N, bits, group_size)
+    if (_slot_numel(qweight_stacked) * qweight_stacked.element_size() != cb
+            or _slot_numel(meta_stacked) * meta_stacked.element_size() != mb
             or not qweight_stacked.is_contiguous() or not meta_stacked.is_contiguous()
             or not scales_stacked.is_contiguous() or scales_stacked.dtype != torch.float16):
         raise ValueError("stacked delta tensors do not match the native layout for these sizes")
     if out is None:
         if accumulate:
             raise ValueError("accumulate needs an output tensor")
-        out = torch.empty((T, N), dtype=torch.float16, device=x.device)
+        out = torch.empty((T, N), dtype=torch.float16, device=device)
+        ldy = N
     else:
         if out.dtype != torch.float16 or out.dim() != 2 or out.shape != (T, N) or out.stride(1) != 1:
             raise ValueError("out must be float16 [T, N] with unit column stride")
-    ldy = out.stride(0)
+        ldy = out.stride(0)
     if T > MAX_TOKENS_FUSED:
         blocks = _usable_blocks(order, T, S)
         plan = None
@@ -1033,20 +1068,19 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
                 and (not _short_chunks(T, K, N, bits, S) if blocks is None else blocks.mixed is not None)):
             plan = _in_mixed_blocks(T, K, N, S, blocks.mix if blocks is not None else None)
         if plan is not None:
-            from .prefill import multi_delta_linear_mixed
-            return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
-                                            bits=bits, out=out, accumulate=accumulate, plan=plan, blocks=blocks,
-                                            base_tiled=base_tiled)
+            return prefill.multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
+                                                    bits=bits, out=out, accumulate=accumulate, plan=plan, blocks=blocks,
+                                                    base_tiled=base_tiled)
         most = _most_row_blocks(T, K, N, bits, S, blocks)
         if most is not None:
-            ws = _workspace(x.device, MAX_TOKENS_FUSED, K, N)
+            ws = _workspace(device, MAX_TOKENS_FUSED, K, N)
             w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
             delta = (qweight_stacked.data_ptr(), meta_stacked.data_ptr(), scales_stacked.data_ptr())
             shape = (T, K, N, 1 if accumulate else 0, ldy)
             wptr, over, L, st = w.data_ptr() if w is not None else None, None, _lib.lib(), _stream()
             if most:                                  # the row blocks if there are few, else the chunks
                 perm, seg_off = segment(indices, S, True)
-                table = torch.empty(4 * most + 1, dtype=torch.int32, device=x.device)
+                table = torch.empty(4 * most + 1, dtype=torch.int32, device=device)
                 over = table[4 * most:].data_ptr()
                 _lib.check(L.dz_build_tiles_rows_upto(seg_off.data_ptr(), S, SHORT_ROWS, most, table.data_ptr(), most,
                                                       over, st), "dz_build_tiles_rows_upto")
@@ -1057,10 +1091,9 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
                                                       out.data_ptr(), T, K, N, S, bits, group_size, *shape[3:], over,
                                                       ws.data_ptr(), ws.numel(), st), "dz_multi_delta_linear_chunks")
             return out
-        from .prefill import multi_delta_linear_prefill
-        return multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
-                                          indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
-                                          base_tiled=base_tiled)
+        return prefill.multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked,
+                                                  indices, bits=bits, out=out, accumulate=accumulate, blocks=blocks,
+                                                  base_tiled=base_tiled)
     blocks, met = None, T
     if isinstance(order, RowBlocks):
         if (order.order is not None and order.T == T and order.S == S and order.mix is not None
@@ -1072,40 +1105,21 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
         met = S
     if (met < T and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT
             and mixes_at_decode(T, K, N, met)):
-        from .prefill import multi_delta_linear_mixed
-        return multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
-                                        bits=bits, out=out, accumulate=accumulate, plan=_decode_plan(T, K, N, met),
-                                        blocks=blocks, base_tiled=base_tiled)
-    ws = _workspace(x.device, T, K, N)
-    optr = _order_ptr(order, T, x.device)
-    if base_tiled is not None:
-        one = lambda p: (C.c_void_p * 1)(p)
-        rc = _lib.lib().dz_multi_delta_linear_batch_tiled(
-            1, one(x2.data_ptr()), one(base_tiled.data_ptr()), one(qweight_stacked.data_ptr()),
-            one(meta_stacked.data_ptr()), one(scales_stacked.data_ptr()), indices.data_ptr(), one(out.data_ptr()),
-            (C.c_int * 1)(N), (C.c_int * 1)(ldy), T, K, S, bits, group_size, 1 if accumulate else 0, optr,
-            ws.data_ptr(), ws.numel(), _stream())
-        _lib.check(rc, "dz_multi_delta_linear_batch_tiled")
-        return out
-    if optr is None:
-        rc = _lib.lib().dz_multi_delta_linear(
-            x2.data_ptr(), base_weight.data_ptr() if base_weight is not None else None,
-            qweight_stacked.data_ptr(), meta_stacked.data_ptr(), scales_stacked.data_ptr(),
-            indices.data_ptr(), out.data_ptr(), T, K, N, S, bits, group_size, 1 if accumulate else 0, ldy,
-            ws.data_ptr(), ws.numel(), _stream())
-    else:
-        one = lambda p: (C.c_void_p * 1)(p)
-        rc = _lib.lib().dz_multi_delta_linear_batch(
-            1, one(x2.data_ptr()), one(base_weight.data_ptr() if base_weight is not None else None),
-            one(qweight_stacked.data_ptr()), one(meta_stacked.data_ptr()), one(scales_stacked.data_ptr()),
-            indices.data_ptr(), one(out.data_ptr()), (C.c_int * 1)(N), (C.c_int * 1)(ldy), T, K, S, bits, group_size,
-            1 if accumulate else 0, optr, ws.data_ptr(), ws.numel(), _stream())
+        return prefill.multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
+                                                bits=bits, out=out, accumulate=accumulate,
+                                                plan=_decode_plan(T, K, N, met), blocks=blocks, base_tiled=base_tiled)
+    ws = _workspace(device, T, K, N)
+    w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
+    rc = _lib.lib().dz_multi_delta_linear_ordered(
+        x2.data_ptr(), w.data_ptr() if w is not None else None, tiled, qweight_stacked.data_ptr(), meta_stacked.data_ptr(),
+        scales_stacked.data_ptr(), indices.data_ptr(), out.data_ptr(), T, K, N, S, bits, group_size, 1 if accumulate else 0,
+        ldy, _order_ptr(order, T, device), ws.data_ptr(), ws.numel(), _stream())
     _lib.check(rc, "dz_multi_delta_linear")
     return out
 
 
 def _bits_from_shapes(qweight_stacked: torch.Tensor, K: int, N: int) -> int:
-    words = qweight_stacked[0].numel()
+    words = _slot_numel(qweight_stacked)
     bits = words * 64 // (K * N)  # words = K*N*bits/64
     if bits not in (2, 4) or words * 64 != K * N * bits:
         raise ValueError("cannot infer the bit width from qweight_stacked")
@@ -1122,7 +1136,7 @@ def apply_delta(x: torch.Tensor, qweight_stacked: torch.Tensor, scales_stacked: 
     bits = _bits_from_shapes(qweight_stacked, K, N)
     y = multi_delta_linear(x, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices, bits=bits,
                            order=order, base_tiled=base_tiled)
-    return y.view(*x.shape[:-1], N)
+    return y if x.dim() == 2 else y.view(*x.shape[:-1], N)
 
 
 def _order_ptr(order: Optional[torch.Tensor], T: int, device) -> Optional[int]:
@@ -1153,9 +1167,9 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     if not (len(xs) == len(qweight_stacked) == len(scales_stacked) == len(meta_stacked) == n) or not 1 <= n <= 4:
         raise ValueError("one x / qweight / scales / meta / base weight per projection, at most 4 projections")
     K = base_weight[0].shape[1]
-    T = xs[0].reshape(-1, K).shape[0]
+    T = xs[0].shape[0] if xs[0].dim() == 2 and xs[0].shape[1] == K else xs[0].reshape(-1, K).shape[0]
     bits = _bits_from_shapes(qweight_stacked[0], K, base_weight[0].shape[0])
-    G = scales_stacked[0][0].numel() // base_weight[0].shape[0]
+    G = _slot_numel(scales_stacked[0]) // base_weight[0].shape[0]
     S = qweight_stacked[0].shape[0]
     if T > MAX_TOKENS_FUSED:
         blocks = order if isinstance(order, RowBlocks) else None
@@ -1180,14 +1194,12 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     x2s, outs, Ns = [], [], []
     for j in range(n):
         N = base_weight[j].shape[0]
-        x2 = xs[j].reshape(-1, K)
+        x2 = xs[j] if xs[j].dim() == 2 and xs[j].shape[1] == K else xs[j].reshape(-1, K)
         if (x2.dtype != torch.float16 or base_weight[j].dtype != torch.float16 or base_weight[j].shape[1] != K
                 or x2.shape[0] != T or not x2.is_contiguous() or not base_weight[j].is_contiguous()):
             raise ValueError("x and base weights must be contiguous float16 with the same K and T")
-        cb, mb, sb = native_sizes(K, N, bits, group_size)
         q, m, sc = qweight_stacked[j], meta_stacked[j], scales_stacked[j]
-        if (q.shape[0] != S or q[0].numel() * q.element_size() != cb or m[0].numel() * m.element_size() != mb
-                or sc[0].numel() * sc.element_size() != sb or sc.dtype != torch.float16
+        if (q.shape[0] != S or _slot_bytes_differ(q, m, sc, _sizes(K, N, bits, group_size)) or sc.dtype != torch.float16
                 or not (q.is_contiguous() and m.is_contiguous() and sc.is_contiguous())):
             raise ValueError("stacked delta tensors do not match the native layout for these sizes")
         x2s.append(x2); Ns.append(N)
@@ -1207,7 +1219,7 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
         indices.data_ptr(), ptrs(outs), (C.c_int * n)(*Ns), (C.c_int * n)(*Ns), T, K, S, bits, group_size, 0,
         _order_ptr(order, T, indices.device), ws.data_ptr(), ws.numel(), _stream())
     _lib.check(rc, "dz_multi_delta_linear_batch")
-    return [outs[j].view(*xs[j].shape[:-1], Ns[j]) for j in range(n)]
+    return [y if v.dim() == 2 else y.view(*v.shape[:-1], y.shape[1]) for y, v in zip(outs, xs)]
 
 
 def add_delta(y: torch.Tensor, x: torch.Tensor, qweight: torch.Tensor, qzeros, scales: torch.Tensor,
@@ -1298,13 +1310,11 @@ def apply_delta_packed_nslice(x: torch.Tensor, qweight_stacked: Sequence[torch.T
         raise ValueError("output must have one row per token")
     bits = _bits_from_shapes(qweight_stacked[0], K, Ns[0])
     S = qweight_stacked[0].shape[0]
-    G = scales_stacked[0][0].numel() // Ns[0]
+    G = _slot_numel(scales_stacked[0]) // Ns[0]
     group_size = -1 if G == 1 else K // G
     for j in range(n):
-        cb, mb, sb = native_sizes(K, Ns[j], bits, group_size)
         q, m, sc = qweight_stacked[j], meta_stacked[j], scales_stacked[j]
-        if (q.shape[0] != S or q[0].numel() * q.element_size() != cb or m[0].numel() * m.element_size() != mb
-                or sc[0].numel() * sc.element_size() != sb or sc.dtype != torch.float16
+        if (q.shape[0] != S or _slot_bytes_differ(q, m, sc, _sizes(K, Ns[j], bits, group_size)) or sc.dtype != torch.float16
                 or not (q.is_contiguous() and m.is_contiguous() and sc.is_contiguous())):
             raise ValueError("stacked delta tensors do not match the native layout for these sizes")
     vp = C.c_void_p * n
@@ -1324,3 +1334,5 @@ def set_ksplit(nsplit: int) -> None:
     """Benchmark hook: force the number of K chunks of the fused kernel (0 = automatic)."""
     _lib.lib().dz_set_ksplit(int(nsplit))
 
+
+from . import prefill  # noqa: E402  (which reads this module when it is called)

@@ -13,7 +13,7 @@ from typing import Optional
 
 import torch
 
-from . import _lib
+from . import _lib, ops
 
 
 def gemm_f16(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = None,
@@ -23,7 +23,7 @@ def gemm_f16(x: torch.Tensor, w: torch.Tensor, out: Optional[torch.Tensor] = Non
     N = w.shape[0]
     if out is None:
         out = torch.empty((T, N), dtype=torch.float16, device=x.device)
-    st = torch.cuda.current_stream().cuda_stream
+    st = ops._stream()
     if w2 is None:
         rc = _lib.lib().dz_gemm_f16(x.data_ptr(), w.data_ptr(), out.data_ptr(), T, K, N,
                                     1 if accumulate else 0, out.stride(0), st)
@@ -43,11 +43,10 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
     host, gathered, scattered or dequantised to memory.  `blocks`: ops.row_blocks(indices, S) when
     the caller made it once for the batch (else made here, per call).  `base_tiled`: the base weight
     in tiles (ops.tile_base), read instead of base_weight when given."""
-    from .ops import _one_wave_of_long_blocks, row_blocks
     T, K = x2.shape
     N = scales_stacked.shape[-1]
     S = qweight_stacked.shape[0]
-    G = scales_stacked[0].numel() // N
+    G = ops._slot_numel(scales_stacked) // N
     group_size = -1 if G == 1 else K // G
     # the kernel addresses an operand with 31-bit byte offsets: very long batches go in pieces
     max_rows = ((1 << 31) - 1) // (2 * K)
@@ -59,10 +58,10 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
                                        accumulate=accumulate, base_tiled=base_tiled)
         return out
     lib = _lib.lib()
-    stream = torch.cuda.current_stream().cuda_stream
-    one_wave = _one_wave_of_long_blocks(T, N, bits)
+    stream = ops._stream()
+    one_wave = ops._one_wave_of_long_blocks(T, N, bits)
     if blocks is None:
-        blocks = row_blocks(indices, S, device_picks=S == 1 and one_wave, features=N, mixed=False)
+        blocks = ops.row_blocks(indices, S, device_picks=S == 1 and one_wave, features=N, mixed=False)
     take_long, take_short = blocks.tiles is not None, blocks.short is not None
     if blocks.host_picks:
         take_long, take_short = one_wave, not one_wave
@@ -92,16 +91,15 @@ def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, m
     """The layer over blocks that hold the tokens of several deltas (dz_multi_delta_gemm_mixed), with a base weight.
     `plan`: ops._mixed_plan(T, K, N).  `blocks`: as for multi_delta_linear_prefill; without them, or where they
     were made for more deltas than this layer's block can hold, the call makes the table it needs."""
-    from .ops import mixed_deltas, own_mixed_table
     small, parts = plan
     T, K = x2.shape
     N, S = scales_stacked.shape[-1], qweight_stacked.shape[0]
-    G = scales_stacked[0].numel() // N
-    L, stream = _lib.lib(), torch.cuda.current_stream().cuda_stream
-    deltas = mixed_deltas(bits, G > 1)
+    G = ops._slot_numel(scales_stacked) // N
+    L, stream = _lib.lib(), ops._stream()
+    deltas = ops.mixed_deltas(bits, G > 1)
     table = blocks.mixed[small] if blocks is not None else None
     if table is None or table.deltas > deltas:
-        table = own_mixed_table(indices, S, small, deltas)
+        table = ops.own_mixed_table(indices, S, small, deltas)
     sums = torch.empty(parts * T * N, dtype=torch.float32, device=x2.device) if parts > 1 else None
     w = base_tiled if base_tiled is not None else base_weight
     rc = L.dz_multi_delta_gemm_mixed(

@@ -279,6 +279,13 @@ int dz_multi_delta_linear_batch_tiled(int ncalls, const uint16_t* const* x,
                                       const int32_t* order, void* workspace, size_t workspace_bytes,
                                       void* stream);
 
+/* dz_multi_delta_linear over either form of the base weight -- row-major [N, K] (w_tiled = 0), the tiles dz_tile_base
+ * writes (w_tiled != 0), or NULL -- with the token order of dz_token_order, or NULL. */
+int dz_multi_delta_linear_ordered(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
+                                  const void* meta_stacked, const void* scales_stacked, const int64_t* indices, uint16_t* y,
+                                  int T, int K, int N, int S, int bits, int group_size, int accumulate, int ldy,
+                                  const int32_t* order, void* workspace, size_t workspace_bytes, void* stream);
+
 /* dz_multi_delta_linear for any T >= 1, DZ_MAX_TOKENS_FUSED tokens at a time (workspace as for that many).
  * w_base is row-major [N, K] (w_tiled = 0), the tiles dz_tile_base writes (w_tiled != 0), or NULL.
  * only_if: NULL, or device memory read when the kernels run: 0 there leaves y as it is. */

@@ -1321,3 +1321,33 @@ def test_compressor_of_whole_rows(dev, n, k, bits):
     q0, m0 = ops.pack_2of4(d, s32, bits)
     torch.cuda.synchronize()
     assert torch.equal(s.view(torch.int16), s16.view(torch.int16)) and torch.equal(q, q0) and torch.equal(m, m0)
+
+
+@pytest.mark.parametrize("t", [1, 32, 33, 128])
+def test_one_call_with_a_token_order(dev, t):
+    """dz_multi_delta_linear_ordered over rows, tiles and no base weight, with the order and without: the bits of the entry
+    for several calls."""
+    from deltazip_amd import _lib
+    n, k, nd = 96, 1280, 5
+    p = make_problem(n, k, 2, -1, nd, t, "uniform", 7 * t, dev)
+    L, st, tiles = _lib.lib(), torch.cuda.current_stream().cuda_stream, ops.tile_base(p["wb"])
+    order = ops.token_order(p["ids"], nd) if t > 32 else None
+    ws = torch.zeros(L.dz_workspace_bytes(t, k, n), dtype=torch.uint8, device=dev)
+    ref = o.forward_ref(p["x_np"], p["wb_np"], p["dts"], p["ids_np"])
+    for w, tiled in ((p["wb"], 0), (tiles, 1), (None, 0)):
+        for perm in ([None, order] if order is not None else [None]):
+            y = torch.full((t, n), float("nan"), dtype=torch.float16, device=dev)
+            assert L.dz_multi_delta_linear_ordered(
+                p["x"].data_ptr(), None if w is None else w.data_ptr(), tiled, p["q"].data_ptr(), p["m"].data_ptr(),
+                p["s"].data_ptr(), p["ids"].data_ptr(), y.data_ptr(), t, k, n, nd, 2, -1, 0, n,
+                None if perm is None else perm.data_ptr(), ws.data_ptr(), ws.numel(), st) == 0
+            torch.cuda.synchronize()
+            if w is not None:
+                assert o.rel_err(y.cpu().numpy(), ref) <= TOL
+            want = torch.zeros_like(y)
+            ops.multi_delta_linear(p["x"], w if not tiled else None, p["q"], p["s"], p["m"], p["ids"], bits=2, out=want,
+                                   accumulate=w is None, order=perm, base_tiled=w if tiled else None)
+            assert torch.equal(y, want)
+    assert L.dz_multi_delta_linear_ordered(None, None, 0, p["q"].data_ptr(), p["m"].data_ptr(), p["s"].data_ptr(),
+                                           p["ids"].data_ptr(), y.data_ptr(), t, k, n, nd, 2, -1, 0, n, None, ws.data_ptr(),
+                                           ws.numel(), st) != 0

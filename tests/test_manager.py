@@ -777,3 +777,21 @@ def test_captured_decode_step_keeps_the_token_order(monkeypatch, made_captured, 
         LinearWithDelta.apply_weights(layer, None)
     assert (seen[0] is blocks) == blocks_go and (blocks_go or torch.equal(seen[0], token_order[:64]))
     assert seen[1] is blocks
+
+
+@pytest.mark.parametrize("shape", [(3, 4, 5), (1, 7), (2, 0), (4,), (0, 3), ()])
+def test_values_per_slot_without_a_view(shape):
+    """The calls' checks count a slot's values by the shape; a stack without slots is refused as indexing it is."""
+    t = torch.zeros(shape)
+    if shape and shape[0]:
+        assert ops._slot_numel(t) == t[0].numel()
+    else:
+        with pytest.raises(IndexError):
+            ops._slot_numel(t)
+
+
+def test_sizes_are_looked_up_once_and_refused_every_time():
+    assert ops._sizes(512, 64, 2, -1) == ops.native_sizes(512, 64, 2, -1) == ops._sizes(512, 64, 2, -1)
+    for _ in range(2):
+        with pytest.raises(ValueError):
+            ops._sizes(500, 64, 2, -1)
