@@ -34,6 +34,8 @@ SIGNATURES = {
     "dz_build_tiles_rows": (_i, [_vp, _i, _i, _vp, _i, _vp]),
     "dz_multi_delta_gemm_rows": (_i, [_vp, _vp, _i, _vp, _vp, _vp, _i, _i, _i, _vp, _i, _vp, _vp, _i, _i, _i, _i, _i, _vp]),
     "dz_mixed_blocks": (_i, [_i, _i, _i, _i]),
+    "dz_mixed_us": (C.c_float, [_i, _i, _i, _i, _i]),
+    "dz_mixed_parts": (_i, [_i, _i, _i, _i, _i]),
     "dz_build_mixed": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _vp]),
     "dz_order_mixed": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp]),
     "dz_build_tables": (_i, [_vp, _vp, _i, _i, _vp, _i, _vp, _i, _i, _i, _vp, _i, _vp, _i, _vp]),

@@ -52,9 +52,15 @@ struct MixedParams {
   const dz_mixed_block* blocks;
   _Float16* y;
   float* part;                   // partial sums [ksplit][T][N], or nullptr
-  int T, K, N, G, accumulate, ldy, tiles_n, NKB, NP, w_tiled, ksplit;
+  int T, K, N, G, accumulate, ldy, tiles_n, NKB, NP, w_tiled;
+  int ksplit;                    // slices of K, or 0: by the number of blocks,
+  unsigned long long parts_of;   // 4 bits for each of 1 to 16 (more: as for 16)
   unsigned gmagic;               // group of a slab: (slab * gmagic) >> 32
 };
+
+__device__ __forceinline__ int slices_for(int used, int ksplit, unsigned long long parts_of) {
+  return ksplit ? ksplit : (int)(parts_of >> (4 * (min(used, 16) - 1))) & 15;
+}
 
 // f(0), f(1), .. f(N - 1) with constant arguments.  (Arrays that a loop indexes stay in memory until it is
 // unrolled, and by then a choice between two of their elements has become a load from a chosen address.)
@@ -83,7 +89,7 @@ struct BlockHead {
 // One block of up to NT tiles and ND deltas, columns of k-blocks [kb0, kb1).  GRP: scales change along K.
 template <int BITS, bool GRP, int ND, int NT>
 __device__ __forceinline__ void mixed_block(const MixedParams& P, unsigned char* smem, const dz_mixed_block* blk,
-                                            const BlockHead& head, int n0, int kb0, int kb1, int slice) {
+                                            const BlockHead& head, int n0, int kb0, int kb1, int slice) {   // slice -1: all of K
   constexpr bool HAS_D = ND > 0;
   constexpr int E = HAS_D ? ND : 1;
   constexpr bool AHEAD = ND < (GRP && BITS == 2 ? 3 : 4) || NT < 8;         // a tile's activations are read during the tile before (else: spills)
@@ -330,7 +336,7 @@ __device__ __forceinline__ void mixed_block(const MixedParams& P, unsigned char*
   for (int b = 0; b < NT; ++b) {
     const int row = blk->row[b * 16 + li];
     if (row < 0) continue;
-    if (P.part) {
+    if (slice >= 0) {
       float* prow = P.part + ((size_t)slice * P.T + row) * P.N + np_own * DZ_NPAIR + 4 * lg;
 #pragma unroll
       for (int a = 0; a < 2; ++a) *(f4_t*)(prow + a * 16) = acc[a][b];
@@ -359,14 +365,15 @@ __global__ __launch_bounds__(64 * MWAVES, 2) void dz_gemm24_mixed_kernel(const M
   // blocks' activations in their L2.  (The grid is for the largest table there could be; workgroups without an
   // item come last and cost nothing that could be measured.)
   const unsigned xcd = blockIdx.x & 7;
-  const unsigned per_slice = (unsigned)(P.tiles_n * used), units = per_slice * (unsigned)P.ksplit;
+  const int ksplit = slices_for(used, P.ksplit, P.parts_of);
+  const unsigned per_slice = (unsigned)(P.tiles_n * used), units = per_slice * (unsigned)ksplit;
   const unsigned item = (unsigned)((unsigned long long)units * xcd >> 3) + (blockIdx.x >> 3);
   if (item >= (unsigned)((unsigned long long)units * (xcd + 1) >> 3)) return;
   const int slice = (int)(item / per_slice), at = (int)(item % per_slice);
   const int group = at / (MG * used), wide = min(MG, P.tiles_n - group * MG), r = at - group * MG * used;
   const int tm = r / wide, tn = group * MG + r % wide;
   const dz_mixed_block* blk = P.blocks + tm;
-  const int kb0 = P.NKB * slice / P.ksplit, kb1 = P.NKB * (slice + 1) / P.ksplit;
+  const int kb0 = P.NKB * slice / ksplit, kb1 = P.NKB * (slice + 1) / ksplit, sums = ksplit > 1 ? slice : -1;
   BlockHead head;
   head.nt = blk->nt;
   head.nd = blk->nd;
@@ -378,12 +385,12 @@ __global__ __launch_bounds__(64 * MWAVES, 2) void dz_gemm24_mixed_kernel(const M
   const int nd = head.nd;
   auto go = [&](auto nt_c) {
     constexpr int NT = decltype(nt_c)::value;
-    if (nd == 0) mixed_block<BITS, GRP, 0, NT>(P, smem, blk, head, tn * MN, kb0, kb1, slice);
-    else if (nd == 1) mixed_block<BITS, GRP, 1, NT>(P, smem, blk, head, tn * MN, kb0, kb1, slice);
-    else if (nd == 2) mixed_block<BITS, GRP, 2, NT>(P, smem, blk, head, tn * MN, kb0, kb1, slice);
+    if (nd == 0) mixed_block<BITS, GRP, 0, NT>(P, smem, blk, head, tn * MN, kb0, kb1, sums);
+    else if (nd == 1) mixed_block<BITS, GRP, 1, NT>(P, smem, blk, head, tn * MN, kb0, kb1, sums);
+    else if (nd == 2) mixed_block<BITS, GRP, 2, NT>(P, smem, blk, head, tn * MN, kb0, kb1, sums);
     else if (NT == 2) return;                    // (as many tiles as deltas)
-    else if (nd == 3 || BITS == 4 || GRP) mixed_block<BITS, GRP, 3, NT>(P, smem, blk, head, tn * MN, kb0, kb1, slice);
-    else mixed_block<BITS, GRP, BITS == 4 || GRP ? 3 : 4, NT>(P, smem, blk, head, tn * MN, kb0, kb1, slice);
+    else if (nd == 3 || BITS == 4 || GRP) mixed_block<BITS, GRP, 3, NT>(P, smem, blk, head, tn * MN, kb0, kb1, sums);
+    else mixed_block<BITS, GRP, BITS == 4 || GRP ? 3 : 4, NT>(P, smem, blk, head, tn * MN, kb0, kb1, sums);
   };
   switch (head.nt) {
     case 1:
@@ -397,10 +404,12 @@ __global__ __launch_bounds__(64 * MWAVES, 2) void dz_gemm24_mixed_kernel(const M
   }
 }
 
-// y = sum of the K-slices' partial sums, in slice order
+// y = sum of the K-slices' partial sums, in slice order (nothing to do where there is one slice)
 __global__ __launch_bounds__(256) void dz_mixed_sum_kernel(const float* __restrict__ part, _Float16* __restrict__ y, int T, int N, int ksplit,
-                                                           int accumulate, int ldy) {
-  const int quads = N / 4;
+                                                           int accumulate, int ldy, const int* __restrict__ count,
+                                                           unsigned long long parts_of) {
+  const int quads = N / 4, used = *count;
+  if (used == 0 || (ksplit = slices_for(used, ksplit, parts_of)) == 1) return;
   const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
   if (i >= (long long)T * quads) return;
   const int row = (int)(i / quads), c = (int)(i % quads) * 4;
@@ -432,6 +441,68 @@ __global__ __launch_bounds__(1024) void dz_order_mixed_kernel(const long long* i
 }
 
 }  // namespace
+
+// Estimated us of a batch in so many blocks and slices of K: 5 for a workgroup's start; a slab of 64 columns 0.9 and
+// 0.08 per tile of 16 tokens with all CUs busy, three quarters of it on an idle GPU; up to two waves of workgroups one after the
+// other, more of them half a wave longer than their number; the second launch, and its pass over the sums at 4 TB/s.
+// Fitted to 307 projections of 129 to 512 tokens, each timed with 1, 2, 3, 4 and 6 slices: the best by it
+// takes 0.3 % longer in the mean than the best there is, 14 % at worst; with the number of blocks taken to be T / 128 it was
+// 6 % and 63 %, for where blocks fill the GPU a little more than once, one more of them is another wave.
+// 333 tokens in four blocks, 1 / 2 / 3 / 4 / 6 slices: 13824 x 5120 214 125 100 129 110 us, 5120 x 27648 218 236 245 245 301.
+struct MixedCost {
+  int T, steps, wide;
+  float pass;                                      // over the sums, per slice
+  MixedCost(int T_, int K, int N) : T(T_), steps(K / DZ_KBLOCK), wide((N + MN - 1) / MN), pass(2e-6f * (float)T_ * (float)N) {}
+  float slab(int blocks) const {
+    const int tiles = (T + 24 * blocks - 1) / (16 * blocks), most = MROWS / 16;   // (a segment ends half a tile early)
+    return 0.9f + 0.08f * (float)(tiles < most ? tiles : most);
+  }
+  float us(int blocks, float slab_us, int walk_slabs, int ksplit) const {
+    const float full = (float)(wide * blocks) * (float)ksplit / 256.f;
+    const float walk = (float)walk_slabs * slab_us * (0.75f + 0.25f * (full < 1.f ? full : 1.f));
+    const float all = (5.f + walk) * (full <= 1.f ? 1.f : full <= 2.f ? 2.f : full + 0.5f);
+    return ksplit == 1 ? all : all + 4.f + pass * (float)ksplit;
+  }
+  int walk_slabs(int ksplit) const { return 4 * ((steps + ksplit - 1) / ksplit); }
+};
+
+extern "C" float dz_mixed_us(int T, int K, int N, int blocks, int ksplit) {
+  if (T < 1 || K < DZ_KBLOCK || N < 1 || blocks < 1 || ksplit < 1 || ksplit > K / DZ_KBLOCK) return 0.f;
+  const MixedCost c(T, K, N);
+  return c.us(blocks, c.slab(blocks), c.walk_slabs(ksplit), ksplit);
+}
+
+// Slices of K for `first` blocks, `first` + 1, .. : `usual`, but where another number is estimated to take a tenth and 3 us
+// less.  (80 estimates a call, on the host's path: nothing is divided twice.)
+static void parts_for(int T, int K, int N, int first, int count, int usual, int* parts) {
+  constexpr int NK = 5;
+  const MixedCost c(T, K, N);
+  const int ks[NK] = {1, 2, 3, 4, 6};
+  int walks[NK];
+  for (int i = 0; i < NK; ++i) walks[i] = ks[i] <= c.steps ? c.walk_slabs(ks[i]) : 0;
+  const int walk = c.walk_slabs(usual);
+  for (int n = 0; n < count; ++n) {
+    const int blocks = first + n;
+    const float slab = c.slab(blocks), now = c.us(blocks, slab, walk, usual);
+    float least = now;
+    int best = usual;
+    for (int i = 0; i < NK && walks[i]; ++i) {
+      const float us = c.us(blocks, slab, walks[i], ks[i]);
+      if (us < least) {
+        least = us;
+        best = ks[i];
+      }
+    }
+    parts[n] = least < 0.9f * now && least < now - 3.f ? best : usual;
+  }
+}
+
+extern "C" int dz_mixed_parts(int T, int K, int N, int blocks, int usual) {
+  if (T < 1 || K < DZ_KBLOCK || N < 1 || blocks < 1 || usual < 1 || usual > K / DZ_KBLOCK) return usual;
+  int parts;
+  parts_for(T, K, N, blocks, 1, usual, &parts);
+  return parts;
+}
 
 // Tiles are at most T / 16 and one more per segment; the blocks that are less than half full are those ended
 // by their number of deltas, the last one, and the last one without deltas.
@@ -475,22 +546,39 @@ extern "C" int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_ba
   if (rc) return rc;
   const int gs = (group_size == -1 || group_size == K) ? K : group_size;
   if (T < 1 || ldy < N || ldy % 4) return DZ_ESHAPE;
-  if (ksplit < 1 || ksplit > K / DZ_KBLOCK) return DZ_ESHAPE;
+  if (ksplit == 0 || ksplit > K / DZ_KBLOCK || ksplit < -K / DZ_KBLOCK || ksplit < -15) return DZ_ESHAPE;
   if (deltas < 1 || deltas > (bits == 2 && gs == K ? DZ_MIXED_DELTAS : 3)) return DZ_ESHAPE;
-  if (ksplit > 1 && !partials) return DZ_EWORKSPACE;
+  const int tiles_n = (N + MN - 1) / MN;
+  int most = ksplit < 0 ? 1 : ksplit;              // slices of K
+  unsigned long long parts_of = 0, units = 0;
+  if (ksplit < 0) {                                // the device picks: the most there can be
+    const int fewest = T < 16 * MROWS ? (T + MROWS - 1) / MROWS : 16;
+    int each[16];
+    parts_for(T, K, N, fewest, 17 - fewest, -ksplit, each + fewest - 1);
+    for (int used = 1; used <= 16; ++used) {
+      const int parts = each[used < fewest ? fewest - 1 : used - 1];
+      const unsigned long long u = (unsigned long long)tiles_n * parts * (unsigned)(used == 16 ? max_blocks : used);
+      parts_of |= (unsigned long long)parts << (4 * (used - 1));
+      most = parts > most ? parts : most;
+      units = u > units && used <= max_blocks ? u : units;
+    }
+    ksplit = 0;
+  } else {
+    units = (unsigned long long)tiles_n * ksplit * (unsigned)max_blocks;
+  }
+  if (most > 1 && !partials) return DZ_EWORKSPACE;
   if (((uintptr_t)x & 15) || ((uintptr_t)w_base & 15) || ((uintptr_t)y & 7) || ((uintptr_t)partials & 15)) return DZ_EALIGN;
   if ((unsigned long long)T * (unsigned)K * 2ull >= (1ull << 31)) return DZ_ESHAPE;   // 32-bit row offsets
   MixedParams P{};
   P.x = (const _Float16*)x; P.w = (const _Float16*)w_base; P.y = (_Float16*)y;
   P.codes = (const u4_t*)codes_stacked; P.meta = (const u4_t*)meta_stacked; P.scales = (const _Float16*)scales_stacked;
   P.meta_slot_u4 = (long long)(mb / 16); P.scales_slot = (long long)(sb / 2);
-  P.count = table; P.blocks = (const dz_mixed_block*)(table + DZ_MIXED_HEADER); P.part = ksplit > 1 ? partials : nullptr;
+  P.count = table; P.blocks = (const dz_mixed_block*)(table + DZ_MIXED_HEADER); P.part = partials;
   P.T = T; P.K = K; P.N = N; P.G = K / gs; P.accumulate = accumulate; P.ldy = ldy;
-  P.NKB = K / DZ_KBLOCK; P.NP = N / DZ_NPAIR; P.w_tiled = w_tiled ? 1 : 0; P.ksplit = ksplit;
-  P.tiles_n = (N + MN - 1) / MN;
+  P.NKB = K / DZ_KBLOCK; P.NP = N / DZ_NPAIR; P.w_tiled = w_tiled ? 1 : 0; P.ksplit = ksplit; P.parts_of = parts_of;
+  P.tiles_n = tiles_n;
   const unsigned gslabs = (unsigned)(gs / 64);
   P.gmagic = (unsigned)((0x100000000ull + gslabs - 1) / gslabs);   // (0 where a group is one slab)
-  const unsigned long long units = (unsigned long long)P.tiles_n * ksplit * (unsigned)max_blocks;
   if (units > 0x7ffffff0ull) return DZ_ESHAPE;
   const unsigned grid = (unsigned)(units + 7) / 8 * 8;
   const int lds = 2 * XSTAGE;
@@ -503,9 +591,9 @@ extern "C" int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_ba
   const bool grp = P.G > 1;
   if (bits == 2) rc = grp ? go(dz_gemm24_mixed_kernel<2, true>, 0) : go(dz_gemm24_mixed_kernel<2, false>, 1);
   else rc = grp ? go(dz_gemm24_mixed_kernel<4, true>, 2) : go(dz_gemm24_mixed_kernel<4, false>, 3);
-  if (rc || ksplit == 1) return rc;
+  if (rc || most == 1) return rc;
   const long long quads = (long long)T * (N / 4);
   hipLaunchKernelGGL(dz_mixed_sum_kernel, dim3((unsigned)((quads + 255) / 256)), dim3(256), 0, (hipStream_t)stream, partials,
-                     (_Float16*)y, T, N, ksplit, accumulate, ldy);
+                     (_Float16*)y, T, N, ksplit, accumulate, ldy, table, parts_of);
   return hipGetLastError() == hipSuccess ? DZ_OK : DZ_ELAUNCH;
 }

@@ -295,6 +295,32 @@ def _parts(T: int, K: int, N: int, blocks: int, slab_us: float, host_us: float =
     return best[1]
 
 
+@lru_cache(maxsize=4096)
+def _parts_of_blocks(T: int, K: int, N: int, S: int, plan: Tuple[int, int], most_deltas: int) -> Tuple[int, int]:
+    """What `_mixed_plan`'s number of parts becomes with a better guess at the number of blocks, which is not T / 128: where
+    they fill the GPU a little more than once, one more is another wave of workgroups.  (parts, less than 0 where
+    the device may take others by the blocks it makes; the most there can be), by `dz_mixed_parts`.
+      up to 512 tokens   where a token's result may depend on the mix, the device picks, if there is a launch for the sums in
+                         any case (333 tokens of 8 deltas in four blocks, three parts instead of four: 13824 x 5120 129 ->
+                         100 us, 5120 x 5120 54 -> 46; over 307 projections 2.8 % in the mean)
+      above              by the sizes alone, each delta ending half a tile early in the mean: another number of parts if it is
+                         the faster one for all numbers of blocks that come to mind, from four fifths of the slots in use (or a
+                         prompt of 40 tokens each) to all of them and a block more (1999 tokens of 8 deltas, 4096 x 4096, 4-bit,
+                         17 blocks: two parts 116 to 126 us, one 127 to 146; 11008 x 4096 280 to 314 against 317 to 372)"""
+    L, (small, parts) = _lib.lib(), plan
+    if T <= 4 * MAX_TOKENS_FUSED:
+        if parts == 1:
+            return 1, 1
+        return -parts, max(L.dz_mixed_parts(T, K, N, b, parts) for b in range(-(-T // 128), 17))
+    rows, deltas = 16 * MIXED_BLOCKS[small][0], min(S + 1, T // 16)
+    few, many = (max(-(-(T + 8 * d) // rows), -(-d // most_deltas)) for d in (min(4 * deltas // 5, T // 40), deltas))
+    may = [{p: L.dz_mixed_us(T, K, N, b, p) for p in (1, 2, 3, 4, 6) if p <= K // 256} for b in range(few, many + 2)]
+    us = {p: sum(m[p] for m in may) for p in may[0]}
+    best = min(us, key=us.get)
+    made = best if us[best] < 0.9 * us[parts] and all(m[best] < m[parts] for m in may) else parts
+    return made, made
+
+
 def mixes_at_decode(T: int, K: int, N: int, deltas: int) -> bool:
     """Whether a batch of 33 to 128 tokens of so many deltas (the base model counts as one) goes in blocks of several
     deltas: the decode kernel makes its products once per 32 tokens and delta, a block once per 16 tokens and never
@@ -1069,7 +1095,9 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
             plan = _in_mixed_blocks(T, K, N, S, blocks.mix if blocks is not None else None)
         if plan is not None:
             return prefill.multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
-                                                    bits=bits, out=out, accumulate=accumulate, plan=plan, blocks=blocks,
+                                                    bits=bits, out=out, accumulate=accumulate, blocks=blocks,
+                                                    plan=(plan[0], *_parts_of_blocks(
+                                                        T, K, N, S, plan, 2 if plan[0] else mixed_deltas(bits, G > 1))),
                                                     base_tiled=base_tiled)
         most = _most_row_blocks(T, K, N, bits, S, blocks)
         if most is not None:
@@ -1105,9 +1133,10 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
         met = S
     if (met < T and (base_weight is not None or base_tiled is not None) and 0 < S <= MAX_SLOTS_SEGMENT
             and mixes_at_decode(T, K, N, met)):
+        parts = _decode_plan(T, K, N, met)[1]
         return prefill.multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices,
                                                 bits=bits, out=out, accumulate=accumulate,
-                                                plan=_decode_plan(T, K, N, met), blocks=blocks, base_tiled=base_tiled)
+                                                plan=(0, parts, parts), blocks=blocks, base_tiled=base_tiled)
     ws = _workspace(device, T, K, N)
     w, tiled = (base_tiled, 1) if base_tiled is not None else (base_weight, 0)
     rc = _lib.lib().dz_multi_delta_linear_ordered(

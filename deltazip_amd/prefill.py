@@ -89,9 +89,9 @@ def multi_delta_linear_prefill(x2, base_weight, qweight_stacked, scales_stacked,
 def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices, *, bits: int,
                              out: torch.Tensor, accumulate: bool, plan, blocks=None, base_tiled=None) -> torch.Tensor:
     """The layer over blocks that hold the tokens of several deltas (dz_multi_delta_gemm_mixed), with a base weight.
-    `plan`: ops._mixed_plan(T, K, N).  `blocks`: as for multi_delta_linear_prefill; without them, or where they
+    `plan`: (0 for full blocks, 1 for small ones; parts of K, or less than 0 where the device may take others; the most there can be).  `blocks`: as for multi_delta_linear_prefill; without them, or where they
     were made for more deltas than this layer's block can hold, the call makes the table it needs."""
-    small, parts = plan
+    small, parts, most = plan
     T, K = x2.shape
     N, S = scales_stacked.shape[-1], qweight_stacked.shape[0]
     G = ops._slot_numel(scales_stacked) // N
@@ -100,7 +100,7 @@ def multi_delta_linear_mixed(x2, base_weight, qweight_stacked, scales_stacked, m
     table = blocks.mixed[small] if blocks is not None else None
     if table is None or table.deltas > deltas:
         table = ops.own_mixed_table(indices, S, small, deltas)
-    sums = torch.empty(parts * T * N, dtype=torch.float32, device=x2.device) if parts > 1 else None
+    sums = torch.empty(most * T * N, dtype=torch.float32, device=x2.device) if most > 1 else None
     w = base_tiled if base_tiled is not None else base_weight
     rc = L.dz_multi_delta_gemm_mixed(
         x2.data_ptr(), w.data_ptr(), 1 if base_tiled is not None else 0, qweight_stacked.data_ptr(),

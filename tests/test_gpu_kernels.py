@@ -1351,3 +1351,37 @@ def test_one_call_with_a_token_order(dev, t):
     assert L.dz_multi_delta_linear_ordered(None, None, 0, p["q"].data_ptr(), p["m"].data_ptr(), p["s"].data_ptr(),
                                            p["ids"].data_ptr(), y.data_ptr(), t, k, n, nd, 2, -1, 0, n, None, ws.data_ptr(),
                                            ws.numel(), st) != 0
+
+
+@pytest.mark.parametrize("n,k,bits,gs,t,usual", [(5120, 2560, 2, -1, 333, 4), (2048, 3072, 4, 128, 512, 3), (1280, 1536, 2, 64, 129, 6),
+                                                 (96, 512, 2, -1, 2300, 2)])
+def test_parts_of_k_by_the_blocks_a_batch_has(dev, n, k, bits, gs, t, usual):
+    """ksplit < 0: the parts that dz_mixed_parts gives for the blocks in the table, bit for bit, from the fewest blocks to more
+    than 16, a whole walk among them (nothing to sum, and the sums stay as they are); without room for sums it is refused."""
+    from deltazip_amd import _lib
+    L, seen = _lib.lib(), set()
+    p = make_problem(n, k, bits, gs, 40, t, "uniform", n + t, dev)
+    fewest = -(-t // 128)
+    room = max(L.dz_mixed_parts(t, k, n, b, usual) for b in range(min(fewest, 16), 17))
+    for deltas in (1, 3, 7, 12, 20, 40):
+        ids = p["ids"] % deltas
+        table = ops.own_mixed_table(ids, 40, 0, 3)
+        used = int(table.table[0])
+        parts = L.dz_mixed_parts(t, k, n, min(max(used, fewest), 16), usual)
+        seen.add(parts)
+        args = (p["x"].data_ptr(), p["wb"].data_ptr(), 0, p["q"].data_ptr(), p["m"].data_ptr(), p["s"].data_ptr(), 40, bits, gs,
+                table.table.data_ptr(), table.max_blocks, table.deltas)
+        st, got = torch.cuda.current_stream().cuda_stream, []
+        for ksplit in (parts, -usual):
+            y = torch.full((t, n), float("nan"), dtype=torch.float16, device=dev)
+            sums = torch.full((room * t * n,), 7.0, dtype=torch.float32, device=dev)
+            assert L.dz_multi_delta_gemm_mixed(*args, y.data_ptr(), t, k, n, 0, n, ksplit, sums.data_ptr(), st) == 0
+            torch.cuda.synchronize()
+            got.append(y)
+            if parts == 1:
+                assert bool((sums == 7.0).all())
+        assert torch.equal(*got) and not torch.isnan(got[0]).any(), (deltas, used, parts)
+    assert len(seen) > 1 or t > 512
+    assert L.dz_multi_delta_gemm_mixed(*args, y.data_ptr(), t, k, n, 0, n, -usual, None, st) != 0
+    assert L.dz_multi_delta_gemm_mixed(*args, y.data_ptr(), t, k, n, 0, n, 0, sums.data_ptr(), st) != 0
+    assert L.dz_multi_delta_gemm_mixed(*args, y.data_ptr(), t, k, n, 0, n, -(k // 256) - 1, sums.data_ptr(), st) != 0

@@ -795,3 +795,23 @@ def test_sizes_are_looked_up_once_and_refused_every_time():
     for _ in range(2):
         with pytest.raises(ValueError):
             ops._sizes(500, 64, 2, -1)
+
+
+def test_parts_by_blocks_keep_the_usual_number_unless_another_is_clearly_faster():
+    from deltazip_amd import _lib
+    L = _lib.lib()
+    for t, k, n in ((333, 13824, 5120), (129, 256, 32), (512, 2560, 1280), (4000, 4096, 4096)):
+        for usual in (1, 2, 4, 6):
+            if usual > k // 256:
+                assert L.dz_mixed_parts(t, k, n, 4, usual) == usual and L.dz_mixed_us(t, k, n, 4, usual) == 0
+                continue
+            for blocks in (1, 4, 5, 16, 40):
+                us = {c: L.dz_mixed_us(t, k, n, blocks, c) for c in {1, 2, 3, 4, 6, usual} if c <= k // 256}
+                got, least = L.dz_mixed_parts(t, k, n, blocks, usual), min(us.values())
+                assert us[got] == least if least < 0.899 * us[usual] and least < us[usual] - 3.01 else \
+                    got == usual or us[got] < us[usual]
+    assert ops._parts_of_blocks(333, 5120, 27648, 16, (0, 1), 4) == (1, 1)             # nothing was to be summed
+    parts, room = ops._parts_of_blocks(333, 13824, 5120, 16, (0, 4), 4)
+    assert parts == -4 and room == max(L.dz_mixed_parts(333, 13824, 5120, b, 4) for b in range(3, 17))
+    assert ops._parts_of_blocks(1999, 11008, 4096, 8, (0, 1), 3) == (2, 2)             # by the sizes alone
+    assert ops._parts_of_blocks(8192, 13824, 5120, 16, (0, 1), 4) == (1, 1)
