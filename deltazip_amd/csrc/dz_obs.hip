@@ -20,7 +20,8 @@
 namespace {
 
 constexpr int OBS_BLOCK = 128;
-constexpr int OBS_TRI = 136 * 64;   // floats of a block of hinv on and above its diagonal, in 8 x 8 pieces
+constexpr int OBS_PIECE = 64 + 4;   // floats from an 8 x 8 piece to the next: 16 lanes that read 16 pieces meet 16 times 4 banks
+constexpr int OBS_TRI = 136 * OBS_PIECE;   // floats of a block of hinv on and above its diagonal, in such pieces
 
 typedef f4_t f4u_t __attribute__((aligned(4)));   // 16 bytes of an array that is aligned to its elements only
 
@@ -241,10 +242,14 @@ __device__ __forceinline__ float div_by(float x, float b, float y) {
   return __builtin_fmaf(__builtin_fmaf(-b, q1, x), y, q1);
 }
 constexpr float W_MIN = 0x1p-40f, X_MIN = 0x1p-80f, X_MAX = 0x1p40f, B_MIN = 0x1p-20f, B_MAX = 0x1p20f;
+constexpr unsigned T_MAX = 0x5C000000u;   // bits of 2^57: w^2 is below 2^97, whose division is as exact
 
 template <int L>
 __device__ __forceinline__ float row_lane(float v) {   // the value of lane L of each row of 16 lanes
   return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x150 + L, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float lane_down(float v) {  // each lane of 16 takes the value of the next, the last that of the first
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x12F, 0xF, 0xF, true));
 }
 template <typename F, int... L>
 __device__ __forceinline__ void for_each_lane(F&& f, std::integer_sequence<int, L...>) {
@@ -261,7 +266,10 @@ __device__ __forceinline__ void for_each_lane(F&& f, std::integer_sequence<int, 
 // and by the row's scale use their reciprocals (`div_by`); a turn that meets a value outside the
 // range where that is the correctly rounded quotient -- zeros among them -- is run again with
 // ordinary divisions.  err_prev: errors of the block before, not yet carried to these columns (they
-// are first), or nullptr.  4096 rows, per block: 145 -> 28 us.
+// are first), or nullptr.
+// Where it stands: 51 vector instructions a column, 16 of them the products, one wavefront per SIMD: 23 us per block of 4096
+// rows (145 with a wavefront per row).  It was 30 while the 16 lanes, which read one row of 16 pieces of hinv, met the same
+// banks (OBS_PIECE; 31 k of the 73 k cycles a CU took were conflicts), and columns were compared through the mask register.
 template <bool QUANT, int M>   // M: columns per pruning group, 0: no pruning
 __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* __restrict__ hinv,
                                            const float* __restrict__ scale, int N, int K, int i1, float maxq,
@@ -270,11 +278,9 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
 #pragma clang fp contract(off)
   float* hs = sm;                                   // 8 x 8 pieces (row group o, column group j >= o), see `piece`
   float* cst = sm + OBS_TRI;                        // [4][128]: d, 1 / d, d^2, 1 / d^2
-  float* outs = cst + 4 * OBS_BLOCK;                // [16 rows][132]: errors of the block before, then w - q
-  constexpr int OLD = OBS_BLOCK + 4;
   const int tid = threadIdx.x, lane = tid & 63, p = lane & 15, rg = tid >> 4;   // rg: row within the workgroup
   const int row = wg * 16 + rg, rowc = min(row, N - 1);
-  auto piece = [](int o, int j) { return (((o * (33 - o)) >> 1) + j - o) * 64; };
+  auto piece = [](int o, int j) { return (((o * (33 - o)) >> 1) + j - o) * OBS_PIECE; };
   // all loads of hinv by a thread are on their way before the first is used
   f4_t hl[16], hh[8];
   auto fetch_tri = [&]() {     // the block's own rows, on and right of the diagonal pieces
@@ -291,7 +297,7 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
   };
   auto place_half = [&]() {
 #pragma unroll
-    for (int l = 0; l < 8; ++l) ((f4_t*)hs)[l * 256 + tid] = hh[l];
+    for (int l = 0; l < 8; ++l) ((f4_t*)hs)[l * 256 + (tid & ~31) + ((tid >> 1) & 15) + 16 * (tid & 1)] = hh[l];   // a lane's two halves of 8 columns 64 floats apart
   };
   if (err_prev) fetch_half(i1 - OBS_BLOCK);
   bool odd = false;   // a divisor outside the range of div_by: every turn takes ordinary divisions
@@ -317,23 +323,30 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
   odd = odd || (QUANT && !(sc >= W_MIN && sc <= X_MAX));
   if (err_prev) {
     const float* ep = err_prev + (size_t)rowc * OBS_BLOCK + 8 * p;
-    *(f4_t*)(outs + rg * OLD + 8 * p) = *(const f4u_t*)ep;
-    *(f4_t*)(outs + rg * OLD + 8 * p + 4) = *(const f4u_t*)(ep + 4);
+    float old[8];                                   // errors of the lane's columns of that block; they move as w does below
+    {
+      const f4_t v0 = *(const f4u_t*)ep, v1 = *(const f4u_t*)(ep + 4);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        old[e] = v0[e];
+        old[4 + e] = v1[e];
+      }
+    }
     float acc[1][8] = {{0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
     for (int half = 0; half < 2; ++half) {
       place_half();
       __syncthreads();
       if (half == 0) fetch_half(i1 - OBS_BLOCK / 2);
-#pragma unroll 2
-      for (int k = 0; k < OBS_BLOCK / 2; k += 4) {
-        const f4_t e4 = *(const f4_t*)(outs + rg * OLD + half * (OBS_BLOCK / 2) + k);
+      for (int k = 0; k < OBS_BLOCK / 2; k += 8) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          const f4_t b = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 8 * p), c = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 8 * p + 4);
-          const float va[1] = {e4[u]}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
+        for (int u = 0; u < 8; ++u) {
+          const f4_t b = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 4 * p), c = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 64 + 4 * p);
+          const float va[1] = {row_lane<0>(old[u])}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
           outer_add(acc, va, vb);
         }
+#pragma unroll
+        for (int u = 0; u < 8; ++u) old[u] = lane_down(old[u]);
       }
       __syncthreads();
     }
@@ -348,6 +361,9 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
   }
   odd = __syncthreads_or(odd);
 
+  float left[8];                                    // w - q of the lane's columns
+#pragma unroll
+  for (int e = 0; e < 8; ++e) left[e] = 0.f;
   for (int o = 0; o < 16; ++o) {
     const float* hp = hs + piece(o, o + min(p, 15 - o));   // (lanes that have wrapped around hold columns that are done)
     // constants of the turn's 8 columns, the same for every lane
@@ -364,7 +380,8 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
     auto turn = [&](auto fast_c) {
       constexpr bool FAST = decltype(fast_c)::value;
       float wmin = 1.f, xmin = 1.f, xmax = 1.f;
-      unsigned pruned = 0;   // bit r: column r of the group that is being decided
+      unsigned tmax = 0;     // bits of the largest w^2 / diag^2 (those of a NaN are larger)
+      int rank[M > 0 ? M : 1];
 #pragma unroll
       for (int r = 0; r < 8; ++r) {
         if constexpr (M > 0) {
@@ -378,27 +395,30 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
               t[c] = FAST ? div_by(ww, dd[r + c], ydd[r + c]) : ww / dd[r + c];
               if (FAST) {
                 wmin = fminf(wmin, fabsf(w[r + c]));
-                xmax = fmaxf(xmax, fabsf(w[r + c]));
+                tmax = max(tmax, __float_as_uint(t[c]));
               }
             }
-            pruned = 0;
+            // how many of the group come behind a column
 #pragma unroll
-            for (int a = 0; a < M; ++a) {
-              int rank = 0;
+            for (int a = 0; a < M; ++a) rank[a] = 0;
 #pragma unroll
-              for (int b = 0; b < M; ++b)
-                if (a != b) rank += (b > a) ? (t[b] > t[a]) : (t[b] >= t[a]);
-              if (rank >= M - prunen) pruned |= 1u << a;
-            }
+            for (int a = 0; a < M; ++a)
+#pragma unroll
+              for (int b = a + 1; b < M; ++b) {
+                // (values that are not negative: their bits compare as they do, without a trip through the mask register)
+                const int less = FAST ? (int)(((unsigned)__float_as_int(t[a]) - (unsigned)__float_as_int(t[b])) >> 31) : t[b] > t[a];
+                rank[a] += less;
+                rank[b] += FAST ? 1 - less : t[a] >= t[b];
+              }
           }
         }
-        const bool pr = M > 0 && ((pruned >> (r % (M > 0 ? M : 1))) & 1u);
+        const bool pr = M > 0 && rank[r % (M > 0 ? M : 1)] >= M - prunen;
         float qv = pr ? 0.f : w[r];
         if (QUANT) {
           // (a pruned column's code is the zero-point: rint(0 / sc) + zero)
           const float quo = FAST ? div_by(w[r], sc, ysc) : w[r] / sc;
-          const float code = fminf(fmaxf(rintf(pr ? 0.f : quo) + zero, 0.f), maxq);
-          qv = sc * (code - zero);
+          // clamp(rint + zero, 0, maxq) - zero; the sum makes a zero positive, as that difference does
+          qv = sc * (__builtin_amdgcn_fmed3f(rintf(pr ? 0.f : quo), -zero, maxq - zero) + 0.f);
         }
         const float diff = w[r] - qv;
         float e;
@@ -414,7 +434,8 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
         q[r] = qv;
         df[r] = diff;
         er[r] = e;
-        const float eb = row_lane<0>(e);
+        float eb = row_lane<0>(e);
+        asm("" : "+v"(eb));                          // (as an operand of the products the move takes a wait in front of each)
         const f4_t h0 = *(const f4_t*)(hp + 8 * r), h1 = *(const f4_t*)(hp + 8 * r + 4);
         const float h[8] = {h0[0], h0[1], h0[2], h0[3], h1[0], h1[1], h1[2], h1[3]};
         // columns that are done -- the first lane's up to r, and whole lanes that have wrapped around
@@ -425,7 +446,7 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
           w[c] = w[c] - pp;
         }
       }
-      if (FAST) bad = !(wmin >= W_MIN && xmin >= X_MIN && xmax <= X_MAX);
+      if (FAST) bad = !(wmin >= W_MIN && xmin >= X_MIN && xmax <= X_MAX && tmax <= T_MAX);
     };
     if (!odd) {
 #pragma unroll
@@ -446,20 +467,21 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
       for (int e = 0; e < 8; e += 4) {
         *(f4u_t*)(wr + e) = (f4_t){q[e], q[e + 1], q[e + 2], q[e + 3]};
         *(f4u_t*)(ep + e) = (f4_t){er[e], er[e + 1], er[e + 2], er[e + 3]};
-        *(f4_t*)(outs + rg * OLD + 8 * o + e) = (f4_t){df[e], df[e + 1], df[e + 2], df[e + 3]};
       }
     }
-    // the next lane's columns move into the deciding lane (row_ror:15 = one lane down)
+    // the next lane's columns move into the deciding lane; what is left of the turn's goes to the lane that loaded them
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-      w[e] = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(w[e]), 0x12F, 0xF, 0xF, true));
+    for (int e = 0; e < 8; ++e) {
+      const float dv = row_lane<0>(df[e]);
+      left[e] = p == o ? dv : left[e];
+      w[e] = lane_down(w[e]);
+    }
   }
   // the row's losses, summed in column order: each lane continues the sum of the lane before it
   float term[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) {
-    const float diff = outs[rg * OLD + 8 * p + e], dd = cst[2 * OBS_BLOCK + 8 * p + e];
-    term[e] = (diff * diff) / dd;
+    term[e] = (left[e] * left[e]) / cst[2 * OBS_BLOCK + 8 * p + e];
   }
   float lsum = 0.f;
   auto chain = [&](auto l_c) {
@@ -472,7 +494,7 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
   if (row < N && p == 0) loss[row] = loss[row] + lsum / 2.f;
 }
 
-constexpr size_t OBS_LDS = (size_t)(OBS_TRI + 4 * OBS_BLOCK + 16 * (OBS_BLOCK + 4)) * 4;   // 44 KiB: three workgroups per CU
+constexpr size_t OBS_LDS = (size_t)(OBS_TRI + 4 * OBS_BLOCK) * 4;   // 38 KiB: four workgroups per CU
 
 // ---- W[:, c0 .. c0 + 127] -= Err @ hinv[i1 .. i1 + 127, c0 ..] for 64 rows, the sum over the block's
 // 128 columns in ascending order (sparsegpt.py:146).  Bound by the multiply-add rate: 4 x 8 values
@@ -533,10 +555,11 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 // One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
 // carrying the errors of the block before, err_prev, to their own columns), the others carry
 // err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
-// the products fill them: at 4096 x 4096, 8.4 -> 2.05 ms for the whole sweep
+// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.88 ms for the
+// whole sweep (2.04 with two beside it, and the sweep's conflicts in LDS)
 // (one kernel after the other: 2.6 ms).
 template <bool QUANT, int M>
-__global__ __launch_bounds__(256, 3) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
+__global__ __launch_bounds__(256, 4) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
                                                           const float* __restrict__ scale, int N, int K, int i1,
                                                           float maxq, float zero, int prunen, int nsweep,
                                                           const float* __restrict__ err_sweep, float* __restrict__ err,

@@ -145,6 +145,23 @@ def test_obs_sweep_values_outside_the_fast_range(dev, n, k, quant, prune):
     assert np.array_equal(loss.cpu().numpy(), want_loss, equal_nan=True)
 
 
+@pytest.mark.parametrize("prune", [(1, 2), (2, 4), (3, 8)])
+def test_obs_sweep_ties_keep_the_lower_column(dev, prune):
+    """Columns of a group that are equally far from zero, in the range of the fast turns: the lower ones are pruned first, as
+    in the oracle.  With an inverse factor that is diagonal no error travels and every group has ties."""
+    n, k = 33, 256
+    rng = np.random.default_rng(11)
+    W0 = (rng.choice([-2e-3, -1e-3, 1e-3, 2e-3], size=(n, k))).astype(np.float32)
+    hinv = np.diag(rng.choice([0.5, 1.0], size=k // 8).repeat(8)).astype(np.float32)
+    sc = o.find_params_sym(W0, 4)[0][:, 0].copy()
+    want, want_loss = o.obs_sweep_ref(W0.copy(), hinv, sc, 4, *prune)
+    Wd = torch.from_numpy(W0.copy()).to(dev)
+    loss = ops.obs_sweep(Wd, torch.from_numpy(hinv).to(dev), torch.from_numpy(sc).to(dev), 4, *prune)
+    torch.cuda.synchronize()
+    assert np.array_equal(Wd.cpu().numpy(), want)
+    assert np.array_equal(loss.cpu().numpy(), want_loss)
+
+
 @pytest.mark.parametrize("prune", [(0, 0), (1, 2), (2, 4), (3, 8)])
 def test_obs_sweep_without_rounding_carries_nan_and_infinity(dev, prune):
     """A weight that is no finite number spoils its row from its column on, and no other row: in the
