@@ -500,29 +500,33 @@ constexpr size_t OBS_LDS = (size_t)(OBS_TRI + 4 * OBS_BLOCK) * 4;   // 38 KiB: f
 // 128 columns in ascending order (sparsegpt.py:146).  Bound by the multiply-add rate: 4 x 8 values
 // per thread; the errors are staged with the row index innermost (with the
 // column innermost the four rows of a thread fell on one bank) and in stages of 32 columns, so that
-// several workgroups fit a CU.
+// several workgroups fit a CU.  NJ = 4: half a tile,
+// 64 columns, for what is left when the others have gone round the CUs (`obs_sweep`).
+template <int NJ>
 __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const float* __restrict__ err,
                                                const float* __restrict__ hinv, int N, int K, int i1, int r0, int c0,
                                                float* sm) {
 #pragma clang fp contract(off)
-  constexpr int KC = 32, ELD = 64 + 4;
+  constexpr int KC = 32, ELD = 64 + 4, C = 16 * NJ, NH = KC * C / 1024;
   float* es = sm;                   // [KC][ELD]
-  float* hs = sm + KC * ELD;        // [KC][128]
-  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;   // rows 4 tr .. + 3, columns 4 tc .. + 3 and 64 + 4 tc .. + 3
-  float acc[4][8];
+  float* hs = sm + KC * ELD;        // [KC][C]
+  const int tid = threadIdx.x, tr = tid >> 4, tc = tid & 15;   // rows 4 tr .. + 3, columns 4 tc .. + 3 (and 64 + 4 tc .. + 3)
+  float acc[4][NJ];
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = 0.f;
+    for (int j = 0; j < NJ; ++j) acc[i][j] = 0.f;
   // stage loads: errors as 16 bytes of a row (row tid / 8 and + 32, columns 4 (tid % 8) .. + 3)
-  f4_t en[2], hn[4];
+  f4_t en[2], hn[NH];
   auto fetch = [&](int k0) {
 #pragma unroll
     for (int l = 0; l < 2; ++l)
       en[l] = *(const f4u_t*)(err + (size_t)min(r0 + l * 32 + (tid >> 3), N - 1) * OBS_BLOCK + k0 + 4 * (tid & 7));
 #pragma unroll
-    for (int l = 0; l < 4; ++l)
-      hn[l] = *(const f4u_t*)(hinv + (size_t)(i1 + k0 + l * 8 + (tid >> 5)) * K + c0 + 4 * (tid & 31));
+    for (int l = 0; l < NH; ++l) {
+      const int at = l * 256 + tid;
+      hn[l] = *(const f4u_t*)(hinv + (size_t)(i1 + k0 + at / (C / 4)) * K + c0 + 4 * (at % (C / 4)));
+    }
   };
   fetch(0);
   for (int k0 = 0; k0 < OBS_BLOCK; k0 += KC) {
@@ -532,17 +536,17 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 #pragma unroll
       for (int e = 0; e < 4; ++e) es[(4 * (tid & 7) + e) * ELD + l * 32 + (tid >> 3)] = en[l][e];
 #pragma unroll
-    for (int l = 0; l < 4; ++l) *(f4_t*)(hs + (l * 8 + (tid >> 5)) * 128 + 4 * (tid & 31)) = hn[l];
+    for (int l = 0; l < NH; ++l) *(f4_t*)(hs + 4 * (l * 256 + tid)) = hn[l];
     __syncthreads();
     if (k0 + KC < OBS_BLOCK) fetch(k0 + KC);
-    outer_steps<KC>(acc, es + 4 * tr, ELD, hs + 4 * tc, 128, 64);
+    outer_steps<KC>(acc, es + 4 * tr, ELD, hs + 4 * tc, C, 64);
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int r = r0 + 4 * tr + i;
     if (r >= N) continue;
 #pragma unroll
-    for (int j = 0; j < 8; j += 4) {
+    for (int j = 0; j < NJ; j += 4) {
       f4u_t* wp = (f4u_t*)(W + (size_t)r * K + c0 + 16 * j + 4 * tc);
       f4_t v = *wp;
 #pragma unroll
@@ -555,13 +559,13 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 // One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
 // carrying the errors of the block before, err_prev, to their own columns), the others carry
 // err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
-// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.88 ms for the
-// whole sweep (2.04 with two beside it, and the sweep's conflicts in LDS)
+// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.80 ms for the
+// whole sweep (2.04 with two beside it, conflicts in LDS and no halves)
 // (one kernel after the other: 2.6 ms).
 template <bool QUANT, int M>
 __global__ __launch_bounds__(256, 4) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
                                                           const float* __restrict__ scale, int N, int K, int i1,
-                                                          float maxq, float zero, int prunen, int nsweep,
+                                                          float maxq, float zero, int prunen, int nsweep, int whole,
                                                           const float* __restrict__ err_sweep, float* __restrict__ err,
                                                           const float* __restrict__ err_prev, int i_prev, int c_lo,
                                                           float* __restrict__ loss) {
@@ -570,8 +574,11 @@ __global__ __launch_bounds__(256, 4) void dz_obs_step_kernel(float* __restrict__
   if (wg < nsweep) {
     sweep_rows<QUANT, M>(W, hinv, scale, N, K, i1, maxq, zero, prunen, err_sweep, err, loss, wg, sm);
   } else {
-    const int nr = (N + 63) / 64, t = wg - nsweep;
-    propagate_tile(W, err_prev, hinv, N, K, i_prev, (t % nr) * 64, c_lo + (t / nr) * 128, sm);
+    const int nr = (N + 63) / 64, at = wg - nsweep;
+    const bool half = at >= whole;
+    const int t = half ? whole + (at - whole) / 2 : at, r0 = t % nr * 64, c0 = c_lo + t / nr * 128;
+    if (half) propagate_tile<4>(W, err_prev, hinv, N, K, i_prev, r0, c0 + ((at - whole) & 1) * 64, sm);
+    else propagate_tile<8>(W, err_prev, hinv, N, K, i_prev, r0, c0, sm);
   }
 }
 
@@ -616,9 +623,14 @@ static int obs_sweep(float* W, const float* hinv_upper, const float* scale, int 
   auto sweep = [&](auto kern) -> int {
     if (!dz_lds_limit_once(attr_done[which], (const void*)kern, (int)OBS_LDS)) return DZ_ELAUNCH;
     auto step = [&](int ns, int i1, const float* err_sweep, float* err_cur, const float* err_prev, int i_prev, int c_lo) {
-      const int grid = ns + (err_prev ? nr * ((K - c_lo) / OBS_BLOCK) : 0);
+      // What goes beyond whole tiles, two by two on the 256 CUs, goes in halves: a tile alone on a CU has one wavefront per
+      // SIMD, which takes its products at half the rate.  Up to 512 tiles are done before the sweep beside them.  (4096 rows,
+      // us per launch, whole / with halves: 576 tiles 56 / 48, 768 60 / 57, 1280 82 / 74; all 4096 columns 1875 / 1800.)
+      const int tiles = err_prev ? nr * ((K - c_lo) / OBS_BLOCK) : 0, over = tiles % 512;
+      const int whole = tiles <= 512 ? tiles : tiles - (over > 256 ? over - 256 : over);
+      const int grid = ns + whole + 2 * (tiles - whole);
       hipLaunchKernelGGL(kern, dim3(grid), dim3(256), OBS_LDS, st, W, hinv_upper, scale, N, K, i1, maxq, zero, prunen,
-                         ns, err_sweep, err_cur, err_prev, i_prev, c_lo, loss);
+                         ns, whole, err_sweep, err_cur, err_prev, i_prev, c_lo, loss);
     };
     for (int i1 = 0, b = 0; i1 < K; i1 += OBS_BLOCK, ++b) {
       const int i2 = i1 + OBS_BLOCK;

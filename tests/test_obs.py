@@ -162,6 +162,25 @@ def test_obs_sweep_ties_keep_the_lower_column(dev, prune):
     assert np.array_equal(loss.cpu().numpy(), want_loss)
 
 
+@pytest.mark.parametrize("n", [2117, 3072])
+def test_obs_sweep_of_many_rows_is_that_of_its_parts(dev, n):
+    """Rows are swept on their own: a call that carries errors in tiles of which the last go in halves (more than 512 of 64 x
+    128 values) gives the bits of calls over a few of the rows, which need none."""
+    k, rows = 2304, 1024
+    g = torch.Generator(device=dev).manual_seed(n)
+    W0 = torch.randn(n, k, device=dev, generator=g) * 1e-3
+    hinv = torch.randn(k, k, device=dev, generator=g).mul_(0.02).triu_(1)
+    hinv.diagonal().copy_(torch.rand(k, device=dev, generator=g) * 0.5 + 0.5)
+    sc = W0.abs().amax(1) / 7
+    W = W0.clone()
+    loss = ops.obs_sweep(W, hinv, sc, 4, 2, 4)
+    for r in range(0, n, rows):
+        part = W0[r:r + rows].clone()
+        assert torch.equal(ops.obs_sweep(part, hinv, sc[r:r + rows].clone(), 4, 2, 4), loss[r:r + rows])
+        assert torch.equal(part, W[r:r + rows])
+    assert torch.isfinite(W).all()
+
+
 @pytest.mark.parametrize("prune", [(0, 0), (1, 2), (2, 4), (3, 8)])
 def test_obs_sweep_without_rounding_carries_nan_and_infinity(dev, prune):
     """A weight that is no finite number spoils its row from its column on, and no other row: in the
