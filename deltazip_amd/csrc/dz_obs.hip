@@ -338,12 +338,18 @@ __device__ __forceinline__ void sweep_rows(float* __restrict__ W, const float* _
       place_half();
       __syncthreads();
       if (half == 0) fetch_half(i1 - OBS_BLOCK / 2);
+      const float* hp = hs + 4 * p;                 // (a row is read while the one before is summed: 10 -> 7 us per block)
+      f4_t b = *(const f4_t*)hp, c = *(const f4_t*)(hp + 64);
       for (int k = 0; k < OBS_BLOCK / 2; k += 8) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) {
-          const f4_t b = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 4 * p), c = *(const f4_t*)(hs + (k + u) * OBS_BLOCK + 64 + 4 * p);
+          hp += u < 7 || k + 8 < OBS_BLOCK / 2 ? OBS_BLOCK : 0;
+          const f4_t bn = *(const f4_t*)hp, cn = *(const f4_t*)(hp + 64);
+          __builtin_amdgcn_sched_barrier(0);
           const float va[1] = {row_lane<0>(old[u])}, vb[8] = {b[0], b[1], b[2], b[3], c[0], c[1], c[2], c[3]};
           outer_add(acc, va, vb);
+          b = bn;
+          c = cn;
         }
 #pragma unroll
         for (int u = 0; u < 8; ++u) old[u] = lane_down(old[u]);
@@ -559,7 +565,7 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 // One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
 // carrying the errors of the block before, err_prev, to their own columns), the others carry
 // err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
-// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.80 ms for the
+// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.81 ms for the
 // whole sweep (2.04 with two beside it, conflicts in LDS and no halves)
 // (one kernel after the other: 2.6 ms).
 template <bool QUANT, int M>
