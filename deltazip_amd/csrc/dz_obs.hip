@@ -267,7 +267,7 @@ __device__ __forceinline__ void for_each_lane(F&& f, std::integer_sequence<int, 
 // range where that is the correctly rounded quotient -- zeros among them -- is run again with
 // ordinary divisions.  err_prev: errors of the block before, not yet carried to these columns (they
 // are first), or nullptr.
-// Where it stands: 51 vector instructions a column, 16 of them the products, one wavefront per SIMD: 23 us per block of 4096
+// Where it stands: 49 vector instructions a column, 16 of them the products, one wavefront per SIMD: 23 us per block of 4096
 // rows (145 with a wavefront per row).  It was 30 while the 16 lanes, which read one row of 16 pieces of hinv, met the same
 // banks (OBS_PIECE; 31 k of the 73 k cycles a CU took were conflicts), and columns were compared through the mask register.
 template <bool QUANT, int M>   // M: columns per pruning group, 0: no pruning
