@@ -1196,7 +1196,9 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     if not (len(xs) == len(qweight_stacked) == len(scales_stacked) == len(meta_stacked) == n) or not 1 <= n <= 4:
         raise ValueError("one x / qweight / scales / meta / base weight per projection, at most 4 projections")
     K = base_weight[0].shape[1]
-    T = xs[0].shape[0] if xs[0].dim() == 2 and xs[0].shape[1] == K else xs[0].reshape(-1, K).shape[0]
+    if any(v.shape[-1:] != (w.shape[1],) for v, w in zip(xs, base_weight)):
+        raise ValueError("x must be [.., K], as wide as the base weight")
+    T = xs[0].shape[0] if xs[0].dim() == 2 else xs[0].reshape(-1, K).shape[0]
     bits = _bits_from_shapes(qweight_stacked[0], K, base_weight[0].shape[0])
     G = _slot_numel(scales_stacked[0]) // base_weight[0].shape[0]
     S = qweight_stacked[0].shape[0]
@@ -1223,7 +1225,7 @@ def apply_delta_batch(x, qweight_stacked: Sequence[torch.Tensor], scales_stacked
     x2s, outs, Ns = [], [], []
     for j in range(n):
         N = base_weight[j].shape[0]
-        x2 = xs[j] if xs[j].dim() == 2 and xs[j].shape[1] == K else xs[j].reshape(-1, K)
+        x2 = xs[j] if xs[j].dim() == 2 else xs[j].reshape(-1, K)
         if (x2.dtype != torch.float16 or base_weight[j].dtype != torch.float16 or base_weight[j].shape[1] != K
                 or x2.shape[0] != T or not x2.is_contiguous() or not base_weight[j].is_contiguous()):
             raise ValueError("x and base weights must be contiguous float16 with the same K and T")

@@ -815,3 +815,30 @@ def test_parts_by_blocks_keep_the_usual_number_unless_another_is_clearly_faster(
     assert parts == -4 and room == max(L.dz_mixed_parts(333, 13824, 5120, b, 4) for b in range(3, 17))
     assert ops._parts_of_blocks(1999, 11008, 4096, 8, (0, 1), 3) == (2, 2)             # by the sizes alone
     assert ops._parts_of_blocks(8192, 13824, 5120, 16, (0, 1), 4) == (1, 1)
+
+
+@pytest.mark.parametrize("t", [4, 128, 256])
+def test_projections_that_share_tokens_refuse_other_widths(launches, t):
+    """A batch of projections takes [.., K] as one projection does: tokens of another width are not cut into rows of K,
+    whatever the number of rows that would make, and nothing is launched for them."""
+    k, n, s = 256, 32, 2
+    stacks = [torch.empty(s, k * n * 2 // 64, dtype=torch.int32)] * 2, [torch.empty(s, 1, n, dtype=torch.float16)] * 2, \
+        [torch.empty(s, n, k // 16, dtype=torch.int16)] * 2
+    w, ids = [torch.empty(n, k, dtype=torch.float16)] * 2, torch.zeros(t, dtype=torch.int64)
+    x = torch.empty(t, k, dtype=torch.float16)
+    for bad in (x.view(t // 2, 2 * k), x.view(2 * t, k // 2), x.view(2, t // 4, 2 * k), x.view(t * k)):
+        for xs in (bad, [x, bad], [bad, x]):
+            with pytest.raises(ValueError):
+                ops.apply_delta_batch(xs, *stacks, ids, w)
+    assert not launches
+    for good in (x, x.view(2, t // 2, k), x.view(t, 1, k)):
+        assert [y.shape for y in ops.apply_delta_batch(good, *stacks, ids, w)] == [(*good.shape[:-1], n)] * 2
+    assert ops.apply_delta_batch(x[0], *stacks, ids[:1], w)[1].shape == (n,)
+    narrow = [torch.empty(t, k, dtype=torch.float16), torch.empty(t, 2 * k, dtype=torch.float16)]   # each its own width: a call each
+    stacks2 = [stacks[0][0], torch.empty(s, k * n * 4 // 64, dtype=torch.int32)], stacks[1], [stacks[2][0], torch.empty(s, n, k // 8, dtype=torch.int16)]
+    both = lambda: ops.apply_delta_batch(narrow, *stacks2, ids, [w[0], torch.empty(n, 2 * k, dtype=torch.float16)])
+    if t > 128:
+        assert [y.shape for y in both()] == [(t, n)] * 2
+    else:
+        with pytest.raises(ValueError):
+            both()
