@@ -473,8 +473,9 @@ extern "C" float dz_mixed_us(int T, int K, int N, int blocks, int ksplit) {
 }
 
 // Slices of K for `first` blocks, `first` + 1, .. : `usual`, but where another number is estimated to take a tenth and 3 us
-// less.  (80 estimates a call, on the host's path: nothing is divided twice.)
-static void parts_for(int T, int K, int N, int first, int count, int usual, int* parts) {
+// less.  (Up to 80 estimates, on the host's path: nothing is divided twice.)  One copy of this code, so that whoever asks for
+// the parts of the same sizes gets the same.
+__attribute__((noinline)) static void parts_for(int T, int K, int N, int first, int count, int usual, int* parts) {
   constexpr int NK = 5;
   const MixedCost c(T, K, N);
   const int ks[NK] = {1, 2, 3, 4, 6};
@@ -502,6 +503,31 @@ extern "C" int dz_mixed_parts(int T, int K, int N, int blocks, int usual) {
   int parts;
   parts_for(T, K, N, blocks, 1, usual, &parts);
   return parts;
+}
+
+// Where the device picks: 4 bits of parts for each of 1 to 16 blocks, and the most of them, which is what the partial sums
+// need room for.
+struct MixedPick {
+  unsigned long long parts_of = 0;
+  int most = 1;
+  int parts(int blocks) const { return (int)(parts_of >> (4 * (blocks - 1))) & 15; }
+};
+static MixedPick pick_parts(int T, int K, int N, int usual) {
+  MixedPick pick;
+  const int fewest = T < 16 * MROWS ? (T + MROWS - 1) / MROWS : 16;
+  int each[16];
+  parts_for(T, K, N, fewest, 17 - fewest, usual, each + fewest - 1);
+  for (int b = 1; b <= 16; ++b) {
+    const int parts = each[b < fewest ? fewest - 1 : b - 1];
+    pick.parts_of |= (unsigned long long)parts << (4 * (b - 1));
+    pick.most = parts > pick.most ? parts : pick.most;
+  }
+  return pick;
+}
+
+extern "C" int dz_mixed_most_parts(int T, int K, int N, int usual) {
+  if (T < 1 || K < DZ_KBLOCK || N < 1 || usual < 1 || usual > K / DZ_KBLOCK || usual > 15) return usual;
+  return pick_parts(T, K, N, usual).most;
 }
 
 // Tiles are at most T / 16 and one more per segment; the blocks that are less than half full are those ended
@@ -549,23 +575,20 @@ extern "C" int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_ba
   if (ksplit == 0 || ksplit > K / DZ_KBLOCK || ksplit < -K / DZ_KBLOCK || ksplit < -15) return DZ_ESHAPE;
   if (deltas < 1 || deltas > (bits == 2 && gs == K ? DZ_MIXED_DELTAS : 3)) return DZ_ESHAPE;
   const int tiles_n = (N + MN - 1) / MN;
-  int most = ksplit < 0 ? 1 : ksplit;              // slices of K
-  unsigned long long parts_of = 0, units = 0;
-  if (ksplit < 0) {                                // the device picks: the most there can be
-    const int fewest = T < 16 * MROWS ? (T + MROWS - 1) / MROWS : 16;
-    int each[16];
-    parts_for(T, K, N, fewest, 17 - fewest, -ksplit, each + fewest - 1);
-    for (int used = 1; used <= 16; ++used) {
-      const int parts = each[used < fewest ? fewest - 1 : used - 1];
-      const unsigned long long u = (unsigned long long)tiles_n * parts * (unsigned)(used == 16 ? max_blocks : used);
-      parts_of |= (unsigned long long)parts << (4 * (used - 1));
-      most = parts > most ? parts : most;
-      units = u > units && used <= max_blocks ? u : units;
+  int most = ksplit;                               // slices of K
+  unsigned long long parts_of = 0, units = (unsigned long long)ksplit * (unsigned)max_blocks;
+  if (ksplit < 0) {                                // the device picks: room and workgroups for the most there can be
+    const MixedPick pick = pick_parts(T, K, N, -ksplit);
+    most = pick.most;
+    parts_of = pick.parts_of;
+    units = 0;
+    for (int used = 1; used <= 16 && used <= max_blocks; ++used) {
+      const unsigned long long u = (unsigned long long)pick.parts(used) * (unsigned)(used == 16 ? max_blocks : used);
+      units = u > units ? u : units;
     }
     ksplit = 0;
-  } else {
-    units = (unsigned long long)tiles_n * ksplit * (unsigned)max_blocks;
   }
+  units *= (unsigned)tiles_n;
   if (most > 1 && !partials) return DZ_EWORKSPACE;
   if (((uintptr_t)x & 15) || ((uintptr_t)w_base & 15) || ((uintptr_t)y & 7) || ((uintptr_t)partials & 15)) return DZ_EALIGN;
   if ((unsigned long long)T * (unsigned)K * 2ull >= (1ull << 31)) return DZ_ESHAPE;   // 32-bit row offsets

@@ -311,7 +311,7 @@ def _parts_of_blocks(T: int, K: int, N: int, S: int, plan: Tuple[int, int], most
     if T <= 4 * MAX_TOKENS_FUSED:
         if parts == 1:
             return 1, 1
-        return -parts, max(L.dz_mixed_parts(T, K, N, b, parts) for b in range(-(-T // 128), 17))
+        return -parts, L.dz_mixed_most_parts(T, K, N, parts)
     rows, deltas = 16 * MIXED_BLOCKS[small][0], min(S + 1, T // 16)
     few, many = (max(-(-(T + 8 * d) // rows), -(-d // most_deltas)) for d in (min(4 * deltas // 5, T // 40), deltas))
     may = [{p: L.dz_mixed_us(T, K, N, b, p) for p in (1, 2, 3, 4, 6) if p <= K // 256} for b in range(few, many + 2)]

@@ -416,13 +416,16 @@ int dz_build_tables(const int32_t* seg_off, const int32_t* perm, int S, int T, d
 float dz_mixed_us(int T, int K, int N, int blocks, int ksplit);
 int dz_mixed_parts(int T, int K, int N, int blocks, int usual);
 
+/* The most parts that ksplit = -usual below comes to, whatever blocks there are: the room that its partials need. */
+int dz_mixed_most_parts(int T, int K, int N, int usual);
+
 /* dz_multi_delta_gemm over blocks of several deltas: every block reads the base weight once, whatever
  * deltas it holds.  deltas: what the table was made with (DZ_MIXED_DELTAS for 2-bit deltas with one scale per
  * row only).  w_base is row-major [N, K] (w_tiled = 0) or the tiles dz_tile_base writes.  ksplit > 1: K is cut
  * into that many parts (1 .. K / 256), computed side by side; partials then holds ksplit * T * N floats.  ksplit < 0
  * (not below -15): into dz_mixed_parts(T, K, N, blocks, -ksplit) parts for the blocks that the table turns out to have (for 16,
- * where there are more), picked on the device; partials then holds T * N floats for each of the most parts that any number
- * of blocks from T / DZ_MIXED_ROWS, rounded up, to 16 comes to. */
+ * where there are more), picked on the device; partials then holds dz_mixed_most_parts(T, K, N, -ksplit) * T * N
+ * floats. */
 int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
                               const void* meta_stacked, const void* scales_stacked, int S, int bits, int group_size,
                               const int32_t* table, int max_blocks, int deltas, uint16_t* y, int T, int K, int N,

@@ -842,3 +842,26 @@ def test_projections_that_share_tokens_refuse_other_widths(launches, t):
     else:
         with pytest.raises(ValueError):
             both()
+
+
+def test_room_for_sums_is_asked_of_the_function_that_picks_the_parts(monkeypatch):
+    """A launch whose parts the device picks writes as many partial sums as that function has it; the caller asks the same
+    one, once for a size, and makes no list of blocks of its own."""
+    from deltazip_amd import _lib
+    L, asked = _lib.lib(), []
+    for t in (129, 195, 333, 512, 2300):
+        for k, n in ((13824, 10784), (4096, 4096), (5120, 2560), (512, 96)):
+            for usual in (1, 2, 4, 6, 15):
+                if usual <= k // 256:
+                    few = min(-(-t // 128), 16)
+                    assert L.dz_mixed_most_parts(t, k, n, usual) == max(L.dz_mixed_parts(t, k, n, b, usual) for b in range(few, 17))
+
+    class Asked:
+        def __getattr__(self, name):
+            asked.append(name)
+            return getattr(L, name)
+    monkeypatch.setattr(_lib, "lib", lambda: Asked())
+    ops._parts_of_blocks.cache_clear()
+    assert [ops._parts_of_blocks(195, 13824, 10784, 2, (0, 2), 4) for _ in range(2)] == [(-2, 6)] * 2
+    assert asked == ["dz_mixed_most_parts"]
+    ops._parts_of_blocks.cache_clear()
