@@ -314,10 +314,7 @@ def _parts_of_blocks(T: int, K: int, N: int, S: int, plan: Tuple[int, int], most
         return -parts, L.dz_mixed_most_parts(T, K, N, parts)
     rows, deltas = 16 * MIXED_BLOCKS[small][0], min(S + 1, T // 16)
     few, many = (max(-(-(T + 8 * d) // rows), -(-d // most_deltas)) for d in (min(4 * deltas // 5, T // 40), deltas))
-    may = [{p: L.dz_mixed_us(T, K, N, b, p) for p in (1, 2, 3, 4, 6) if p <= K // 256} for b in range(few, many + 2)]
-    us = {p: sum(m[p] for m in may) for p in may[0]}
-    best = min(us, key=us.get)
-    made = best if us[best] < 0.9 * us[parts] and all(m[best] < m[parts] for m in may) else parts
+    made = L.dz_mixed_parts_between(T, K, N, few, many + 1, parts)
     return made, made
 
 

@@ -865,3 +865,29 @@ def test_room_for_sums_is_asked_of_the_function_that_picks_the_parts(monkeypatch
     assert [ops._parts_of_blocks(195, 13824, 10784, 2, (0, 2), 4) for _ in range(2)] == [(-2, 6)] * 2
     assert asked == ["dz_mixed_most_parts"]
     ops._parts_of_blocks.cache_clear()
+
+
+def test_parts_above_512_tokens_cost_one_call_of_the_library(monkeypatch):
+    """Prefill meets a new number of tokens at nearly every step: the estimates behind its parts are made in one call, and
+    come to what they do one by one."""
+    from deltazip_amd import _lib
+    L, asked = _lib.lib(), []
+
+    class Asked:
+        def __getattr__(self, name):
+            asked.append(name)
+            return getattr(L, name)
+    monkeypatch.setattr(_lib, "lib", lambda: Asked())
+    ops._parts_of_blocks.cache_clear()
+    for t in (513, 1999, 8192):
+        for k, n in ((4096, 4096), (1536, 1536), (11008, 4096)):
+            asked.clear()
+            assert ops._parts_of_blocks(t, k, n, 8, ops._mixed_plan(t, k, n), 3)[0] >= 1 and len(asked) == 1
+            for few, many in ((1, 1), (-(-t // 128), -(-t // 128) + 5)):
+                us = {p: [L.dz_mixed_us(t, k, n, b, p) for b in range(few, many + 1)] for p in (1, 2, 3, 4, 6)}
+                for usual in us:
+                    best = min(us, key=lambda p: sum(us[p]))
+                    want = best if sum(us[best]) < 0.9 * sum(us[usual]) and all(a < b for a, b in zip(us[best], us[usual])) else usual
+                    assert L.dz_mixed_parts_between(t, k, n, few, many, usual) == want
+    ops._parts_of_blocks.cache_clear()
+    assert L.dz_mixed_parts_between(999, 512, 96, 8, 9, 3) == 3 and L.dz_mixed_parts_between(999, 512, 96, 0, 9, 2) == 2
