@@ -36,7 +36,7 @@ SIGNATURES = {
     "dz_mixed_blocks": (_i, [_i, _i, _i, _i]),
     "dz_mixed_us": (C.c_float, [_i, _i, _i, _i, _i]),
     "dz_mixed_parts": (_i, [_i, _i, _i, _i, _i]),
-    "dz_mixed_parts_between": (_i, [_i, _i, _i, _i, _i, _i]),
+    "dz_mixed_parts_between": (_i, [_i, _i, _i, _i, _i, _i, _i]),
     "dz_mixed_most_parts": (_i, [_i, _i, _i, _i]),
     "dz_build_mixed": (_i, [_vp, _vp, _i, _i, _i, _i, _vp, _i, _vp]),
     "dz_order_mixed": (_i, [_vp, _i, _i, _i, _i, _vp, _vp, _i, _vp, _vp]),

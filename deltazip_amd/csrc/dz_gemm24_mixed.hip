@@ -505,29 +505,30 @@ extern "C" int dz_mixed_parts(int T, int K, int N, int blocks, int usual) {
   return parts;
 }
 
-// Slices of K by the sizes alone: `usual`, but the number that is fastest for `few` blocks to `many` in their mean where it
-// is a tenth faster and faster for each of them.
-extern "C" int dz_mixed_parts_between(int T, int K, int N, int few, int many, int usual) {
+// Slices of K by the sizes alone: `usual`, but another number (`only` this one, or 0: any) where it is faster for each number of
+// blocks from `few` to `many` and a tenth faster in their mean; the one that saves the largest share.
+extern "C" int dz_mixed_parts_between(int T, int K, int N, int few, int many, int usual, int only) {
   if (T < 1 || K < DZ_KBLOCK || N < 1 || few < 1 || usual < 1 || usual > K / DZ_KBLOCK) return usual;
   const MixedCost c(T, K, N);
-  auto us = [&](int blocks, int ksplit) { return c.us(blocks, c.slab(blocks), c.walk_slabs(ksplit), ksplit); };
-  auto mean = [&](int ksplit) {
-    double sum = 0.;
-    for (int b = few; b <= many; ++b) sum += us(b, ksplit);
-    return sum;
-  };
-  int best = 1;
-  double least = mean(1);
-  for (int ksplit : {2, 3, 4, 6}) {
-    const double m = ksplit <= c.steps ? mean(ksplit) : least;
-    if (m < least) {
-      least = m;
+  const int walk = c.walk_slabs(usual);
+  int best = usual;
+  double share = 0.9;
+  for (int ksplit : {1, 2, 3, 4, 6}) {
+    if (ksplit > c.steps || ksplit == usual || (only && ksplit != only)) continue;
+    const int walk_k = c.walk_slabs(ksplit);
+    double sum = 0., sum_usual = 0.;
+    bool faster = true;
+    for (int b = few; b <= many && faster; ++b) {
+      const float slab = c.slab(b), us = c.us(b, slab, walk_k, ksplit), now = c.us(b, slab, walk, usual);
+      faster = us < now;
+      sum += us;
+      sum_usual += now;
+    }
+    if (faster && sum < share * sum_usual) {
+      share = sum / sum_usual;
       best = ksplit;
     }
   }
-  if (!(least < 0.9 * mean(usual))) return usual;
-  for (int b = few; b <= many; ++b)
-    if (!(us(b, best) < us(b, usual))) return usual;
   return best;
 }
 

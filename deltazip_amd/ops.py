@@ -303,18 +303,25 @@ def _parts_of_blocks(T: int, K: int, N: int, S: int, plan: Tuple[int, int], most
       up to 512 tokens   where a token's result may depend on the mix, the device picks, if there is a launch for the sums in
                          any case (333 tokens of 8 deltas in four blocks, three parts instead of four: 13824 x 5120 129 ->
                          100 us, 5120 x 5120 54 -> 46; over 307 projections 2.8 % in the mean)
-      above              by the sizes alone, each delta ending half a tile early in the mean: another number of parts if it is
-                         the faster one for all numbers of blocks that come to mind, from four fifths of the slots in use (or a
-                         prompt of 40 tokens each) to all of them and a block more (1999 tokens of 8 deltas, 4096 x 4096, 4-bit,
-                         17 blocks: two parts 116 to 126 us, one 127 to 146; 11008 x 4096 280 to 314 against 317 to 372)"""
+      above              by the sizes alone: another number of parts if it is the faster one for all numbers of blocks that
+                         there can be, from full ones to all slots in use and blocks that end by their deltas; or, of five slots
+                         and more in full blocks, twice as many, if those are faster from four fifths of the slots (or a prompt of
+                         40 tokens each) on that end half a tile early in the mean.  One in 77 drawn
+                         projections; 500 of them timed both ways, a mix each: 6.9 % less in the mean, 39 take 2 % more and
+                         the worst 14 % (1999 tokens of 8 deltas, 4-bit, 17 blocks, two parts for one: 4096 x 4096 127 to 146
+                         us -> 116 to 126, 11008 x 4096 317 to 372 -> 280 to 314).  With the second range for any
+                         number of parts it was one in 29, 8 % less in the mean, but 15 % of them took 2 % more and the worst 37 %"""
     L, (small, parts) = _lib.lib(), plan
     if T <= 4 * MAX_TOKENS_FUSED:
         if parts == 1:
             return 1, 1
         return -parts, L.dz_mixed_most_parts(T, K, N, parts)
     rows, deltas = 16 * MIXED_BLOCKS[small][0], min(S + 1, T // 16)
-    few, many = (max(-(-(T + 8 * d) // rows), -(-d // most_deltas)) for d in (min(4 * deltas // 5, T // 40), deltas))
-    made = L.dz_mixed_parts_between(T, K, N, few, many + 1, parts)
+    early, ended = lambda d: -(-(T + 8 * d) // rows), lambda d: -(-d // most_deltas)
+    made = L.dz_mixed_parts_between(T, K, N, -(-T // rows), early(deltas) + ended(deltas) + 1, parts, 0)
+    if made == parts <= 3 and not small and S >= 5:
+        d = min(4 * deltas // 5, T // 40)
+        made = L.dz_mixed_parts_between(T, K, N, max(early(d), ended(d)), early(deltas) + ended(deltas) - 1, parts, 2 * parts)
     return made, made
 
 

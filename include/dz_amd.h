@@ -413,10 +413,10 @@ int dz_build_tables(const int32_t* seg_off, const int32_t* perm, int S, int T, d
 
 /* Estimated microseconds of a batch of T tokens in that many blocks with K in that many parts (1 .. K / 256), and the
  * number of parts for it: `usual`, but where 1, 2, 3, 4 or 6 are estimated to be clearly faster, for these blocks or for
- * every number of them from `few` to `many`. */
+ * every number of them from `few` to `many` (only: 0, or the one number that may be taken). */
 float dz_mixed_us(int T, int K, int N, int blocks, int ksplit);
 int dz_mixed_parts(int T, int K, int N, int blocks, int usual);
-int dz_mixed_parts_between(int T, int K, int N, int few, int many, int usual);
+int dz_mixed_parts_between(int T, int K, int N, int few, int many, int usual, int only);
 
 /* The most parts that ksplit = -usual below comes to, whatever blocks there are: the room that its partials need. */
 int dz_mixed_most_parts(int T, int K, int N, int usual);

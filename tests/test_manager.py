@@ -867,8 +867,8 @@ def test_room_for_sums_is_asked_of_the_function_that_picks_the_parts(monkeypatch
     ops._parts_of_blocks.cache_clear()
 
 
-def test_parts_above_512_tokens_cost_one_call_of_the_library(monkeypatch):
-    """Prefill meets a new number of tokens at nearly every step: the estimates behind its parts are made in one call, and
+def test_parts_above_512_tokens_cost_few_calls_of_the_library(monkeypatch):
+    """Prefill meets a new number of tokens at nearly every step: the estimates behind its parts are made in a call or two, and
     come to what they do one by one."""
     from deltazip_amd import _lib
     L, asked = _lib.lib(), []
@@ -882,12 +882,22 @@ def test_parts_above_512_tokens_cost_one_call_of_the_library(monkeypatch):
     for t in (513, 1999, 8192):
         for k, n in ((4096, 4096), (1536, 1536), (11008, 4096)):
             asked.clear()
-            assert ops._parts_of_blocks(t, k, n, 8, ops._mixed_plan(t, k, n), 3)[0] >= 1 and len(asked) == 1
-            for few, many in ((1, 1), (-(-t // 128), -(-t // 128) + 5)):
+            assert ops._parts_of_blocks(t, k, n, 8, ops._mixed_plan(t, k, n), 3)[0] >= 1 and len(asked) <= 2
+            for few, many in ((1, 1), (-(-t // 128), -(-t // 128)), (-(-t // 128), -(-t // 128) + 5)):
                 us = {p: [L.dz_mixed_us(t, k, n, b, p) for b in range(few, many + 1)] for p in (1, 2, 3, 4, 6)}
-                for usual in us:
-                    best = min(us, key=lambda p: sum(us[p]))
-                    want = best if sum(us[best]) < 0.9 * sum(us[usual]) and all(a < b for a, b in zip(us[best], us[usual])) else usual
-                    assert L.dz_mixed_parts_between(t, k, n, few, many, usual) == want
+                for usual, now in us.items():
+                    share = {p: sum(v) / sum(now) for p, v in us.items() if all(a < b for a, b in zip(v, now))}
+                    for only in (0, 2, 5):
+                        may = {usual: 0.9, **{p: v for p, v in share.items() if only in (0, p)}}
+                        assert L.dz_mixed_parts_between(t, k, n, few, many, usual, only) == min(may, key=may.get)
     ops._parts_of_blocks.cache_clear()
-    assert L.dz_mixed_parts_between(999, 512, 96, 8, 9, 3) == 3 and L.dz_mixed_parts_between(999, 512, 96, 0, 9, 2) == 2
+    assert L.dz_mixed_parts_between(999, 512, 96, 8, 9, 3, 0) == 3 and L.dz_mixed_parts_between(999, 512, 96, 0, 9, 2, 0) == 2
+
+
+@pytest.mark.parametrize("t,k,n,slots,deltas,usual", [
+    (541, 3072, 6656, 6, 2, (1, 1)), (1268, 3072, 3072, 2, 4, (0, 2)), (620, 5888, 4352, 4, 3, (0, 3)),     # full blocks fit one round
+    (588, 3840, 3840, 38, 3, (0, 3)), (986, 4096, 4096, 17, 4, (0, 2)), (1876, 11008, 1024, 34, 3, (0, 4))])  # one part leaves CUs idle
+def test_parts_above_512_tokens_stay_where_some_mix_would_lose(t, k, n, slots, deltas, usual):
+    """Sizes at which a batch whose blocks come out a few more or fewer than the mean took up to 1.3 times as long in the
+    other number of parts."""
+    assert ops._mixed_plan(t, k, n) == usual and ops._parts_of_blocks(t, k, n, slots, usual, deltas) == (usual[1],) * 2
