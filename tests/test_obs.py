@@ -181,6 +181,24 @@ def test_obs_sweep_of_many_rows_is_that_of_its_parts(dev, n):
     assert torch.isfinite(W).all()
 
 
+@pytest.mark.parametrize("n,k", [(3072, 2688), (3050, 2688)])
+def test_obs_sweep_keeps_the_first_half_round_of_the_rest_whole(dev, n, k):
+    """Up to 912 tiles, 400 beyond 512: 256 of those stay whole and 144 go in halves, launch by launch fewer.  The bits are
+    those of calls over 512 rows, whose tiles (152 and fewer) all stay whole."""
+    g = torch.Generator(device=dev).manual_seed(n + k)
+    W0 = torch.randn(n, k, device=dev, generator=g) * 1e-3
+    hinv = torch.randn(k, k, device=dev, generator=g).mul_(0.02).triu_(1)
+    hinv.diagonal().copy_(torch.rand(k, device=dev, generator=g) * 0.5 + 0.5)
+    sc = W0.abs().amax(1) / 7
+    W = W0.clone()
+    loss = ops.obs_sweep(W, hinv, sc, 4, 2, 4)
+    for r in range(0, n, 512):
+        part = W0[r:r + 512].clone()
+        assert torch.equal(ops.obs_sweep(part, hinv, sc[r:r + 512].clone(), 4, 2, 4), loss[r:r + 512])
+        assert torch.equal(part, W[r:r + 512])
+    assert torch.isfinite(W).all()
+
+
 @pytest.mark.parametrize("prune", [(0, 0), (1, 2), (2, 4), (3, 8)])
 def test_obs_sweep_without_rounding_carries_nan_and_infinity(dev, prune):
     """A weight that is no finite number spoils its row from its column on, and no other row: in the
