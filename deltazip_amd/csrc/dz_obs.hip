@@ -565,9 +565,8 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 // One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
 // carrying the errors of the block before, err_prev, to their own columns), the others carry
 // err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
-// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.81 ms for the
-// whole sweep (2.04 with two beside it, conflicts in LDS and no halves)
-// (one kernel after the other: 2.6 ms).
+// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.79 ms for the
+// whole sweep (2.04 with two beside it, conflicts in LDS and no halves; one kernel after the other: 2.6 ms).
 template <bool QUANT, int M>
 __global__ __launch_bounds__(256, 4) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
                                                           const float* __restrict__ scale, int N, int K, int i1,
@@ -630,10 +629,12 @@ static int obs_sweep(float* W, const float* hinv_upper, const float* scale, int 
     if (!dz_lds_limit_once(attr_done[which], (const void*)kern, (int)OBS_LDS)) return DZ_ELAUNCH;
     auto step = [&](int ns, int i1, const float* err_sweep, float* err_cur, const float* err_prev, int i_prev, int c_lo) {
       // What goes beyond whole tiles, two by two on the 256 CUs, goes in halves: a tile alone on a CU has one wavefront per
-      // SIMD, which takes its products at half the rate.  Up to 512 tiles are done before the sweep beside them.  (4096 rows,
-      // us per launch, whole / with halves: 576 tiles 56 / 48, 768 60 / 57, 1280 82 / 74; all 4096 columns 1875 / 1800.)
+      // SIMD, which takes its products at half the rate.  Up to 256 tiles are done before the sweep beside them: launches with 0
+      // to 256 take 33 to 35 us, with 320 43.  (us per launch, whole / with halves, 4096 rows: 576 tiles 56 / 48, 768 60 / 57, 1280 82 / 74;
+      // whole sweeps with halves beyond 512 tiles / beyond 256: 2560 columns, 1760 rows 639 / 622, 2048 x 2048 477 / 468, 4096
+      // columns, 1024 rows 928 / 917, 3072, 1344 rows 729 / 722; 4096 x 4096, none at all / beyond 512 1875 / 1800.)
       const int tiles = err_prev ? nr * ((K - c_lo) / OBS_BLOCK) : 0, over = tiles % 512;
-      const int whole = tiles <= 512 ? tiles : tiles - (over > 256 ? over - 256 : over);
+      const int whole = tiles <= 256 ? tiles : tiles - (over > 256 ? over - 256 : over);
       const int grid = ns + whole + 2 * (tiles - whole);
       hipLaunchKernelGGL(kern, dim3(grid), dim3(256), OBS_LDS, st, W, hinv_upper, scale, N, K, i1, maxq, zero, prunen,
                          ns, whole, err_sweep, err_cur, err_prev, i_prev, c_lo, loss);

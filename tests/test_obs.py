@@ -181,9 +181,10 @@ def test_obs_sweep_of_many_rows_is_that_of_its_parts(dev, n):
     assert torch.isfinite(W).all()
 
 
-@pytest.mark.parametrize("n,k", [(3072, 2688), (3050, 2688)])
+@pytest.mark.parametrize("n,k", [(3072, 2688), (3050, 2688), (1024, 2432), (1460, 2304)])
 def test_obs_sweep_keeps_the_first_half_round_of_the_rest_whole(dev, n, k):
-    """Up to 912 tiles, 400 beyond 512: 256 of those stay whole and 144 go in halves, launch by launch fewer.  The bits are
+    """Up to 912 tiles, 400 beyond 512: 256 of those stay whole and 144 go in halves, launch by launch fewer; 272 and 368 tiles,
+    of which 16 and 112 go in halves, and fewer, which stay whole.  The bits are
     those of calls over 512 rows, whose tiles (152 and fewer) all stay whole."""
     g = torch.Generator(device=dev).manual_seed(n + k)
     W0 = torch.randn(n, k, device=dev, generator=g) * 1e-3
