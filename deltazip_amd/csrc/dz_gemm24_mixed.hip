@@ -22,7 +22,7 @@
 // CUs busy and the base weight of 256 features per CU coming from memory 1.7 us, 4.9 to 5.9 TB/s.  5120 x
 // 27648, 2-bit, against one delta per block and against 256 x 256 tiles: 333 tokens of 10 deltas 250 -> 215 us, 1000
 // of 32 950 -> 700, 8192 of 16 3460 -> 3020; 13824 x 5120, 333 tokens 160 -> 100 (K in three parts, by the
-// number of blocks; in four 129).  A layer of 5120/13824, 333 tokens: 770 -> 521 us.
+// number of blocks; in four 129).  A layer of 5120/13824, 333 tokens: 770 -> 521 us (by the card 483 to 557).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 

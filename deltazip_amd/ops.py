@@ -249,8 +249,10 @@ def mixed_deltas(bits: int, grouped: bool) -> int:
 def _mixed_plan(T: int, K: int, N: int) -> Optional[Tuple[int, int]]:
     """How a batch of more than 128 tokens takes blocks of several deltas: (0 for full blocks, 1 for small
     ones; parts K is cut into), or None where they do not pay.  By the sizes alone, so that above 512 tokens a token's
-    result depends on neither the mix nor its place in the batch (up to 512 `_in_mixed_blocks` and `_short_chunks` may
-    choose another kernel, whose fp32 sums have another order).
+    result depends on neither the mix nor its place in the batch.  Up to 512 it may: `_in_mixed_blocks` and `_short_chunks`
+    may choose another kernel, and where this plan has more than one part the device takes a number of them by the blocks
+    that the batch came to (`_parts_of_blocks`), in every call, direct ones and replays among them.  Another kernel or number
+    of parts is another order of fp32 sums.
 
     Fitted to 2240 timed batches of 129 to 1700 tokens and 3780 of 129 to 8192 (1 to 64 slots, sorted ids and
     requests, both bit widths, K from 512 to 13824, N to 27648): the choice takes 6.6 % longer in the mean than
@@ -1048,7 +1050,9 @@ def multi_delta_linear(x: torch.Tensor, base_weight: Optional[torch.Tensor], qwe
     caller already has for this batch -- the result of `token_order(indices, S)` (up to 128
     tokens) or of `row_blocks(indices, S)` (more).
     `base_tiled`: `tile_base(base_weight)`, read instead of the row-major weight (the results are
-    the same bit for bit); base_weight may then be None -- a layer that keeps only the tiled copy."""
+    the same bit for bit); base_weight may then be None -- a layer that keeps only the tiled copy.
+    The order of the fp32 sums goes by the sizes, and at 129 to 512 tokens also by the ids of the batch: the other tokens'
+    deltas set the number of blocks, and that the parts K is cut into, also when a graph is replayed over other ids."""
     _need_cuda(x, base_weight, qweight_stacked, scales_stacked, meta_stacked, indices)
     if x.dtype != torch.float16:
         raise ValueError("x must be float16")

@@ -427,7 +427,7 @@ int dz_mixed_most_parts(int T, int K, int N, int usual);
  * into that many parts (1 .. K / 256), computed side by side; partials then holds ksplit * T * N floats.  ksplit < 0
  * (not below -15): into dz_mixed_parts(T, K, N, blocks, -ksplit) parts for the blocks that the table turns out to have (for 16,
  * where there are more), picked on the device; partials then holds dz_mixed_most_parts(T, K, N, -ksplit) * T * N
- * floats. */
+ * floats, and the order of a token's sums follows the table, which is to say the ids of all tokens, at every replay. */
 int dz_multi_delta_gemm_mixed(const uint16_t* x, const uint16_t* w_base, int w_tiled, const void* codes_stacked,
                               const void* meta_stacked, const void* scales_stacked, int S, int bits, int group_size,
                               const int32_t* table, int max_blocks, int deltas, uint16_t* y, int T, int K, int N,
