@@ -566,7 +566,7 @@ __device__ __forceinline__ void propagate_tile(float* __restrict__ W, const floa
 // One launch of the sweep: its first `nsweep` workgroups sweep the block at column i1 (after
 // carrying the errors of the block before, err_prev, to their own columns), the others carry
 // err_prev to the columns `c_lo` and beyond.  The sweep leaves most of the GPU's issue slots free and
-// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.79 ms for the
+// the products fill them, three workgroups of them beside one of the sweep on a CU: at 4096 x 4096, 8.4 -> 2.04 -> 1.80 ms for the
 // whole sweep (2.04 with two beside it, conflicts in LDS and no halves; one kernel after the other: 2.6 ms).
 template <bool QUANT, int M>
 __global__ __launch_bounds__(256, 4) void dz_obs_step_kernel(float* __restrict__ W, const float* __restrict__ hinv,
