@@ -446,7 +446,7 @@ __global__ __launch_bounds__(1024) void dz_order_mixed_kernel(const long long* i
 // 0.08 per tile of 16 tokens with all CUs busy, three quarters of it on an idle GPU; up to two waves of workgroups one after the
 // other, more of them half a wave longer than their number; the second launch, and its pass over the sums at 4 TB/s.
 // Fitted to 307 projections of 129 to 512 tokens, each timed with 1, 2, 3, 4 and 6 slices: the best by it
-// takes 0.3 % longer in the mean than the best there is, 14 % at worst; with the number of blocks taken to be T / 128 it was
+// takes 0.3 % longer in the mean than the best there is, 14 % at worst (of 700 others 1.3 % and 44 %); with the number of blocks taken to be T / 128 it was
 // 6 % and 63 %, for where blocks fill the GPU a little more than once, one more of them is another wave.
 // 333 tokens in four blocks, 1 / 2 / 3 / 4 / 6 slices: 13824 x 5120 214 125 100 129 110 us, 5120 x 27648 218 236 245 245 301.
 struct MixedCost {
